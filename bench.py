@@ -601,7 +601,7 @@ def main() -> int:
             "matched_pairs": main_t["matched"],
             "embeddings": res["num_matches"] if args.find_all else None,
             "dfs_steps": res["dfs_steps"],
-            "join_lane_use": (round(res["dfs_steps"] / (64.0 * res["join_wave_steps"]), 4) if res.get("join_wave_steps") else None),
+            "join_steps_per_lane": (round(res["dfs_steps"] / (64.0 * res["join_wave_steps"]), 4) if res.get("join_wave_steps") else None),
             "form": head,
             **({"tuning": getattr(args, "tuning", None)} if "batched" in forms else {}),
             "graph": bool(args.graph and args.config != 3),

@@ -254,7 +254,7 @@ typedef struct sigmo_pipeline_result {
   double phase_ms[SIGMO_PHASE_COUNT];
   double total_ms;         /* device time from first signature kernel to join completion */
   uint64_t dfs_steps;      /* join DFS frame steps (accepts + backtracks + leaves)         */
-  uint64_t join_wave_steps; /* join loop iterations summed over wavefronts (lane use = dfs_steps / (64 x this)) */
+  uint64_t join_wave_steps; /* join loop iterations summed over wavefronts (an iteration takes up to three DFS steps of each lane) */
 } sigmo_pipeline_result;
 /* Runs gen(D), gen(Q), filter, R x {refsig(D,r), refsig(Q,r), refine}, GMCR, join on
  * device-resident graphs, with one launch per phase; allocates and frees its buffers.  With
@@ -323,7 +323,7 @@ typedef struct sigmo_batch_tuning {
   uint32_t filter_blocks_per_cu; /* pair evaluation: 4-wavefront blocks per CU (capped by residency); 0: all that stay resident (<= 8) */
   uint32_t filter_claim;         /* molecule mode: molecules a wavefront claims at a time (0: ~count / (4 x wavefronts), 1..64);
                                     list mode: 64-pair groups a wavefront claims at a time (0: 2) */
-  uint32_t join_blocks_per_cu;   /* lane join: 2-wavefront blocks per CU (1..4); 0: 4 */
+  uint32_t join_blocks_per_cu;   /* lane join: quarters of the wavefronts its LDS keeps resident (1..4); 0: 4 */
   uint32_t join_chunk;           /* GMCR pairs per claim of the lane join; 0: ~P / (16 x wavefronts), 64..1024 */
   uint32_t filter_mode;          /* pair evaluation: 1 molecule by molecule from LDS-staged planes, 2 pair by pair from the
                                     pre-tested pair list; 0: list mode below 256 query graphs */

@@ -44,12 +44,6 @@ constexpr uint16_t kEndToken = 0xFFFF;    // closes a query node's token segment
 // word, so the reader's one-word lookahead stays inside the segment.
 __host__ __device__ constexpr uint32_t token_segment(uint32_t R) { return ((2 + 16 * R + 3) & ~3u) + 4; }
 
-// Orders this wavefront's LDS accesses across lanes (the compiler may not move them across).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // Level-r sphere of every node, one BFS layer per call (the reachables of the reference are
 // the BFS ball of the previous level when levels are refined in order).  Positions are taken
 // mod 64: bit b of the frontier expands node prev + b, as in signature.hpp:336-390.
@@ -2083,21 +2077,21 @@ hipError_t launch_scatter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Lane join over P pairs (molecules of <= 64 nodes; the others are listed in wide_pairs): a
-// shallow first pass and a full-depth pass over the pairs of deeper queries (deep_pairs).
+// Lane join over P pairs (molecules of <= 64 nodes; the others are listed in wide_pairs): for many
+// pairs a shallow first pass and a second over the pairs of deeper queries (deep_pairs).
 hipError_t launch_join(sigmo_batch* b, const RunShape& L, hipStream_t s, unsigned long long* stats, uint64_t P, int find_first,
                        const unsigned long long* P_dev = nullptr) {
   if (!P) return hipSuccess;
-  const uint32_t per_cu = b->tune.join_blocks_per_cu ? std::min<uint32_t>(b->tune.join_blocks_per_cu, 4) : 4;
+  const uint32_t quarters = b->tune.join_blocks_per_cu ? std::min<uint32_t>(b->tune.join_blocks_per_cu, 4) : 4;
   return sigmo_k::launch_join_lanes(s, L.qd, L.dd, sigmo_k::ArenaMasks{b->arena, b->mask_off, b->counters + 3}, b->indices, b->pair_graph, P,
-                                    find_first, b->counts, stats, b->wide_pairs, L.cus, P_dev, b->deep_pairs, per_cu, b->tune.join_chunk);
+                                    find_first, b->counts, stats, b->wide_pairs, L.cus, P_dev, b->deep_pairs, quarters, b->tune.join_chunk);
 }
 
 // Lane join over the nw listed pairs of 65..128-node molecules (two-word positions).
 hipError_t launch_join_wide(sigmo_batch* b, const RunShape& L, hipStream_t s, unsigned long long* stats, uint64_t nw, int find_first,
                             const unsigned long long* nw_dev = nullptr) {
   return sigmo_k::launch_join_wide(s, L.qd, L.dd, sigmo_k::ArenaMasks{b->arena, b->mask_off, b->counters + 3}, b->indices, b->pair_graph,
-                                   b->wide_pairs, nw, find_first, b->counts, stats, L.cus, nw_dev, b->deep_pairs);
+                                   b->wide_pairs, nw, find_first, b->counts, stats, L.cus, nw_dev);
 }
 
 // Buffers of a run that do not depend on its results.
@@ -2282,7 +2276,7 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
 
 int sigmo_batch_set_tuning(sigmo_batch* b, const sigmo_batch_tuning* t) {
   if (!b || !t) return sigmo_err::set(SIGMO_ERR_INVALID, "null argument");
-  if (t->join_blocks_per_cu > 4) return sigmo_err::set(SIGMO_ERR_INVALID, "join_blocks_per_cu must be 0..4 (LDS keeps 4 resident)");
+  if (t->join_blocks_per_cu > 4) return sigmo_err::set(SIGMO_ERR_INVALID, "join_blocks_per_cu must be 0..4");
   if (t->filter_claim > 64) return sigmo_err::set(SIGMO_ERR_INVALID, "filter_claim must be 0..64");
   if (t->filter_mode > 2) return sigmo_err::set(SIGMO_ERR_INVALID, "filter_mode must be 0 (automatic), 1 (molecule) or 2 (list)");
   b->tune = *t;

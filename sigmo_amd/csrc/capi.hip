@@ -1263,7 +1263,7 @@ int sigmo_join(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_graph* data
     if (nw)
       SIGMO_HIP_TRY(sigmo_k::join_lanes_wide(s, query->dev(), data->dev(), c->bits, c->W64, m->indices, m->pair_graph, mm->wide_pairs, nw,
                                              find_first, mm->pair_counts, ctx->stats, ctx->num_cus,
-                                             ctx->capturing ? ctx->stats + 5 : nullptr, mm->deep_pairs));
+                                             ctx->capturing ? ctx->stats + 5 : nullptr));
   }
   SIGMO_TRY(ps.close());
   SIGMO_HIP_TRY(hipMemcpyAsync(ctx->stats_host, ctx->stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));

@@ -23,6 +23,12 @@ __device__ __forceinline__ uint32_t uniform32(uint32_t v) {
 __device__ __forceinline__ uint64_t uniform64(uint64_t v) {
   return static_cast<uint64_t>(uniform32(static_cast<uint32_t>(v))) | (static_cast<uint64_t>(uniform32(static_cast<uint32_t>(v >> 32))) << 32);
 }
+// Orders this wavefront's LDS accesses across lanes (the compiler may not move them across).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Bits at positions >= pos of a 64-bit word (0 when pos >= 64).
 __device__ __forceinline__ uint64_t bits_from(uint32_t pos) { return pos >= 64 ? 0ull : (~0ull << pos); }
 

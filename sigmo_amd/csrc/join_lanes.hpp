@@ -31,8 +31,9 @@ struct ArenaMasks {
     lo = arena[static_cast<uint64_t>(base) + 2 * depth];
     hi = arena[static_cast<uint64_t>(base) + 2 * depth + 1];
   }
-  // The masks of query nodes 0..k-1 (0 from k on), two per 16-byte load: a pair's block starts on a
-  // 4-word boundary and spans a multiple of 4 words, so a load that starts below k stays inside it.
+  // The masks of query nodes 0..k-1 (entries from k on are not to be read), two per 16-byte load: a
+  // pair's block starts on a 4-word boundary and spans a multiple of 4 words, so a load that starts
+  // below k stays inside it.
   template <int N>
   __device__ __forceinline__ void masks(uint32_t base, uint32_t, uint32_t k, uint32_t, uint32_t, uint64_t (&m)[N]) const {
     static_assert(N % 2 == 0, "masks come in pairs");
@@ -41,7 +42,7 @@ struct ArenaMasks {
       uint4 v = make_uint4(0, 0, 0, 0);
       if (t < k) v = *reinterpret_cast<const uint4*>(arena + static_cast<uint64_t>(base) + t);
       m[t] = static_cast<uint64_t>(v.x) | (static_cast<uint64_t>(v.y) << 32);
-      m[t + 1] = t + 1 < k ? (static_cast<uint64_t>(v.z) | (static_cast<uint64_t>(v.w) << 32)) : 0ull;
+      m[t + 1] = static_cast<uint64_t>(v.z) | (static_cast<uint64_t>(v.w) << 32);
     }
   }
   // The two-word masks of query nodes 0..k-1, one 16-byte load per node.
@@ -103,203 +104,426 @@ struct BitsetMasks {
   }
 };
 
-constexpr uint32_t kJoinLaneWaves = 2;  // wavefronts per block of the lane-per-pair join
-
-// Query depth the first lane-join pass holds in LDS.  Surviving pairs are mostly small queries
-// (on 20 M molecules x 2,000 queries of U[4,32] nodes: 89% have k <= 8, 98.5% k <= 12), so the
-// first pass keeps 12 levels per lane (6.75 KB per wavefront instead of 18 KB, 2.5x the resident
-// wavefronts) and lists the deeper pairs for a second pass that keeps all 32.
-constexpr int kJoinShallow = 12;
+// Query levels the lane join holds in LDS per lane.  Surviving pairs are mostly small queries (on
+// LogNormal molecules and U[4,32]-node queries 92% have k <= 8, and they take 89% of the DFS
+// steps), so a large join lists the pairs of deeper queries for a second pass; a small one runs
+// them all in one pass that holds 12 levels and reaches deeper ones through global memory.
+constexpr int kJoinShallow = 8;
+constexpr int kJoinLevels = 12;
 constexpr uint64_t kJoinTwoPassPairs = 1ull << 24;  // pair counts from which the lane join runs in two passes
+constexpr uint32_t kJoinDeepChunk = 128;            // pairs a wavefront claims at a time of the deep queries' list
+constexpr uint32_t kJoinRefill = 24;                // idle lanes that make a wavefront hand out new pairs
 
-// Join with one lane per GMCR pair, for molecules of <= 64 nodes (the rest are listed in
-// `wide` for the two-word kernel) and queries of <= KMAX nodes (the rest are listed in `deep`
-// for a second pass of this kernel with KMAX = 32 over that list).  Each lane runs the reference
-// DFS of isomorphism.hpp:270-381 for its own pair with the reference's bookkeeping: every
-// mapping entry starts at local node 0, an exhausted frame unsets the visited bit of its
-// (possibly stale) mapping entry, `visited` is cleared when depth 1 is exhausted, and a frame
-// resumes at mapping[depth] + 1.  The validity test of isomorphism.hpp:150-168 -- for every
-// j < depth, qAdj(j, depth) == dAdj(mapping[j], c) -- becomes set algebra on adjacency rows:
-// adjacency is symmetric, so the candidates that pass are those in the row of every mapped query
-// neighbour and in the row of no other mapped node.  The rows of the mapped positions and the
-// mapping sit in LDS (depth-major, one column per lane).  With `list` the pairs are list[0..P),
-// claimed through stats[cursor]; without it they are 0..P through stats[kStatCursor].
-template <bool FIND_FIRST, class Src, int KMAX = 32>
-__global__ __launch_bounds__(kJoinLaneWaves * 64) void k_join_lanes(GraphDev q, GraphDev d, Src src, const uint32_t* __restrict__ indices,
-                                                                   const uint32_t* __restrict__ pair_graph, uint64_t P, uint32_t chunk,
-                                                                   int32_t* __restrict__ counts, unsigned long long* __restrict__ stats,
-                                                                   uint32_t* __restrict__ wide, const unsigned long long* __restrict__ P_dev,
-                                                                   const uint32_t* __restrict__ list = nullptr, uint32_t* __restrict__ deep = nullptr,
-                                                                   uint32_t cursor = kStatCursor) {
-  static_assert(KMAX >= 2 && KMAX <= 32, "query depth");
-  __shared__ uint64_t rows_all[kJoinLaneWaves][KMAX][kWave];
-  if (src.aborted()) return;  // block-uniform: no barrier follows
+// One wavefront's LDS: per level t and lane, the adjacency row of the position mapped at t and the
+// candidates frame t started from (t < L = KC - 1), the candidate mask of query node t + 1, and
+// the mapping (a byte per level); then the queue of the next pairs.
+template <int KC, bool DEEP, bool WIDE>
+struct JoinLds {
+  static constexpr int L = KC - 1;
+  static constexpr int H = WIDE ? 2 : 1;
+  static constexpr int M = DEEP ? 40 : 8;  // mapping bytes per lane
+  uint64_t row[H][L][kWave];
+  uint64_t base[H][L][kWave];
+  uint64_t mask[H][L][kWave];
+  alignas(8) uint8_t map[kWave][M];
+  uint64_t q_adj[kWave];
+  uint32_t q_pair[kWave], q_start[kWave], q_qoff[kWave], q_base[kWave];
+  uint16_t q_nk[kWave];
+  uint32_t listed[(WIDE ? 0 : 1) + (DEEP ? 0 : 1) ? (WIDE ? 0 : 1) + (DEEP ? 0 : 1) : 1][2 * kWave];  // pairs for other passes: deep, then wide
+};
+template <int KC, bool DEEP, bool WIDE>
+constexpr uint32_t join_waves_per_cu() {  // wavefronts the 160 KB of LDS hold
+  return static_cast<uint32_t>(160 * 1024 / ((sizeof(JoinLds<KC, DEEP, WIDE>) + 511) / 512 * 512));
+}
+
+// Positions above c of a 64-position word.
+__device__ __forceinline__ uint64_t bits_above(uint32_t c) { return (~0ull << c) << 1; }
+__device__ __forceinline__ uint64_t bit_of(uint32_t c) { return 1ull << (c & 63u); }
+// A candidate set after the row of one mapped node: x & row where `a` is all ones (a query
+// neighbour), x & ~row where it is 0.  x & ~(row ^ a), table 0x90, one operation per 32 positions.
+__device__ __forceinline__ uint64_t and_row(uint64_t x, uint64_t row, uint32_t a) {
+  const uint32_t lo = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(x), static_cast<uint32_t>(row), a, 0x90);
+  const uint32_t hi = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(x >> 32), static_cast<uint32_t>(row >> 32), a, 0x90);
+  return lo | (static_cast<uint64_t>(hi) << 32);
+}
+// All ones when bit t (< 32) of q is set.
+__device__ __forceinline__ uint32_t bit_spread(uint32_t q, uint32_t t) {
+  return static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(q), t, 1u));
+}
+
+// Join with one lane per GMCR pair: the reference DFS of isomorphism.hpp:270-381 for the lane's
+// pair with the reference's bookkeeping -- every mapping entry starts at local node 0, an
+// exhausted frame unsets the visited bit of its (possibly stale) mapping entry, `visited` is
+// cleared when depth 1 is exhausted, and a frame resumes at mapping[depth] + 1.  The validity
+// test of isomorphism.hpp:150-168 -- for every j < depth, qAdj(j, depth) == dAdj(mapping[j], c)
+// -- is set algebra on adjacency rows: adjacency is symmetric, so the candidates that pass are
+// those in the row of every mapped query neighbour and in the row of no other mapped node.
+//
+// An iteration takes several DFS steps of a lane: it pops an exhausted frame, accepts the frame's
+// next candidate, and forms the next frame's candidates at once; when those are none, the next
+// frame's exhaustion is taken here too and the lane stays.  Most failing searches are accept /
+// exhaust pairs two or three levels down (LogNormal molecules, U[4,32] queries: 16.8 steps per
+// pair in 9.5 accepts).  A frame's candidates are kept in LDS for its return.  Rows at and above
+// the current depth are kept zero, so the rows of all levels apply without a test per lane (a
+// zero row at a non-adjacent level keeps every position), and their LDS reads go out together.
+//
+// Pairs come 64 at a time through three loading stages, a pair per lane, into a queue in LDS;
+// idle lanes take queued pairs and load their masks.  Loads return in order, so a step's wait for
+// its adjacency row also waits for every load issued before: the stages and the masks are
+// therefore all issued together, when kJoinRefill lanes are idle, and a wavefront stalls on them
+// once per that many pairs (16, 24 and 32 measure the same, 40 is 4% slower).
+//
+// Bound by VALU issue (about two thirds of it on 68 M pairs) at 12 wavefronts per CU by LDS.  One
+// DFS step per iteration, all rows tested per lane and an atomic per listed batch took, for 1 M
+// LogNormal molecules x 1,000 queries, 10.8 + 1.4 ms (molecules of <= 64 nodes) and 2.5 + 1.6 ms
+// (wider ones); this takes 6.0 + 1.9 and 1.65 ms, and 33,331 molecules x 257 queries find-all,
+// whose last lanes run long searches, 2.3 ms less.
+//
+// Molecules of <= 64 nodes (!WIDE; pairs of larger ones are listed in `wide`) or, with WIDE, of
+// 65..128 nodes: positions then span two words, and `visited` stays one word addressed by
+// position mod 64, the reference's Bitset aliasing (utils.hpp:71-73).  Queries of up to KC nodes;
+// deeper ones are listed in `deep` (their count in stats[deep_stat]), or, with DEEP, run here
+// with the levels past LDS read through global memory.  With `list` the pairs are list[0..P).
+template <bool FIND_FIRST, class Src, int KC, bool DEEP, bool WIDE>
+__global__ __launch_bounds__(64) void k_join_lanes(GraphDev q, GraphDev d, Src src, const uint32_t* __restrict__ indices,
+                                                   const uint32_t* __restrict__ pair_graph, uint64_t P, uint32_t chunk,
+                                                   int32_t* __restrict__ counts, unsigned long long* __restrict__ stats,
+                                                   uint32_t* __restrict__ wide, const unsigned long long* __restrict__ P_dev,
+                                                   const uint32_t* __restrict__ list, uint32_t* __restrict__ deep, uint32_t cursor,
+                                                   uint32_t deep_stat) {
+  static_assert(KC == 8 || KC == 12, "levels in LDS");
+  constexpr uint32_t L = KC - 1;
+  __shared__ JoinLds<KC, DEEP, WIDE> sh;
+  if (src.aborted()) return;
   // the pair (or list) count left on the device; P, what the arrays were sized for, bounds it
   if (P_dev) P = min(P, static_cast<uint64_t>(*P_dev));
-  __shared__ uint8_t maps_all[kJoinLaneWaves][KMAX][kWave];
   const uint32_t lane = static_cast<uint32_t>(lane_id());
-  const uint32_t wave = threadIdx.x / kWave;
-  uint64_t (*rows)[kWave] = rows_all[wave];
-  uint8_t (*maps)[kWave] = maps_all[wave];
   const uint64_t below = (1ull << lane) - 1;
-  uint64_t next = 0, end = 0;  // claimed pairs [next, end) (wave-uniform)
-  bool exhausted = false;
+  const uint32_t* qfold = reinterpret_cast<const uint32_t*>(q.fold);  // query rows fit the low word (k <= 32)
   uint64_t sum = 0, matched = 0, steps = 0, overflow = 0, wave_iters = 0;
 
-  bool have = false;
-  uint64_t j = 0, visited = 0, count = 0;
-  uint32_t s = 0, n = 0, qoff = 0, k = 0, base = 0, depth = 0, pos = 0;
-  // A shallow pass keeps its pair's candidate masks in registers, loaded together when the pair
-  // is taken: the DFS then reads no mask from memory (each of them used to be one dependent load
-  // per step, and the pairs' masks do not stay in L2 meanwhile).
-  constexpr bool kRegMasks = KMAX <= 16;
-  uint64_t mk[kRegMasks ? KMAX : 1];
+  // pairs on their way to the queue, one per lane and stage: graphs and mask base (a), sizes and
+  // offsets (b), query adjacency (c)
+  // claimed pairs [next, end) (wave-uniform): a wavefront's first claim is its own, later ones come
+  // from the cursor
+  uint64_t next = static_cast<uint64_t>(blockIdx.x) * chunk, end = next + chunk < P ? next + chunk : P;
+  const uint64_t claimed = static_cast<uint64_t>(gridDim.x) * chunk;
+  bool exhausted = false, have_a = false, have_b = false, have_c = false;
+  uint32_t qhead = 0, qcount = 0;
+  bool av = false, bv = false, cv = false;
+  uint32_t aj = 0, ag = 0, aq = 0, abase = 0;
+  uint32_t bj = 0, bbase = 0, bs = 0, be = 0, bq = 0, bqe = 0;
+  uint32_t cj = 0, cbase = 0, cs = 0, cn = 0, cq = 0, ck = 0;
+  uint32_t ca[8];
 #pragma unroll
-  for (int t = 0; t < (kRegMasks ? KMAX : 1); ++t) mk[t] = 0;
-  // Loads a step needs are issued a step ahead: `qad` is the query adjacency row of `depth`, and
-  // after an accept the new mapped node's row waits in `nrow` (`fresh`) until the next step, which
-  // uses it last and then stores it to LDS.
-  uint32_t qad = 0;
-  uint64_t nrow = 0;
-  bool fresh = false;
-  // Each lane prefetches its next pair while it runs the current one: nst = 1 once the pair's
-  // index is claimed and its molecule, query graph and mask base are loading; nst = 2 once its
-  // offsets and sizes are loading too.  A lane that finishes its pair takes the prefetched one
-  // without waiting on that chain of dependent loads.
-  uint32_t nst = 0, nj = 0, ndg = 0, nqg = 0, nbase = 0, ns = 0, nn = 0, nqoff = 0, nk = 0;
+  for (int t = 0; t < 8; ++t) ca[t] = 0;
+
+  // the lane's pair; `loading`: taken, its candidate masks on their way
+  bool have = false, loading = false;
+  uint64_t mlo[KC], mhi[WIDE ? KC : 1];
+#pragma unroll
+  for (int t = 0; t < KC; ++t) mlo[t] = 0;
+#pragma unroll
+  for (int t = 0; t < (WIDE ? KC : 1); ++t) mhi[t] = 0;
+  uint32_t j = 0, s = 0, n = 0, qoff = 0, k = 0, base = 0, depth = 0;
+  uint64_t adj = 0, visited = 0, count = 0;      // adj: byte t = query row of node t < 8 over nodes < 8
+  uint64_t cur = 0, cur_hi = 0, rem = 0, rem_hi = 0;  // the frame's candidates; positions past its last accept
+
+  // Pairs for another pass gather in LDS and go out 64 at a time: an atomic per batch of 64 pairs on
+  // one address (about 10 ns each across the XCDs) took 11 ms for 68 M pairs and bound the kernel.
+  uint32_t ndeep = 0, nwide = 0;
+  auto list_flush = [&](uint32_t* buf, uint32_t cnt, uint32_t* out, unsigned long long* total) {
+    unsigned long long b = 0;
+    if (lane == 0) b = atomicAdd(total, static_cast<unsigned long long>(cnt));
+    const uint64_t ob = uniform64(__shfl(b, 0));
+    if (lane < cnt) out[ob + lane] = buf[lane];
+  };
+  auto list_pairs = [&](bool mine, uint32_t pair, uint32_t* buf, uint32_t& cnt, uint32_t* out, unsigned long long* total) {
+    const uint64_t m = __ballot(mine);
+    if (!m) return;
+    if (mine) buf[cnt + __popcll(m & below)] = pair;
+    wave_sync();
+    cnt += static_cast<uint32_t>(__popcll(m));
+    if (cnt >= kWave) {
+      list_flush(buf, kWave, out, total);
+      cnt -= kWave;
+      const uint32_t left = buf[kWave + lane];
+      wave_sync();
+      buf[lane] = left;
+      wave_sync();
+    }
+  };
+  // rows of the mapped positions at levels below `upto` (and, in LDS, the zero rows above)
+  // applied to a candidate set; qm: the query row's bits below `upto`
+  auto apply_rows = [&](uint32_t qm, uint32_t upto, uint64_t& lo, uint64_t& hi) {
+    auto group = [&](uint32_t t0, uint32_t t1) {
+      uint64_t r[4], rh[4];
+#pragma unroll
+      for (uint32_t t = t0; t < t1; ++t) {
+        r[t - t0] = sh.row[0][t][lane];
+        if constexpr (WIDE) rh[t - t0] = sh.row[1][t][lane];
+      }
+#pragma unroll
+      for (uint32_t t = t0; t < t1; ++t) {
+        const uint32_t a = bit_spread(qm, t);
+        lo = and_row(lo, r[t - t0], a);
+        if constexpr (WIDE) hi = and_row(hi, rh[t - t0], a);
+      }
+    };
+    group(0, 4);
+    if (__any(upto > 4)) {
+      group(4, L < 8 ? L : 8);
+      if constexpr (L > 8)
+        if (__any(upto > 8)) group(8, L);
+    }
+    if constexpr (DEEP)
+      for (uint32_t t = L; t < upto; ++t) {
+        const uint64_t v = static_cast<uint64_t>(s) + sh.map[lane][t];
+        const uint32_t a = bit_spread(qm, t);
+        if constexpr (WIDE) {
+          lo = and_row(lo, d.adj[2 * v], a);
+          hi = and_row(hi, d.adj[2 * v + 1], a);
+        } else {
+          lo = and_row(lo, d.fold[v], a);
+        }
+      }
+  };
+  // the query adjacency row of node t < k (with bits of later rows above bit 7 when t < 8)
+  auto query_row = [&](uint32_t t) -> uint32_t {
+    uint32_t r = static_cast<uint32_t>(adj >> ((8 * t) & 63u));
+    if constexpr (DEEP)
+      if (t >= 8) r = qfold[2 * (static_cast<uint64_t>(qoff) + t)];
+    return r;
+  };
+  // the candidate mask of query node t >= 1
+  auto node_mask = [&](uint32_t t, uint64_t& lo, uint64_t& hi) {
+    const uint32_t at = DEEP ? min(t - 1, L - 1) : t - 1;
+    lo = sh.mask[0][at][lane];
+    if constexpr (WIDE) hi = sh.mask[1][at][lane];
+    if constexpr (DEEP)
+      if (t > L) {
+        if constexpr (WIDE) src.mask2(base, qoff + t, t, s, n, lo, hi);
+        else lo = src.mask(base, qoff + t, t, s, n);
+      }
+  };
+
   while (true) {
-    if (!have && nst == 2) {  // take the prefetched pair
-      j = nj;
-      s = ns;
-      n = nn;
-      qoff = nqoff;
-      k = nk;
-      base = nbase;
-      for (uint32_t t = 0; t < k; ++t) maps[t][lane] = 0;  // every mapping entry starts at local node 0
-      if constexpr (kRegMasks) src.masks(base, qoff, k, s, n, mk);
-      qad = static_cast<uint32_t>(q.fold[qoff]);
-      fresh = false;
+    if (loading) {  // the taken pair's masks have arrived: start it
+#pragma unroll
+      for (int t = 0; t < (DEEP ? 32 : 8); t += 8) *reinterpret_cast<uint64_t*>(&sh.map[lane][t]) = 0;  // every entry: local node 0
+#pragma unroll
+      for (uint32_t t = 0; t < L; ++t) {
+        sh.row[0][t][lane] = 0;
+        sh.mask[0][t][lane] = mlo[t + 1];
+        if constexpr (WIDE) {
+          sh.row[1][t][lane] = 0;
+          sh.mask[1][t][lane] = mhi[t + 1];
+        }
+      }
+      cur = mlo[0];
+      rem = ~0ull;
+      if constexpr (WIDE) {
+        cur_hi = mhi[0];
+        rem_hi = ~0ull;
+      }
       depth = 0;
-      pos = 0;
       visited = 0;
       count = 0;
       have = true;
-      nst = 0;
+      loading = false;
     }
-    bool wide_pair = false, deep_pair = false;
-    if (nst == 1) {  // the prefetched pair's offsets and sizes
-      ns = d.go[ndg];
-      nn = d.go[ndg + 1] - ns;
-      nqoff = q.go[nqg];
-      nk = q.go[nqg + 1] - nqoff;
-      wide_pair = nn > 64;
-      deep_pair = KMAX < 32 && !wide_pair && nk > static_cast<uint32_t>(KMAX);
-      nst = wide_pair || deep_pair ? 0u : 2u;
-    }
-    const uint64_t wm = __ballot(wide_pair);  // molecules of > 64 nodes go to the two-word kernel
-    if (wm) {
-      unsigned long long b = 0;
-      if (lane == 0) b = atomicAdd(&stats[kStatWide], static_cast<unsigned long long>(__popcll(wm)));
-      const uint64_t wb = uniform64(__shfl(b, 0));
-      if (wide_pair) wide[wb + __popcll(wm & below)] = nj;
-    }
-    const uint64_t dm = KMAX < 32 ? __ballot(deep_pair) : 0ull;  // queries deeper than KMAX go to the second pass
-    if (dm) {
-      unsigned long long b = 0;
-      if (lane == 0) b = atomicAdd(&stats[kStatDeep], static_cast<unsigned long long>(__popcll(dm)));
-      const uint64_t db = uniform64(__shfl(b, 0));
-      if (deep_pair) deep[db + __popcll(dm & below)] = nj;
-    }
-    uint64_t need = __ballot(nst == 0);  // lanes with nothing prefetched claim a pair
-    while (need && !exhausted) {
-      if (next >= end) {
-        unsigned long long b = 0;
-        if (lane == 0) b = atomicAdd(&stats[cursor], static_cast<unsigned long long>(chunk));
-        next = uniform64(__shfl(b, 0));
-        end = next + chunk < P ? next + chunk : P;
-        if (next >= P) {
+    const uint64_t idle = __ballot(!have);
+    if (static_cast<uint32_t>(__popcll(idle)) >= kJoinRefill || idle == ~0ull) {  // wave-uniform
+      if (qcount == 0 && have_c) {  // the third stage has arrived: queue its pairs
+        const bool wide_pair = !WIDE && cv && cn > 64;  // molecules of > 64 nodes go to the two-word pass
+        const bool deep_pair = !DEEP && cv && !wide_pair && ck > static_cast<uint32_t>(KC);
+        if constexpr (!DEEP) list_pairs(deep_pair, cj, sh.listed[0], ndeep, deep, &stats[deep_stat]);
+        if constexpr (!WIDE) list_pairs(wide_pair, cj, sh.listed[DEEP ? 0 : 1], nwide, wide, &stats[kStatWide]);
+        const bool mine = cv && !wide_pair && !deep_pair;
+        const uint64_t mm = __ballot(mine);
+        if (mine) {
+          uint64_t a = 0;
+#pragma unroll
+          for (uint32_t t = 0; t < 8; ++t) a |= static_cast<uint64_t>(ca[t] & 0xFFu) << (8 * t);
+          const uint32_t at = __popcll(mm & below);
+          sh.q_adj[at] = a;
+          sh.q_pair[at] = cj;
+          sh.q_start[at] = cs;
+          sh.q_qoff[at] = cq;
+          sh.q_base[at] = cbase;
+          sh.q_nk[at] = static_cast<uint16_t>(cn | (ck << 8));
+        }
+        wave_sync();
+        qhead = 0;
+        qcount = static_cast<uint32_t>(__popcll(mm));
+        have_c = false;
+      }
+      if (!have_c && have_b) {
+        cv = bv;
+        cj = bj;
+        cbase = bbase;
+        cs = bs;
+        cn = be - bs;
+        cq = bq;
+        ck = bqe - bq;
+        if (cv) {
+#pragma unroll
+          for (uint32_t t = 0; t < 8; ++t) ca[t] = t < ck ? qfold[2 * (static_cast<uint64_t>(cq) + t)] : 0u;
+        }
+        have_c = true;
+        have_b = false;
+      }
+      if (!have_b && have_a) {
+        bv = av;
+        bj = aj;
+        bbase = abase;
+        if (bv) {
+          bs = d.go[ag];
+          be = d.go[ag + 1];
+          bq = q.go[aq];
+          bqe = q.go[aq + 1];
+        }
+        have_b = true;
+        have_a = false;
+      }
+      if (!have_a && !exhausted) {
+        if (next >= end && claimed < P) {
+          unsigned long long b = 0;
+          if (lane == 0) b = atomicAdd(&stats[cursor], static_cast<unsigned long long>(chunk));
+          next = claimed + uniform64(__shfl(b, 0));
+          end = next + chunk < P ? next + chunk : P;
+        }
+        if (next >= end) {
           exhausted = true;
-          break;
+        } else {
+          av = next + lane < end;
+          if (av) {
+            aj = list ? list[next + lane] : static_cast<uint32_t>(next + lane);
+            ag = pair_graph[aj];
+            aq = indices[aj];
+            abase = src.base(aj);
+          }
+          next += kWave;
+          have_a = true;
         }
       }
-      const uint32_t cnt = min(static_cast<uint32_t>(end - next), static_cast<uint32_t>(__popcll(need)));
-      const uint32_t rn = __popcll(need & below);
-      const bool take = ((need >> lane) & 1ull) && rn < cnt;
-      if (take) {
-        nj = list ? list[next + rn] : static_cast<uint32_t>(next + rn);
-        ndg = pair_graph[nj];
-        nqg = indices[nj];
-        nbase = src.base(nj);
-        nst = 1;
+      if (qcount) {  // hand queued pairs to idle lanes
+        const uint32_t cnt = min(qcount, static_cast<uint32_t>(__popcll(idle)));
+        const uint32_t rn = __popcll(idle & below);
+        if (!have && rn < cnt) {
+          const uint32_t at = qhead + rn;
+          adj = sh.q_adj[at];
+          j = sh.q_pair[at];
+          s = sh.q_start[at];
+          qoff = sh.q_qoff[at];
+          base = sh.q_base[at];
+          n = sh.q_nk[at] & 0xFFu;
+          k = sh.q_nk[at] >> 8;
+          if constexpr (WIDE) src.masks2(base, qoff, k, s, n, mlo, mhi);
+          else src.masks(base, qoff, k, s, n, mlo);
+          loading = true;
+        }
+        qhead += cnt;
+        qcount -= cnt;
       }
-      next += cnt;
-      need &= ~__ballot(take);
+      if (__ballot(have || loading) == 0) {
+        if (exhausted && !have_a && !have_b && !have_c && qcount == 0) break;
+        continue;
+      }
     }
-    if (__ballot(have || nst != 0) == 0) break;
     ++wave_iters;
     if (have) {
-      ++steps;
       bool done = false;
-      if (depth == k) {  // leaf (:336-344)
-        ++count;
-        if (FIND_FIRST) {
-          done = true;
-        } else {
-          // the pending row is the leaf's last node's, which no step reads
-          fresh = false;
-          depth = k - 1;
-          pos = static_cast<uint32_t>(maps[depth][lane]) + 1;
-          qad = static_cast<uint32_t>(q.fold[static_cast<uint64_t>(qoff) + depth]);
-        }
-      } else {
-        // adjacency rows as 8-byte folded words: query graphs (<= 32 nodes) and these molecules
-        // (<= 64 nodes) have no neighbour at positions >= 64, so fold = the low row word
-        // candidates in the row of every mapped query neighbour and in no row of another mapped
-        // node: AND over t of row_t, complemented where t is not adjacent to `depth`
-        uint64_t md = 0;
-        if (kRegMasks) {
-#pragma unroll
-          for (uint32_t t = 0; t < (kRegMasks ? KMAX : 1); ++t) md = t == depth ? mk[t] : md;
-        } else {
-          md = src.mask(base, qoff + depth, depth, s, n);
-        }
-        uint64_t el = md & ~visited & bits_from(pos);
-        const uint32_t lim = fresh ? depth - 1 : depth;
-        if (kRegMasks) {  // unrolled over KMAX; the compiler branches around the rows at t >= lim
-#pragma unroll
-          for (uint32_t t = 0; t < (kRegMasks ? KMAX : 1); ++t) {
-            const uint64_t rw = rows[t][lane];
-            if (t < lim) el &= rw ^ (static_cast<uint64_t>(((qad >> t) & 1u)) - 1ull);
+      uint32_t st = 0;
+      uint64_t el = cur & ~visited & rem, eh = WIDE ? cur_hi & ~visited & rem_hi : 0ull;
+      if ((el | eh) == 0) {  // exhausted frame (:346-354)
+        st = 1;
+        done = depth == 0;
+        const uint32_t up = done ? 0u : depth - 1;
+        const uint32_t m = sh.map[lane][depth], c = sh.map[lane][up];
+        visited &= ~bit_of(m);
+        if (depth == 1) visited = 0;
+        if (!DEEP || up < L) {
+          cur = sh.base[0][up][lane];
+          sh.row[0][up][lane] = 0;
+          if constexpr (WIDE) {
+            cur_hi = sh.base[1][up][lane];
+            sh.row[1][up][lane] = 0;
           }
         } else {
-          for (uint32_t t = 0; t < lim; ++t) el &= rows[t][lane] ^ (static_cast<uint64_t>(((qad >> t) & 1u)) - 1ull);
+          node_mask(up, cur, cur_hi);
+          const uint32_t qr = query_row(up);
+          apply_rows(qr & ((1u << up) - 1u), up, cur, cur_hi);
         }
-        if (fresh) {
-          el &= nrow ^ (static_cast<uint64_t>(((qad >> lim) & 1u)) - 1ull);
-          rows[lim][lane] = nrow;
-          fresh = false;
+        depth = up;
+        if constexpr (WIDE) {
+          rem = c < 64 ? bits_above(c) : 0ull;
+          rem_hi = c < 64 ? ~0ull : bits_above(c - 64);
+          eh = done ? 0ull : cur_hi & ~visited & rem_hi;
+        } else {
+          rem = bits_above(c);
         }
-        if (el) {  // accept (:366-370)
-          const uint32_t c = static_cast<uint32_t>(__builtin_ctzll(el));
-          maps[depth][lane] = static_cast<uint8_t>(c);
-          nrow = d.fold[static_cast<uint64_t>(s) + c];
-          fresh = true;
-          visited |= 1ull << c;
-          ++depth;
-          pos = 0;
-          if (depth < k) qad = static_cast<uint32_t>(q.fold[static_cast<uint64_t>(qoff) + depth]);
-        } else {  // exhausted frame (:346-354)
-          visited &= ~(1ull << (maps[depth][lane] & 63u));
-          if (depth == 0) {
-            done = true;
-          } else {
-            if (depth == 1) visited = 0;
-            --depth;
-            pos = static_cast<uint32_t>(maps[depth][lane]) + 1;
-            qad = static_cast<uint32_t>(q.fold[static_cast<uint64_t>(qoff) + depth]);
+        el = done ? 0ull : cur & ~visited & rem;
+      }
+      if (el | eh) {  // accept (:366-370)
+        uint32_t c;
+        if constexpr (WIDE) {
+          c = el ? static_cast<uint32_t>(__builtin_ctzll(el)) : 64u + static_cast<uint32_t>(__builtin_ctzll(eh));
+          rem = c < 64 ? bits_above(c) : 0ull;
+          rem_hi = c < 64 ? ~0ull : bits_above(c - 64);
+          visited |= bit_of(c);
+        } else {
+          c = static_cast<uint32_t>(__builtin_ctzll(el));
+          const uint64_t bit = el & (0ull - el);
+          rem = 0ull - (bit << 1);  // positions above c
+          visited |= bit;
+        }
+        const uint64_t v = static_cast<uint64_t>(s) + c;
+        uint64_t rlo, rhi = 0, nlo = 0, nhi = 0;
+        if constexpr (WIDE) {
+          rlo = d.adj[2 * v];
+          rhi = d.adj[2 * v + 1];
+        } else {
+          rlo = d.fold[v];
+        }
+        const uint32_t nd = depth + 1;
+        const bool leaf = nd == k;
+        const uint32_t qr = query_row(leaf ? 0u : nd);
+        node_mask(leaf ? 1u : nd, nlo, nhi);
+        sh.map[lane][depth] = static_cast<uint8_t>(c);
+        const uint32_t stale = sh.map[lane][leaf ? 0u : nd];
+        apply_rows(qr & ((1u << depth) - 1u), depth, nlo, nhi);
+        const uint32_t a = bit_spread(qr, depth);
+        nlo = and_row(nlo, rlo, a);
+        if constexpr (WIDE) nhi = and_row(nhi, rhi, a);
+        const bool some = ((nlo & ~visited) | (WIDE ? nhi & ~visited : 0ull)) != 0;
+        if (leaf) {  // (:336-344): the frame resumes past it
+          ++count;
+          done = FIND_FIRST;
+        }
+        if (!leaf && some) {  // the next frame
+          st += 1;
+          if (!DEEP || depth < L) {
+            sh.base[0][depth][lane] = cur;
+            sh.row[0][depth][lane] = rlo;
+            if constexpr (WIDE) {
+              sh.base[1][depth][lane] = cur_hi;
+              sh.row[1][depth][lane] = rhi;
+            }
           }
+          depth = nd;
+          cur = nlo;
+          rem = ~0ull;
+          if constexpr (WIDE) {
+            cur_hi = nhi;
+            rem_hi = ~0ull;
+          }
+        } else {  // the leaf, or the next frame's exhaustion
+          st += 2;
+          if (!leaf) visited = nd == 1 ? 0ull : visited & ~bit_of(stale);
         }
       }
+      steps += st;
       if (done) {
         if (count > 0x7FFFFFFFull) overflow = 1;
         counts[j] = static_cast<int32_t>(count > 0x7FFFFFFFull ? 0x7FFFFFFFull : count);
@@ -309,6 +533,10 @@ __global__ __launch_bounds__(kJoinLaneWaves * 64) void k_join_lanes(GraphDev q, 
       }
     }
   }
+  if constexpr (!DEEP)
+    if (ndeep) list_flush(sh.listed[0], ndeep, deep, &stats[deep_stat]);
+  if constexpr (!WIDE)
+    if (nwide) list_flush(sh.listed[DEEP ? 0 : 1], nwide, wide, &stats[kStatWide]);
 #pragma unroll
   for (int o = kWave / 2; o > 0; o >>= 1) {
     sum += __shfl_xor(sum, o);
@@ -325,297 +553,76 @@ __global__ __launch_bounds__(kJoinLaneWaves * 64) void k_join_lanes(GraphDev q, 
   }
 }
 
-// The same lane-per-pair DFS for the pairs listed in `list` (molecules of 65..128 nodes).  The
-// positions span two words: candidates and the adjacency rows of mapped positions are (lo, hi)
-// pairs, while `visited` stays one word addressed by position mod 64, the reference's Bitset
-// aliasing (utils.hpp:71-73), exactly as the wavefront join does for these molecules.  LDS holds
-// two row words per depth and lane: with KMAX = kJoinShallow (12.75 KB per wavefront) the pass
-// lists the pairs of deeper queries in `deep` (count in stats[kStatWideDeep]) for a second pass
-// with KMAX = 32 (34.8 KB).  The shallow pass keeps its pair's masks in registers and, as the
-// narrow lane join, prefetches its next pair, issues each step's loads a step ahead and unrolls
-// its row loop.
-template <bool FIND_FIRST, class Src, int KMAX = 32>
-__global__ __launch_bounds__(64) void k_join_lanes_wide(GraphDev q, GraphDev d, Src src, const uint32_t* __restrict__ indices,
-                                                        const uint32_t* __restrict__ pair_graph, const uint32_t* __restrict__ list, uint64_t P,
-                                                        uint32_t chunk, uint32_t cursor, int32_t* __restrict__ counts,
-                                                        unsigned long long* __restrict__ stats,
-                                                        const unsigned long long* __restrict__ P_dev = nullptr,
-                                                        uint32_t* __restrict__ deep = nullptr) {
-  static_assert(KMAX >= 2 && KMAX <= 32, "query depth");
-  __shared__ uint64_t rows_lo[KMAX][kWave];
-  __shared__ uint64_t rows_hi[KMAX][kWave];
-  __shared__ uint8_t maps[KMAX][kWave];
-  if (src.aborted()) return;
-  // the list's length as the lane join left it on the device, bounded by what the caller sized
-  if (P_dev) P = min(P, static_cast<uint64_t>(*P_dev));
-  const uint32_t lane = static_cast<uint32_t>(lane_id());
-  const uint64_t below = (1ull << lane) - 1;
-  uint64_t next = 0, end = 0;
-  bool exhausted = false;
-  uint64_t sum = 0, matched = 0, steps = 0, overflow = 0, wave_iters = 0;
-
-  bool have = false;
-  uint64_t j = 0, visited = 0, count = 0;
-  uint32_t s = 0, n = 0, qoff = 0, k = 0, base = 0, depth = 0, pos = 0;
-  constexpr bool kReg = KMAX <= 16;
-  uint64_t mlo[kReg ? KMAX : 1], mhi[kReg ? KMAX : 1];
-#pragma unroll
-  for (int t = 0; t < (kReg ? KMAX : 1); ++t) mlo[t] = mhi[t] = 0;
-  uint32_t qad = 0;
-  uint64_t nlo = 0, nhi = 0;  // the accepted node's row words, stored to LDS by the next step
-  bool fresh = false;
-  uint32_t nst = 0, nj = 0, ndg = 0, nqg = 0, nbase = 0, ns = 0, nn = 0, nqoff = 0, nk = 0;
-  while (true) {
-    if (!have && nst == 2) {  // take the prefetched pair
-      j = nj;
-      s = ns;
-      n = nn;
-      qoff = nqoff;
-      k = nk;
-      base = nbase;
-      for (uint32_t t = 0; t < k; ++t) maps[t][lane] = 0;  // every mapping entry starts at local node 0
-      if constexpr (kReg) src.masks2(base, qoff, k, s, n, mlo, mhi);
-      qad = static_cast<uint32_t>(q.adj[2 * static_cast<uint64_t>(qoff)]);
-      fresh = false;
-      depth = 0;
-      pos = 0;
-      visited = 0;
-      count = 0;
-      have = true;
-      nst = 0;
-    }
-    bool deep_pair = false;
-    if (nst == 1) {  // the prefetched pair's offsets and sizes
-      ns = d.go[ndg];
-      nn = d.go[ndg + 1] - ns;
-      nqoff = q.go[nqg];
-      nk = q.go[nqg + 1] - nqoff;
-      deep_pair = KMAX < 32 && nk > static_cast<uint32_t>(KMAX);
-      nst = deep_pair ? 0u : 2u;
-    }
-    const uint64_t dm = KMAX < 32 ? __ballot(deep_pair) : 0ull;  // queries deeper than KMAX go to the second pass
-    if (dm) {
-      unsigned long long b = 0;
-      if (lane == 0) b = atomicAdd(&stats[kStatWideDeep], static_cast<unsigned long long>(__popcll(dm)));
-      const uint64_t db = uniform64(__shfl(b, 0));
-      if (deep_pair) deep[db + __popcll(dm & below)] = nj;
-    }
-    uint64_t need = __ballot(nst == 0);  // lanes with nothing prefetched claim a pair
-    while (need && !exhausted) {
-      if (next >= end) {
-        unsigned long long b = 0;
-        if (lane == 0) b = atomicAdd(&stats[cursor], static_cast<unsigned long long>(chunk));
-        next = uniform64(__shfl(b, 0));
-        end = next + chunk < P ? next + chunk : P;
-        if (next >= P) {
-          exhausted = true;
-          break;
-        }
-      }
-      const uint32_t cnt = min(static_cast<uint32_t>(end - next), static_cast<uint32_t>(__popcll(need)));
-      const uint32_t rn = __popcll(need & below);
-      const bool take = ((need >> lane) & 1ull) && rn < cnt;
-      if (take) {
-        nj = list[next + rn];
-        ndg = pair_graph[nj];
-        nqg = indices[nj];
-        nbase = src.base(nj);
-        nst = 1;
-      }
-      next += cnt;
-      need &= ~__ballot(take);
-    }
-    if (__ballot(have || nst != 0) == 0) break;
-    ++wave_iters;
-    if (have) {
-      ++steps;
-      bool done = false;
-      if (depth == k) {  // leaf (:336-344)
-        ++count;
-        if (FIND_FIRST) {
-          done = true;
-        } else {
-          fresh = false;  // the pending rows are the leaf's last node's, which no step reads
-          depth = k - 1;
-          pos = static_cast<uint32_t>(maps[depth][lane]) + 1;
-          qad = static_cast<uint32_t>(q.adj[2 * (static_cast<uint64_t>(qoff) + depth)]);
-        }
-      } else {
-        uint64_t clo = 0, chi = 0;
-        if (kReg) {
-#pragma unroll
-          for (uint32_t t = 0; t < (kReg ? KMAX : 1); ++t) {
-            clo = t == depth ? mlo[t] : clo;
-            chi = t == depth ? mhi[t] : chi;
-          }
-        } else {
-          src.mask2(base, qoff + depth, depth, s, n, clo, chi);
-        }
-        clo &= ~visited & bits_from(pos);
-        chi &= ~visited & (pos <= 64 ? ~0ull : bits_from(pos - 64));
-        uint64_t el = clo, eh = chi;
-        const uint32_t lim = fresh ? depth - 1 : depth;
-        if (kReg) {  // unrolled over KMAX; the compiler branches around the rows at t >= lim
-#pragma unroll
-          for (uint32_t t = 0; t < (kReg ? KMAX : 1); ++t) {
-            const uint64_t rl = rows_lo[t][lane], rh = rows_hi[t][lane];
-            if (t < lim) {
-              const uint64_t flip = static_cast<uint64_t>(((qad >> t) & 1u)) - 1ull;  // all ones where t is not adjacent
-              el &= rl ^ flip;
-              eh &= rh ^ flip;
-            }
-          }
-        } else {
-          for (uint32_t t = 0; t < lim; ++t) {
-            const uint64_t flip = static_cast<uint64_t>(((qad >> t) & 1u)) - 1ull;
-            el &= rows_lo[t][lane] ^ flip;
-            eh &= rows_hi[t][lane] ^ flip;
-          }
-        }
-        if (fresh) {
-          const uint64_t flip = static_cast<uint64_t>(((qad >> lim) & 1u)) - 1ull;
-          el &= nlo ^ flip;
-          eh &= nhi ^ flip;
-          rows_lo[lim][lane] = nlo;
-          rows_hi[lim][lane] = nhi;
-          fresh = false;
-        }
-        if (el | eh) {  // accept (:366-370)
-          const uint32_t c = el ? static_cast<uint32_t>(__builtin_ctzll(el)) : 64u + static_cast<uint32_t>(__builtin_ctzll(eh));
-          maps[depth][lane] = static_cast<uint8_t>(c);
-          nlo = d.adj[2 * (static_cast<uint64_t>(s) + c)];
-          nhi = d.adj[2 * (static_cast<uint64_t>(s) + c) + 1];
-          fresh = true;
-          visited |= 1ull << (c & 63);
-          ++depth;
-          pos = 0;
-          if (depth < k) qad = static_cast<uint32_t>(q.adj[2 * (static_cast<uint64_t>(qoff) + depth)]);
-        } else {  // exhausted frame (:346-354)
-          visited &= ~(1ull << (maps[depth][lane] & 63u));
-          if (depth == 0) {
-            done = true;
-          } else {
-            if (depth == 1) visited = 0;
-            --depth;
-            pos = static_cast<uint32_t>(maps[depth][lane]) + 1;
-            qad = static_cast<uint32_t>(q.adj[2 * (static_cast<uint64_t>(qoff) + depth)]);
-          }
-        }
-      }
-      if (done) {
-        if (count > 0x7FFFFFFFull) overflow = 1;
-        counts[j] = static_cast<int32_t>(count > 0x7FFFFFFFull ? 0x7FFFFFFFull : count);
-        sum += count;
-        matched += count > 0;
-        have = false;
-      }
-    }
-  }
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) {
-    sum += __shfl_xor(sum, o);
-    matched += __shfl_xor(matched, o);
-    steps += __shfl_xor(steps, o);
-    overflow |= __shfl_xor(overflow, o);
-  }
-  if (lane == 0) {
-    if (sum) atomicAdd(&stats[0], static_cast<unsigned long long>(sum));
-    if (matched) atomicAdd(&stats[1], static_cast<unsigned long long>(matched));
-    if (overflow) atomicOr(&stats[3], 1ull);
-    atomicAdd(&stats[4], static_cast<unsigned long long>(steps));
-    atomicAdd(&stats[7], static_cast<unsigned long long>(wave_iters));
-  }
+// Wavefronts (one-wavefront blocks) for `pairs` pairs: as many as stay resident by LDS, or the
+// tuned share of them in quarters, and no more than have a pair each.
+template <int KC, bool DEEP, bool WIDE>
+uint64_t join_blocks(uint64_t pairs, int num_cus, uint32_t quarters) {
+  const uint64_t cus = static_cast<uint64_t>(num_cus > 0 ? num_cus : 256);
+  const uint64_t per_cu = std::max<uint64_t>(1, uint64_t(join_waves_per_cu<KC, DEEP, WIDE>()) * quarters / 4);
+  return std::max<uint64_t>(1, std::min<uint64_t>((pairs + 63) / 64, cus * per_cu));
 }
 
 // The lane join over P pairs: with `deep`, a kJoinShallow-level pass over all of them that lists
-// the deeper queries, then a full-depth pass over that list (its length read on the device);
-// without it, one full-depth pass.  blocks_per_cu (<= 4 by LDS at full depth) and chunk (0: ~16
-// claims per wavefront) shape the first pass.
+// the deeper queries, then a pass over that list (its length read on the device); without it, one
+// pass.  `quarters` (1..4: share of the resident wavefronts) and chunk (0: ~4 claims per
+// wavefront, at most 1024 pairs: a claim is an atomic on one address) shape the first pass.
 template <class Src>
 hipError_t launch_join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const Src& src, const uint32_t* indices,
                              const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts, unsigned long long* stats,
-                             uint32_t* wide, int num_cus, const unsigned long long* P_dev, uint32_t* deep, uint32_t blocks_per_cu,
+                             uint32_t* wide, int num_cus, const unsigned long long* P_dev, uint32_t* deep, uint32_t quarters,
                              uint32_t chunk) {
   if (!P) return hipSuccess;
-  // Two passes pay off once the pairs fill the device many times over (1.4 x 10^8 pairs of a
-  // 1 M-molecule x 2,000-query chunk: 50.6 -> 45.4 ms); on 1.5 x 10^6 pairs the second pass's
-  // serial tail costs more than the first pass gains (0.53 -> 0.83 ms), so small joins run one
-  // full-depth pass.
   if (P < kJoinTwoPassPairs) deep = nullptr;
-  const uint64_t cus = static_cast<uint64_t>(num_cus > 0 ? num_cus : 256);
-  // the shallow pass keeps 2.75x the wavefronts resident: up to 11 blocks per CU (13.5 KB of LDS
-  // each, 80 VGPRs), which the LDS holds at once
-  const uint64_t per_cu = deep ? static_cast<uint64_t>(blocks_per_cu) * 11 / 4 : blocks_per_cu;
-  const uint64_t blocks = std::max<uint64_t>(1, std::min<uint64_t>((P + 127) / 128, cus * per_cu));
-  const uint32_t ch = chunk ? chunk
-                            : static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, P / (blocks * kJoinLaneWaves * 16))));
-  const dim3 grid(static_cast<unsigned>(blocks)), block(kJoinLaneWaves * 64);
+  const auto claim = [&](uint64_t blocks) {
+    return chunk ? chunk : static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, P / (blocks * 4) / 64 * 64)));
+  };
   if (!deep) {
+    const uint64_t blocks = join_blocks<kJoinLevels, true, false>(P, num_cus, quarters);
+    const dim3 grid(static_cast<unsigned>(blocks));
     if (find_first)
-      hipLaunchKernelGGL((k_join_lanes<true, Src, 32>), grid, block, 0, s, q, d, src, indices, pair_graph, P, ch, counts, stats, wide, P_dev,
-                         nullptr, nullptr, kStatCursor);
+      hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinLevels, true, false>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, claim(blocks),
+                         counts, stats, wide, P_dev, nullptr, nullptr, kStatCursor, kStatDeep);
     else
-      hipLaunchKernelGGL((k_join_lanes<false, Src, 32>), grid, block, 0, s, q, d, src, indices, pair_graph, P, ch, counts, stats, wide, P_dev,
-                         nullptr, nullptr, kStatCursor);
+      hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinLevels, true, false>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, claim(blocks),
+                         counts, stats, wide, P_dev, nullptr, nullptr, kStatCursor, kStatDeep);
     return hipGetLastError();
   }
+  const uint64_t blocks = join_blocks<kJoinShallow, false, false>(P, num_cus, quarters);
+  const dim3 grid(static_cast<unsigned>(blocks));
   if (find_first)
-    hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinShallow>), grid, block, 0, s, q, d, src, indices, pair_graph, P, ch, counts, stats, wide,
-                       P_dev, nullptr, deep, kStatCursor);
+    hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinShallow, false, false>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, claim(blocks),
+                       counts, stats, wide, P_dev, nullptr, deep, kStatCursor, kStatDeep);
   else
-    hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinShallow>), grid, block, 0, s, q, d, src, indices, pair_graph, P, ch, counts, stats, wide,
-                       P_dev, nullptr, deep, kStatCursor);
+    hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinShallow, false, false>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, claim(blocks),
+                       counts, stats, wide, P_dev, nullptr, deep, kStatCursor, kStatDeep);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  // the deep list is short (queries of more than kJoinShallow nodes): small claims, full depth
-  const uint64_t dblocks = std::max<uint64_t>(1, std::min<uint64_t>((P + 127) / 128, cus * 4));
-  const dim3 dgrid(static_cast<unsigned>(dblocks));
+  const dim3 dgrid(static_cast<unsigned>(join_blocks<kJoinLevels, true, false>(P, num_cus, 4)));
   if (find_first)
-    hipLaunchKernelGGL((k_join_lanes<true, Src, 32>), dgrid, block, 0, s, q, d, src, indices, pair_graph, P, 16u, counts, stats, wide,
-                       stats + kStatDeep, deep, nullptr, kStatDeepCursor);
+    hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinLevels, true, false>), dgrid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, kJoinDeepChunk, counts,
+                       stats, wide, stats + kStatDeep, deep, nullptr, kStatDeepCursor, kStatDeep);
   else
-    hipLaunchKernelGGL((k_join_lanes<false, Src, 32>), dgrid, block, 0, s, q, d, src, indices, pair_graph, P, 16u, counts, stats, wide,
-                       stats + kStatDeep, deep, nullptr, kStatDeepCursor);
+    hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinLevels, true, false>), dgrid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, kJoinDeepChunk, counts,
+                       stats, wide, stats + kStatDeep, deep, nullptr, kStatDeepCursor, kStatDeep);
   return hipGetLastError();
 }
 
 // The two-word lane join over the nw pairs listed in `list` (their count also at nw_dev when
-// given, nw then only bounding the grid).  With `deep` (capacity nw) a kJoinShallow-level pass
-// (12 resident one-wavefront blocks per CU) lists the deeper queries for a full-depth pass over
-// that list (4 blocks per CU); without it, one full-depth pass.
+// given, nw then only bounding the grid).
 template <class Src>
 hipError_t launch_join_wide(hipStream_t s, const GraphDev& q, const GraphDev& d, const Src& src, const uint32_t* indices,
                             const uint32_t* pair_graph, const uint32_t* list, uint64_t nw, int find_first, int32_t* counts,
-                            unsigned long long* stats, int num_cus, const unsigned long long* nw_dev, uint32_t* deep) {
+                            unsigned long long* stats, int num_cus, const unsigned long long* nw_dev) {
   if (!nw) return hipSuccess;
-  const uint64_t cus = static_cast<uint64_t>(num_cus > 0 ? num_cus : 256);
-  const uint64_t per_cu = deep ? 12 : 4;
-  const uint64_t blocks = std::max<uint64_t>(1, std::min<uint64_t>((nw + 63) / 64, cus * per_cu));
-  const uint32_t chunk = static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, nw / (blocks * 16))));
-  if (!deep) {
-    if (find_first)
-      hipLaunchKernelGGL((k_join_lanes_wide<true, Src, 32>), dim3(static_cast<unsigned>(blocks)), dim3(64), 0, s, q, d, src, indices, pair_graph,
-                         list, nw, chunk, static_cast<uint32_t>(kStatWideCursor), counts, stats, nw_dev, nullptr);
-    else
-      hipLaunchKernelGGL((k_join_lanes_wide<false, Src, 32>), dim3(static_cast<unsigned>(blocks)), dim3(64), 0, s, q, d, src, indices, pair_graph,
-                         list, nw, chunk, static_cast<uint32_t>(kStatWideCursor), counts, stats, nw_dev, nullptr);
-    return hipGetLastError();
-  }
+  const uint64_t blocks = join_blocks<kJoinShallow, true, true>(nw, num_cus, 4);
+  const uint32_t chunk = static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, nw / (blocks * 4) / 64 * 64)));
+  const dim3 grid(static_cast<unsigned>(blocks));
   if (find_first)
-    hipLaunchKernelGGL((k_join_lanes_wide<true, Src, kJoinShallow>), dim3(static_cast<unsigned>(blocks)), dim3(64), 0, s, q, d, src, indices,
-                       pair_graph, list, nw, chunk, static_cast<uint32_t>(kStatWideCursor), counts, stats, nw_dev, deep);
+    hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinShallow, true, true>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, nw, chunk, counts,
+                       stats, nullptr, nw_dev, list, nullptr, static_cast<uint32_t>(kStatWideCursor), static_cast<uint32_t>(kStatDeep));
   else
-    hipLaunchKernelGGL((k_join_lanes_wide<false, Src, kJoinShallow>), dim3(static_cast<unsigned>(blocks)), dim3(64), 0, s, q, d, src, indices,
-                       pair_graph, list, nw, chunk, static_cast<uint32_t>(kStatWideCursor), counts, stats, nw_dev, deep);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const uint64_t dblocks = std::max<uint64_t>(1, std::min<uint64_t>((nw + 63) / 64, cus * 4));
-  if (find_first)
-    hipLaunchKernelGGL((k_join_lanes_wide<true, Src, 32>), dim3(static_cast<unsigned>(dblocks)), dim3(64), 0, s, q, d, src, indices, pair_graph,
-                       deep, nw, 16u, static_cast<uint32_t>(kStatWideDeepCursor), counts, stats, stats + kStatWideDeep, nullptr);
-  else
-    hipLaunchKernelGGL((k_join_lanes_wide<false, Src, 32>), dim3(static_cast<unsigned>(dblocks)), dim3(64), 0, s, q, d, src, indices, pair_graph,
-                       deep, nw, 16u, static_cast<uint32_t>(kStatWideDeepCursor), counts, stats, stats + kStatWideDeep, nullptr);
+    hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinShallow, true, true>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, nw, chunk, counts,
+                       stats, nullptr, nw_dev, list, nullptr, static_cast<uint32_t>(kStatWideCursor), static_cast<uint32_t>(kStatDeep));
   return hipGetLastError();
 }
 

@@ -1078,8 +1078,8 @@ hipError_t join_wildcard(hipStream_t s, const GraphDev& q, const GraphDev& d, co
 
 hipError_t join_lanes_wide(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint64_t* bits, uint64_t W64, const uint32_t* indices,
                            const uint32_t* pair_graph, const uint32_t* list, uint64_t nw, int find_first, int32_t* counts,
-                           unsigned long long* stats, int num_cus, const unsigned long long* nw_dev, uint32_t* deep) {
-  return launch_join_wide(s, q, d, BitsetMasks{bits, W64}, indices, pair_graph, list, nw, find_first, counts, stats, num_cus, nw_dev, deep);
+                           unsigned long long* stats, int num_cus, const unsigned long long* nw_dev) {
+  return launch_join_wide(s, q, d, BitsetMasks{bits, W64}, indices, pair_graph, list, nw, find_first, counts, stats, num_cus, nw_dev);
 }
 
 }  // namespace sigmo_k

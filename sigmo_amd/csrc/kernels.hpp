@@ -115,18 +115,16 @@ enum : uint32_t {
   kStatWide = 5,       // pairs listed for the two-word join (molecules of > 64 nodes)
   kStatWideCursor = 6, // its work cursor
   kStatWaveIters = 7,  // loop iterations summed over wavefronts
-  kStatDeep = 8,       // pairs listed for the full-depth pass of the lane join
-  kStatDeepCursor = 9, // its work cursor
-  kStatWideDeep = 10,  // pairs listed for the full-depth pass of the two-word join
-  kStatWideDeepCursor = 11  // its work cursor
+  kStatDeep = 8,       // pairs listed for the second pass of the lane join
+  kStatDeepCursor = 9  // its work cursor
 };
 constexpr uint32_t kJoinStatWords = 16;
 
 // Join.  stats[0] += sum of counts, stats[1] += pairs with count > 0, stats[2] = work cursor
-// (zeroed by the caller), stats[3] |= 1 on int32 overflow.  With `deep` (capacity P) the join
-// runs in two passes: a first that holds kJoinShallow query levels per lane in LDS and lists
-// the pairs of deeper queries in `deep` (count in stats[8]), then a full-depth pass over that
-// list; without it, one full-depth pass.
+// (zeroed by the caller), stats[3] |= 1 on int32 overflow.  With `deep` (capacity P) a
+// large join runs in two passes: a first over the queries of at most kJoinShallow nodes, which
+// lists the other pairs in `deep` (count in stats[8]), then one over that list; without it, one
+// pass.
 // Lane-per-pair join of the pairs whose molecule has <= 64 nodes; the others are appended to
 // `wide` (count in stats[5]) for join_lanes_wide.  With P_dev the kernel reads the pair count
 // from the device and P only bounds the grid.
@@ -140,9 +138,9 @@ hipError_t join_wildcard(hipStream_t s, const GraphDev& q, const GraphDev& d, co
                          unsigned long long* stats, int num_cus);
 // The lane-per-pair join over the `nw` listed pairs of molecules with 65..128 nodes
 // (stats[kStatWideCursor] is the work counter).  With nw_dev the kernel reads the list's length on
-// the device, bounded by nw.  With `deep` (capacity nw) it runs in two passes as join_lanes does.
+// the device, bounded by nw.
 hipError_t join_lanes_wide(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint64_t* bits, uint64_t W64, const uint32_t* indices,
                            const uint32_t* pair_graph, const uint32_t* list, uint64_t nw, int find_first, int32_t* counts,
-                           unsigned long long* stats, int num_cus, const unsigned long long* nw_dev = nullptr, uint32_t* deep = nullptr);
+                           unsigned long long* stats, int num_cus, const unsigned long long* nw_dev = nullptr);
 
 }  // namespace sigmo_k

@@ -435,8 +435,7 @@ def main() -> int:
                          "per-kernel times then overlap): 1 / 2 / 3 workers take 1.38 / 1.33 / 1.30 s per pass")
     ap.add_argument("--autotune", action="store_true", help="batched form: pick launch shapes with the autotuner before timing")
     ap.add_argument("--filter-mode", type=int, default=0, choices=(0, 1, 2),
-                    help="configs 1-2, batched form: pair evaluation by molecule (1) or from the pre-tested pair list (2); "
-                         "0 (default): the library's choice (list mode below 256 query graphs)")
+                    help="accepted, without effect (the batched form's pair evaluation has one form)")
     ap.add_argument("--graph", action="store_true",
                     help="configs 1-2: capture one whole step (the same kernel launches and work; the batched form's "
                          "includes the database refresh) as a hipGraph and time its replays; per-kernel figures then "

@@ -320,13 +320,11 @@ typedef struct sigmo_batch_result {
 } sigmo_batch_result;
 /* Launch shape of the batched form's persistent kernels; 0 fields keep the built-in choice. */
 typedef struct sigmo_batch_tuning {
-  uint32_t filter_blocks_per_cu; /* pair evaluation: 4-wavefront blocks per CU (capped by residency); 0: all that stay resident (<= 8) */
-  uint32_t filter_claim;         /* molecule mode: molecules a wavefront claims at a time (0: ~count / (4 x wavefronts), 1..64);
-                                    list mode: 64-pair groups a wavefront claims at a time (0: 2) */
+  uint32_t filter_blocks_per_cu; /* pair evaluation: 8-wavefront blocks per CU (capped by residency); 0: all that stay resident */
+  uint32_t filter_claim;         /* 0..64: accepted, without effect (the pair evaluation has one form, which takes its work by groups) */
   uint32_t join_blocks_per_cu;   /* lane join: quarters of the wavefronts its LDS keeps resident (1..4); 0: 4 */
-  uint32_t join_chunk;           /* GMCR pairs per claim of the lane join; 0: ~P / (16 x wavefronts), 64..1024 */
-  uint32_t filter_mode;          /* pair evaluation: 1 molecule by molecule from LDS-staged planes, 2 pair by pair from the
-                                    pre-tested pair list; 0: list mode below 256 query graphs */
+  uint32_t join_chunk;           /* GMCR pairs per claim of the lane join; 0: ~P / (4 x wavefronts), 64..1024 */
+  uint32_t filter_mode;          /* 0..2: accepted, without effect (as filter_claim) */
 } sigmo_batch_tuning;
 int sigmo_db_prepare(sigmo_ctx* ctx, const sigmo_graph* data, uint32_t refinement_steps, sigmo_db** out);
 /* Recompute the level planes from the data graph's current device contents (same result as a

@@ -36,7 +36,6 @@ namespace sigmo_k {
 namespace {
 
 constexpr uint32_t kMaxLevels = 8;        // token encoding keeps 3 bits of level
-constexpr uint32_t kNoWide = 0xFFFFFFFFu;
 constexpr uint16_t kEndToken = 0xFFFF;    // closes a query node's token segment
 
 // Tokens of one query node: [label] [requirement]* [end], requirement = r | l << 3 | c << 7
@@ -90,9 +89,9 @@ __device__ __forceinline__ uint64_t wave_nib_max(uint64_t x) {
 }
 
 
-// Per-molecule facts the pair pre-test reads, stored in width-class order.
-struct MolInfo {
-  uint32_t m, s, n, x, wi, mlab;  // molecule, first node, nodes, plane index, wide index, labels < 16 present
+// Per-molecule facts the pair filter reads, stored in width-class order.
+struct alignas(16) MolInfo {
+  uint32_t m, s, n, mlab;  // molecule, first node, nodes, labels < 16 present
 };
 
 // Per-query-graph facts the pair pre-test reads.
@@ -154,18 +153,31 @@ __global__ __launch_bounds__(256) void k_db_order_keys(uint32_t G, const uint32_
   keys[m] = (cls << 23) | (labels << 7) | ((n - 1) & 127u);
 }
 
-// Level planes, bit p = bit i of the level-(r+1) signature of position p for plane i =
-// 4*label + bit, go to one of two arrays by the molecule's width class: planes32[(x*R + r)*64
-// + i] (u32) for molecules of <= 32 nodes, planes64[(x*R + r)*64 + i] (u64) otherwise, x =
-// pidx[m]; planes_hi holds positions 64..127 and lab_hi[w*16+l] the positions 64..127 with
-// label l (w = wide_idx[m]; positions 0..63 use the graph's label masks).  Wavefront c handles
-// molecule m = cls_list[c] (width-class order, grouped by k_db_order_keys) and writes minfo[c], dmax[c*R + r], the
-// nibble-wise max of the level-(r+1) signatures over the molecule's positions, and
-// cmax[(k*R + r)*G + c], the same max over the positions labelled cl.l[k] (0 if none).
-__global__ __launch_bounds__(256) void k_db_prepare(GraphDev g, uint32_t R, const uint32_t* __restrict__ cls_list,
-                                                    const uint32_t* __restrict__ pidx, const uint32_t* __restrict__ wide_idx,
-                                                    uint32_t* __restrict__ planes32, uint64_t* __restrict__ planes64,
-                                                    uint64_t* __restrict__ planes_hi, uint64_t* __restrict__ lab_hi,
+// The level planes are laid out for 64-lane groups of the width-class order.  A lane holds 32
+// positions of a molecule: molecules of <= 32 nodes take one lane, of 33..64 two, wider ones four,
+// so a group is 64, 32 or 16 neighbours of one class (the last group of a class may be short).
+// planes[((group*R + r)*16 + l)*64 + lane] is the four plane words (bits 0..3 of the count of label
+// l at level r+1) of the lane's positions, labs[(group*16 + l)*64 + lane] its positions labelled l:
+// a group's words of one level and label are one coalesced kilobyte.
+struct GroupOrder {
+  uint32_t count[3];  // molecules of <= 32, 33..64 and 65..128 nodes, one class after another
+  __host__ __device__ uint32_t groups(int cls) const { return (count[cls] + (64u >> cls) - 1) / (64u >> cls); }
+  __host__ __device__ uint32_t total() const { return groups(0) + groups(1) + groups(2); }
+};
+// Group and first lane of the `at`-th molecule of a class.
+__device__ __forceinline__ void group_place(const GroupOrder& o, int cls, uint32_t at, uint64_t& group, uint32_t& lane0) {
+  const uint32_t per = 64u >> cls;
+  group = at / per + (cls > 0 ? o.groups(0) : 0u) + (cls > 1 ? o.groups(1) : 0u);
+  lane0 = (at % per) << cls;
+}
+
+// One wavefront per molecule of more than 32 nodes (width-class entries c0 and up), lane p =
+// position p (and p+64 for molecules of 65..128 nodes): writes the molecule's planes and label
+// masks, minfo[c], dmax[c*R + r], the nibble-wise max of the level-(r+1) signatures over the
+// molecule's positions, and cmax[(k*R + r)*G + c], the same max over the positions labelled
+// cl.l[k] (0 if none).
+__global__ __launch_bounds__(256) void k_db_prepare(GraphDev g, uint32_t R, const uint32_t* __restrict__ cls_list, GroupOrder order,
+                                                    uint32_t* __restrict__ planes, uint32_t* __restrict__ labs,
                                                     uint64_t* __restrict__ dmax, MolInfo* __restrict__ minfo, ClassLabels cl,
                                                     uint64_t* __restrict__ cmax, uint32_t c0) {
   __shared__ uint64_t fold_all[4][kWave];
@@ -174,6 +186,10 @@ __global__ __launch_bounds__(256) void k_db_prepare(GraphDev g, uint32_t R, cons
   if (c >= g.G) return;  // wave-uniform
   const uint64_t m = cls_list[c];
   const uint32_t s = g.go[m], n = g.go[m + 1] - s;
+  const int cls = c < static_cast<uint64_t>(order.count[0]) + order.count[1] ? 1 : 2;
+  uint64_t group;
+  uint32_t lane0;
+  group_place(order, cls, static_cast<uint32_t>(c - order.count[0] - (cls > 1 ? order.count[1] : 0u)), group, lane0);
   const uint64_t* lm = g.lmask + m * 16;
   // the label masks of positions 0..63 and the labels that occur there (wave-uniform): the
   // histogram only visits those labels
@@ -184,16 +200,13 @@ __global__ __launch_bounds__(256) void k_db_prepare(GraphDev g, uint32_t R, cons
     lmv[l] = lm[l];
     if (lmv[l]) present |= 1u << l;
   }
-  const uint32_t halves = n > 64 ? 2 : 1;
-  const uint64_t x = pidx[m];
-  const uint32_t wi = wide_idx[m];
   // Only positions 0..63 are ever expanded (frontier bit b expands node s + b), each by its
   // neighbours folded mod 64: stage those 64 words in LDS once.
   uint64_t* fold = fold_all[threadIdx.x / kWave];
   fold[lane] = lane < n ? g.fold[static_cast<uint64_t>(s) + lane] : 0ull;
   wave_sync();
   uint32_t labels = 0;
-  for (uint32_t h = 0; h < halves; ++h) {
+  for (uint32_t h = 0; h < static_cast<uint32_t>(cls); ++h) {
     const uint32_t pos = lane + 64 * h;
     const bool valid = pos < n;
     const uint32_t mylab = valid ? g.nl[s + pos] : 0x100u;
@@ -218,28 +231,29 @@ __global__ __launch_bounds__(256) void k_db_prepare(GraphDev g, uint32_t R, cons
             sig |= static_cast<uint64_t>(cnt) << (4 * l);
           }
       }
-      const uint64_t col = transpose64(sig);
-      if (h == 1) planes_hi[(static_cast<uint64_t>(wi) * R + r) * 64 + lane] = col;
-      else if (n <= 32) planes32[(x * R + r) * 64 + lane] = static_cast<uint32_t>(col);
-      else planes64[(x * R + r) * 64 + lane] = col;
+      const uint64_t col = transpose64(sig);  // lane i: plane i = 4*label + bit over the 64 positions
+      uint32_t* dst = planes + ((((group * R + r) * 16 + (lane >> 2)) * 64 + lane0 + 2 * h) * 4 + (lane & 3u));
+      dst[0] = static_cast<uint32_t>(col);
+      dst[4] = static_cast<uint32_t>(col >> 32);
       const uint64_t mx = planes_nib_max(col);
       if (lane == 0) dmax[c * R + r] = h == 0 ? mx : nib_max(dmax[c * R + r], mx);
 #pragma unroll
       for (uint32_t k = 0; k < kClasses; ++k) {
         const uint64_t cm = planes_nib_max(col & cpos[k]);
-        uint64_t* dst = cmax + (static_cast<uint64_t>(k) * R + r) * g.G + c;
-        if (lane == 0) *dst = h == 0 ? cm : nib_max(*dst, cm);
+        uint64_t* cd = cmax + (static_cast<uint64_t>(k) * R + r) * g.G + c;
+        if (lane == 0) *cd = h == 0 ? cm : nib_max(*cd, cm);
       }
     }
-    if (h == 1) {
-      const uint32_t lab = valid ? g.nl[s + pos] : 0xFFu;
-      uint64_t mine = 0;
+    uint64_t mine = 0;
 #pragma unroll
-      for (int l = 0; l < 16; ++l) {
-        const uint64_t b = __ballot(lab == static_cast<uint32_t>(l));
-        if (lane == static_cast<uint32_t>(l)) mine = b;
-      }
-      if (lane < 16) lab_hi[static_cast<uint64_t>(wi) * 16 + lane] = mine;
+    for (int l = 0; l < 16; ++l) {
+      const uint64_t b = __ballot(mylab == static_cast<uint32_t>(l));
+      if (lane == static_cast<uint32_t>(l)) mine = b;
+    }
+    if (lane < 16) {
+      uint32_t* dst = labs + (group * 16 + lane) * 64 + lane0 + 2 * h;
+      dst[0] = static_cast<uint32_t>(mine);
+      dst[1] = static_cast<uint32_t>(mine >> 32);
     }
   }
 #pragma unroll
@@ -249,8 +263,6 @@ __global__ __launch_bounds__(256) void k_db_prepare(GraphDev g, uint32_t R, cons
     info.m = static_cast<uint32_t>(m);
     info.s = s;
     info.n = n;
-    info.x = static_cast<uint32_t>(x);
-    info.wi = wi;
     info.mlab = labels;
     minfo[c] = info;
   }
@@ -291,7 +303,7 @@ __device__ __forceinline__ void planes_nib_max2(uint64_t col, uint64_t& lo, uint
 // its own molecule's positions; one 64 x 64 transpose gives both molecules' level planes (low and
 // high 32 bits of each plane word), so the transposes, and the lanes, serve two molecules.
 __global__ __launch_bounds__(256) void k_db_prepare_pairs(GraphDev g, uint32_t R, uint32_t count, const uint32_t* __restrict__ cls_list,
-                                                          const uint32_t* __restrict__ pidx, uint32_t* __restrict__ planes32,
+                                                          uint32_t* __restrict__ planes, uint32_t* __restrict__ labs,
                                                           uint64_t* __restrict__ dmax, MolInfo* __restrict__ minfo, ClassLabels cl,
                                                           uint64_t* __restrict__ cmax) {
   __shared__ uint64_t fold_all[4][kWave];
@@ -325,7 +337,8 @@ __global__ __launch_bounds__(256) void k_db_prepare_pairs(GraphDev g, uint32_t R
   uint64_t cpos[kClasses];
 #pragma unroll
   for (uint32_t k = 0; k < kClasses; ++k) cpos[k] = __ballot(mylab == cl.l[k]);
-  const uint64_t xA = pidx[cls_list[cA]], xB = hasB ? pidx[cls_list[cB]] : 0;
+  const uint64_t group = cA / 64;  // both molecules, on neighbouring lanes
+  const uint32_t lane0 = static_cast<uint32_t>(cA % 64);
   uint64_t self = 1ull << p, ball = self, frontier = self;
   for (uint32_t r = 0; r < R; ++r) {
     uint64_t sig = 0;
@@ -344,8 +357,9 @@ __global__ __launch_bounds__(256) void k_db_prepare_pairs(GraphDev g, uint32_t R
         }
     }
     const uint64_t col = transpose64(sig);
-    planes32[(xA * R + r) * 64 + lane] = static_cast<uint32_t>(col);
-    if (hasB) planes32[(xB * R + r) * 64 + lane] = static_cast<uint32_t>(col >> 32);
+    uint32_t* dst = planes + ((((group * R + r) * 16 + (lane >> 2)) * 64 + lane0) * 4 + (lane & 3u));
+    dst[0] = static_cast<uint32_t>(col);
+    if (hasB) dst[4] = static_cast<uint32_t>(col >> 32);
     uint64_t ma, mb;
     planes_nib_max2(col, ma, mb);
     if (lane == 0) dmax[cA * R + r] = ma;
@@ -357,6 +371,17 @@ __global__ __launch_bounds__(256) void k_db_prepare_pairs(GraphDev g, uint32_t R
       if (lane == 1 && hasB) cmax[(static_cast<uint64_t>(k) * R + r) * g.G + cB] = mb;
     }
   }
+  uint64_t mine = 0;
+#pragma unroll
+  for (int l = 0; l < 16; ++l) {
+    const uint64_t b = __ballot(mylab == static_cast<uint32_t>(l));
+    if (lane == static_cast<uint32_t>(l)) mine = b;
+  }
+  if (lane < 16) {
+    uint32_t* dst = labs + (group * 16 + lane) * 64 + lane0;
+    dst[0] = static_cast<uint32_t>(mine);
+    if (hasB) dst[1] = static_cast<uint32_t>(mine >> 32);
+  }
 #pragma unroll
   for (int o = 16; o > 0; o >>= 1) labels |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(labels), o));  // within each half
   if (p == 0 && live) {
@@ -364,8 +389,6 @@ __global__ __launch_bounds__(256) void k_db_prepare_pairs(GraphDev g, uint32_t R
     info.m = static_cast<uint32_t>(m);
     info.s = s;
     info.n = n;
-    info.x = static_cast<uint32_t>(half ? xB : xA);
-    info.wi = kNoWide;
     info.mlab = labels;
     minfo[c] = info;
   }
@@ -532,7 +555,6 @@ struct PretestArgs {
   const uint64_t* qmax;          // [g * R + r]
   const uint64_t* qcmax;         // [(g * 3 + k) * R + r]
   unsigned long long* surv;      // [m * W + w] out: bit g of word w = pair (g, m) passes
-  uint32_t* pcnt;                // [c] out: passing pairs of the molecule
 };
 
 // Nibble-wise a <= b for the 16 four-bit fields of several words, bit-sliced: bit b of every
@@ -597,7 +619,6 @@ __global__ __launch_bounds__(256) void k_pair_pretest(PretestArgs a) {
       for (uint32_t b = 0; b < 4; ++b) mc[k][r / 4][b] |= nib_plane(x, b, r % 4);
     }
   }
-  uint32_t cnt = 0;
   for (uint32_t w = 0; w < a.W; ++w) {
     __syncthreads();  // the previous tile has been read
     for (uint32_t t = threadIdx.x; t < kWave * S; t += 256) {
@@ -643,33 +664,6 @@ __global__ __launch_bounds__(256) void k_pair_pretest(PretestArgs a) {
       word |= static_cast<uint64_t>(fits) << j;
     }
     if (valid) a.surv[static_cast<uint64_t>(m) * a.W + w] = word;
-    cnt += static_cast<uint32_t>(__popcll(word));
-  }
-  if (valid) a.pcnt[c] = cnt;
-}
-
-// The pre-tested pairs listed in (width-class order, query graph) order: entry = c | g << 32,
-// molecule c's pairs from poff[c] (the exclusive scan of pcnt).  Entries past `cap` are not
-// written; a list longer than `cap` sets the overflow flag (counters[3]) and the host repeats the
-// run with the demand (the scan's total, counters[7]).
-__global__ __launch_bounds__(256) void k_pair_expand(uint32_t G, uint32_t W, const MolInfo* __restrict__ minfo,
-                                                     const unsigned long long* __restrict__ surv, const uint32_t* __restrict__ poff,
-                                                     uint64_t* __restrict__ list, uint64_t cap, unsigned long long* __restrict__ counters) {
-  const uint64_t c = blockIdx.x * 256ull + threadIdx.x;
-  if (c == 0 && counters[7] > cap) atomicOr(&counters[3], 1ull);
-  if (c >= G) return;
-  uint64_t pos = poff[c];
-  const uint64_t end = poff[c + 1];
-  if (pos == end) return;
-  const uint64_t m = minfo[c].m;
-  for (uint32_t w = 0; w < W && pos < end; ++w) {
-    uint64_t x = surv[m * W + w];
-    while (x) {
-      const uint32_t g = w * kWave + static_cast<uint32_t>(__builtin_ctzll(x));
-      x &= x - 1;
-      if (pos < cap) list[pos] = c | (static_cast<uint64_t>(g) << 32);
-      ++pos;
-    }
   }
 }
 
@@ -679,579 +673,299 @@ __global__ __launch_bounds__(256) void k_pair_expand(uint32_t G, uint32_t W, con
 // rounded up to a whole 32-byte group.
 __host__ __device__ __forceinline__ uint32_t pair_words(uint32_t k, uint32_t stride) { return (k * stride + 3) & ~3u; }
 
-constexpr uint32_t kSurviveWaves = 4;     // wavefronts per block
-constexpr uint32_t kLaneChunk = 64;       // arena words a lane owns at a time (>= the largest pair, 2 x 32)
-constexpr uint32_t kWaveChunk = 64 * kLaneChunk;
+constexpr uint32_t kGroupWaves = 8;       // wavefronts per block of the pair evaluation
+constexpr uint32_t kGroupStatSlots = 32;  // one address would take every wavefront's sums one after another (~10 ns each)
 
-// Candidate masks of one width class: NW = 1 (<= 32 positions, u32), 2 (<= 64, u64) or
-// 4 (<= 128, two u64 words).
-template <int NW>
-struct Mask {
-  using T = typename std::conditional<NW == 1, uint32_t, uint64_t>::type;
-  T lo = 0;
-  uint64_t hi = 0;  // NW == 4 only
-  __device__ __forceinline__ bool any() const { return NW == 4 ? ((static_cast<uint64_t>(lo) | hi) != 0) : (lo != 0); }
-};
-
-// One lane's walk over a pair's token words.
-template <int NW>
-struct PairWalk {
-  Mask<NW> mask;
-  uint64_t tw = 0;        // the current token word
-  uint64_t nodebase = 0;  // token index of the current node's stream
-  uint64_t base = 0;      // the pair's first arena word
-  uint32_t i = 0, k = 0, tp = 0;  // current node, nodes, token offset within the node's stream
-  // node masks are held four words at a time and stored as one aligned 32-byte group (pair
-  // blocks start on a 4-word boundary and take a multiple of 4 words): whole sectors go out
-  // together, and a pair that dies never stores its open group
-  uint64_t buf[4] = {0, 0, 0, 0};
-};
-
-enum : int { kWalkOn = 0, kWalkDied = 1, kWalkSurvived = 2 };
-
-// One token word of a pair: a node's label token sets its mask to the filter's label test
-// (isomorphism.hpp:49), each requirement token ANDs one bit-sliced refine test
-// (isomorphism.hpp:103-110), and the end token stores the node's mask.  The pair dies at the
-// first node without candidates (the GMCR predicate, gmcr.hpp:56-61) and survives when its last
-// node ends.  `P` gives the four plane words of (level r, label l) and the position masks of a
-// label; `ns()` gives the molecule's node count and first node (read only for labels >= 16).  All
-// four tokens' plane reads and the next word's load are issued together; requirements of a node
-// commute, so their order within the word is free.
-template <int NW, class Planes, class NS>
-__device__ __forceinline__ int walk_step(const Planes& P, NS ns, const uint8_t* __restrict__ nl, const uint64_t* __restrict__ tok64,
-                                         uint32_t R, PairWalk<NW>& w, uint64_t* __restrict__ arena, uint64_t arena_cap) {
-  using T = typename Mask<NW>::T;
-  constexpr uint32_t stride = NW == 4 ? 2u : 1u;
-  uint32_t tok[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) tok[j] = static_cast<uint32_t>(w.tw >> (16 * j)) & 0xFFFFu;
-  const uint32_t e = tok[0] == kEndToken ? 0u : tok[1] == kEndToken ? 1u : tok[2] == kEndToken ? 2u : tok[3] == kEndToken ? 3u : 4u;
-  const bool last = e < 4 && w.i + 1 == w.k;  // the pair's last node ends in this word
-  uint64_t tw_next = 0;
-  if (!last) tw_next = tok64[(w.nodebase + w.tp + 4) / 4];  // this node's next word, or the next node's first
-  uint64_t pv[4][4], ph[4][4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) P.load(min(tok[j] & 7u, R - 1), (tok[j] >> 3) & 15u, pv[j], ph[j]);  // clamped, masked below
-  const uint32_t ql = tok[0];
-  if (w.tp == 0) {  // the node's label token: the filter's label test (isomorphism.hpp:49)
-    if (ql < 16u) {
-      uint64_t lo = 0, hi = 0;
-      P.lab(ql, lo, hi);
-      w.mask.lo = static_cast<T>(lo);
-      if (NW == 4) w.mask.hi = hi;
-    } else {
-      const uint2 mns = ns();  // (n, s)
-      if (ql == 255u) {
-        w.mask.lo = static_cast<T>(mns.x >= 64 ? ~0ull : ((1ull << mns.x) - 1));
-        if (NW == 4) w.mask.hi = mns.x >= 128 ? ~0ull : ((1ull << (mns.x - 64)) - 1);
-      } else {
-        uint64_t l0 = 0, l1 = 0;
-        for (uint32_t p = 0; p < mns.x; ++p)
-          if (nl[mns.y + p] == ql) {
-            if (p < 64) l0 |= 1ull << p;
-            else l1 |= 1ull << (p - 64);
-          }
-        w.mask.lo = static_cast<T>(l0);
-        if (NW == 4) w.mask.hi = l1;
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {  // count_q(l) <= count_p(l) at level r (isomorphism.hpp:103-110)
-    const bool req = static_cast<uint32_t>(j) < e && (w.tp != 0 || j != 0);
-    const uint32_t c = req ? (tok[j] >> 7) & 15u : 0u;  // c = 0: always true
-    w.mask.lo &= static_cast<T>(ge4_bits<T>(static_cast<T>(pv[j][0]), static_cast<T>(pv[j][1]), static_cast<T>(pv[j][2]),
-                                            static_cast<T>(pv[j][3]), c));
-    if (NW == 4) w.mask.hi &= ge4_bits<uint64_t>(ph[j][0], ph[j][1], ph[j][2], ph[j][3], c);
-  }
-  int out = kWalkOn;
-  if (!w.mask.any()) {
-    out = kWalkDied;
-  } else if (e < 4) {  // node done: its mask joins the register group, stored when full or last
-    const uint32_t wd = w.i * stride;  // the node's first word in the pair's block
-#pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) {
-      if (j == (wd & 3u)) w.buf[j] = static_cast<uint64_t>(w.mask.lo);
-      if (NW == 4 && j == (wd & 3u) + 1) w.buf[j] = w.mask.hi;
-    }
-    if ((wd & 3u) + stride == 4u || w.i + 1 == w.k) {
-      const uint64_t at = w.base + (wd & ~3u);
-      if (at + 4 <= arena_cap) {  // 32-byte aligned: two 16-byte stores
-        uint4* dst = reinterpret_cast<uint4*>(arena + at);
-        dst[0] = make_uint4(static_cast<uint32_t>(w.buf[0]), static_cast<uint32_t>(w.buf[0] >> 32), static_cast<uint32_t>(w.buf[1]),
-                            static_cast<uint32_t>(w.buf[1] >> 32));
-        dst[1] = make_uint4(static_cast<uint32_t>(w.buf[2]), static_cast<uint32_t>(w.buf[2] >> 32), static_cast<uint32_t>(w.buf[3]),
-                            static_cast<uint32_t>(w.buf[3] >> 32));
-      }
-    }
-    ++w.i;
-    if (w.i == w.k) {
-      out = kWalkSurvived;
-    } else {
-      w.nodebase += w.tp + 4;  // the next node's stream starts at the next word
-      w.tp = 0;
-    }
-  } else {
-    w.tp += 4;
-  }
-  w.tw = tw_next;
-  return out;
-}
-
-// A lane's arena sub-chunk and its wavefront's chunk: lanes whose sub-chunk cannot hold a new
-// pair of `need` words get a fresh one from the wavefront's chunk, which claims kWaveChunk words
-// of the arena at a time (setting the overflow flag, counters[3], past the arena's end).
-struct ArenaCursor {
-  uint64_t wc_next = 0, wc_end = 0;  // the wavefront's chunk (wave-uniform)
-  uint64_t lc_next = 0, lc_end = 0;  // the lane's sub-chunk
-  __device__ __forceinline__ void reserve(bool take, uint32_t need, uint64_t below, unsigned long long* counters, uint64_t arena_cap) {
-    const bool fresh = take && lc_next + need > lc_end;
-    const uint64_t fm = __ballot(fresh);
-    if (fm) {
-      const uint32_t nf = __popcll(fm);
-      if (wc_next + static_cast<uint64_t>(nf) * kLaneChunk > wc_end) {
-        unsigned long long b = 0;
-        if (lane_id() == 0) {
-          b = atomicAdd(&counters[1], static_cast<unsigned long long>(kWaveChunk));
-          if (b + kWaveChunk > arena_cap) atomicOr(&counters[3], 1ull);
-        }
-        wc_next = uniform64(__shfl(b, 0));
-        wc_end = wc_next + kWaveChunk;
-      }
-      if (fresh) {
-        lc_next = wc_next + static_cast<uint64_t>(__popcll(fm & below)) * kLaneChunk;
-        lc_end = lc_next + kLaneChunk;
-      }
-      wc_next += static_cast<uint64_t>(nf) * kLaneChunk;
-    }
-  }
-};
-
-// A pre-tested (query graph, molecule) pair waiting for a lane.
-struct PairEntry {
-  uint32_t slot, qg, qoff, k;
-  uint64_t tw;  // first token word of the pair's first query node
-};
-
-struct SurviveArgs {
-  GraphDev q, d;
-  uint32_t R, Gq, W;       // W: survival-bitmask words per molecule
-  uint32_t count;          // molecules of the width class
-  uint32_t claim;          // molecules a wavefront claims at a time
-  const MolInfo* minfo;    // the width class's molecules, ascending
-  const uint32_t* pcnt;    // the width class's pre-tested pair counts
-  const uint32_t* planes32;
-  const uint64_t* planes64;
-  const uint64_t* planes_hi;
-  const uint64_t* lab_hi;
-  const uint64_t* tok64;   // token segments as 64-bit words
+struct GroupArgs {
+  GraphDev d;
+  GroupOrder order;
+  uint32_t R, Gq, W;
+  uint32_t parts;          // blocks that share a group's query graphs (a power of two, <= 64 / kGroupWaves)
+  uint32_t slots;          // labels whose planes LDS holds
+  uint32_t chunk;          // arena words a wavefront claims at a time
+  const MolInfo* minfo;    // width-class order
+  const uint4* planes;     // [((group*R + r)*16 + l)*64 + lane]
+  const uint32_t* labs;    // [(group*16 + l)*64 + lane]
+  const uint16_t* tokens;
   const QueryInfo* qinfo;
-  uint64_t* arena;         // survivor masks: k words (2k, interleaved, for molecules of > 64 nodes)
+  uint64_t* arena;
   uint64_t arena_cap;
   unsigned long long* surv;      // [Gd][W] in: the pre-test's pairs; out: bit qg of row m = the pair survives GMCR
   uint32_t* pair_off;            // [Gd * Gq] arena offset of each surviving pair
-  unsigned long long* counters;  // [0] molecule cursor, [1] arena top, [3] overflow, [4..5] statistics
+  unsigned long long* counters;  // [1] arena words claimed past the wavefronts' first chunks, [2] item cursor, [3] overflow
+  unsigned long long* stats;     // kGroupStatSlots x 16: [0] node evaluations, [1] their live lanes, [2] pre-tested pairs
 };
 
-// Molecule slots per wavefront and LDS words (u64) per slot, by width class.
-__host__ __device__ constexpr uint32_t ring_slots(int nw) { return nw == 1 ? 4u : (nw == 2 ? 3u : 2u); }
-__host__ __device__ constexpr uint32_t slot_words(uint32_t R, int nw) {
-  return nw == 1 ? R * 32 + 8 : (nw == 2 ? R * 64 + 16 : 2 * R * 64 + 32);
+// LDS: planes [label slot][level][lane] (16 bytes), label masks [label slot][lane], the next item.
+__host__ __device__ constexpr uint32_t group_lds_bytes(uint32_t slots, uint32_t R) { return slots * (R * 1024 + 256) + 16; }
+
+// The value of lane ^ 1 and lane ^ 2 (quad permutations).
+__device__ __forceinline__ uint32_t quad_xor1(uint32_t x) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0xB1, 0xF, 0xF, false));
 }
-__host__ __device__ constexpr uint32_t plist_words() { return kWave * sizeof(PairEntry) / 8; }
-__host__ __device__ constexpr uint32_t survive_lds_bytes(uint32_t R, int nw) {
-  return kSurviveWaves * (ring_slots(nw) * slot_words(R, nw) + plist_words()) * 8;
+__device__ __forceinline__ uint32_t quad_xor2(uint32_t x) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x4E, 0xF, 0xF, false));
 }
 
-// The plane words of a molecule staged in an LDS slot (layout of k_pair_survive).
-template <int NW>
-struct SlotPlanes {
-  const uint64_t* slot;
-  uint32_t R;
-  __device__ __forceinline__ void load(uint32_t r, uint32_t l, uint64_t pv[4], uint64_t ph[4]) const {
-    if (NW == 1) {
-      const uint4 v = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint32_t*>(slot) + r * 64 + l * 4);
-      pv[0] = v.x;
-      pv[1] = v.y;
-      pv[2] = v.z;
-      pv[3] = v.w;
-    } else {
-#pragma unroll
-      for (int b = 0; b < 4; ++b) pv[b] = slot[r * 64 + l * 4 + b];
-      if (NW == 4) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) ph[b] = slot[R * 64 + r * 64 + l * 4 + b];
-      }
-    }
-  }
-  __device__ __forceinline__ void lab(uint32_t l, uint64_t& lo, uint64_t& hi) const {
-    const uint32_t lm_at = NW == 1 ? 2 * R * 32 : (NW == 4 ? 2 * R * 64 : R * 64);  // u32 index for NW == 1
-    lo = NW == 1 ? reinterpret_cast<const uint32_t*>(slot)[lm_at + l] : slot[lm_at + l];
-    hi = NW == 4 ? slot[lm_at + 16 + l] : 0ull;
-  }
+// A wavefront's arena chunk and statistics (wave-uniform but `live`).
+struct GroupState {
+  uint64_t next, end, first_chunks;
+  uint64_t nodes = 0, scans = 0;
+  uint32_t live = 0;  // per lane
 };
 
-// The plane words of a molecule read from the database in device memory.
-template <int NW>
-struct GlobalPlanes {
-  const uint32_t* p32;  // the molecule's planes (NW == 1)
-  const uint64_t* p64;  // the molecule's planes (NW >= 2)
-  const uint64_t* phi;  // positions 64..127 (NW == 4)
-  const uint64_t* lm;   // label masks of positions 0..63
-  const uint64_t* lmh;  // label masks of positions 64..127 (NW == 4)
-  __device__ __forceinline__ void load(uint32_t r, uint32_t l, uint64_t pv[4], uint64_t ph[4]) const {
-    if (NW == 1) {
-      const uint4 v = *reinterpret_cast<const uint4*>(p32 + r * 64 + l * 4);
-      pv[0] = v.x;
-      pv[1] = v.y;
-      pv[2] = v.z;
-      pv[3] = v.w;
-    } else {
-      const uint4* s = reinterpret_cast<const uint4*>(p64 + r * 64 + l * 4);
-      const uint4 v0 = s[0], v1 = s[1];
-      pv[0] = v0.x | (static_cast<uint64_t>(v0.y) << 32);
-      pv[1] = v0.z | (static_cast<uint64_t>(v0.w) << 32);
-      pv[2] = v1.x | (static_cast<uint64_t>(v1.y) << 32);
-      pv[3] = v1.z | (static_cast<uint64_t>(v1.w) << 32);
-      if (NW == 4) {
-        const uint4* t = reinterpret_cast<const uint4*>(phi + r * 64 + l * 4);
-        const uint4 u0 = t[0], u1 = t[1];
-        ph[0] = u0.x | (static_cast<uint64_t>(u0.y) << 32);
-        ph[1] = u0.z | (static_cast<uint64_t>(u0.w) << 32);
-        ph[2] = u1.x | (static_cast<uint64_t>(u1.y) << 32);
-        ph[3] = u1.z | (static_cast<uint64_t>(u1.w) << 32);
-      }
-    }
-  }
-  __device__ __forceinline__ void lab(uint32_t l, uint64_t& lo, uint64_t& hi) const {
-    lo = lm[l];
-    hi = NW == 4 ? lmh[l] : 0ull;
-  }
-};
+// One requirement on 32 positions (isomorphism.hpp:103-110), count_q(l) <= count_p(l) at level r:
+// the decoded token is a scalar, so the count's bit masks (bits 20..23) are too.
+__device__ __forceinline__ uint32_t group_test(uint32_t tk, const uint4& v) {
+  uint32_t ge = ge_first(v.x, static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(tk), 20, 1)));
+  ge = ge_stage(v.y, static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(tk), 21, 1)), ge);
+  ge = ge_stage(v.z, static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(tk), 22, 1)), ge);
+  return ge_stage(v.w, static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(tk), 23, 1)), ge);
+}
 
-// Persistent pair evaluation of one width class, molecule by molecule.  Each wavefront keeps a
-// ring of molecule slots in LDS -- the molecule's level planes and label masks, staged with
-// coalesced loads when the wavefront claims it (molecules with no pre-tested pair are skipped) --
-// and lists the open molecule's pre-tested pairs, 64 query graphs at a time, in an LDS list from
-// which idle lanes take pairs of any slot.  A slot is reused once its molecule's list is done and
-// none of its pairs is pending.  Each lane owns an arena sub-chunk: node masks go straight to the
-// pair's final place, and a pair that dies leaves its space to the lane's next pair (and clears
-// its pre-test bit).  Suited to many pairs per molecule (large query batches).
-template <int NW>
-__global__ __launch_bounds__(256) void k_pair_survive(SurviveArgs a) {
-  constexpr uint32_t stride = NW == 4 ? 2u : 1u;
-  constexpr uint32_t S = ring_slots(NW);
-  extern __shared__ uint64_t lds[];
+// One group of a class against the wavefront's share of the query graphs.
+template <int CLS>
+__device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uint32_t part, uint32_t wave, uint4* planes_lds, uint32_t* labs_lds,
+                                           uint32_t off_mask, GroupState& st) {
   const uint32_t lane = static_cast<uint32_t>(lane_id());
-  const uint32_t wave = threadIdx.x / kWave;
-  const uint32_t R = a.R, Gq = a.Gq;
-  const uint32_t sw = slot_words(R, NW);
-  uint64_t* ring = lds + static_cast<uint64_t>(wave) * (S * sw + plist_words());
-  PairEntry* plist = reinterpret_cast<PairEntry*>(ring + S * sw);
+  const uint32_t R = a.R;
   const uint32_t seg = token_segment(R);
-  const uint64_t below = (1ull << lane) - 1;
-
-  // wave-uniform state
-  ArenaCursor ac;
-  uint32_t lhead = 0, lcount = 0;             // pending list entries [lhead, lcount)
-  uint32_t pending[S];                        // listed pairs of the slot's molecule not yet finished
-  MolInfo smol[S];                            // the slot's molecule
-  uint32_t open = S, scan_qg = 0;             // slot being listed (S: none) and its next query graph
-  // With at most 64 bitmask words per molecule the open molecule's words sit in registers (lane i:
-  // word i, listed bits cleared), loaded with one coalesced load when it is opened.
-  const bool reg_words = a.W <= kWave;
-  uint64_t mw = 0;
-  uint32_t om = 0;                            // the open molecule
-  bool exhausted = false;
-  uint64_t mc_next = 0, mc_end = 0;           // claimed molecules [mc_next, mc_end)
+  const uint32_t first = (CLS > 0 ? a.order.count[0] : 0u) + (CLS > 1 ? a.order.count[1] : 0u);
+  const uint64_t group = grp + (CLS > 0 ? a.order.groups(0) : 0u) + (CLS > 1 ? a.order.groups(1) : 0u);
+  const uint32_t at = grp * (64u >> CLS) + (lane >> CLS);  // the lane's molecule within its class
+  const uint32_t h = lane & ((1u << CLS) - 1u);            // its 32 positions within the molecule
+  const bool valid = at < a.order.count[CLS];
+  MolInfo mi = {};
+  if (valid) mi = a.minfo[first + at];
+  constexpr uint64_t leaders = CLS == 0 ? ~0ull : (CLS == 1 ? 0x5555555555555555ull : 0x1111111111111111ull);
+  const uint64_t below = (1ull << (lane & ~((1u << CLS) - 1u))) - 1;
+  uint32_t present = 0;  // labels that occur in the group
 #pragma unroll
-  for (uint32_t sl = 0; sl < S; ++sl) pending[sl] = 0;
-  uint64_t wave_steps = 0, lane_steps = 0;    // statistics
+  for (uint32_t l = 0; l < 16; ++l) present |= static_cast<uint32_t>(__ballot((mi.mlab >> l) & 1u) != 0ull) << l;
+  present = uniform32(present);
+  const uint32_t occur = static_cast<uint32_t>(__popc(present)), staged = min(occur, a.slots);
+  auto label_of = [&](uint32_t slot) -> uint32_t {  // the slot-th label that occurs
+    uint32_t left = present;
+    for (uint32_t x = 0; x < slot; ++x) left &= left - 1;
+    return static_cast<uint32_t>(__builtin_ctz(left));
+  };
+  // the wavefronts take every eighth (label, level), four loads in flight each
+  for (uint32_t e0 = wave; e0 < staged * R; e0 += 4 * kGroupWaves) {
+    uint4 v[4];
+#pragma unroll
+    for (uint32_t x = 0; x < 4; ++x) {
+      const uint32_t e = e0 + x * kGroupWaves;
+      v[x] = make_uint4(0, 0, 0, 0);
+      if (e < staged * R && valid) v[x] = a.planes[((group * R + e % R) * 16 + label_of(e / R)) * 64 + lane];
+    }
+#pragma unroll
+    for (uint32_t x = 0; x < 4; ++x) {
+      const uint32_t e = e0 + x * kGroupWaves;
+      if (e < staged * R) planes_lds[e * kWave + lane] = v[x];
+    }
+  }
+  for (uint32_t slot = wave; slot < staged; slot += kGroupWaves)
+    labs_lds[slot * kWave + lane] = valid ? a.labs[(group * 16 + label_of(slot)) * 64 + lane] : 0u;
+  __syncthreads();
 
-  // per-lane pair state
-  bool have = false;
-  uint32_t sl_of = 0, qg = 0;
-  PairWalk<NW> pw;
-  while (true) {
-    uint64_t need = __ballot(!have);
-    while (need) {
-      if (lhead < lcount) {  // hand waiting pairs to idle lanes
-        const uint32_t cnt = min(lcount - lhead, static_cast<uint32_t>(__popcll(need)));
-        const uint32_t rn = __popcll(need & below);
-        const bool take = ((need >> lane) & 1ull) && rn < cnt;
-        if (take) {
-          const PairEntry& e = plist[lhead + rn];
-          sl_of = e.slot;
-          qg = e.qg;
-          pw.k = e.k;
-          pw.tw = e.tw;
-          pw.nodebase = static_cast<uint64_t>(e.qoff) * seg;
-          pw.i = 0;
-          pw.tp = 0;
-          have = true;
+  const uint32_t workers = kGroupWaves * a.parts;  // wavefronts that share the query graphs (a power of two <= 64)
+  uint64_t mine = 0;
+  for (uint32_t t = part * kGroupWaves + wave; t < 64; t += workers) mine |= 1ull << t;
+  for (uint32_t w = 0; w < a.W; ++w) {
+    const uint64_t word = valid ? a.surv[static_cast<uint64_t>(mi.m) * a.W + w] : 0ull;
+    uint32_t any_lo = static_cast<uint32_t>(word), any_hi = static_cast<uint32_t>(word >> 32);
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      any_lo |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(any_lo), o));
+      any_hi |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(any_hi), o));
+    }
+    uint64_t dead = 0;
+    for (uint64_t bits = uniform64(any_lo | (static_cast<uint64_t>(any_hi) << 32)) & mine; bits; bits &= bits - 1) {  // wave-uniform
+      const uint32_t jb = static_cast<uint32_t>(__builtin_ctzll(bits));
+      const uint32_t g = w * kWave + jb;
+      const bool act = (word >> jb) & 1ull;
+      const uint64_t am = __ballot(act) & leaders;
+      const uint32_t qoff = uniform32(a.qinfo[g].qoff), k = uniform32(a.qinfo[g].k);
+      const uint32_t cnt = static_cast<uint32_t>(__popcll(am)), pw = pair_words(k, CLS == 2 ? 2u : 1u);
+      st.scans += cnt;
+      if (st.next + static_cast<uint64_t>(cnt) * pw > st.end) {
+        unsigned long long b = 0;
+        if (lane == 0) {
+          b = st.first_chunks + atomicAdd(&a.counters[1], static_cast<unsigned long long>(a.chunk));
+          if (b + a.chunk > a.arena_cap) atomicOr(&a.counters[3], 1ull);
         }
-        wave_sync();
-        lhead += cnt;
-        need &= ~__ballot(take);
-        ac.reserve(take, pair_words(pw.k, stride), below, a.counters, a.arena_cap);
-        if (take) pw.base = ac.lc_next;
-        continue;
+        st.next = uniform64(__shfl(b, 0));
+        st.end = st.next + a.chunk;
       }
-      if (reg_words && open < S && __ballot(mw != 0ull)) {
-        // list the open molecule's next pre-tested pairs: the words from the lowest unlisted one up
-        // whose pairs fit the 64-entry list (the first always does), then each entry's query graph
-        // fields, one load per entry, all in flight together
-        const uint32_t pc = static_cast<uint32_t>(__popcll(mw));
-        uint32_t incl = pc;
-#pragma unroll
-        for (int d = 1; d < kWave; d <<= 1) {
-          const uint32_t y = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), d));
-          if (lane >= static_cast<uint32_t>(d)) incl += y;
-        }
-        const bool sel = pc != 0 && incl <= kWave;
-        const uint64_t selm = __ballot(sel);
-        for (uint64_t f = selm; f; f &= f - 1) {  // wave-uniform
-          const int w = static_cast<int>(__builtin_ctzll(f));
-          const uint64_t x = __shfl(mw, w);
-          const uint32_t at = static_cast<uint32_t>(__shfl(static_cast<int>(incl - pc), w));
-          if ((x >> lane) & 1ull) {
-            PairEntry& e = plist[at + __popcll(x & below)];
-            e.slot = open;
-            e.qg = static_cast<uint32_t>(w) * kWave + lane;
+      const uint64_t base = st.next + static_cast<uint64_t>(__popcll(am & below)) * pw;
+      st.next += static_cast<uint64_t>(cnt) * pw;
+      const bool room = st.end <= a.arena_cap;
+
+      // the graph's tokens, 64 at a time and one per lane, decoded once: a requirement becomes its
+      // planes' byte offset in LDS (bits 10..16) and its count (bits 20..23); `far` is set when a
+      // label's planes are not there
+      const uint16_t* tok = a.tokens + static_cast<uint64_t>(qoff) * seg;
+      const uint32_t total = k * seg;
+      uint32_t pos = 0, p = 0, raw = 0, dec = 0;
+      uint64_t ends = 0;
+      bool far = false;
+      auto load_tokens = [&](uint32_t from) {
+        pos = from;
+        p = 0;
+        raw = tok[min(from + lane, total - 1)];
+        const uint32_t slot = static_cast<uint32_t>(__popc(present & ((1u << ((raw >> 3) & 15u)) - 1u)));
+        dec = (((slot * R + (raw & 7u)) * (kWave * 16)) & 0x1FC00u) | (((raw >> 7) & 15u) << 20);
+        far = staged < occur && __ballot(raw != kEndToken && slot >= staged) != 0;
+        ends = __ballot(raw == kEndToken);
+      };
+      auto planes = [&](uint32_t tk) -> uint4 {
+        return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(planes_lds) + ((tk & off_mask) | (lane * 16)));
+      };
+      // the candidates of the next node among this lane's positions; leaves p at the node after
+      auto node_mask = [&]() -> uint32_t {
+        if (p >= kWave || (ends >> p) == 0) load_tokens(pos + p);  // the node's stream (at most 33 tokens) crosses the 64
+        const uint32_t e = p + static_cast<uint32_t>(__builtin_ctzll(ends >> p));
+        // its label token: the filter's label test (isomorphism.hpp:49)
+        const uint32_t ql = rl32(raw, p);
+        uint32_t mask = 0, t = p + 1;
+        p = (e & ~3u) + 4;
+        if (ql < 16u) {
+          const uint32_t slot = static_cast<uint32_t>(__popc(present & ((1u << ql) - 1u)));
+          if (slot < staged) mask = labs_lds[slot * kWave + lane];
+          else if (valid) mask = a.labs[(group * 16 + ql) * 64 + lane];
+        } else {
+          const uint32_t positions = mi.n > 32 * h ? min(32u, mi.n - 32 * h) : 0u;
+          if (ql == 255u) {
+            mask = positions >= 32 ? ~0u : (1u << positions) - 1u;
+          } else if (act) {
+            for (uint32_t x = 0; x < positions; ++x)
+              if (a.d.nl[static_cast<uint64_t>(mi.s) + 32 * h + x] == ql) mask |= 1u << x;
           }
         }
-        const uint32_t cnt = static_cast<uint32_t>(__shfl(static_cast<int>(incl), 63 - static_cast<int>(__builtin_clzll(selm))));
-        if (sel) mw = 0;
-        wave_sync();
-        if (lane < cnt) {
-          PairEntry& e = plist[lane];
-          const QueryInfo qi = a.qinfo[e.qg];
-          e.qoff = qi.qoff;
-          e.k = qi.k;
-          e.tw = qi.first;
-        }
-        wave_sync();
-        lhead = 0;
-        lcount = cnt;
-#pragma unroll
-        for (uint32_t sl = 0; sl < S; ++sl)
-          if (sl == open) pending[sl] += lcount;
-        continue;
-      }
-      if (!reg_words && open < S && scan_qg < Gq) {  // list the open molecule's pre-tested pairs of the next 64 query graphs
-        const uint64_t word = a.surv[static_cast<uint64_t>(om) * a.W + scan_qg / kWave];
-        const uint32_t g = scan_qg + lane;
-        const bool ok = (word >> lane) & 1ull;
-        if (ok) {
-          const QueryInfo qi = a.qinfo[g];
-          PairEntry& e = plist[__popcll(word & below)];
-          e.slot = open;
-          e.qg = g;
-          e.qoff = qi.qoff;
-          e.k = qi.k;
-          e.tw = qi.first;
-        }
-        wave_sync();
-        lhead = 0;
-        lcount = __popcll(word);
-#pragma unroll
-        for (uint32_t sl = 0; sl < S; ++sl)
-          if (sl == open) pending[sl] += lcount;
-        scan_qg += kWave;
-        continue;
-      }
-      // the open molecule is fully listed: open the next one with pairs in a free slot
-      if (exhausted) break;
-      uint32_t free_slot = S;
-#pragma unroll
-      for (uint32_t sl = 0; sl < S; ++sl)
-        if (free_slot == S && pending[sl] == 0) free_slot = sl;
-      if (free_slot == S) break;  // every slot still has pairs in flight
-      if (mc_next >= mc_end) {  // claim the next few molecules (one atomic per claim)
-        unsigned long long b = 0;
-        if (lane == 0) b = atomicAdd(&a.counters[0], static_cast<unsigned long long>(a.claim));
-        mc_next = uniform64(__shfl(b, 0));
-        mc_end = mc_next + a.claim < a.count ? mc_next + a.claim : a.count;
-      }
-      if (mc_next >= a.count) {
-        exhausted = true;
-        open = S;
-        break;
-      }
-      const uint64_t c = mc_next++;
-      if (a.pcnt[c] == 0) continue;  // nothing passed the pre-test: not staged
-      const MolInfo mi = a.minfo[c];
-      uint64_t* slot = ring + free_slot * sw;
-      if (NW == 1) {
-        const uint64_t* src = reinterpret_cast<const uint64_t*>(a.planes32 + static_cast<uint64_t>(mi.x) * R * 64);
-        for (uint32_t t = lane; t < R * 32; t += kWave) slot[t] = src[t];
-        if (lane < 16) reinterpret_cast<uint32_t*>(slot + R * 32)[lane] = static_cast<uint32_t>(a.d.lmask[static_cast<uint64_t>(mi.m) * 16 + lane]);
-      } else {
-        const uint64_t* src = a.planes64 + static_cast<uint64_t>(mi.x) * R * 64;
-        for (uint32_t t = lane; t < R * 64; t += kWave) slot[t] = src[t];
-        const uint32_t lm_at = NW == 4 ? 2 * R * 64 : R * 64;
-        if (lane < 16) slot[lm_at + lane] = a.d.lmask[static_cast<uint64_t>(mi.m) * 16 + lane];
-        if (NW == 4) {
-          const uint64_t* srch = a.planes_hi + static_cast<uint64_t>(mi.wi) * R * 64;
-          for (uint32_t t = lane; t < R * 64; t += kWave) slot[R * 64 + t] = srch[t];
-          if (lane < 16) slot[lm_at + 16 + lane] = a.lab_hi[static_cast<uint64_t>(mi.wi) * 16 + lane];
-        }
-      }
-      wave_sync();
-#pragma unroll
-      for (uint32_t sl = 0; sl < S; ++sl)
-        if (sl == free_slot) smol[sl] = mi;
-      open = free_slot;
-      om = mi.m;
-      scan_qg = 0;
-      if (reg_words) mw = lane < a.W ? a.surv[static_cast<uint64_t>(om) * a.W + lane] : 0ull;
-    }
-    const uint64_t active = __ballot(have);
-    if (active == 0) break;
-    ++wave_steps;
-    lane_steps += __popcll(active);
-    bool finished = false;
-    if (have) {
-      const SlotPlanes<NW> P{ring + sl_of * sw, R};
-      auto ns = [&]() {
-        MolInfo mi = {};
-#pragma unroll
-        for (uint32_t sl = 0; sl < S; ++sl)
-          if (sl == sl_of) mi = smol[sl];
-        return make_uint2(mi.n, mi.s);
-      };
-      const int st = walk_step<NW>(P, ns, a.d.nl, a.tok64, R, pw, a.arena, a.arena_cap);
-      if (st != kWalkOn) {
-        uint32_t m = 0;
-#pragma unroll
-        for (uint32_t sl = 0; sl < S; ++sl)
-          if (sl == sl_of) m = smol[sl].m;
-        if (st == kWalkSurvived) {  // every query node has a candidate: the pair survives GMCR
-          a.pair_off[static_cast<uint64_t>(m) * Gq + qg] = static_cast<uint32_t>(pw.base);
-          ac.lc_next = pw.base + pair_words(pw.k, stride);
+        if (!far) {
+          for (; t + 4 <= e; t += 4) {
+            const uint32_t k0 = rl32(dec, t), k1 = rl32(dec, t + 1), k2 = rl32(dec, t + 2), k3 = rl32(dec, t + 3);
+            const uint4 v0 = planes(k0), v1 = planes(k1), v2 = planes(k2), v3 = planes(k3);
+            mask &= group_test(k0, v0) & group_test(k1, v1);
+            mask &= group_test(k2, v2) & group_test(k3, v3);
+          }
+          if (t + 2 <= e) {
+            const uint32_t k0 = rl32(dec, t), k1 = rl32(dec, t + 1);
+            const uint4 v0 = planes(k0), v1 = planes(k1);
+            mask &= group_test(k0, v0) & group_test(k1, v1);
+            t += 2;
+          }
+          if (t < e) {
+            const uint32_t k0 = rl32(dec, t);
+            mask &= group_test(k0, planes(k0));
+          }
         } else {
-          atomicAnd(&a.surv[static_cast<uint64_t>(m) * a.W + (qg >> 6)], ~(1ull << (qg & 63)));
+          for (; t < e; ++t) {
+            const uint32_t tw = rl32(raw, t), l = (tw >> 3) & 15u, k0 = rl32(dec, t);
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (static_cast<uint32_t>(__popc(present & ((1u << l) - 1u))) < staged) v = planes(k0);
+            else if (valid) v = a.planes[((group * R + (tw & 7u)) * 16 + l) * 64 + lane];
+            mask &= group_test(k0, v);
+          }
         }
-        have = false;
-        finished = true;
+        ++st.nodes;
+        return mask;
+      };
+      // whether the lane's molecule keeps a candidate
+      auto some = [&](uint32_t mask) -> bool {
+        if (CLS >= 1) mask |= quad_xor1(mask);
+        if (CLS == 2) mask |= quad_xor2(mask);
+        return mask != 0;
+      };
+      load_tokens(0);
+      bool alive = act;
+      // two nodes at a time, whose masks go out together (the second past the last node falls in the
+      // block's padding); a pair dies at its first node without candidates (gmcr.hpp:56-61)
+      for (uint32_t i = 0; i < k; i += 2) {  // wave-uniform
+        st.live += alive;
+        const uint32_t m0 = node_mask();
+        alive = alive && some(m0);
+        if (__ballot(alive) == 0) break;
+        uint32_t m1 = 0;
+        if (i + 1 < k) {
+          st.live += alive;
+          m1 = node_mask();
+          alive = alive && some(m1);
+          if (__ballot(alive) == 0) break;
+        }
+        if (CLS == 0) {
+          if (alive && room) *reinterpret_cast<uint4*>(a.arena + base + i) = make_uint4(m0, 0, m1, 0);
+        } else if (CLS == 1) {  // the lanes of a molecule swap halves: each stores one node's word
+          const uint32_t other = quad_xor1(h ? m0 : m1);
+          if (alive && room) reinterpret_cast<uint2*>(a.arena + base + i)[h] = h ? make_uint2(other, m1) : make_uint2(m0, other);
+        } else if (alive && room) {
+          uint32_t* dst = reinterpret_cast<uint32_t*>(a.arena + base + 2 * i);
+          dst[h] = m0;
+          dst[4 + h] = m1;
+        }
       }
+      if (alive && h == 0) a.pair_off[static_cast<uint64_t>(mi.m) * a.Gq + g] = static_cast<uint32_t>(base);
+      if (act && !alive) dead |= 1ull << jb;
     }
-    // pairs finished this step release their slot's count
-#pragma unroll
-    for (uint32_t sl = 0; sl < S; ++sl) pending[sl] -= __popcll(__ballot(finished && sl_of == sl));
-  }
-  if (lane == 0) {
-    atomicAdd(&a.counters[4], static_cast<unsigned long long>(wave_steps));
-    atomicAdd(&a.counters[5], static_cast<unsigned long long>(lane_steps));
+    if (dead && h == 0) atomicAnd(&a.surv[static_cast<uint64_t>(mi.m) * a.W + w], ~dead);
   }
 }
 
-struct EvalArgs {
-  GraphDev d;
-  uint32_t R, Gq, W;
-  const MolInfo* minfo;    // width-class order (all classes)
-  const uint32_t* planes32;
-  const uint64_t* planes64;
-  const uint64_t* planes_hi;
-  const uint64_t* lab_hi;
-  const uint64_t* tok64;
-  const QueryInfo* qinfo;
-  const uint64_t* list;    // pre-tested pairs, c | g << 32
-  const uint32_t* poff;    // list offset of each molecule (width-class order)
-  uint64_t list_cap;
-  uint32_t first, count;   // the width class's molecules [first, first + count)
-  uint32_t chunk;          // list entries a wavefront claims at a time
-  uint64_t* arena;
-  uint64_t arena_cap;
-  unsigned long long* surv;
-  uint32_t* pair_off;
-  unsigned long long* counters;  // [0] list cursor, [1] arena top, [3] overflow, [4..5] statistics
-};
-
-// Persistent pair evaluation of one width class, pair by pair: lanes take the class's entries of
-// the pre-tested pair list as they become idle and read the molecule's planes from device memory
-// (neighbouring entries mostly share a molecule, so the reads share cache lines).  No molecule is
-// staged, so every lane has a pair however few pairs a molecule has (small query batches).
-// Survivors and deaths are recorded as in k_pair_survive.
-template <int NW>
-__global__ __launch_bounds__(256) void k_pair_eval(EvalArgs a) {
-  constexpr uint32_t stride = NW == 4 ? 2u : 1u;
-  const uint32_t lane = static_cast<uint32_t>(lane_id());
-  const uint32_t R = a.R, Gq = a.Gq;
-  const uint32_t seg = token_segment(R);
-  const uint64_t below = (1ull << lane) - 1;
-  const uint64_t lo = a.poff[a.first];
-  const uint64_t hi = min(static_cast<uint64_t>(a.poff[a.first + a.count]), a.list_cap);
-  ArenaCursor ac;
-  uint64_t next = 0, end = 0;  // claimed entries [next, end) (wave-uniform)
-  bool exhausted = lo >= hi;
-  uint64_t wave_steps = 0, lane_steps = 0;
-
-  bool have = false;
-  uint32_t qg = 0, m = 0, n = 0, s = 0;
-  GlobalPlanes<NW> P{};
-  PairWalk<NW> pw;
-  while (true) {
-    uint64_t need = __ballot(!have);
-    while (need && !exhausted) {
-      if (next >= end) {
-        unsigned long long b = 0;
-        if (lane == 0) b = atomicAdd(&a.counters[0], static_cast<unsigned long long>(a.chunk));
-        next = lo + uniform64(__shfl(b, 0));
-        end = next + a.chunk < hi ? next + a.chunk : hi;
-        if (next >= hi) {
-          exhausted = true;
-          break;
-        }
-      }
-      const uint32_t cnt = min(static_cast<uint32_t>(end - next), static_cast<uint32_t>(__popcll(need)));
-      const uint32_t rn = __popcll(need & below);
-      const bool take = ((need >> lane) & 1ull) && rn < cnt;
-      if (take) {
-        const uint64_t e = a.list[next + rn];
-        const MolInfo mi = a.minfo[static_cast<uint32_t>(e)];
-        qg = static_cast<uint32_t>(e >> 32);
-        const QueryInfo qi = a.qinfo[qg];
-        m = mi.m;
-        n = mi.n;
-        s = mi.s;
-        P.p32 = a.planes32 + static_cast<uint64_t>(mi.x) * R * 64;
-        P.p64 = a.planes64 + static_cast<uint64_t>(mi.x) * R * 64;
-        P.phi = a.planes_hi + static_cast<uint64_t>(NW == 4 ? mi.wi : 0u) * R * 64;
-        P.lm = a.d.lmask + static_cast<uint64_t>(mi.m) * 16;
-        P.lmh = a.lab_hi + static_cast<uint64_t>(NW == 4 ? mi.wi : 0u) * 16;
-        pw.k = qi.k;
-        pw.tw = qi.first;
-        pw.nodebase = static_cast<uint64_t>(qi.qoff) * seg;
-        pw.i = 0;
-        pw.tp = 0;
-        have = true;
-      }
-      next += cnt;
-      need &= ~__ballot(take);
-      ac.reserve(take, pair_words(pw.k, stride), below, a.counters, a.arena_cap);
-      if (take) pw.base = ac.lc_next;
-    }
-    const uint64_t active = __ballot(have);
-    if (active == 0) break;
-    ++wave_steps;
-    lane_steps += __popcll(active);
-    if (have) {
-      auto ns = [&]() { return make_uint2(n, s); };
-      const int st = walk_step<NW>(P, ns, a.d.nl, a.tok64, R, pw, a.arena, a.arena_cap);
-      if (st == kWalkSurvived) {
-        a.pair_off[static_cast<uint64_t>(m) * Gq + qg] = static_cast<uint32_t>(pw.base);
-        ac.lc_next = pw.base + pair_words(pw.k, stride);
-        have = false;
-      } else if (st == kWalkDied) {
-        atomicAnd(&a.surv[static_cast<uint64_t>(m) * a.W + (qg >> 6)], ~(1ull << (qg & 63)));
-        have = false;
-      }
-    }
+// Pair evaluation: the exact candidates of every pre-tested pair's query nodes (isomorphism.hpp:49
+// and :103-110), keeping the masks of the pairs that survive GMCR.
+//
+// A wavefront takes one query graph and one group, 64 lanes of neighbours in the width-class
+// order, so a requirement's level, label and count are scalars: a test is one 16-byte LDS read and
+// seven vector operations for 64 x 32 positions.  A lane that walked a pair of its own decoded
+// every token for itself and gathered its token words and planes, about 40 operations a test, and
+// a wavefront waited for its longest pair.  The order groups molecules of one label set and
+// similar size, so a query graph passes the pre-test for none of a group's molecules three times
+// out of four and for half of them otherwise (1 M LogNormal molecules, U[4,32]-node queries).
+//
+// A block of eight wavefronts stages the group's planes and label masks for the labels that occur
+// in it (the first a.slots of them; the rest are read from the database) and shares its query
+// graphs out by index.  Node masks go straight to the pairs' arena blocks, which a wavefront takes
+// from a chunk of its own; pairs that die clear their pre-test bits, one atomic per molecule and
+// 64 query graphs.  80 registers: six wavefronts per SIMD, which its scalar token decode needs to
+// hide (20 waves with 4-wavefront blocks: 8.1 instead of 6.8 ms).
+//
+// Measured, in place of one launch per size class with a lane per pair: 2,000 molecules x 20 query
+// graphs 219 -> 12 us (three serial chains of ~100 us), 100,000 x 100 475 -> 125 us, 1 M x 25
+// 1,242 -> 392 us, 1 M x 1,000 10.7 -> 6.8 ms.
+__global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a) {
+  extern __shared__ uint4 lds4[];
+  uint32_t* labs = reinterpret_cast<uint32_t*>(lds4 + static_cast<uint64_t>(a.slots) * a.R * kWave);
+  unsigned long long* next_item = reinterpret_cast<unsigned long long*>(labs + a.slots * kWave);
+  const uint32_t wave = uniform32(threadIdx.x / kWave);
+  const uint32_t g0 = a.order.groups(0), g1 = a.order.groups(1);
+  const uint64_t items = static_cast<uint64_t>(a.order.total()) * a.parts;
+  GroupState st;
+  st.next = (static_cast<uint64_t>(blockIdx.x) * kGroupWaves + wave) * a.chunk;
+  st.end = st.next + a.chunk;
+  st.first_chunks = static_cast<uint64_t>(gridDim.x) * kGroupWaves * a.chunk;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && st.first_chunks > a.arena_cap) atomicOr(&a.counters[3], 1ull);
+  uint32_t off_mask = 0x1FC00u;
+  asm volatile("" : "+v"(off_mask));  // in a vector register: the and-or of a token's offset and the lane's is then one operation
+  for (uint64_t item = blockIdx.x; item < items;) {
+    const uint32_t part = static_cast<uint32_t>(item & (a.parts - 1));
+    const uint32_t grp = static_cast<uint32_t>(item / a.parts);
+    if (grp < g0) group_item<0>(a, grp, part, wave, lds4, labs, off_mask, st);
+    else if (grp < g0 + g1) group_item<1>(a, grp - g0, part, wave, lds4, labs, off_mask, st);
+    else group_item<2>(a, grp - g0 - g1, part, wave, lds4, labs, off_mask, st);
+    if (gridDim.x >= items) break;
+    __syncthreads();  // the staged planes have been read
+    if (threadIdx.x == 0) *next_item = gridDim.x + atomicAdd(&a.counters[2], 1ull);
+    __syncthreads();
+    item = uniform64(*next_item);
   }
-  if (lane == 0) {
-    atomicAdd(&a.counters[4], static_cast<unsigned long long>(wave_steps));
-    atomicAdd(&a.counters[5], static_cast<unsigned long long>(lane_steps));
+  uint32_t live = st.live;
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) live += static_cast<uint32_t>(__shfl_xor(static_cast<int>(live), o));
+  if (lane_id() == 0 && st.scans) {
+    unsigned long long* out = a.stats + (blockIdx.x % kGroupStatSlots) * 16;
+    atomicAdd(&out[0], static_cast<unsigned long long>(st.nodes));
+    atomicAdd(&out[1], static_cast<unsigned long long>(live));
+    atomicAdd(&out[2], static_cast<unsigned long long>(st.scans));
   }
 }
 
@@ -1381,19 +1095,17 @@ __global__ __launch_bounds__(256) void k_request_stats(uint64_t P, const uint32_
 
 // The first `small` width-class entries (molecules of <= 32 nodes) two per wavefront, the rest one
 // per wavefront.
-hipError_t db_prepare(hipStream_t s, const GraphDev& g, uint32_t R, const uint32_t* cls_list, const uint32_t* pidx, const uint32_t* wide_idx,
-                      uint32_t* planes32, uint64_t* planes64, uint64_t* planes_hi, uint64_t* lab_hi, uint64_t* dmax, MolInfo* minfo,
-                      const ClassLabels& cl, uint64_t* cmax, uint32_t small) {
+hipError_t db_prepare(hipStream_t s, const GraphDev& g, uint32_t R, const uint32_t* cls_list, const GroupOrder& order, uint32_t* planes,
+                      uint32_t* labs, uint64_t* dmax, MolInfo* minfo, const ClassLabels& cl, uint64_t* cmax) {
   if (!g.G) return hipSuccess;
+  const uint32_t small = order.count[0];
   if (small) {
     const uint32_t waves = (small + 1) / 2;
-    k_db_prepare_pairs<<<(waves + 3) / 4, 256, 0, s>>>(g, R, small, cls_list, pidx, planes32, dmax, minfo, cl, cmax);
+    k_db_prepare_pairs<<<(waves + 3) / 4, 256, 0, s>>>(g, R, small, cls_list, planes, labs, dmax, minfo, cl, cmax);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if (g.G > small)
-    k_db_prepare<<<(g.G - small + 3) / 4, 256, 0, s>>>(g, R, cls_list, pidx, wide_idx, planes32, planes64, planes_hi, lab_hi, dmax, minfo, cl,
-                                                       cmax, small);
+  if (g.G > small) k_db_prepare<<<(g.G - small + 3) / 4, 256, 0, s>>>(g, R, cls_list, order, planes, labs, dmax, minfo, cl, cmax, small);
   return hipGetLastError();
 }
 
@@ -1495,10 +1207,8 @@ using namespace sigmo_internal;
 
 // Pair spaces up to this size run with one host synchronisation (sigmo_batch_run).
 constexpr uint64_t kOneSyncPairs = 1ull << 25;
-// Query graphs per batch below which the pair evaluation runs pair by pair from the list: with
-// fewer, a molecule has too few pre-tested pairs to keep a wavefront's lanes busy from the few
-// molecules its LDS ring holds.
-constexpr uint32_t kListModeGraphs = 256;
+// A run's device counters: 16 words, then the group evaluation's statistics.
+constexpr uint64_t kCounterWords = 16 + 16 * sigmo_k::kGroupStatSlots;
 
 struct sigmo_batch;
 namespace sigmo_internal {
@@ -1510,17 +1220,16 @@ struct sigmo_db {
   const sigmo_graph* data = nullptr;
   uint32_t R = 0;
   uint32_t num_wide = 0;
-  uint32_t cls_count[3] = {0, 0, 0};  // molecules of <= 32, 33..64 and 65..128 nodes
+  uint32_t num_labels = 0;            // node labels < 16 that occur in the data
+  sigmo_k::GroupOrder order{{0, 0, 0}};  // molecules of <= 32, 33..64 and 65..128 nodes
   uint32_t* cls_list = nullptr;       // the three classes' molecules one after another, grouped by label set and size
-  uint32_t* pidx = nullptr;           // index of the molecule's planes in planes32 or planes64
-  uint32_t* wide_idx = nullptr;
-  uint32_t* planes32 = nullptr;
-  uint64_t *planes64 = nullptr, *planes_hi = nullptr, *lab_hi = nullptr, *dmax = nullptr;  // dmax in width-class order
+  uint32_t *planes = nullptr, *labs = nullptr;  // level planes and label masks by group (GroupOrder)
+  uint64_t* dmax = nullptr;                     // width-class order
   uint64_t* cmax = nullptr;                                                                // per-class maxima, [(k*R + r)*G + c]
   sigmo_k::MolInfo* minfo = nullptr;                                                       // width-class order
   sigmo_k::ClassLabels cls{{0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}};                        // the pre-test's class labels
   uint64_t bytes = 0;
-  uint64_t cap_G = 0, cap_32 = 0, cap_64 = 0, cap_hi = 0, cap_dmax = 0, cap_lab = 0, cap_cmax = 0;  // allocated elements
+  uint64_t cap_G = 0, cap_planes = 0, cap_labs = 0, cap_dmax = 0, cap_cmax = 0;  // allocated elements
   uint64_t generation = 0;  // bumped whenever a rebind changes the data or any buffer address
   uint32_t* order_keys = nullptr;  // 2G: the sort keys and their sorted copy
   uint8_t* sort_tmp = nullptr;
@@ -1529,12 +1238,8 @@ struct sigmo_db {
     bfree(order_keys);
     bfree(sort_tmp);
     bfree(cls_list);
-    bfree(pidx);
-    bfree(wide_idx);
-    bfree(planes32);
-    bfree(planes64);
-    bfree(planes_hi);
-    bfree(lab_hi);
+    bfree(planes);
+    bfree(labs);
     bfree(dmax);
     bfree(cmax);
     bfree(minfo);
@@ -1550,11 +1255,6 @@ struct sigmo_batch {
   uint64_t* qmax = nullptr;
   uint64_t* qcmax = nullptr;  // per-class maxima, [(g*3 + k)*R + r]
   uint64_t cap_tokens = 0, cap_qinfo = 0, cap_qmax = 0, cap_qcmax = 0;
-  // pre-test: passing pairs per molecule (width-class order), their scan and the pair list
-  uint32_t *pcnt = nullptr, *poff = nullptr;
-  uint64_t cap_pcnt = 0, cap_poff = 0;
-  uint64_t* list = nullptr;
-  uint64_t cap_list = 0;
   // pair evaluation
   uint64_t* arena = nullptr;
   uint64_t cap_arena = 0;
@@ -1577,14 +1277,14 @@ struct sigmo_batch {
   uint64_t cap_wide = 0;
   uint32_t* deep_pairs = nullptr;  // pairs of queries deeper than the lane join's first pass holds
   uint64_t cap_deep = 0;
-  unsigned long long* run_host = nullptr;  // pinned: a one-sync run's filter counters [0..7] and GMCR total [8]
+  unsigned long long* run_host = nullptr;  // pinned: a run's filter counters, then the GMCR total
   uint32_t* req_offsets = nullptr;        // per-request statistics
   unsigned long long* req_out = nullptr;
   sigmo_batch_tuning tune{};               // 0 fields: the built-in heuristics
   // a captured run (sigmo_batch_capture): the graph, its sizes and its pinned readback
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
-  unsigned long long* graph_host = nullptr;  // [0..7] filter counters, [8] GMCR total, [9..16] join stats
+  unsigned long long* graph_host = nullptr;  // filter counters, GMCR total, 8 words of join stats
   uint64_t graph_P = 0, graph_nw = 0, graph_db_generation = 0;
   uint32_t graph_Gq = 0;
   int graph_find_first = 0;
@@ -1609,9 +1309,6 @@ struct sigmo_batch {
     bfree(qinfo);
     bfree(qmax);
     bfree(qcmax);
-    bfree(pcnt);
-    bfree(poff);
-    bfree(list);
     bfree(arena);
     bfree(surv);
     bfree(pair_off);
@@ -1650,6 +1347,8 @@ int choose_classes(sigmo_db* db, const sigmo_graph* data, hipStream_t s) {
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   bfree(hist);
   if (e != hipSuccess) return sigmo_err::set(SIGMO_ERR_HIP, std::string("label histogram: ") + hipGetErrorString(e));
+  db->num_labels = 0;
+  for (uint32_t l = 0; l < 16; ++l) db->num_labels += h[l] != 0;
   for (uint32_t k = 0; k < sigmo_k::kClasses; ++k) {
     uint32_t best = 0xFFFFFFFFu;
     for (uint32_t l = 0; l < 16; ++l)
@@ -1669,40 +1368,27 @@ int db_fill(sigmo_db* db, const sigmo_graph* data) {
   BATCH_TRY(ctx_info(db->ctx, &device, &s, &cus, &st, &sh));
   const auto& go = graph_host_offsets(data);
   const uint32_t G = static_cast<uint32_t>(go.size() - 1);
-  std::vector<uint32_t> widx(G, sigmo_k::kNoWide), pidx(G, 0);
-  uint32_t nw = 0, n32 = 0, n64 = 0, count[3] = {0, 0, 0};
+  sigmo_k::GroupOrder order{{0, 0, 0}};
   for (uint32_t g = 0; g < G; ++g) {
     const uint32_t n = go[g + 1] - go[g];
-    const int c = n <= 32 ? 0 : (n <= 64 ? 1 : 2);
-    ++count[c];
-    pidx[g] = c == 0 ? n32++ : n64++;
-    if (c == 2) widx[g] = nw++;
+    ++order.count[n <= 32 ? 0 : (n <= 64 ? 1 : 2)];
   }
-  const uint64_t R = db->R;
+  const uint64_t R = db->R, groups = order.total();
   uint64_t cap_g = db->cap_G;
   BATCH_TRY(bgrow(&db->cls_list, cap_g, G));
-  cap_g = db->cap_G;
-  BATCH_TRY(bgrow(&db->pidx, cap_g, G));
-  cap_g = db->cap_G;
-  BATCH_TRY(bgrow(&db->wide_idx, cap_g, G));
   cap_g = db->cap_G;
   BATCH_TRY(bgrow(&db->minfo, cap_g, G));
   db->cap_G = cap_g;
   BATCH_TRY(bgrow(&db->dmax, db->cap_dmax, uint64_t(G) * R));
   BATCH_TRY(bgrow(&db->cmax, db->cap_cmax, uint64_t(G) * R * sigmo_k::kClasses));
-  BATCH_TRY(bgrow_slack(&db->planes32, db->cap_32, uint64_t(n32) * R * 64));
-  BATCH_TRY(bgrow_slack(&db->planes64, db->cap_64, uint64_t(n64) * R * 64));
-  BATCH_TRY(bgrow_slack(&db->planes_hi, db->cap_hi, uint64_t(nw) * R * 64));
-  BATCH_TRY(bgrow_slack(&db->lab_hi, db->cap_lab, uint64_t(nw) * 16));
+  BATCH_TRY(bgrow_slack(&db->planes, db->cap_planes, groups * R * 16 * 64 * 4));
+  BATCH_TRY(bgrow_slack(&db->labs, db->cap_labs, groups * 16 * 64));
   db->data = data;
   db->generation++;
-  db->num_wide = nw;
-  for (int c = 0; c < 3; ++c) db->cls_count[c] = count[c];
-  db->bytes = G * (12ull + sizeof(sigmo_k::MolInfo)) + (uint64_t(n32) * 256 + (uint64_t(n64) + nw) * 512) * R + nw * 128ull +
-              uint64_t(G) * R * 8 * (1 + sigmo_k::kClasses);
+  db->num_wide = order.count[2];
+  db->order = order;
+  db->bytes = G * (4ull + sizeof(sigmo_k::MolInfo)) + groups * 16 * 64 * (16 * R + 4) + uint64_t(G) * R * 8 * (1 + sigmo_k::kClasses);
   BATCH_TRY(choose_classes(db, data, s));
-  BATCH_HIP_TRY(hipMemcpyAsync(db->wide_idx, widx.data(), G * 4ull, hipMemcpyHostToDevice, s));
-  BATCH_HIP_TRY(hipMemcpyAsync(db->pidx, pidx.data(), G * 4ull, hipMemcpyHostToDevice, s));
   // the width-class order: molecules sorted by (class, label set, size), stably (by index within a key)
   BATCH_TRY(bgrow_slack(&db->order_keys, db->cap_keys, 2ull * G));
   const sigmo_k::GraphDev gd = graph_dev(data);
@@ -1713,7 +1399,6 @@ int db_fill(sigmo_db* db, const sigmo_graph* data) {
   BATCH_HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, db->order_keys, db->order_keys + G, ids, db->cls_list, G, 0u, 25u, s));
   BATCH_TRY(bgrow_slack(&db->sort_tmp, db->cap_sort, std::max<uint64_t>(tmp_bytes, 1)));
   BATCH_HIP_TRY(rocprim::radix_sort_pairs(db->sort_tmp, tmp_bytes, db->order_keys, db->order_keys + G, ids, db->cls_list, G, 0u, 25u, s));
-  BATCH_HIP_TRY(hipStreamSynchronize(s));  // the host vectors go out of scope
   BATCH_TRY(sigmo_db_refresh(db));
   BATCH_HIP_TRY(hipStreamSynchronize(s));
   return SIGMO_OK;
@@ -1761,8 +1446,7 @@ int sigmo_db_refresh(sigmo_db* db) {
   const double bytes = 4.0 * (double(g.N) + 1.0) + 4.0 * double(graph_edges(db->data)) + double(g.N) + 8.0 * db->R * double(g.N);
   void* tok = nullptr;
   BATCH_TRY(ctx_timed(db->ctx, SIGMO_PHASE_SIG_DATA, SIGMO_KERNEL_DB_PREPARE, bytes, true, &tok));
-  BATCH_HIP_TRY(sigmo_k::db_prepare(s, g, db->R, db->cls_list, db->pidx, db->wide_idx, db->planes32, db->planes64, db->planes_hi, db->lab_hi,
-                                    db->dmax, db->minfo, db->cls, db->cmax, db->cls_count[0]));
+  BATCH_HIP_TRY(sigmo_k::db_prepare(s, g, db->R, db->cls_list, db->order, db->planes, db->labs, db->dmax, db->minfo, db->cls, db->cmax));
   BATCH_TRY(ctx_timed(db->ctx, 0, 0, 0.0, false, &tok));
   return SIGMO_OK;
 }
@@ -1792,7 +1476,7 @@ int sigmo_batch_create(sigmo_ctx* ctx, const sigmo_db* db, sigmo_batch** out) {
   auto* b = new sigmo_batch();
   b->ctx = ctx;
   b->db = db;
-  int stt = balloc(&b->counters, 16);
+  int stt = balloc(&b->counters, kCounterWords);
   if (stt == SIGMO_OK) stt = balloc(&b->total, 1);
   if (stt != SIGMO_OK) {
     delete b;
@@ -1814,17 +1498,13 @@ int sigmo_batch_workspace_bytes(const sigmo_batch* b, uint32_t num_query_graphs,
   // for the pairs that survive otherwise, priced at the arena's guess of 1/8 of the pairs (plus
   // 4 B per pair for the list of wide-molecule pairs).  A run whose survivors exceed the guess
   // grows the arena and those arrays to the measured demand; a batch keeps its buffers at their
-  // largest size, so a caller admitting by this figure should leave room for that growth.  In
-  // list mode (below 256 query graphs by default) the pre-tested pair list takes 8 B per listed
-  // pair, priced at its first sizing (a quarter of the pairs; every pair on the one-sync path).
+  // largest size, so a caller admitting by this figure should leave room for that growth.
   const uint64_t guess = std::min<uint64_t>(std::max<uint64_t>(pairs / 8, 1 << 16), 1ull << 26);
   const uint64_t arena_words = static_cast<uint64_t>(double(guess) * (mean_k + 1.0) * (db->num_wide ? 2.0 : 1.0));
   const bool one_sync = !db->num_wide && pairs && pairs <= kOneSyncPairs;
   const uint64_t gmcr_pairs = one_sync ? pairs : guess;
-  const bool list_mode = b->tune.filter_mode == 2 || (b->tune.filter_mode == 0 && Gq < kListModeGraphs);
-  const uint64_t list = !list_mode ? 0 : (one_sync ? pairs : std::min<uint64_t>(pairs, pairs / 4 + 65536));
   *bytes = query_nodes * sigmo_k::token_segment(static_cast<uint32_t>(R)) * 2 + Gq * (sizeof(sigmo_k::QueryInfo) + 8 * R * (1 + sigmo_k::kClasses)) +
-           Gd * W * 8 + pairs * 4 + arena_words * 8 + gmcr_pairs * 16 + (db->num_wide ? guess * 4 : 0) + (Gd + 1) * 8 + list * 8;
+           Gd * W * 8 + pairs * 4 + arena_words * 8 + gmcr_pairs * 16 + (db->num_wide ? guess * 4 : 0) + (Gd + 1) * 8;
   return SIGMO_OK;
 }
 
@@ -1881,11 +1561,9 @@ struct RunShape {
   uint32_t R = 0, Gq = 0, Gd = 0, W = 0;
   uint64_t pairs = 0, ksum = 0;
   int cus = 0;
-  bool list_mode = false;  // pair evaluation from the pre-tested pair list (k_pair_eval)
-  uint32_t lds_bytes[3] = {0, 0, 0};
-  uint64_t cls_blocks[3] = {0, 0, 0}, waves_total = 0;
+  uint32_t group_blocks = 0, group_parts = 1, group_slots = 1, group_chunk = 0;  // the pair evaluation's launch
+  uint64_t first_chunks = 0;  // arena words its wavefronts start with
 };
-
 
 int shape_run(const sigmo_batch* b, const sigmo_graph* query, int cus, RunShape& L) {
   const sigmo_db* db = b->db;
@@ -1904,53 +1582,34 @@ int shape_run(const sigmo_batch* b, const sigmo_graph* query, int cus, RunShape&
   L.R = db->R;
   L.W = (L.Gq + 63) / 64;
   L.pairs = uint64_t(L.Gq) * L.Gd;
-  L.list_mode = b->tune.filter_mode == 2 || (b->tune.filter_mode == 0 && L.Gq < kListModeGraphs);
-  // one persistent launch per width class, as many 4-wave blocks as registers and LDS keep
-  // resident (or the tuned count, capped by residency)
-  const void* kern[3] = {reinterpret_cast<const void*>(sigmo_k::k_pair_survive<1>), reinterpret_cast<const void*>(sigmo_k::k_pair_survive<2>),
-                         reinterpret_cast<const void*>(sigmo_k::k_pair_survive<4>)};
-  const void* kern_list[3] = {reinterpret_cast<const void*>(sigmo_k::k_pair_eval<1>), reinterpret_cast<const void*>(sigmo_k::k_pair_eval<2>),
-                              reinterpret_cast<const void*>(sigmo_k::k_pair_eval<4>)};
-  for (int c = 0; c < 3; ++c) L.lds_bytes[c] = L.list_mode ? 0u : sigmo_k::survive_lds_bytes(L.R, c == 0 ? 1 : (c == 1 ? 2 : 4));
-  for (int c = 0; c < 3; ++c) {
-    if (!db->cls_count[c]) continue;
-    if (L.list_mode) {
-      int resident = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern_list[c], 256, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        resident = 4;
-      }
-      // two blocks per CU unless tuned: each lane reads its pair's molecule planes from device
-      // memory, and fewer molecules in flight per XCD keep more of them in L2 (10 M molecules x 25
-      // query graphs: 17.6 -> 16.2 ms with 2 blocks instead of 8; x 64: 24.2 -> 22.4 ms)
-      uint64_t per_cu = std::max<uint64_t>(1, std::min<uint64_t>(2, static_cast<uint64_t>(resident)));
-      if (b->tune.filter_blocks_per_cu) per_cu = std::min<uint64_t>(static_cast<uint64_t>(std::max(1, resident)), b->tune.filter_blocks_per_cu);
-      L.cls_blocks[c] = uint64_t(cus) * per_cu;
-      L.waves_total += L.cls_blocks[c] * sigmo_k::kSurviveWaves;
-      continue;
-    }
-    if (L.lds_bytes[c] > 64 * 1024) return sigmo_err::set(SIGMO_ERR_UNSUPPORTED, "molecule slots exceed 64 KB of LDS per block");
-    int resident = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern[c], 256, L.lds_bytes[c]) != hipSuccess) {
-      (void)hipGetLastError();
-      resident = 2;
-    }
-    uint64_t per_cu = std::max<uint64_t>(1, std::min<uint64_t>(8, static_cast<uint64_t>(resident)));
-    if (b->tune.filter_blocks_per_cu) per_cu = std::min<uint64_t>(per_cu, b->tune.filter_blocks_per_cu);
-    L.cls_blocks[c] = std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(cus) * per_cu, (uint64_t(db->cls_count[c]) + 3) / 4));
-    L.waves_total += L.cls_blocks[c] * sigmo_k::kSurviveWaves;
-  }
+  const uint64_t groups = db->order.total(), ucus = static_cast<uint64_t>(cus);
+  // a group's query graphs go to one block, or to more where the groups alone leave CUs idle
+  while (L.group_parts < 64 / sigmo_k::kGroupWaves && groups * L.group_parts < 2 * ucus && sigmo_k::kGroupWaves * L.group_parts < L.Gq)
+    L.group_parts *= 2;
+  const uint64_t items = groups * L.group_parts;
+  // LDS for every label that occurs, within 64 KB; with blocks to spare within 52 KB, so that three
+  // stay resident (a group of neighbours in the width-class order holds 4 to 6 labels)
+  const uint32_t lds = (items > 2 * ucus ? 52u : 64u) * 1024;
+  L.group_slots = std::max<uint32_t>(1, std::min<uint32_t>(db->num_labels, lds / sigmo_k::group_lds_bytes(1, L.R)));
+  uint64_t per_cu = std::max<uint64_t>(1, std::min<uint64_t>(32 / sigmo_k::kGroupWaves, 160 * 1024 / sigmo_k::group_lds_bytes(L.group_slots, L.R)));
+  if (b->tune.filter_blocks_per_cu) per_cu = std::min<uint64_t>(per_cu, b->tune.filter_blocks_per_cu);
+  L.group_blocks = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(items, ucus * per_cu)));
+  // a wavefront's arena chunk holds the largest query graph for a whole group (2,048 words) and, for
+  // many pairs, more: claims meet on one address
+  const uint64_t waves = uint64_t(L.group_blocks) * sigmo_k::kGroupWaves;
+  uint64_t chunk = 2048;
+  while (chunk < 16384 && chunk * waves * 64 < L.pairs) chunk *= 2;
+  L.group_chunk = static_cast<uint32_t>(chunk);
+  L.first_chunks = waves * chunk;
   return SIGMO_OK;
 }
 
-// Pair evaluation: the pre-test over every pair (its bits in surv), the scan of its per-molecule
-// counts (total in counters[7]) and, per width class, the evaluation of the passing pairs --
-// molecule by molecule from LDS-staged planes (k_pair_survive) or, in list mode, pair by pair
-// from the pre-tested pair list (k_pair_expand, then k_pair_eval).  Counters are cleared by a
-// kernel.  Deaths clear their pre-test bit, so surv ends as the GMCR survival bitmask.
+// Pair filter: the pre-test over every pair (its bits in surv), then the evaluation of the passing
+// pairs.  Counters are cleared by a kernel.  Deaths clear their pre-test bit, so surv ends as the
+// GMCR survival bitmask.
 hipError_t launch_filter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
   const sigmo_db* db = b->db;
-  hipError_t e = sigmo_k::fill_u64(s, reinterpret_cast<uint64_t*>(b->counters), 16, 0);
+  hipError_t e = sigmo_k::fill_u64(s, reinterpret_cast<uint64_t*>(b->counters), kCounterWords, 0);
   if (e != hipSuccess || !L.Gd || !L.Gq) return e;
   sigmo_k::PretestArgs p;
   p.R = L.R;
@@ -1964,7 +1623,6 @@ hipError_t launch_filter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
   p.qmax = b->qmax;
   p.qcmax = b->qcmax;
   p.surv = b->surv;
-  p.pcnt = b->pcnt;
   const dim3 pgrid((L.Gd + 255) / 256);
   switch (L.R) {  // one instantiation per level count keeps the molecule's maxima in registers
     case 1: hipLaunchKernelGGL(sigmo_k::k_pair_pretest<1>, pgrid, dim3(256), 0, s, p); break;
@@ -1977,79 +1635,41 @@ hipError_t launch_filter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
     default: hipLaunchKernelGGL(sigmo_k::k_pair_pretest<8>, pgrid, dim3(256), 0, s, p); break;
   }
   e = hipGetLastError();
-  if (e == hipSuccess) e = sigmo_k::exclusive_scan(s, b->pcnt, L.Gd, b->poff, b->scan_tmp, reinterpret_cast<uint64_t*>(b->counters + 7));
-  if (e == hipSuccess && L.list_mode) {
-    hipLaunchKernelGGL(sigmo_k::k_pair_expand, dim3((L.Gd + 255) / 256), dim3(256), 0, s, L.Gd, L.W, db->minfo, b->surv, b->poff, b->list,
-                       b->cap_list, b->counters);
-    e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  sigmo_k::GroupArgs a;
+  a.d = L.dd;
+  a.order = db->order;
+  a.R = L.R;
+  a.Gq = L.Gq;
+  a.W = L.W;
+  a.parts = L.group_parts;
+  a.slots = L.group_slots;
+  a.chunk = L.group_chunk;
+  a.minfo = db->minfo;
+  a.planes = reinterpret_cast<const uint4*>(db->planes);
+  a.labs = db->labs;
+  a.tokens = b->tokens;
+  a.qinfo = b->qinfo;
+  a.arena = b->arena;
+  a.arena_cap = b->cap_arena;
+  a.surv = b->surv;
+  a.pair_off = b->pair_off;
+  a.counters = b->counters;
+  a.stats = b->counters + 16;
+  hipLaunchKernelGGL(sigmo_k::k_pair_group, dim3(L.group_blocks), dim3(sigmo_k::kGroupWaves * 64),
+                     sigmo_k::group_lds_bytes(L.group_slots, L.R), s, a);
+  return hipGetLastError();
+}
+
+// The filter's statistics and arena demand from its counters on the host.
+uint64_t read_counters(uint64_t first_chunks, const unsigned long long* cnt, sigmo_batch_result* res) {
+  res->filter_wave_steps = res->filter_lane_steps = res->filter_scans = 0;
+  for (uint32_t i = 0; i < sigmo_k::kGroupStatSlots; ++i) {
+    res->filter_wave_steps += cnt[16 + 16 * i];
+    res->filter_lane_steps += cnt[16 + 16 * i + 1];
+    res->filter_scans += cnt[16 + 16 * i + 2];
   }
-  uint64_t first = 0;
-  for (int c = 0; c < 3 && e == hipSuccess; ++c) {
-    const uint32_t count = db->cls_count[c];
-    const uint64_t at = first;
-    first += count;
-    if (!count) continue;
-    const int nw = c == 0 ? 1 : (c == 1 ? 2 : 4);
-    e = sigmo_k::fill_u64(s, reinterpret_cast<uint64_t*>(b->counters), 1, 0);  // each launch starts its own cursor
-    if (e != hipSuccess) break;
-    const dim3 grid(static_cast<unsigned>(L.cls_blocks[c]));
-    if (L.list_mode) {
-      sigmo_k::EvalArgs a;
-      a.d = L.dd;
-      a.R = L.R;
-      a.Gq = L.Gq;
-      a.W = L.W;
-      a.minfo = db->minfo;
-      a.planes32 = db->planes32;
-      a.planes64 = db->planes64;
-      a.planes_hi = db->planes_hi;
-      a.lab_hi = db->lab_hi;
-      a.tok64 = reinterpret_cast<const uint64_t*>(b->tokens);
-      a.qinfo = b->qinfo;
-      a.list = b->list;
-      a.poff = b->poff;
-      a.list_cap = b->cap_list;
-      a.first = static_cast<uint32_t>(at);
-      a.count = count;
-      a.chunk = 64u * (b->tune.filter_claim ? b->tune.filter_claim : 2u);
-      a.arena = b->arena;
-      a.arena_cap = b->cap_arena;
-      a.surv = b->surv;
-      a.pair_off = b->pair_off;
-      a.counters = b->counters;
-      if (nw == 1) hipLaunchKernelGGL(sigmo_k::k_pair_eval<1>, grid, dim3(256), 0, s, a);
-      else if (nw == 2) hipLaunchKernelGGL(sigmo_k::k_pair_eval<2>, grid, dim3(256), 0, s, a);
-      else hipLaunchKernelGGL(sigmo_k::k_pair_eval<4>, grid, dim3(256), 0, s, a);
-    } else {
-      sigmo_k::SurviveArgs a;
-      a.q = L.qd;
-      a.d = L.dd;
-      a.R = L.R;
-      a.Gq = L.Gq;
-      a.W = L.W;
-      a.count = count;
-      a.minfo = db->minfo + at;
-      a.pcnt = b->pcnt + at;
-      a.planes32 = db->planes32;
-      a.planes64 = db->planes64;
-      a.planes_hi = db->planes_hi;
-      a.lab_hi = db->lab_hi;
-      a.tok64 = reinterpret_cast<const uint64_t*>(b->tokens);
-      a.qinfo = b->qinfo;
-      a.arena = b->arena;
-      a.arena_cap = b->cap_arena;
-      a.surv = b->surv;
-      a.pair_off = b->pair_off;
-      a.counters = b->counters;
-      const uint64_t auto_claim = std::max<uint64_t>(1, std::min<uint64_t>(16, count / (L.cls_blocks[c] * sigmo_k::kSurviveWaves * 4)));
-      a.claim = static_cast<uint32_t>(b->tune.filter_claim ? std::min<uint32_t>(b->tune.filter_claim, 64) : auto_claim);
-      if (nw == 1) hipLaunchKernelGGL(sigmo_k::k_pair_survive<1>, grid, dim3(256), L.lds_bytes[0], s, a);
-      else if (nw == 2) hipLaunchKernelGGL(sigmo_k::k_pair_survive<2>, grid, dim3(256), L.lds_bytes[1], s, a);
-      else hipLaunchKernelGGL(sigmo_k::k_pair_survive<4>, grid, dim3(256), L.lds_bytes[2], s, a);
-    }
-    e = hipGetLastError();
-  }
-  return e;
+  return cnt[1] + first_chunks;
 }
 
 // GMCR: survivors per molecule and their exclusive scan (total in b->total).
@@ -2102,8 +1722,6 @@ int size_fixed_buffers(sigmo_batch* b, const RunShape& L) {
   BATCH_TRY(b->grow(&b->qinfo, b->cap_qinfo, L.Gq));
   BATCH_TRY(b->grow(&b->qmax, b->cap_qmax, uint64_t(L.Gq) * L.R));
   BATCH_TRY(b->grow(&b->qcmax, b->cap_qcmax, uint64_t(L.Gq) * L.R * sigmo_k::kClasses));
-  BATCH_TRY(b->grow(&b->pcnt, b->cap_pcnt, uint64_t(L.Gd) + 1));
-  BATCH_TRY(b->grow(&b->poff, b->cap_poff, uint64_t(L.Gd) + 1));
   BATCH_TRY(b->grow(&b->surv, b->cap_surv, uint64_t(L.Gd) * L.W));
   BATCH_TRY(b->grow(&b->pair_off, b->cap_pair_off, L.pairs));
   BATCH_TRY(b->grow(&b->mol_count, b->cap_mc, uint64_t(L.Gd) + 1));
@@ -2143,8 +1761,8 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
   // On overflow the counter still holds the exact demand, so one replay with that size
   // suffices; the capacity is kept for later runs.
   const double mean_k = Gq ? double(L.ksum) / Gq : 0.0;
-  // every wavefront may leave its chunk's tail and each lane its sub-chunk's tail unused
-  const uint64_t slack_arena = L.waves_total * 2 * sigmo_k::kWaveChunk;
+  // every wavefront starts with a chunk and may leave its last one's tail unused
+  const uint64_t slack_arena = 2 * L.first_chunks;
   const uint64_t guess = std::min<uint64_t>(std::max<uint64_t>(L.pairs / 8, 1 << 16), 1ull << 26);
   uint64_t want_arena = static_cast<uint64_t>(double(guess) * (mean_k + 1.0) * (db->num_wide ? 2.0 : 1.0)) + slack_arena;
   want_arena = std::max(want_arena, b->cap_arena);
@@ -2154,41 +1772,38 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
   // total are read after the join.  An arena overflow (data that changed) falls back to the
   // sized path below, which repeats the run.
   const uint64_t bound = uint64_t(Gq) * Gd;
+  if (!b->run_host) BATCH_HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&b->run_host), (kCounterWords + 1) * sizeof(unsigned long long)));
+  const unsigned long long* cnt = b->run_host;
   if (sized && !db->num_wide && bound && bound <= kOneSyncPairs && b->arena && b->cap_arena >= want_arena) {
-    if (!b->run_host) BATCH_HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&b->run_host), 16 * sizeof(unsigned long long)));
     BATCH_TRY(b->grow(&b->indices, b->cap_idx, bound));
     BATCH_TRY(b->grow(&b->pair_graph, b->cap_pg, bound));
     BATCH_TRY(b->grow(&b->mask_off, b->cap_mo, bound));
     BATCH_TRY(b->grow(&b->counts, b->cap_counts, bound));
     BATCH_TRY(b->grow(&b->deep_pairs, b->cap_deep, bound));
-    if (L.list_mode) BATCH_TRY(b->grow(&b->list, b->cap_list, bound));
     const double reads = (1.0 + 8.0 * R) * double(L.dd.N) + double(L.qd.N) * (1.0 + 2.0 * 16.0 * R) + double(Gq) * (4.0 + 8.0 * R);
     void* tok = nullptr;
     BATCH_TRY(ctx_timed(b->ctx, SIGMO_PHASE_FILTER, SIGMO_KERNEL_PAIR_FILTER, reads, true, &tok));
     BATCH_HIP_TRY(launch_filter(b, L, s));
     BATCH_TRY(ctx_timed(b->ctx, 0, 0, 0.0, false, &tok));
     res->one_sync = 1;
-    BATCH_HIP_TRY(hipMemcpyAsync(b->run_host, b->counters, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    BATCH_HIP_TRY(hipMemcpyAsync(b->run_host, b->counters, kCounterWords * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     BATCH_TRY(ctx_timed(b->ctx, SIGMO_PHASE_GMCR, -1, 0.0, true, &tok));
     BATCH_HIP_TRY(launch_count_scan(b, L, s));
     BATCH_HIP_TRY(launch_scatter(b, L, s));
     BATCH_TRY(ctx_timed(b->ctx, 0, 0, 0.0, false, &tok));
-    BATCH_HIP_TRY(hipMemcpyAsync(b->run_host + 8, b->total, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    BATCH_HIP_TRY(hipMemcpyAsync(b->run_host + kCounterWords, b->total, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     BATCH_TRY(ctx_timed(b->ctx, SIGMO_PHASE_JOIN, SIGMO_KERNEL_JOIN, 0.0, true, &tok));
     BATCH_HIP_TRY(sigmo_k::fill_u64(s, reinterpret_cast<uint64_t*>(stats), sigmo_k::kJoinStatWords, 0));
     BATCH_HIP_TRY(launch_join(b, L, s, stats, bound, find_first, reinterpret_cast<const unsigned long long*>(b->total)));
     BATCH_TRY(ctx_timed(b->ctx, 0, 0, 0.0, false, &tok));
     BATCH_HIP_TRY(hipMemcpyAsync(stats_host, stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     BATCH_HIP_TRY(hipStreamSynchronize(s));
-    const unsigned long long* cnt = b->run_host;
+    const uint64_t demand = read_counters(L.first_chunks, cnt, res);
     if (!cnt[3]) {
-      const uint64_t P = b->run_host[8];
+      const uint64_t P = b->run_host[kCounterWords];
       if (P >= (1ull << 32)) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "GMCR pair count exceeds u32");
       if (stats_host[3]) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "a per-pair match count exceeded int32");
-      ctx_add_bytes(b->ctx, SIGMO_KERNEL_PAIR_FILTER, double(cnt[1]) * 8.0 + double(Gd) * W * 8.0);
-      res->filter_wave_steps = cnt[4];
-      res->filter_lane_steps = cnt[5];
-      res->filter_scans = cnt[7];
+      ctx_add_bytes(b->ctx, SIGMO_KERNEL_PAIR_FILTER, double(demand) * 8.0 + double(Gd) * W * 8.0);
       b->P = P;
       b->Gq = Gq;
       b->ran = true;
@@ -2199,14 +1814,11 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
       res->join_wave_steps = stats_host[7];
       return SIGMO_OK;
     }
-    want_arena = std::max<uint64_t>(want_arena + 1, cnt[1] + cnt[1] / 8 + slack_arena);  // overflowed: size and repeat
+    want_arena = std::max<uint64_t>(want_arena + 1, demand + demand / 8 + slack_arena);  // overflowed: size and repeat
     res->arena_repeats = 1;
   }
-  // the pre-tested pair list (list mode): a quarter of the pairs at first, then the measured demand
-  uint64_t want_list = L.list_mode ? std::max<uint64_t>(b->cap_list, std::min<uint64_t>(L.pairs, L.pairs / 4 + 65536)) : 0;
   for (int attempt = 0; attempt < 4; ++attempt) {
     BATCH_TRY(b->grow(&b->arena, b->cap_arena, want_arena));
-    if (L.list_mode) BATCH_TRY(b->grow(&b->list, b->cap_list, want_list));
     if (b->cap_arena >= (1ull << 32)) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "candidate arena exceeds 2^32 words");
     // algorithmic reads: the data side once per run -- a label byte and R level signatures per
     // data node, (1 + 8R) D -- plus the query side; writes are added once they are known.
@@ -2215,22 +1827,18 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
     BATCH_TRY(ctx_timed(b->ctx, SIGMO_PHASE_FILTER, SIGMO_KERNEL_PAIR_FILTER, reads, true, &tok));
     BATCH_HIP_TRY(launch_filter(b, L, s));
     BATCH_TRY(ctx_timed(b->ctx, 0, 0, 0.0, false, &tok));
-    unsigned long long cnt[8];
-    BATCH_HIP_TRY(hipMemcpyAsync(cnt, b->counters, sizeof(cnt), hipMemcpyDeviceToHost, s));
+    BATCH_HIP_TRY(hipMemcpyAsync(b->run_host, b->counters, kCounterWords * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     BATCH_HIP_TRY(hipStreamSynchronize(s));
-    res->filter_wave_steps = cnt[4];
-    res->filter_lane_steps = cnt[5];
-    res->filter_scans = cnt[7];
-    if (cnt[7] >= (1ull << 32)) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "pre-tested pairs of one run exceed 2^32");
+    const uint64_t demand = read_counters(L.first_chunks, cnt, res);
+    if (res->filter_scans >= (1ull << 32)) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "pre-tested pairs of one run exceed 2^32");
     // writes: candidate masks, the survival bits and arena offsets
-    ctx_add_bytes(b->ctx, SIGMO_KERNEL_PAIR_FILTER, double(cnt[1]) * 8.0 + double(Gd) * W * 8.0);
+    ctx_add_bytes(b->ctx, SIGMO_KERNEL_PAIR_FILTER, double(demand) * 8.0 + double(Gd) * W * 8.0);
     if (!cnt[3]) break;
-    if (attempt == 3) return sigmo_err::set(SIGMO_ERR_NOMEM, "candidate arena or pair list overflowed repeatedly");
+    if (attempt == 3) return sigmo_err::set(SIGMO_ERR_NOMEM, "candidate arena overflowed repeatedly");
     res->arena_repeats++;
     // replay with the demand just measured; the claim order (and so the space left unused at
-    // sub-chunk ends) varies between runs, hence the 1/8 margin.  The list's demand is exact.
-    if (L.list_mode && cnt[7] > b->cap_list) want_list = cnt[7];
-    if (cnt[1] > b->cap_arena) want_arena = std::max<uint64_t>(want_arena + 1, cnt[1] + cnt[1] / 8 + slack_arena);
+    // chunk ends) varies between runs, hence the 1/8 margin
+    if (demand > b->cap_arena) want_arena = std::max<uint64_t>(want_arena + 1, demand + demand / 8 + slack_arena);
   }
   // canonical GMCR: count survivors per molecule, scan, scatter in (molecule, query graph) order
   void* tok = nullptr;
@@ -2278,7 +1886,7 @@ int sigmo_batch_set_tuning(sigmo_batch* b, const sigmo_batch_tuning* t) {
   if (!b || !t) return sigmo_err::set(SIGMO_ERR_INVALID, "null argument");
   if (t->join_blocks_per_cu > 4) return sigmo_err::set(SIGMO_ERR_INVALID, "join_blocks_per_cu must be 0..4");
   if (t->filter_claim > 64) return sigmo_err::set(SIGMO_ERR_INVALID, "filter_claim must be 0..64");
-  if (t->filter_mode > 2) return sigmo_err::set(SIGMO_ERR_INVALID, "filter_mode must be 0 (automatic), 1 (molecule) or 2 (list)");
+  if (t->filter_mode > 2) return sigmo_err::set(SIGMO_ERR_INVALID, "filter_mode must be 0..2");
   b->tune = *t;
   return SIGMO_OK;
 }
@@ -2309,10 +1917,8 @@ int sigmo_batch_autotune(sigmo_batch* b, const sigmo_graph* query, int find_firs
   sigmo_batch_tuning best_t{};
   double best = 0;
   BATCH_TRY(time_with(best_t, &best));
-  // coordinate search: pair evaluation mode and shape, then the join's
-  const uint32_t filter_modes[] = {1, 2};
+  // coordinate search: the pair evaluation's blocks, then the join's shape
   const uint32_t filter_blocks[] = {1, 2, 4, 0};
-  const uint32_t filter_claims[] = {2, 8, 32, 0};
   const uint32_t join_blocks[] = {2, 3, 4};
   const uint32_t join_chunks[] = {16, 64, 256, 0};
   auto sweep = [&](uint32_t sigmo_batch_tuning::*field, const uint32_t* vals, size_t n) -> int {
@@ -2329,9 +1935,7 @@ int sigmo_batch_autotune(sigmo_batch* b, const sigmo_graph* query, int find_firs
     }
     return SIGMO_OK;
   };
-  BATCH_TRY(sweep(&sigmo_batch_tuning::filter_mode, filter_modes, 2));
   BATCH_TRY(sweep(&sigmo_batch_tuning::filter_blocks_per_cu, filter_blocks, 4));
-  BATCH_TRY(sweep(&sigmo_batch_tuning::filter_claim, filter_claims, 4));
   BATCH_TRY(sweep(&sigmo_batch_tuning::join_blocks_per_cu, join_blocks, 3));
   BATCH_TRY(sweep(&sigmo_batch_tuning::join_chunk, join_chunks, 4));
   b->tune = best_t;
@@ -2352,14 +1956,13 @@ int sigmo_batch_capture(sigmo_batch* b, const sigmo_graph* query, int find_first
   const uint64_t nw = stats_host[5];
   RunShape L;
   BATCH_TRY(shape_run(b, query, cus, L));
-  if (!b->graph_host) BATCH_HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&b->graph_host), 32 * sizeof(unsigned long long)));
+  if (!b->graph_host) BATCH_HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&b->graph_host), (kCounterWords + 16) * sizeof(unsigned long long)));
   b->drop_graph();
   const sigmo_db* db = b->db;
   BATCH_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   hipError_t e = hipSuccess;
   if (refresh_db)
-    e = sigmo_k::db_prepare(s, L.dd, db->R, db->cls_list, db->pidx, db->wide_idx, db->planes32, db->planes64, db->planes_hi, db->lab_hi,
-                            db->dmax, db->minfo, db->cls, db->cmax, db->cls_count[0]);
+    e = sigmo_k::db_prepare(s, L.dd, db->R, db->cls_list, db->order, db->planes, db->labs, db->dmax, db->minfo, db->cls, db->cmax);
   if (e == hipSuccess) e = sigmo_k::query_prepare(s, L.qd, L.R, b->tokens, b->qinfo, b->qmax, db->cls, b->qcmax);
   if (e == hipSuccess) e = launch_filter(b, L, s);
   if (e == hipSuccess) e = launch_count_scan(b, L, s);
@@ -2369,9 +1972,9 @@ int sigmo_batch_capture(sigmo_batch* b, const sigmo_graph* query, int find_first
   // replay on changed data reads only entries the replay itself wrote
   if (e == hipSuccess) e = launch_join(b, L, s, stats, b->P, find_first, reinterpret_cast<const unsigned long long*>(b->total));
   if (e == hipSuccess && db->num_wide) e = launch_join_wide(b, L, s, stats, nw, find_first, stats + 5);
-  if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host, b->counters, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host + 8, b->total, sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host + 9, stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host, b->counters, kCounterWords * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host + kCounterWords, b->total, sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host + kCounterWords + 1, stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
   hipGraph_t g = nullptr;
   const hipError_t end = hipStreamEndCapture(s, &g);
   if (e != hipSuccess || end != hipSuccess) {
@@ -2406,21 +2009,20 @@ int sigmo_batch_replay(sigmo_batch* b, sigmo_batch_result* res) {
   BATCH_TRY(ctx_timed(b->ctx, 0, 0, 0.0, false, &tok));
   BATCH_HIP_TRY(hipStreamSynchronize(s));
   const unsigned long long* h = b->graph_host;
-  if (h[3] || h[8] != b->graph_P || (b->db->num_wide && h[9 + 5] != b->graph_nw)) {
+  const unsigned long long* js = h + kCounterWords + 1;  // join statistics
+  if (h[3] || h[kCounterWords] != b->graph_P || (b->db->num_wide && js[5] != b->graph_nw)) {
     return sigmo_err::set(SIGMO_ERR_INVALID, "the captured graph no longer matches the data (arena or pair counts changed): capture again");
   }
-  if (h[9 + 3]) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "a per-pair match count exceeded int32");
+  if (js[3]) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "a per-pair match count exceeded int32");
   b->P = b->graph_P;
   b->Gq = b->graph_Gq;
   b->ran = true;
-  res->num_matches = h[9 + 0];
-  res->matched_pairs = h[9 + 1];
+  res->num_matches = js[0];
+  res->matched_pairs = js[1];
   res->gmcr_pairs = b->graph_P;
-  res->dfs_steps = h[9 + 4];
-  res->join_wave_steps = h[9 + 7];
-  res->filter_wave_steps = h[4];
-  res->filter_lane_steps = h[5];
-  res->filter_scans = h[7];
+  res->dfs_steps = js[4];
+  res->join_wave_steps = js[7];
+  read_counters(0, h, res);
   return SIGMO_OK;
 }
 

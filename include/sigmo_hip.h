@@ -258,9 +258,12 @@ typedef struct sigmo_pipeline_result {
 } sigmo_pipeline_result;
 /* Runs gen(D), gen(Q), filter, R x {refsig(D,r), refsig(Q,r), refine}, GMCR, join on
  * device-resident graphs, with one launch per phase; allocates and frees its buffers.  With
- * R >= 1 the filter runs after the level-1 signature passes, fused with the first refine into one
- * launch (the same bits: the filter reads no signatures, the signature passes no candidates);
- * sigmo_kernel_stats then counts that launch under SIGMO_KERNEL_FILTER and R - 1 refines. */
+ * 1 <= R <= 8 (and memory for every level's signature planes) each side's signatures of all levels
+ * are one launch, and the filter with all refinements is another, which writes each bitset word
+ * once (the same bits: the filter reads no signatures, the signature passes no candidates, and the
+ * tests AND); otherwise the filter is fused with the first refine.  sigmo_kernel_stats counts a
+ * launch that does several's work once for each -- one SIG_GENERATE and R SIG_REFINE, one FILTER and
+ * R - 1 REFINE -- with its time and bytes shared out equally. */
 int sigmo_pipeline_run(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_graph* data, uint32_t refinement_steps,
                        int find_first, sigmo_pipeline_result* result);
 

@@ -39,25 +39,14 @@ constexpr uint32_t kMaxLevels = 8;        // token encoding keeps 3 bits of leve
 constexpr uint16_t kEndToken = 0xFFFF;    // closes a query node's token segment
 
 // Tokens of one query node: [label] [requirement]* [end], requirement = r | l << 3 | c << 7
-// (level r < 8, label l < 16, count 1 <= c <= 15).  Segments are 4-token aligned with one spare
+// (level r < 8, label l < 16, count 1 <= c <= 15; those of counts up to kNearCount first).  Segments are 4-token aligned with one spare
 // word, so the reader's one-word lookahead stays inside the segment.
 __host__ __device__ constexpr uint32_t token_segment(uint32_t R) { return ((2 + 16 * R + 3) & ~3u) + 4; }
 
-// Level-r sphere of every node, one BFS layer per call (the reachables of the reference are
-// the BFS ball of the previous level when levels are refined in order).  Positions are taken
-// mod 64: bit b of the frontier expands node prev + b, as in signature.hpp:336-390.
-__device__ __forceinline__ uint64_t next_layer(const GraphDev& g, uint32_t prev, uint64_t& ball, uint64_t& frontier) {
-  uint64_t next = 0, f = frontier;
-  while (f) {
-    const uint32_t b = __builtin_ctzll(f);
-    f &= f - 1;
-    const uint64_t u = static_cast<uint64_t>(prev) + b;
-    next |= g.fold[u];
-  }
-  next &= ~ball;
-  ball |= next;
-  frontier = next;
-  return next;
+// Bit 0 of every nonzero nibble.
+__device__ __forceinline__ uint64_t nibbles_set(uint64_t x) {
+  x |= x >> 2;
+  return (x | (x >> 1)) & 0x1111111111111111ull;
 }
 
 // 16 four-bit label counts of the nodes in r (labels >= 16 are not counted; counts saturate
@@ -97,7 +86,6 @@ struct alignas(16) MolInfo {
 // Per-query-graph facts the pair pre-test reads.
 struct QueryInfo {
   uint32_t qoff, k, qlab, qcls;  // first node, nodes, labels < 16 present, signature classes present (bit c)
-  uint64_t first;                // first token word of the graph's first node
 };
 
 // The database's signature classes: up to three labels (< 16), the database's most frequent, for
@@ -402,25 +390,33 @@ __global__ __launch_bounds__(256) void k_db_prepare_pairs(GraphDev g, uint32_t R
 // starts at the word after the one holding the current node's end token.
 __global__ __launch_bounds__(256) void k_query_prepare(GraphDev q, uint32_t R, uint16_t* __restrict__ tokens,
                                                        QueryInfo* __restrict__ qinfo, uint64_t* __restrict__ qmax) {
+  __shared__ uint64_t fold_all[4][kWave];
   const uint32_t lane = static_cast<uint32_t>(lane_id());
   const uint64_t g = static_cast<uint64_t>(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave;
-  if (g >= q.G) return;  // wave-uniform
+  if (g >= q.G) return;  // wave-uniform; no block barrier follows
   const uint32_t prev = q.go[g], k = q.go[g + 1] - prev;
   const bool valid = lane < k;
   const uint32_t seg = token_segment(R);
   const uint32_t label = valid ? q.nl[prev + lane] : 0u;
+  // the graph's adjacency in LDS: a level's expansion then waits on no memory
+  uint64_t* fold = fold_all[threadIdx.x / kWave];
+  fold[lane] = valid ? q.fold[static_cast<uint64_t>(prev) + lane] : 0ull;
+  wave_sync();
   // the node's level signatures, and its token count: label + one per nonzero nibble + end
   uint64_t sig[kMaxLevels];
-  uint64_t self = 1ull << (lane & 63), ball = self, frontier = self;
+  uint64_t self = 1ull << (lane & 63), ball = self, frontier = valid ? self : 0ull;
   uint32_t ntok = 2;
 #pragma unroll
   for (uint32_t r = 0; r < kMaxLevels; ++r) {
     sig[r] = 0;
     if (r < R) {
-      if (valid) {
-        sig[r] = histogram16(next_layer(q, prev, ball, frontier), q.lmask + g * 16);
-        for (uint32_t l = 0; l < 16; ++l) ntok += ((sig[r] >> (4 * l)) & 15u) != 0;
-      }
+      uint64_t next = 0;
+      for (; frontier; frontier &= frontier - 1) next |= fold[__builtin_ctzll(frontier)];
+      next &= ~ball;
+      ball |= next;
+      frontier = next;
+      if (next) sig[r] = histogram16(next, q.lmask + g * 16);
+      ntok += static_cast<uint32_t>(__popcll(nibbles_set(sig[r])));
       const uint64_t mx = wave_nib_max(sig[r]);
       if (lane == 0) qmax[g * R + r] = mx;
     }
@@ -434,24 +430,20 @@ __global__ __launch_bounds__(256) void k_query_prepare(GraphDev q, uint32_t R, u
     if (lane >= static_cast<uint32_t>(o)) incl += y;
   }
   uint16_t* t = tokens + static_cast<uint64_t>(prev) * seg + (incl - len);
-  uint64_t first = label;  // lane 0: the first four tokens of node 0
-  uint32_t cnt = 1;
   if (valid) {
     t[0] = static_cast<uint16_t>(label);
+    uint32_t at = 1, back = ntok - 1;  // near requirements from the front, the others from the back
+    t[back] = kEndToken;
 #pragma unroll
     for (uint32_t r = 0; r < kMaxLevels; ++r)
       if (r < R)
-        for (uint32_t l = 0; l < 16; ++l) {
-          const uint32_t c = static_cast<uint32_t>(sig[r] >> (4 * l)) & 15u;
-          if (c) {
-            const uint32_t tk = r | (l << 3) | (c << 7);
-            if (cnt < 4) first |= static_cast<uint64_t>(tk) << (16 * cnt);
-            t[cnt++] = static_cast<uint16_t>(tk);
-          }
+        for (uint64_t nz = nibbles_set(sig[r]); nz; nz &= nz - 1) {
+          const uint32_t sh = static_cast<uint32_t>(__builtin_ctzll(nz)), c = static_cast<uint32_t>(sig[r] >> sh) & 15u;
+          const uint16_t tk = static_cast<uint16_t>(r | (sh << 1) | (c << 7));  // label = sh / 4, at bit 3
+          if (c <= kNearCount) t[at++] = tk;
+          else t[--back] = tk;
         }
-    t[cnt] = kEndToken;
   }
-  if (cnt < 4) first |= static_cast<uint64_t>(kEndToken) << (16 * cnt);
   uint32_t bits = valid && label < 16 ? 1u << label : 0u;
 #pragma unroll
   for (int o = kWave / 2; o > 0; o >>= 1) bits |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), o));
@@ -461,7 +453,6 @@ __global__ __launch_bounds__(256) void k_query_prepare(GraphDev q, uint32_t R, u
     info.k = k;
     info.qlab = bits;
     info.qcls = 0;  // set by k_query_classes
-    info.first = first;
     qinfo[g] = info;
   }
 }
@@ -696,7 +687,7 @@ struct GroupArgs {
   unsigned long long* stats;     // kGroupStatSlots x 16: [0] node evaluations, [1] their live lanes, [2] pre-tested pairs
 };
 
-// LDS: planes [label slot][level][lane] (16 bytes), label masks [label slot][lane], the next item.
+// LDS: near planes [label slot][level][count][lane], label masks [label slot][lane], the next item.
 __host__ __device__ constexpr uint32_t group_lds_bytes(uint32_t slots, uint32_t R) { return slots * (R * 1024 + 256) + 16; }
 
 // The value of lane ^ 1 and lane ^ 2 (quad permutations).
@@ -714,19 +705,10 @@ struct GroupState {
   uint32_t live = 0;  // per lane
 };
 
-// One requirement on 32 positions (isomorphism.hpp:103-110), count_q(l) <= count_p(l) at level r:
-// the decoded token is a scalar, so the count's bit masks (bits 20..23) are too.
-__device__ __forceinline__ uint32_t group_test(uint32_t tk, const uint4& v) {
-  uint32_t ge = ge_first(v.x, static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(tk), 20, 1)));
-  ge = ge_stage(v.y, static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(tk), 21, 1)), ge);
-  ge = ge_stage(v.z, static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(tk), 22, 1)), ge);
-  return ge_stage(v.w, static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(tk), 23, 1)), ge);
-}
-
 // One group of a class against the wavefront's share of the query graphs.
 template <int CLS>
-__device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uint32_t part, uint32_t wave, uint4* planes_lds, uint32_t* labs_lds,
-                                           uint32_t off_mask, GroupState& st) {
+__device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uint32_t part, uint32_t wave, uint32_t* near_lds, uint32_t* labs_lds,
+                                           GroupState& st) {
   const uint32_t lane = static_cast<uint32_t>(lane_id());
   const uint32_t R = a.R;
   const uint32_t seg = token_segment(R);
@@ -761,7 +743,7 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
 #pragma unroll
     for (uint32_t x = 0; x < 4; ++x) {
       const uint32_t e = e0 + x * kGroupWaves;
-      if (e < staged * R) planes_lds[e * kWave + lane] = v[x];
+      if (e < staged * R) stage_near(near_lds, e, v[x]);
     }
   }
   for (uint32_t slot = wave; slot < staged; slot += kGroupWaves)
@@ -801,25 +783,21 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
       st.next += static_cast<uint64_t>(cnt) * pw;
       const bool room = st.end <= a.arena_cap;
 
-      // the graph's tokens, 64 at a time and one per lane, decoded once: a requirement becomes its
-      // planes' byte offset in LDS (bits 10..16) and its count (bits 20..23); `far` is set when a
-      // label's planes are not there
+      // the graph's tokens, 64 at a time and one per lane, decoded once: a near requirement becomes
+      // its plane's offset in LDS; `fars` marks the others (a large count, or a label whose planes
+      // are not there)
       const uint16_t* tok = a.tokens + static_cast<uint64_t>(qoff) * seg;
       const uint32_t total = k * seg;
       uint32_t pos = 0, p = 0, raw = 0, dec = 0;
-      uint64_t ends = 0;
-      bool far = false;
+      uint64_t ends = 0, fars = 0;
       auto load_tokens = [&](uint32_t from) {
         pos = from;
         p = 0;
         raw = tok[min(from + lane, total - 1)];
-        const uint32_t slot = static_cast<uint32_t>(__popc(present & ((1u << ((raw >> 3) & 15u)) - 1u)));
-        dec = (((slot * R + (raw & 7u)) * (kWave * 16)) & 0x1FC00u) | (((raw >> 7) & 15u) << 20);
-        far = staged < occur && __ballot(raw != kEndToken && slot >= staged) != 0;
+        const uint32_t r = raw & 7u, c = (raw >> 7) & 15u, slot = static_cast<uint32_t>(__popc(present & ((1u << ((raw >> 3) & 15u)) - 1u)));
+        dec = near_offset(slot * R + r, c);
+        fars = __ballot(c > kNearCount || slot >= staged);
         ends = __ballot(raw == kEndToken);
-      };
-      auto planes = [&](uint32_t tk) -> uint4 {
-        return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(planes_lds) + ((tk & off_mask) | (lane * 16)));
       };
       // the candidates of the next node among this lane's positions; leaves p at the node after
       auto node_mask = [&]() -> uint32_t {
@@ -842,30 +820,18 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
               if (a.d.nl[static_cast<uint64_t>(mi.s) + 32 * h + x] == ql) mask |= 1u << x;
           }
         }
-        if (!far) {
-          for (; t + 4 <= e; t += 4) {
-            const uint32_t k0 = rl32(dec, t), k1 = rl32(dec, t + 1), k2 = rl32(dec, t + 2), k3 = rl32(dec, t + 3);
-            const uint4 v0 = planes(k0), v1 = planes(k1), v2 = planes(k2), v3 = planes(k3);
-            mask &= group_test(k0, v0) & group_test(k1, v1);
-            mask &= group_test(k2, v2) & group_test(k3, v3);
-          }
-          if (t + 2 <= e) {
-            const uint32_t k0 = rl32(dec, t), k1 = rl32(dec, t + 1);
-            const uint4 v0 = planes(k0), v1 = planes(k1);
-            mask &= group_test(k0, v0) & group_test(k1, v1);
-            t += 2;
-          }
-          if (t < e) {
-            const uint32_t k0 = rl32(dec, t);
-            mask &= group_test(k0, planes(k0));
-          }
-        } else {
-          for (; t < e; ++t) {
-            const uint32_t tw = rl32(raw, t), l = (tw >> 3) & 15u, k0 = rl32(dec, t);
+        // near requirements come first in a node's stream
+        const uint64_t fm = t < kWave ? fars >> t : 0ull;
+        const uint32_t near = fm ? min(e, t + static_cast<uint32_t>(__builtin_ctzll(fm))) : e;
+        mask = near_tests(near_lds, dec, t, near, mask);
+        for (t = near; t < e; ++t) {
+          if (!((fars >> t) & 1ull)) {
+            mask &= near_plane(near_lds, rl32(dec, t));
+          } else {
+            const uint32_t tw = rl32(raw, t);
             uint4 v = make_uint4(0, 0, 0, 0);
-            if (static_cast<uint32_t>(__popc(present & ((1u << l) - 1u))) < staged) v = planes(k0);
-            else if (valid) v = a.planes[((group * R + (tw & 7u)) * 16 + l) * 64 + lane];
-            mask &= group_test(k0, v);
+            if (valid) v = a.planes[((group * R + (tw & 7u)) * 16 + ((tw >> 3) & 15u)) * 64 + lane];
+            mask &= ge4_bits<uint32_t>(v.x, v.y, v.z, v.w, (tw >> 7) & 15u);
           }
         }
         ++st.nodes;
@@ -915,8 +881,8 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
 // and :103-110), keeping the masks of the pairs that survive GMCR.
 //
 // A wavefront takes one query graph and one group, 64 lanes of neighbours in the width-class
-// order, so a requirement's level, label and count are scalars: a test is one 16-byte LDS read and
-// seven vector operations for 64 x 32 positions.  A lane that walked a pair of its own decoded
+// order, so a requirement's level, label and count are scalars: a near test is one LDS read and
+// three vector operations for 64 x 32 positions.  A lane that walked a pair of its own decoded
 // every token for itself and gathered its token words and planes, about 40 operations a test, and
 // a wavefront waited for its longest pair.  The order groups molecules of one label set and
 // similar size, so a query graph passes the pre-test for none of a group's molecules three times
@@ -933,8 +899,8 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
 // graphs 219 -> 12 us (three serial chains of ~100 us), 100,000 x 100 475 -> 125 us, 1 M x 25
 // 1,242 -> 392 us, 1 M x 1,000 10.7 -> 6.8 ms.
 __global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a) {
-  extern __shared__ uint4 lds4[];
-  uint32_t* labs = reinterpret_cast<uint32_t*>(lds4 + static_cast<uint64_t>(a.slots) * a.R * kWave);
+  extern __shared__ uint32_t near_lds[];
+  uint32_t* labs = near_lds + static_cast<uint64_t>(a.slots) * a.R * kNearCount * kWave;
   unsigned long long* next_item = reinterpret_cast<unsigned long long*>(labs + a.slots * kWave);
   const uint32_t wave = uniform32(threadIdx.x / kWave);
   const uint32_t g0 = a.order.groups(0), g1 = a.order.groups(1);
@@ -944,14 +910,12 @@ __global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a)
   st.end = st.next + a.chunk;
   st.first_chunks = static_cast<uint64_t>(gridDim.x) * kGroupWaves * a.chunk;
   if (blockIdx.x == 0 && threadIdx.x == 0 && st.first_chunks > a.arena_cap) atomicOr(&a.counters[3], 1ull);
-  uint32_t off_mask = 0x1FC00u;
-  asm volatile("" : "+v"(off_mask));  // in a vector register: the and-or of a token's offset and the lane's is then one operation
   for (uint64_t item = blockIdx.x; item < items;) {
     const uint32_t part = static_cast<uint32_t>(item & (a.parts - 1));
     const uint32_t grp = static_cast<uint32_t>(item / a.parts);
-    if (grp < g0) group_item<0>(a, grp, part, wave, lds4, labs, off_mask, st);
-    else if (grp < g0 + g1) group_item<1>(a, grp - g0, part, wave, lds4, labs, off_mask, st);
-    else group_item<2>(a, grp - g0 - g1, part, wave, lds4, labs, off_mask, st);
+    if (grp < g0) group_item<0>(a, grp, part, wave, near_lds, labs, st);
+    else if (grp < g0 + g1) group_item<1>(a, grp - g0, part, wave, near_lds, labs, st);
+    else group_item<2>(a, grp - g0 - g1, part, wave, near_lds, labs, st);
     if (gridDim.x >= items) break;
     __syncthreads();  // the staged planes have been read
     if (threadIdx.x == 0) *next_item = gridDim.x + atomicAdd(&a.counters[2], 1ull);

@@ -67,6 +67,8 @@ struct sigmo_ctx {
     double bytes;
     uint64_t seq;
     bool shared_a;  // `a` is the previous phase's end event (returned to the pool with it)
+    int kernel2;    // a launch that does several's work counts `n` times for kernel and `n2` for kernel2,
+    uint32_t n, n2; // its time and bytes shared out equally
   };
   uint64_t launch_seq = 0;          // sequence number of the next timed launch
   uint64_t launch_base = 0;         // sequence number of launch_ms[0]
@@ -108,10 +110,16 @@ struct sigmo_ctx {
         if (launch_ms.size() <= i) launch_ms.resize(i + 1, 0.0);
         launch_ms[i] = ms;
       }
+      const double share = 1.0 / (t.n + t.n2);
       if (t.kernel >= 0) {
-        k_launches[t.kernel] += 1;
-        k_ms[t.kernel] += ms;
-        k_bytes[t.kernel] += t.bytes;
+        k_launches[t.kernel] += t.n;
+        k_ms[t.kernel] += ms * t.n * share;
+        k_bytes[t.kernel] += t.bytes * t.n * share;
+      }
+      if (t.kernel2 >= 0) {
+        k_launches[t.kernel2] += t.n2;
+        k_ms[t.kernel2] += ms * t.n2 * share;
+        k_bytes[t.kernel2] += t.bytes * t.n2 * share;
       }
       if (!t.shared_a) pool.push_back(t.a);
       pool.push_back(t.b);
@@ -138,7 +146,10 @@ struct PhaseScope {
   hipEvent_t a = nullptr;
   bool shared_a = false;
   int status = SIGMO_OK;
-  PhaseScope(sigmo_ctx* ctx, int ph, int k = -1, double by = 0) : c(ctx), phase(ph), kernel(k), bytes(by) {
+  int kernel2;
+  uint32_t n, n2;
+  PhaseScope(sigmo_ctx* ctx, int ph, int k = -1, double by = 0, uint32_t cnt = 1, int k2 = -1, uint32_t cnt2 = 0)
+      : c(ctx), phase(ph), kernel(k), bytes(by), kernel2(k2), n(cnt), n2(cnt2) {
     if (c->capturing) return;  // a graph records no timing events
     if (c->chain && c->chain_end) {
       a = c->chain_end;
@@ -155,7 +166,7 @@ struct PhaseScope {
     hipEvent_t b;
     SIGMO_TRY(c->event(&b));
     SIGMO_HIP_TRY(hipEventRecord(b, c->stream));
-    c->pending.push_back({a, b, phase, kernel, bytes, c->launch_seq++, shared_a});
+    c->pending.push_back({a, b, phase, kernel, bytes, c->launch_seq++, shared_a, kernel2, n, n2});
     if (c->chain) c->chain_end = b;
     a = nullptr;
     return SIGMO_OK;
@@ -1352,6 +1363,10 @@ struct sigmo_pipeline {
   sigmo_candidates* cand = nullptr;
   sigmo_gmcr* gm = nullptr;
   bool has_counts = false;
+  // every level's data planes and query tokens (k_sig_levels, k_query_levels)
+  uint8_t* lvl = nullptr;
+  uint32_t* qtok = nullptr;
+  uint64_t cap_lvl = 0, cap_qtok = 0;
   // a captured execute (sigmo_pipeline_capture)
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
@@ -1366,6 +1381,8 @@ struct sigmo_pipeline {
   ~sigmo_pipeline() {
     drop_graph();
     if (replay_host) (void)hipHostFree(replay_host);
+    dev_free(lvl);
+    dev_free(qtok);
     sigmo_signatures_free(sig);
     sigmo_candidates_free(cand);
     sigmo_gmcr_free(gm);
@@ -1388,6 +1405,17 @@ int candidates_filter_refine(sigmo_ctx* ctx, sigmo_candidates* c, const sigmo_gr
   return ps.close();
 }
 
+// Room for every level's planes and tokens, when the levels fit the sweep's token and LDS layout and
+// the device has the memory (U/2 bytes per data node and level); otherwise the pipeline refines
+// level by level.
+bool pipeline_levels(sigmo_pipeline* p, uint32_t R) {
+  const sigmo_k::LabelSlots& slots = p->q->slots;
+  if (R < 1 || R > 8 || slots.count < 1 || !p->q->N || !p->d->N) return false;
+  const uint64_t lvl = sigmo_k::level_planes_bytes(std::max(p->sig->capD, p->d->N), R, static_cast<uint32_t>(slots.count));
+  if (p->ctx->capturing) return p->lvl && p->qtok && p->cap_lvl >= lvl && p->cap_qtok >= sigmo_k::level_tokens(p->q->N);
+  return grow(&p->qtok, p->cap_qtok, sigmo_k::level_tokens(p->q->N)) == SIGMO_OK && grow(&p->lvl, p->cap_lvl, lvl) == SIGMO_OK;
+}
+
 int pipeline_enqueue(sigmo_pipeline* p, uint32_t refinement_steps, int find_first, uint64_t* matches) {
   sigmo_ctx* ctx = p->ctx;
   sigmo_signatures* sig = p->sig;
@@ -1402,6 +1430,31 @@ int pipeline_enqueue(sigmo_pipeline* p, uint32_t refinement_steps, int find_firs
       c->chain_end = nullptr;
     }
   } chain(ctx);
+  if (pipeline_levels(p, refinement_steps)) {
+    const uint32_t R = refinement_steps;
+    const sigmo_k::LabelSlots& slots = p->q->slots;
+    const sigmo_candidates* c = p->cand;
+    const double level_bytes = 0.5 * slots.count * c->D * R;  // planes of every level
+    {
+      PhaseScope ps(ctx, SIGMO_PHASE_SIG_DATA, SIGMO_KERNEL_SIG_GENERATE, 4.0 * (p->d->N + 1) + 4.0 * p->d->E + p->d->N + level_bytes, 1,
+                    SIGMO_KERNEL_SIG_REFINE, R);
+      SIGMO_HIP_TRY(sigmo_k::sig_levels(ctx->stream, p->d->dev(), R, slots, p->lvl));
+      SIGMO_TRY(ps.close());
+    }
+    {
+      PhaseScope ps(ctx, SIGMO_PHASE_SIG_QUERY, -1, 0.0);
+      SIGMO_HIP_TRY(sigmo_k::query_levels(ctx->stream, p->q->dev(), R, slots, p->qtok));
+      SIGMO_TRY(ps.close());
+    }
+    {
+      PhaseScope ps(ctx, SIGMO_PHASE_FILTER, SIGMO_KERNEL_FILTER, 8.0 * c->Q * c->W64 + c->D + level_bytes + 128.0 * c->Q, 1,
+                    SIGMO_KERNEL_REFINE, R - 1);
+      SIGMO_HIP_TRY(sigmo_k::filter_levels(ctx->stream, p->qtok, c->Q, p->d->lplanes, p->lvl, c->D, R, slots, c->bits, ctx->num_cus));
+      SIGMO_TRY(ps.close());
+    }
+    SIGMO_TRY(gmcr_generate(ctx, p->gm, p->q, p->d, p->cand, true));
+    return sigmo_join(ctx, p->q, p->d, p->cand, p->gm, find_first, matches, nullptr);
+  }
   // every run starts from the constructor's state: zero signatures and empty reachables, taken
   // as such by the first generate and the first refinement (no clearing pass)
   sig->dstate.reset();

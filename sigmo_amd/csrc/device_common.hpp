@@ -128,4 +128,47 @@ __device__ __forceinline__ T ge4_bits(T x0, T x1, T x2, T x3, uint32_t c) {
   }
 }
 
+// The pair evaluation and the pipeline's sweep test 32 positions per lane against requirements
+// (label l at level r, count c >= 1) that are scalars.  For c <= 4, nine of ten or more, LDS holds
+// the positions whose count reaches c (thermometer planes, made from the bit planes when they are
+// staged), so a test is one 4-byte read and one AND; larger counts compare the bit planes.
+constexpr uint32_t kNearCount = 4;
+
+// The thermometer planes of counts 1..4 from a label's four bit planes.
+__device__ __forceinline__ void thermometer(const uint4& x, uint32_t t[kNearCount]) {
+  const uint32_t high = x.z | x.w;
+  t[0] = x.x | x.y | high;
+  t[1] = x.y | high;
+  t[2] = (x.x & x.y) | high;
+  t[3] = high;
+}
+// Byte offset in LDS of the plane of count c for entry e = label slot * R + level.
+__device__ __forceinline__ uint32_t near_offset(uint32_t e, uint32_t c) { return (e * kNearCount + c - 1) * (kWave * 4); }
+// A wavefront stages entry e.
+__device__ __forceinline__ void stage_near(uint32_t* lds, uint32_t e, const uint4& x) {
+  uint32_t t[kNearCount];
+  thermometer(x, t);
+#pragma unroll
+  for (uint32_t c = 0; c < kNearCount; ++c) lds[(e * kNearCount + c) * kWave + lane_id()] = t[c];
+}
+__device__ __forceinline__ uint32_t near_plane(const uint32_t* lds, uint32_t off) {
+  return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(lds) + (off | static_cast<uint32_t>(lane_id() * 4)));
+}
+// ANDs the near requirements of lanes [t, e) of `dec` (their byte offsets) into mask.
+__device__ __forceinline__ uint32_t near_tests(const uint32_t* lds, uint32_t dec, uint32_t t, uint32_t e, uint32_t mask) {
+  for (; t + 4 <= e; t += 4) {
+    const uint32_t v0 = near_plane(lds, rl32(dec, t)), v1 = near_plane(lds, rl32(dec, t + 1));
+    const uint32_t v2 = near_plane(lds, rl32(dec, t + 2)), v3 = near_plane(lds, rl32(dec, t + 3));
+    mask &= v0 & v1;
+    mask &= v2 & v3;
+  }
+  if (t + 2 <= e) {
+    const uint32_t v0 = near_plane(lds, rl32(dec, t)), v1 = near_plane(lds, rl32(dec, t + 1));
+    mask &= v0 & v1;
+    t += 2;
+  }
+  if (t < e) mask &= near_plane(lds, rl32(dec, t));
+  return mask;
+}
+
 }  // namespace sigmo_k

@@ -646,6 +646,171 @@ __global__ __launch_bounds__(kBitsBlock) void k_filter_refine(const uint8_t* __r
   }
 }
 
+// ---- all levels at once (the pipeline) ------------------------------------------------------
+//
+// The pipeline's filter and R refinements AND independent tests, so they run as one sweep over the
+// bitset once every level's signatures are known: each word is written once, where a pass per
+// level read the bitset and wrote most of it again.
+
+constexpr uint32_t kStripNodes = 2048;    // data nodes of one strip: 64 lanes of 32
+constexpr uint32_t kLevelTokens = 32;     // words per query node: up to 31 requirements, then count | label << 8
+constexpr uint32_t kLevelWaves = 16;      // wavefronts per block of the sweep
+
+// Data signatures of levels 1..R (signature.hpp:336-390 with view sizes 1, 2, ..., R from empty
+// reachables), as bit planes of the labels in `slots`: lvl[((strip*R + r)*U + u)*64 + lane] holds
+// the four planes of label slots.label[u] at level r+1 over the lane's 32 nodes.  The BFS state
+// stays in registers from level to level; as one launch per level it took 57 bytes per node and
+// level through HBM (100,000 molecules, R = 6: 319 us in seven launches, 113 us here).
+__global__ __launch_bounds__(kSigBlock) void k_sig_levels(GraphDev g, uint32_t R, LabelSlots slots, uint4* __restrict__ lvl) {
+  constexpr uint32_t WPB = kSigBlock / kWave;
+  __shared__ uint64_t tile[2][64 * WPB];
+  __shared__ uint64_t lms[kStagedGraphs * 16];
+  __shared__ uint64_t fold[kStagedRows];
+  const uint64_t v = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
+  const bool live = v < g.N;
+  const uint32_t gid = live ? g.node_graph[v] : 0u;
+  const uint32_t prev = live ? g.go[gid] : 0u;
+  uint32_t g0 = 0;
+  uint64_t a0 = 0;
+  const bool staged = stage_block(g, lms, fold, g0, a0);
+  const uint32_t U = static_cast<uint32_t>(slots.count);
+  const uint64_t* lm = staged ? nullptr : g.lmask + static_cast<uint64_t>(gid) * 16;
+  const uint64_t strip = static_cast<uint64_t>(blockIdx.x) * kSigBlock / kStripNodes;
+  const uint32_t lane0 = static_cast<uint32_t>(blockIdx.x * static_cast<uint64_t>(kSigBlock) % kStripNodes / 32);
+  const uint64_t self = live ? 1ull << ((static_cast<uint32_t>(v) - prev) & 63u) : 0ull;
+  uint64_t ball = self, frontier = self;
+  for (uint32_t r = 0; r < R; ++r) {
+    uint64_t s = 0;
+    if (frontier) {
+      uint64_t next = staged ? expand_frontier_lds(fold, prev - a0, frontier) : expand_frontier(g.fold, prev, frontier);
+      next &= ~ball;
+      ball |= next;
+      frontier = next;
+      if (next)
+        for (uint32_t u = 0; u < U; ++u) {  // counts saturate at 15 (signature.hpp:44-51)
+          const uint32_t l = slots.label[u];
+          uint32_t c = static_cast<uint32_t>(__popcll(next & (staged ? lms[(gid - g0) * 16 + l] : lm[l])));
+          c = c < 15 ? c : 15;
+          s |= static_cast<uint64_t>(c) << (4 * l);
+        }
+    }
+    uint64_t* t = tile[r & 1];  // two tiles: one barrier a level
+    t[lane_id() * WPB + threadIdx.x / kWave] = transpose64(s);
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < U * 2 * WPB; e += kSigBlock) {
+      const uint32_t u = e / (2 * WPB), x = e % (2 * WPB), p = 4u * slots.label[u];
+      uint32_t w[4];
+#pragma unroll
+      for (uint32_t b = 0; b < 4; ++b) {
+        const uint64_t q = t[(p + b) * WPB + x / 2];
+        w[b] = static_cast<uint32_t>((x & 1u) ? q >> 32 : q);
+      }
+      lvl[((strip * R + r) * U + u) * 64 + lane0 + x] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  }
+}
+
+// Query signatures of levels 1..R as requirement tokens, a wavefront per query graph (<= 32 nodes)
+// and a lane per node: for each nonzero count of label slots.label[u] at level r+1 (at most 31: each
+// needs a node of its own) the LDS offset of its plane when it is near (near_offset), else
+// (u*R + r) << 8 | count; near ones first, as long as their label is one of the first `staged`.
+// tok[node*32 + 31] = near tokens | all tokens << 8 | node label << 16.
+__global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, LabelSlots slots, uint32_t staged, uint32_t* __restrict__ tok) {
+  __shared__ uint64_t fold_all[4][kWave];
+  const uint32_t lane = static_cast<uint32_t>(lane_id());
+  const uint32_t g = blockIdx.x * 4 + threadIdx.x / kWave;
+  if (g >= q.G) return;  // wave-uniform; no block barrier follows
+  const uint32_t s = q.go[g], k = q.go[g + 1] - s;
+  uint64_t* fold = fold_all[threadIdx.x / kWave];
+  fold[lane] = lane < k ? q.fold[static_cast<uint64_t>(s) + lane] : 0ull;
+  wave_sync();
+  if (lane >= k) return;
+  uint32_t* out = tok + (static_cast<uint64_t>(s) + lane) * kLevelTokens;
+  uint64_t ball = 1ull << lane, frontier = ball;
+  uint32_t near = 0, far = kLevelTokens - 1;  // far tokens from the back, moved up at the end
+  for (uint32_t r = 0; r < R && frontier; ++r) {
+    uint64_t next = 0;
+    for (; frontier; frontier &= frontier - 1) next |= fold[__builtin_ctzll(frontier)];
+    next &= ~ball;
+    ball |= next;
+    frontier = next;
+    for (uint32_t u = 0; u < static_cast<uint32_t>(slots.count) && next; ++u) {
+      uint32_t c = static_cast<uint32_t>(__popcll(next & q.lmask[static_cast<uint64_t>(g) * 16 + slots.label[u]]));
+      c = c < 15 ? c : 15;
+      if (!c || near >= far) continue;
+      if (c <= kNearCount && u < staged) out[near++] = near_offset(u * R + r, c);
+      else out[--far] = ((u * R + r) << 8) | c;
+    }
+  }
+  uint32_t all = near;
+  for (uint32_t i = far; i < kLevelTokens - 1; ++i) out[all++] = out[i];
+  out[kLevelTokens - 1] = near | (all << 8) | (static_cast<uint32_t>(q.nl[static_cast<uint64_t>(s) + lane]) << 16);
+}
+
+// filterCandidates<Query> (isomorphism.hpp:22-62) and every refineCandidates<Query> pass (:64-127)
+// as one sweep.  A block stages a strip's planes (of the first `staged` labels of slots) and its
+// wavefronts take the query nodes in turn: a lane holds 32 data nodes and the query node's tokens
+// are scalars, so a near requirement is one LDS read and three vector operations for 2,048 nodes,
+// and each word is written once.  Bound by issue (about a third each vector, scalar and LDS) and
+// the words written.  In place of the fused filter and R - 1 refine passes: 100,000 molecules x
+// 100 queries 823 -> 229 us, 150,000 LogNormal x 300 6.07 -> 1.68 ms (2.6 GB of words, 1.6 TB/s);
+// with four bit planes per entry in LDS instead of the near planes 276 us and 2.10 ms.
+__global__ __launch_bounds__(kLevelWaves * 64, 8) void k_filter_levels(const uint32_t* __restrict__ tok, uint64_t Q,
+                                                                       const uint64_t* __restrict__ lplanes, const uint4* __restrict__ lvl,
+                                                                       uint64_t D, uint32_t R, uint32_t U, uint32_t staged,
+                                                                       uint64_t* __restrict__ bits, uint32_t rpb, uint32_t chunks) {
+  extern __shared__ uint32_t near_lds[];
+  const uint64_t W32 = (D + 63) / 64 * 2;  // a row's 32-node words
+  const uint64_t strips = (W32 + kWave - 1) / kWave;
+  uint64_t strip, chunk;
+  if (!xcd_tile(blockIdx.x, strips, chunks, strip, chunk)) return;  // block-uniform
+  const uint32_t lane = static_cast<uint32_t>(lane_id());
+  const uint32_t wave = uniform32(threadIdx.x / kWave);
+  const uint64_t w = strip * kWave + lane;
+  const bool in = w < W32;
+  const uint4* src = lvl + strip * R * U * kWave;
+  for (uint32_t e0 = wave; e0 < staged * R; e0 += 4 * kLevelWaves) {
+    uint4 v[4];
+#pragma unroll
+    for (uint32_t x = 0; x < 4; ++x) {
+      const uint32_t e = e0 + x * kLevelWaves;  // LDS order: label slot, then level
+      v[x] = make_uint4(0, 0, 0, 0);
+      if (e < staged * R) v[x] = src[((e % R) * U + e / R) * kWave + lane];
+    }
+#pragma unroll
+    for (uint32_t x = 0; x < 4; ++x) {
+      const uint32_t e = e0 + x * kLevelWaves;
+      if (e < staged * R) stage_near(near_lds, e, v[x]);
+    }
+  }
+  uint32_t L[8];
+#pragma unroll
+  for (int b = 0; b < 8; ++b) L[b] = in ? reinterpret_cast<const uint32_t*>(lplanes)[((w >> 1) * 8 + b) * 2 + (w & 1)] : 0u;
+  const uint64_t n0 = w * 32;
+  const uint32_t valid = n0 + 32 <= D ? ~0u : (n0 < D ? (1u << (D - n0)) - 1u : 0u);
+  __syncthreads();
+  const uint64_t q0 = chunk * rpb, q1 = q0 + rpb < Q ? q0 + rpb : Q;
+  uint64_t q = q0 + wave;
+  uint32_t next = q < q1 ? tok[q * kLevelTokens + (lane & 31u)] : 0u;
+  for (; q < q1; q += kLevelWaves) {  // wave-uniform
+    const uint32_t dec = next;
+    if (q + kLevelWaves < q1) next = tok[(q + kLevelWaves) * kLevelTokens + (lane & 31u)];
+    const uint32_t meta = rl32(dec, kLevelTokens - 1), near = meta & 0xFFu, all = (meta >> 8) & 0xFFu, ql = meta >> 16;
+    uint32_t mask = valid;
+    if (ql != 255u) {
+#pragma unroll
+      for (uint32_t b = 0; b < 8; ++b) mask = and_xor(mask, L[b], bit_mask(~ql, b));
+    }
+    mask = near_tests(near_lds, dec, 0, near, mask);
+    for (uint32_t t = near; t < all; ++t) {
+      const uint32_t tk = rl32(dec, t), e = tk >> 8;  // e = u*R + r
+      const uint4 x = src[((e % R) * U + e / R) * kWave + lane];
+      mask &= ge4_bits<uint32_t>(x.x, x.y, x.z, x.w, tk & 15u);
+    }
+    if (in) reinterpret_cast<uint32_t*>(bits)[q * W32 + w] = mask;
+  }
+}
+
 __global__ __launch_bounds__(256) void k_row_counts(const uint64_t* __restrict__ bits, uint64_t W64, uint32_t* __restrict__ counts) {
   __shared__ uint32_t part[256 / kWave];
   const uint64_t q = blockIdx.x;
@@ -1014,6 +1179,43 @@ hipError_t filter_refine(hipStream_t s, const uint8_t* qlabels, const uint64_t* 
 #undef SIGMO_FILTER_REFINE_CASE
     default: return hipErrorInvalidValue;
   }
+}
+
+uint64_t level_planes_bytes(uint64_t D, uint32_t R, uint32_t labels) {
+  return (D + kStripNodes - 1) / kStripNodes * R * labels * kWave * sizeof(uint4);
+}
+uint64_t level_tokens(uint64_t Q) { return Q * kLevelTokens; }
+
+hipError_t sig_levels(hipStream_t s, const GraphDev& g, uint32_t R, const LabelSlots& slots, void* lvl) {
+  if (!g.N) return hipSuccess;
+  const unsigned blocks = static_cast<unsigned>((g.N + kSigBlock - 1) / kSigBlock);
+  k_sig_levels<<<blocks, kSigBlock, 0, s>>>(g, R, slots, static_cast<uint4*>(lvl));
+  return hipGetLastError();
+}
+
+// Labels whose planes the sweep's LDS holds: 52 KB, so that 32 wavefronts stay resident per CU.
+static uint32_t staged_labels(const LabelSlots& slots, uint32_t R) { return std::min<uint32_t>(static_cast<uint32_t>(slots.count), 52u / R); }
+
+hipError_t query_levels(hipStream_t s, const GraphDev& q, uint32_t R, const LabelSlots& slots, uint32_t* tok) {
+  if (!q.G) return hipSuccess;
+  k_query_levels<<<(q.G + 3) / 4, 256, 0, s>>>(q, R, slots, staged_labels(slots, R), tok);
+  return hipGetLastError();
+}
+
+hipError_t filter_levels(hipStream_t s, const uint32_t* tok, uint64_t Q, const uint64_t* lplanes, const void* lvl, uint64_t D, uint32_t R,
+                         const LabelSlots& slots, uint64_t* bits, int num_cus) {
+  const uint64_t strips = (D + kStripNodes - 1) / kStripNodes;
+  if (!Q || !strips) return hipSuccess;
+  const uint32_t U = static_cast<uint32_t>(slots.count), staged = staged_labels(slots, R);
+  // row chunks only until the blocks fill the device four times (staging is paid per block), and of at
+  // least two rows per wavefront
+  const uint64_t target = static_cast<uint64_t>(num_cus > 0 ? num_cus : 256) * 12;
+  const uint64_t chunks0 = std::max<uint64_t>(1, std::min<uint64_t>((Q + 2 * kLevelWaves - 1) / (2 * kLevelWaves), (target + strips - 1) / strips));
+  const uint32_t rpb = static_cast<uint32_t>((Q + chunks0 - 1) / chunks0), chunks = static_cast<uint32_t>((Q + rpb - 1) / rpb);
+  if (xcd_grid(strips, chunks) > 0x7fffffffull) return hipErrorInvalidValue;
+  k_filter_levels<<<static_cast<unsigned>(xcd_grid(strips, chunks)), kLevelWaves * 64, staged * R * 1024, s>>>(
+      tok, Q, lplanes, static_cast<const uint4*>(lvl), D, R, U, staged, bits, rpb, chunks);
+  return hipGetLastError();
 }
 
 hipError_t row_counts(hipStream_t s, const uint64_t* bits, uint64_t Q, uint64_t W64, uint32_t* counts) {

@@ -89,6 +89,15 @@ hipError_t refine(hipStream_t s, const uint64_t* qsig, uint64_t Q, const uint64_
 // filter followed by one refine against the given level's signatures, each word written once.
 hipError_t filter_refine(hipStream_t s, const uint8_t* qlabels, const uint64_t* qsig, uint64_t Q, const uint64_t* lplanes,
                          const uint64_t* planes, uint64_t D, const LabelSlots& slots, uint64_t* bits, int num_cus);
+// Every level at once (the pipeline; 1 <= R <= 8, slots not empty, query graphs of <= 32 nodes): data
+// signatures of levels 1..R as planes of the slots' labels, query signatures as requirement tokens,
+// and the filter with all R refinements, writing every word of the Q x W64 bitset once.
+uint64_t level_planes_bytes(uint64_t D, uint32_t R, uint32_t labels);
+uint64_t level_tokens(uint64_t Q);  // 32-bit words
+hipError_t sig_levels(hipStream_t s, const GraphDev& g, uint32_t R, const LabelSlots& slots, void* lvl);
+hipError_t query_levels(hipStream_t s, const GraphDev& q, uint32_t R, const LabelSlots& slots, uint32_t* tok);
+hipError_t filter_levels(hipStream_t s, const uint32_t* tok, uint64_t Q, const uint64_t* lplanes, const void* lvl, uint64_t D, uint32_t R,
+                         const LabelSlots& slots, uint64_t* bits, int num_cus);
 // Per-row popcounts.
 hipError_t row_counts(hipStream_t s, const uint64_t* bits, uint64_t Q, uint64_t W64, uint32_t* counts);
 // Copy into the reference layout (uint32 words, stride ceil(D/32)).

@@ -1301,8 +1301,10 @@ int sigmo_join_wildcard(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_gr
   hipStream_t s = ctx->stream;
   PhaseScope ps(ctx, SIGMO_PHASE_JOIN, SIGMO_KERNEL_JOIN, 0.0);
   SIGMO_HIP_TRY(sigmo_k::fill_u64(s, reinterpret_cast<uint64_t*>(ctx->stats), sigmo_k::kJoinStatWords, 0));
+  const bool wide = data->max_nodes > 64;
+  if (wide) SIGMO_TRY(grow_slack(&mm->wide_pairs, mm->cap_wide, m->P));
   SIGMO_HIP_TRY(sigmo_k::join_wildcard(s, query->dev(), data->dev(), query->el, data->el, c->bits, c->W64, m->indices, m->pair_graph, m->P,
-                                       find_first, mm->pair_counts, ctx->stats, ctx->num_cus));
+                                       find_first, mm->pair_counts, ctx->stats, ctx->num_cus, wide ? mm->wide_pairs : nullptr));
   SIGMO_TRY(ps.close());
   SIGMO_HIP_TRY(hipMemcpyAsync(ctx->stats_host, ctx->stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   if (per_pair_counts && m->P)

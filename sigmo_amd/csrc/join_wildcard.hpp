@@ -1,5 +1,5 @@
 // The reference's wildcard/edge-label join, joinWildcardCandidates (isomorphism.hpp:428-556),
-// one lane per GMCR pair.
+// one lane per search from a candidate of the first node.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -7,29 +7,38 @@
 #include <cstdint>
 
 #include "device_common.hpp"
+#include "join_lanes.hpp"
 #include "kernels.hpp"
 
 namespace sigmo_k {
 namespace {
 
-constexpr uint32_t kWildcardWaves = 4;  // wavefronts per block
-
 // Label of the first CSR entry of row a that points at b (graph.hpp:88-93), 255 if none.
-__device__ __forceinline__ uint8_t first_edge_label(const uint32_t* __restrict__ ro, const uint32_t* __restrict__ ci,
-                                                    const uint8_t* __restrict__ el, uint32_t a, uint32_t b) {
+__device__ __forceinline__ uint32_t first_edge_label(const uint32_t* __restrict__ ro, const uint32_t* __restrict__ ci,
+                                                     const uint8_t* __restrict__ el, uint32_t a, uint32_t b) {
   for (uint32_t i = ro[a], e = ro[a + 1]; i < e; ++i)
     if (ci[i] == b) return el[i];
   return 0xFFu;
 }
 
-// Position of the idx-th set bit (ascending) of the 128-bit set (lo, hi).
-__device__ __forceinline__ uint32_t nth_bit128(uint64_t lo, uint64_t hi, uint32_t idx) {
-  const uint32_t cl = static_cast<uint32_t>(__popcll(lo));
-  uint64_t x = idx < cl ? lo : hi;
-  uint32_t r = idx < cl ? idx : idx - cl;
-  for (; r; --r) x &= x - 1;
-  return (idx < cl ? 0u : 64u) + static_cast<uint32_t>(__builtin_ctzll(x));
-}
+constexpr int kWildcardLevels = 8;
+constexpr uint32_t kWildcardRefill = 16;  // free pair slots that make a wavefront load new pairs
+
+template <bool WIDE>
+struct WildcardLds {
+  static constexpr int L = kWildcardLevels - 1;
+  static constexpr int H = WIDE ? 2 : 1;
+  // per lane: the DFS it runs
+  uint64_t row[H][L][kWave];   // adjacency row of the position mapped at order position t
+  uint64_t base[H][L][kWave];  // candidates frame t started from
+  alignas(8) uint8_t map[kWave][40];
+  // per pair slot
+  uint64_t mask[H][L][kWave];  // candidate mask of order position t + 1
+  unsigned long long count[kWave];
+  uint32_t start[kWave], qoff[kWave], shape[kWave];  // molecule's first node; query's; nodes | k << 8 | first << 16
+  uint32_t running[kWave];                           // searches taken and not yet done
+  uint8_t root[kWave], turn[kWave];                  // the next search's root; slots by turn
+};
 
 // Per pair, as the reference kernel does per sub-group:
 //  * matching order (defineMatchingOrder, :383-408): the query node with most candidates in
@@ -39,135 +48,303 @@ __device__ __forceinline__ uint32_t nth_bit128(uint64_t lo, uint64_t hi, uint32_
 //    entry = local node 0), summed into the pair's count; find-first ends a DFS at its first
 //    leaf;
 //  * a candidate is valid when, for every earlier node of the order, query and data adjacency
-//    agree and adjacent pairs carry equal edge labels (isValidMapping, :410-426): adjacency by
-//    set algebra on the mapped positions' rows, labels by the first CSR entry of each pair;
+//    agree and adjacent pairs carry equal edge labels (isValidMapping, :410-426);
 //  * an exhausted frame unsets its node's (possibly stale) mapping, and a pop that leaves one
 //    frame resets `visited` to the first node's candidate (:521-526); `visited` is one word
 //    indexed by position mod 64 (utils.hpp:71-73).
 // A frame resumes after its last accepted candidate, which is what advancing the reference's
 // candidate index past it does.
-template <bool FIND_FIRST>
-__global__ __launch_bounds__(kWildcardWaves * 64) void k_join_wildcard(GraphDev q, GraphDev d, const uint8_t* __restrict__ qel,
-                                                                       const uint8_t* __restrict__ del, const uint64_t* __restrict__ bits,
-                                                                       uint64_t W64, const uint32_t* __restrict__ indices,
-                                                                       const uint32_t* __restrict__ pair_graph, uint64_t P,
-                                                                       int32_t* __restrict__ counts, unsigned long long* __restrict__ stats) {
-  __shared__ uint8_t maps_all[kWildcardWaves][32][kWave];
-  __shared__ uint8_t order_all[kWildcardWaves][32][kWave];
+//
+// A wavefront holds up to 64 pairs in slots, loaded together, and its lanes take the searches of
+// their roots as they become idle, a lane per search: a pair's searches are independent, and the
+// longest pair takes 1,600 accepts where the longest search takes 73 (20,011 molecules x 64 query
+// graphs; means 60 and 5).  The frames are k_join_lanes's: an accept forms the next frame's
+// candidates at once, from rows and masks in LDS, less the neighbours of a mapped query neighbour
+// whose edge label differs from the query's; frames past the seventh read masks and rows from
+// memory.  That join took 4.35 ms with a lane per pair and every step rereading masks, rows and
+// labels from memory, 2.6 ms with a lane per pair in these frames, and takes 0.92 ms with a lane per
+// search: what bounds it is the chain of dependent steps, few waves in flight by LDS.
+// Molecules of <= 64 nodes (!WIDE; pairs of larger ones are listed in `wide`) or, with WIDE, the
+// listed pairs of larger ones.
+template <bool FIND_FIRST, bool WIDE>
+__global__ __launch_bounds__(64) void k_join_wildcard(GraphDev q, GraphDev d, const uint8_t* __restrict__ qel, const uint8_t* __restrict__ del,
+                                                      BitsetMasks src, const uint32_t* __restrict__ indices,
+                                                      const uint32_t* __restrict__ pair_graph, uint64_t P, uint32_t chunk,
+                                                      int32_t* __restrict__ counts, unsigned long long* __restrict__ stats,
+                                                      uint32_t* __restrict__ wide, const uint32_t* __restrict__ list,
+                                                      const unsigned long long* __restrict__ P_dev, uint32_t cursor) {
+  constexpr uint32_t L = kWildcardLevels - 1;
+  __shared__ WildcardLds<WIDE> sh;
+  if (P_dev) P = min(P, static_cast<uint64_t>(*P_dev));
   const uint32_t lane = static_cast<uint32_t>(lane_id());
-  const uint32_t wave = threadIdx.x / kWave;
-  uint8_t (*maps)[kWave] = maps_all[wave];
-  uint8_t (*order)[kWave] = order_all[wave];
+  const uint64_t below = (1ull << lane) - 1;
+  const uint32_t* qfold = reinterpret_cast<const uint32_t*>(q.fold);  // query rows fit the low word (k <= 32)
   uint64_t sum = 0, matched = 0, overflow = 0;
-  // candidates of query node t of the pair inside the molecule, as (lo, hi) position words
-  auto mask2 = [&](uint32_t qrow, uint32_t s, uint32_t n, uint64_t& lo, uint64_t& hi) {
-    const uint64_t* row = bits + static_cast<uint64_t>(qrow) * W64;
-    const uint32_t w0 = s >> 6, last = (s + n - 1) >> 6, sh = s & 63;
-    const uint64_t x0 = row[w0];
-    const uint64_t x1 = w0 + 1 <= last ? row[w0 + 1] : 0ull;
-    const uint64_t x2 = w0 + 2 <= last ? row[w0 + 2] : 0ull;
-    lo = sh ? (x0 >> sh) | (x1 << (64 - sh)) : x0;
-    hi = sh ? (x1 >> sh) | (x2 << (64 - sh)) : x1;
-    if (n < 64) {
-      lo &= (1ull << n) - 1;
-      hi = 0;
-    } else if (n == 64) {
-      hi = 0;
-    } else if (n < 128) {
-      hi &= (1ull << (n - 64)) - 1;
+  // a wavefront's first claim is its own, later ones come from the cursor
+  uint64_t next = static_cast<uint64_t>(blockIdx.x) * chunk, end = next + chunk < P ? next + chunk : P;
+  const uint64_t claimed = static_cast<uint64_t>(gridDim.x) * chunk;
+  bool exhausted = false;
+  // the lane's slot: its pair and the roots not yet taken
+  bool held = false;
+  uint32_t pj = 0;
+  uint64_t roots = 0, roots_hi = 0;
+  // the lane's search
+  bool have = false;
+  uint32_t slot = 0, s = 0, n = 0, qoff = 0, k = 0, first = 0, depth = 0;
+  uint64_t visited = 0, count = 0, cur = 0, cur_hi = 0, rem = 0, rem_hi = 0;
+
+  auto node_of = [&](uint32_t t) -> uint32_t { return t == 0 ? first : (t <= first ? t - 1 : t); };  // query node at order position t
+  // the query row of order position t, its bits by order position
+  auto query_row = [&](uint32_t t) -> uint32_t {
+    const uint32_t r = qfold[2 * (static_cast<uint64_t>(qoff) + node_of(t))], bit = 1u << first;
+    return ((r & (bit - 1u)) << 1) | ((r >> first) & 1u) | (r & ~(bit | (bit - 1u)));
+  };
+  auto node_mask = [&](uint32_t t, uint64_t& lo, uint64_t& hi) {  // the candidate mask of order position t >= 1
+    if (t <= L) {
+      lo = sh.mask[0][t - 1][slot];
+      if constexpr (WIDE) hi = sh.mask[1][t - 1][slot];
+    } else if constexpr (WIDE) {
+      src.mask2(0, qoff + node_of(t), 0, s, n, lo, hi);
+    } else {
+      lo = src.mask(0, qoff + node_of(t), 0, s, n);
     }
   };
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  for (uint64_t j = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; j < P; j += stride) {
-    const uint32_t dg = pair_graph[j], qg = indices[j];
-    const uint32_t s = d.go[dg], n = d.go[dg + 1] - s;
-    const uint32_t qoff = q.go[qg], k = q.go[qg + 1] - qoff;
-    // matching order
-    uint32_t first = 0, maxc = 0;
-    for (uint32_t t = 0; t < k; ++t) {
-      uint64_t lo, hi;
-      mask2(qoff + t, s, n, lo, hi);
-      const uint32_t c = static_cast<uint32_t>(__popcll(lo) + __popcll(hi));
-      if (c >= maxc) {
-        maxc = c;
-        first = t;
+  // order position t's candidate set after the mapped positions below it: rows and, for query
+  // neighbours, edge labels
+  auto frame = [&](uint32_t t, uint64_t& lo, uint64_t& hi) {
+    node_mask(t, lo, hi);
+    const uint32_t qr = query_row(t);
+    for (uint32_t x = 0; x < t; ++x) {
+      const uint32_t a = bit_spread(qr, x);
+      uint64_t rl, rh = 0;
+      if (x < L) {
+        rl = sh.row[0][x][lane];
+        if constexpr (WIDE) rh = sh.row[1][x][lane];
+      } else {
+        const uint64_t v = static_cast<uint64_t>(s) + sh.map[lane][x];
+        rl = d.adj[2 * v];
+        if constexpr (WIDE) rh = d.adj[2 * v + 1];
+      }
+      lo = and_row(lo, rl, a);
+      if constexpr (WIDE) hi = and_row(hi, rh, a);
+    }
+    const uint32_t qn = qoff + node_of(t);
+    for (uint32_t nb = qr & ((1u << t) - 1u); nb && (lo | hi); nb &= nb - 1) {
+      const uint32_t x = static_cast<uint32_t>(__builtin_ctz(nb));
+      const uint32_t want = first_edge_label(q.ro, q.ci, qel, qoff + node_of(x), qn);
+      const uint32_t v = s + sh.map[lane][x];
+      uint64_t seen_lo = 0, seen_hi = 0;  // neighbours whose first CSR entry has passed
+      for (uint32_t i = d.ro[v], e = d.ro[v + 1]; i < e; ++i) {
+        const uint32_t c = d.ci[i] - s;
+        const uint64_t bit = bit_of(c);
+        uint64_t& seen = c < 64 ? seen_lo : seen_hi;
+        if (!(seen & bit) && del[i] != want) {
+          if (c < 64) lo &= ~bit;
+          else hi &= ~bit;
+        }
+        seen |= bit;
       }
     }
-    order[0][lane] = static_cast<uint8_t>(first);
-    for (uint32_t t = 0, o = 1; t < k; ++t)
-      if (t != first) order[o++][lane] = static_cast<uint8_t>(t);
-    uint64_t flo, fhi;
-    mask2(qoff + first, s, n, flo, fhi);
-    uint64_t count = 0;
-    for (uint32_t start = 0; start < maxc; ++start) {
-      for (uint32_t t = 0; t < k; ++t) maps[t][lane] = 0;  // every mapping entry starts at local node 0
-      const uint32_t root = nth_bit128(flo, fhi, start);
-      maps[first][lane] = static_cast<uint8_t>(root);
-      uint64_t visited = 1ull << (root & 63);
-      uint32_t depth = 1, pos = 0;
-      while (depth > 0) {
-        if (depth == k) {  // leaf
-          ++count;
-          if (FIND_FIRST) break;
-          depth = k - 1;
-          pos = static_cast<uint32_t>(maps[order[depth][lane]][lane]) + 1;
-          continue;
+  };
+  // Accepts c at `depth` and forms the next frame (or counts the leaf); true when the search ends.
+  auto accept = [&](uint32_t c) -> bool {
+    sh.map[lane][depth] = static_cast<uint8_t>(c);
+    const uint32_t nd = depth + 1;
+    if (nd == k) {
+      ++count;
+      return FIND_FIRST;
+    }
+    if (depth < L) {
+      const uint64_t v = static_cast<uint64_t>(s) + c;
+      sh.row[0][depth][lane] = d.adj[2 * v];
+      sh.base[0][depth][lane] = cur;
+      if constexpr (WIDE) {
+        sh.row[1][depth][lane] = d.adj[2 * v + 1];
+        sh.base[1][depth][lane] = cur_hi;
+      }
+    }
+    uint64_t nlo = 0, nhi = 0;
+    frame(nd, nlo, nhi);
+    if ((nlo & ~visited) | (WIDE ? nhi & ~visited : 0ull)) {
+      depth = nd;
+      cur = nlo;
+      cur_hi = nhi;
+      rem = rem_hi = ~0ull;
+      return false;
+    }
+    // it would be exhausted at once
+    visited &= ~bit_of(sh.map[lane][nd]);
+    if (depth == 1) visited = bit_of(sh.map[lane][0]);
+    return depth == 0;
+  };
+
+  while (true) {
+    uint64_t idle = __ballot(!have);
+    // finished pairs leave their slots; new ones are loaded when the slots' roots no longer feed the
+    // idle lanes
+    if (__popcll(idle) > __popcll(__ballot(held && (roots | roots_hi)))) {  // wave-uniform
+      if (held && !(roots | roots_hi) && sh.running[lane] == 0) {
+        const uint64_t total = sh.count[lane];
+        if (total > 0x7FFFFFFFull) overflow = 1;
+        counts[pj] = static_cast<int32_t>(total > 0x7FFFFFFFull ? 0x7FFFFFFFull : total);
+        sum += total;
+        matched += total > 0;
+        held = false;
+      }
+      const uint64_t room = __ballot(!held);
+      if (!exhausted && (static_cast<uint32_t>(__popcll(room)) >= kWildcardRefill || idle == ~0ull)) {
+        if (next >= end && claimed < P) {
+          unsigned long long b = 0;
+          if (lane == 0) b = atomicAdd(&stats[cursor], static_cast<unsigned long long>(chunk));
+          next = claimed + uniform64(__shfl(b, 0));
+          end = next + chunk < P ? next + chunk : P;
         }
-        const uint32_t qn = order[depth][lane];
-        uint64_t clo, chi;
-        mask2(qoff + qn, s, n, clo, chi);
-        clo &= ~visited & bits_from(pos);
-        chi &= ~visited & (pos <= 64 ? ~0ull : bits_from(pos - 64));
-        // adjacency agreement with every earlier node of the order
-        uint64_t must_lo = ~0ull, must_hi = ~0ull, not_lo = 0, not_hi = 0;
-        uint32_t nbr = 0;  // orders i < depth whose node is a query neighbour of qn
-        for (uint32_t i = 0; i < depth; ++i) {
-          const uint32_t qi = order[i][lane];
-          const uint32_t m = maps[qi][lane];
-          const uint64_t rl = d.adj[2 * (static_cast<uint64_t>(s) + m)], rh = d.adj[2 * (static_cast<uint64_t>(s) + m) + 1];
-          if ((static_cast<uint32_t>(q.adj[2 * (static_cast<uint64_t>(qoff) + qi)]) >> qn) & 1u) {
-            must_lo &= rl;
-            must_hi &= rh;
-            nbr |= 1u << i;
+        if (next >= end) {
+          exhausted = true;
+        } else {
+          const uint32_t cnt = min(static_cast<uint32_t>(end - next), static_cast<uint32_t>(__popcll(room)));
+          const uint32_t rn = __popcll(room & below);
+          const bool take = !held && rn < cnt;
+          bool wide_pair = false;
+          uint32_t ps = 0, pn = 0, pq = 0, pk = 0;
+          if (take) {
+            pj = list ? list[next + rn] : static_cast<uint32_t>(next + rn);
+            const uint32_t dg = pair_graph[pj], qg = indices[pj];
+            ps = d.go[dg];
+            pn = d.go[dg + 1] - ps;
+            pq = q.go[qg];
+            pk = q.go[qg + 1] - pq;
+            wide_pair = !WIDE && pn > 64;
+          }
+          next += cnt;
+          if constexpr (!WIDE) {
+            const uint64_t wm = __ballot(wide_pair);
+            if (wm) {
+              unsigned long long b = 0;
+              if (lane == 0) b = atomicAdd(&stats[kStatWide], static_cast<unsigned long long>(__popcll(wm)));
+              const uint64_t wb = uniform64(__shfl(b, 0));
+              if (wide_pair) wide[wb + __popcll(wm & below)] = pj;
+            }
+          }
+          if (take && !wide_pair) {
+            // the first node of the matching order, then the masks by order position
+            uint32_t maxc = 0, lead = 0;
+            for (uint32_t t = 0; t < pk; ++t) {
+              uint64_t lo = 0, hi = 0;
+              if constexpr (WIDE) src.mask2(0, pq + t, 0, ps, pn, lo, hi);
+              else lo = src.mask(0, pq + t, 0, ps, pn);
+              const uint32_t c = static_cast<uint32_t>(__popcll(lo) + __popcll(hi));
+              // until a later node takes its place as the first, node t's order position is t + 1
+              if (t < L) {
+                sh.mask[0][t][lane] = lo;
+                if constexpr (WIDE) sh.mask[1][t][lane] = hi;
+              }
+              if (c >= maxc) {
+                maxc = c;
+                lead = t;
+                roots = lo;
+                roots_hi = hi;
+              }
+            }
+            // nodes after the first keep their index as order position: masks move one place down
+            for (uint32_t t = lead + 1; t < pk && t <= L; ++t) {
+              uint64_t lo = 0, hi = 0;
+              if (t < L) {
+                lo = sh.mask[0][t][lane];
+                if constexpr (WIDE) hi = sh.mask[1][t][lane];
+              } else if constexpr (WIDE) {
+                src.mask2(0, pq + t, 0, ps, pn, lo, hi);
+              } else {
+                lo = src.mask(0, pq + t, 0, ps, pn);
+              }
+              sh.mask[0][t - 1][lane] = lo;
+              if constexpr (WIDE) sh.mask[1][t - 1][lane] = hi;
+            }
+            sh.start[lane] = ps;
+            sh.qoff[lane] = pq;
+            sh.shape[lane] = pn | (pk << 8) | (lead << 16);
+            sh.count[lane] = 0;
+            sh.running[lane] = 0;
+            held = true;
+          }
+        }
+      }
+      if (exhausted && __ballot(held || have) == 0) break;
+    }
+    // each slot with roots left hands one to an idle lane
+    const uint64_t ready = __ballot(held && (roots | roots_hi));
+    if (ready && idle) {  // wave-uniform
+      const uint32_t cnt = min(static_cast<uint32_t>(__popcll(ready)), static_cast<uint32_t>(__popcll(idle)));
+      const uint32_t rank = __popcll(ready & below);
+      if (((ready >> lane) & 1ull) && rank < cnt) {
+        uint32_t c;
+        if (roots) {
+          c = static_cast<uint32_t>(__builtin_ctzll(roots));
+          roots &= roots - 1;
+        } else {
+          c = 64u + static_cast<uint32_t>(__builtin_ctzll(roots_hi));
+          roots_hi &= roots_hi - 1;
+        }
+        sh.root[lane] = static_cast<uint8_t>(c);
+        sh.turn[rank] = static_cast<uint8_t>(lane);
+        atomicAdd(&sh.running[lane], 1u);
+      }
+      wave_sync();
+      const uint32_t rn = __popcll(idle & below);
+      if (!have && rn < cnt) {  // a search from one root, from fresh state
+        slot = sh.turn[rn];
+        s = sh.start[slot];
+        qoff = sh.qoff[slot];
+        n = sh.shape[slot] & 0xFFu;
+        k = (sh.shape[slot] >> 8) & 0xFFu;
+        first = sh.shape[slot] >> 16;
+        const uint32_t c = sh.root[slot];
+#pragma unroll
+        for (int t = 0; t < 32; t += 8) *reinterpret_cast<uint64_t*>(&sh.map[lane][t]) = 0;  // every entry: local node 0
+        visited = bit_of(c);
+        count = 0;
+        depth = 0;
+        have = !accept(c);  // queries have two nodes or more: no leaf yet
+        if (!have) atomicSub(&sh.running[slot], 1u);
+      }
+      wave_sync();
+    }
+    if (have) {
+      bool done = false;
+      uint64_t el = cur & ~visited & rem, eh = WIDE ? cur_hi & ~visited & rem_hi : 0ull;
+      if ((el | eh) == 0) {  // exhausted frame: pop
+        visited &= ~bit_of(sh.map[lane][depth]);
+        --depth;
+        if (depth == 0) {
+          done = true;
+        } else {
+          if (depth == 1) visited = bit_of(sh.map[lane][0]);
+          const uint32_t c = sh.map[lane][depth];
+          if (depth < L) {
+            cur = sh.base[0][depth][lane];
+            if constexpr (WIDE) cur_hi = sh.base[1][depth][lane];
           } else {
-            not_lo |= rl;
-            not_hi |= rh;
+            frame(depth, cur, cur_hi);
           }
-        }
-        uint64_t el = clo & must_lo & ~not_lo, eh = chi & must_hi & ~not_hi;
-        int accepted = -1;
-        while (el | eh) {  // ascending; the first whose edge labels all agree
-          const uint32_t c = el ? static_cast<uint32_t>(__builtin_ctzll(el)) : 64u + static_cast<uint32_t>(__builtin_ctzll(eh));
-          if (el) el &= el - 1;
-          else eh &= eh - 1;
-          bool ok = true;
-          for (uint32_t b = nbr; b && ok; b &= b - 1) {
-            const uint32_t qi = order[__builtin_ctz(b)][lane];
-            const uint32_t m = maps[qi][lane];
-            ok = first_edge_label(d.ro, d.ci, del, s + m, s + c) == first_edge_label(q.ro, q.ci, qel, qoff + qi, qoff + qn);
-          }
-          if (ok) {
-            accepted = static_cast<int>(c);
-            break;
-          }
-        }
-        if (accepted >= 0) {
-          maps[qn][lane] = static_cast<uint8_t>(accepted);
-          visited |= 1ull << (accepted & 63);
-          ++depth;
-          pos = 0;
-        } else {  // exhausted frame: pop
-          visited &= ~(1ull << (maps[qn][lane] & 63u));
-          --depth;
-          if (depth == 1) visited = 1ull << (maps[first][lane] & 63u);
-          if (depth > 0) pos = static_cast<uint32_t>(maps[order[depth][lane]][lane]) + 1;
+          rem = c < 64 ? bits_above(c) : 0ull;
+          rem_hi = c < 64 ? ~0ull : bits_above(c - 64);
+          el = cur & ~visited & rem;
+          eh = WIDE ? cur_hi & ~visited & rem_hi : 0ull;
         }
       }
+      if (!done && (el | eh)) {
+        const uint32_t c = el ? static_cast<uint32_t>(__builtin_ctzll(el)) : 64u + static_cast<uint32_t>(__builtin_ctzll(eh));
+        rem = c < 64 ? bits_above(c) : 0ull;
+        rem_hi = c < 64 ? ~0ull : bits_above(c - 64);
+        visited |= bit_of(c);
+        done = accept(c);
+      }
+      if (done) {
+        if (count) atomicAdd(&sh.count[slot], static_cast<unsigned long long>(count));
+        atomicSub(&sh.running[slot], 1u);
+        have = false;
+      }
     }
-    if (count > 0x7FFFFFFFull) overflow = 1;
-    counts[j] = static_cast<int32_t>(count > 0x7FFFFFFFull ? 0x7FFFFFFFull : count);
-    sum += count;
-    matched += count > 0;
   }
 #pragma unroll
   for (int o = kWave / 2; o > 0; o >>= 1) {

@@ -1267,14 +1267,27 @@ hipError_t join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const
 
 hipError_t join_wildcard(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint8_t* qel, const uint8_t* del, const uint64_t* bits,
                          uint64_t W64, const uint32_t* indices, const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts,
-                         unsigned long long* stats, int num_cus) {
+                         unsigned long long* stats, int num_cus, uint32_t* wide) {
   if (!P) return hipSuccess;
+  const BitsetMasks src{bits, W64};
   const uint64_t cus = static_cast<uint64_t>(num_cus > 0 ? num_cus : 256);
-  const unsigned blocks = static_cast<unsigned>(std::max<uint64_t>(1, std::min<uint64_t>((P + 255) / 256, cus * 8)));
-  if (find_first)
-    k_join_wildcard<true><<<blocks, kWildcardWaves * 64, 0, s>>>(q, d, qel, del, bits, W64, indices, pair_graph, P, counts, stats);
-  else
-    k_join_wildcard<false><<<blocks, kWildcardWaves * 64, 0, s>>>(q, d, qel, del, bits, W64, indices, pair_graph, P, counts, stats);
+  // wavefronts by LDS, about four claims each
+  const auto shape = [&](uint64_t lds, uint64_t& blocks, uint32_t& chunk) {
+    blocks = std::max<uint64_t>(1, std::min<uint64_t>((P + 63) / 64, cus * (160 * 1024 / ((lds + 511) / 512 * 512))));
+    chunk = static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, P / (blocks * 4))));
+  };
+  uint64_t blocks;
+  uint32_t chunk;
+  shape(sizeof(WildcardLds<false>), blocks, chunk);
+  const auto narrow = find_first ? k_join_wildcard<true, false> : k_join_wildcard<false, false>;
+  narrow<<<static_cast<unsigned>(blocks), 64, 0, s>>>(q, d, qel, del, src, indices, pair_graph, P, chunk, counts, stats, wide, nullptr, nullptr,
+                                                      kStatCursor);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !wide) return e;
+  shape(sizeof(WildcardLds<true>), blocks, chunk);
+  const auto pass = find_first ? k_join_wildcard<true, true> : k_join_wildcard<false, true>;
+  pass<<<static_cast<unsigned>(blocks), 64, 0, s>>>(q, d, qel, del, src, indices, pair_graph, P, 64, counts, stats, nullptr, wide,
+                                                    stats + kStatWide, kStatWideCursor);
   return hipGetLastError();
 }
 

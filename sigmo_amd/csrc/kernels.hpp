@@ -141,10 +141,12 @@ hipError_t join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const
                       const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts, unsigned long long* stats, uint32_t* wide,
                       int num_cus, const unsigned long long* P_dev = nullptr, uint32_t* deep = nullptr);
 // joinWildcardCandidates: matching order by candidate count, edge labels compared, one DFS per
-// candidate of the first node; one lane per pair (qel/del: edge labels of the CSR entries).
+// candidate of the first node; one lane per pair (qel/del: edge labels of the CSR entries).  `wide`
+// (capacity P) takes the pairs of molecules of more than 64 nodes for a second pass; null when the
+// data has none.
 hipError_t join_wildcard(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint8_t* qel, const uint8_t* del, const uint64_t* bits,
                          uint64_t W64, const uint32_t* indices, const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts,
-                         unsigned long long* stats, int num_cus);
+                         unsigned long long* stats, int num_cus, uint32_t* wide);
 // The lane-per-pair join over the `nw` listed pairs of molecules with 65..128 nodes
 // (stats[kStatWideCursor] is the work counter).  With nw_dev the kernel reads the list's length on
 // the device, bounded by nw.

@@ -660,9 +660,11 @@ __global__ __launch_bounds__(256) void k_pair_pretest(PretestArgs a) {
 
 // ---- pair evaluation ----------------------------------------------------------------------------
 
-// Arena words of a pair's block: its k node masks (two words each for molecules of > 64 nodes),
-// rounded up to a whole 32-byte group.
-__host__ __device__ __forceinline__ uint32_t pair_words(uint32_t k, uint32_t stride) { return (k * stride + 3) & ~3u; }
+// Arena words of a pair's block: its k node masks (half a word each for molecules of <= 32 nodes,
+// one for 33..64, two for wider ones), rounded up to four nodes, or to two of the wide ones.
+__device__ __forceinline__ uint32_t pair_words(uint32_t k, int cls) {
+  return cls == 0 ? ((k + 3) & ~3u) / 2 : (cls == 1 ? (k + 3) & ~3u : ((k + 1) & ~1u) * 2);
+}
 
 constexpr uint32_t kGroupWaves = 8;       // wavefronts per block of the pair evaluation
 constexpr uint32_t kGroupStatSlots = 32;  // one address would take every wavefront's sums one after another (~10 ns each)
@@ -682,7 +684,7 @@ struct GroupArgs {
   uint64_t* arena;
   uint64_t arena_cap;
   unsigned long long* surv;      // [Gd][W] in: the pre-test's pairs; out: bit qg of row m = the pair survives GMCR
-  uint32_t* pair_off;            // [Gd * Gq] arena offset of each surviving pair
+  uint4* blocks;                 // [group * Gq + g] where the masks of group and query graph are: pair_block
   unsigned long long* counters;  // [1] arena words claimed past the wavefronts' first chunks, [2] item cursor, [3] overflow
   unsigned long long* stats;     // kGroupStatSlots x 16: [0] node evaluations, [1] their live lanes, [2] pre-tested pairs
 };
@@ -696,6 +698,12 @@ __device__ __forceinline__ uint32_t quad_xor1(uint32_t x) {
 }
 __device__ __forceinline__ uint32_t quad_xor2(uint32_t x) {
   return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x4E, 0xF, 0xF, false));
+}
+
+// The record of a group and a query graph, {base, words, lanes lo, lanes hi}: the pre-tested pairs
+// have consecutive blocks of `words` from `base` on, in the order of their molecules' first lanes.
+__device__ __forceinline__ uint32_t pair_block(uint32_t base, uint32_t words, uint64_t lanes, uint32_t lane0) {
+  return base + static_cast<uint32_t>(__popcll(lanes & ((1ull << lane0) - 1))) * words;
 }
 
 // A wavefront's arena chunk and statistics (wave-uniform but `live`).
@@ -768,7 +776,7 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
       const bool act = (word >> jb) & 1ull;
       const uint64_t am = __ballot(act) & leaders;
       const uint32_t qoff = uniform32(a.qinfo[g].qoff), k = uniform32(a.qinfo[g].k);
-      const uint32_t cnt = static_cast<uint32_t>(__popcll(am)), pw = pair_words(k, CLS == 2 ? 2u : 1u);
+      const uint32_t cnt = static_cast<uint32_t>(__popcll(am)), pw = pair_words(k, CLS);
       st.scans += cnt;
       if (st.next + static_cast<uint64_t>(cnt) * pw > st.end) {
         unsigned long long b = 0;
@@ -779,7 +787,7 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
         st.next = uniform64(__shfl(b, 0));
         st.end = st.next + a.chunk;
       }
-      const uint64_t base = st.next + static_cast<uint64_t>(__popcll(am & below)) * pw;
+      const uint64_t base0 = st.next, base = base0 + static_cast<uint64_t>(__popcll(am & below)) * pw;
       st.next += static_cast<uint64_t>(cnt) * pw;
       const bool room = st.end <= a.arena_cap;
 
@@ -845,32 +853,44 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
       };
       load_tokens(0);
       bool alive = act;
-      // two nodes at a time, whose masks go out together (the second past the last node falls in the
-      // block's padding); a pair dies at its first node without candidates (gmcr.hpp:56-61)
-      for (uint32_t i = 0; i < k; i += 2) {  // wave-uniform
+      // masks go out four nodes at a time, in 16-byte stores (nodes past the last fall in the block's
+      // padding); a pair dies at its first node without candidates (gmcr.hpp:56-61)
+      uint32_t m0 = 0, m1 = 0, m2 = 0, m3 = 0;
+      for (uint32_t i = 0; i < k; ++i) {  // wave-uniform
         st.live += alive;
-        const uint32_t m0 = node_mask();
-        alive = alive && some(m0);
+        m0 = m1;
+        m1 = m2;
+        m2 = m3;
+        m3 = node_mask();
+        alive = alive && some(m3);
         if (__ballot(alive) == 0) break;
-        uint32_t m1 = 0;
-        if (i + 1 < k) {
-          st.live += alive;
-          m1 = node_mask();
-          alive = alive && some(m1);
-          if (__ballot(alive) == 0) break;
+        if ((i & 3u) != 3u) {
+          if (i + 1 < k) continue;
+          for (uint32_t x = i & 3u; x < 3; ++x) {
+            m0 = m1;
+            m1 = m2;
+            m2 = m3;
+            m3 = 0;
+          }
         }
+        const uint32_t i0 = i & ~3u;
         if (CLS == 0) {
-          if (alive && room) *reinterpret_cast<uint4*>(a.arena + base + i) = make_uint4(m0, 0, m1, 0);
-        } else if (CLS == 1) {  // the lanes of a molecule swap halves: each stores one node's word
-          const uint32_t other = quad_xor1(h ? m0 : m1);
-          if (alive && room) reinterpret_cast<uint2*>(a.arena + base + i)[h] = h ? make_uint2(other, m1) : make_uint2(m0, other);
+          if (alive && room) *reinterpret_cast<uint4*>(a.arena + base + i0 / 2) = make_uint4(m0, m1, m2, m3);
+        } else if (CLS == 1) {  // the lanes of a molecule swap halves: each stores two nodes' words
+          const uint32_t o0 = quad_xor1(h ? m0 : m2), o1 = quad_xor1(h ? m1 : m3);
+          if (alive && room) reinterpret_cast<uint4*>(a.arena + base + i0)[h] = h ? make_uint4(o0, m2, o1, m3) : make_uint4(m0, o0, m1, o1);
         } else if (alive && room) {
-          uint32_t* dst = reinterpret_cast<uint32_t*>(a.arena + base + 2 * i);
-          dst[h] = m0;
-          dst[4 + h] = m1;
+          uint32_t* dst = reinterpret_cast<uint32_t*>(a.arena + base + 2 * i0) + h;
+          dst[0] = m0;
+          dst[4] = m1;
+          if (i0 + 2 < k) {
+            dst[8] = m2;
+            dst[12] = m3;
+          }
         }
       }
-      if (alive && h == 0) a.pair_off[static_cast<uint64_t>(mi.m) * a.Gq + g] = static_cast<uint32_t>(base);
+      if (__ballot(alive) && lane == 0)
+        a.blocks[group * a.Gq + g] = make_uint4(static_cast<uint32_t>(base0), pw, static_cast<uint32_t>(am), static_cast<uint32_t>(am >> 32));
       if (act && !alive) dead |= 1ull << jb;
     }
     if (dead && h == 0) atomicAnd(&a.surv[static_cast<uint64_t>(mi.m) * a.W + w], ~dead);
@@ -893,11 +913,13 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
 // graphs out by index.  Node masks go straight to the pairs' arena blocks, which a wavefront takes
 // from a chunk of its own; pairs that die clear their pre-test bits, one atomic per molecule and
 // 64 query graphs.  80 registers: six wavefronts per SIMD, which its scalar token decode needs to
-// hide (20 waves with 4-wavefront blocks: 8.1 instead of 6.8 ms).
+// hide (20 waves with 4-wavefront blocks: 8.1 instead of 6.8 ms).  With 64-bit
+// masks for every molecule and an offset per pair, stored 4 KB apart, 174 M writes went to memory
+// instead of 73 M, in 6.7 instead of 5.6 ms.
 //
 // Measured, in place of one launch per size class with a lane per pair: 2,000 molecules x 20 query
 // graphs 219 -> 12 us (three serial chains of ~100 us), 100,000 x 100 475 -> 125 us, 1 M x 25
-// 1,242 -> 392 us, 1 M x 1,000 10.7 -> 6.8 ms.
+// 1,242 -> 353 us, 1 M x 1,000 10.7 -> 5.6 ms.
 __global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a) {
   extern __shared__ uint32_t near_lds[];
   uint32_t* labs = near_lds + static_cast<uint64_t>(a.slots) * a.R * kNearCount * kWave;
@@ -944,69 +966,86 @@ __global__ __launch_bounds__(256) void k_surv_count(uint32_t Gd, uint32_t W, con
 }
 
 // Canonical GMCR arrays (gmcr.hpp:73-115 order: molecules ascending, query graphs ascending
-// within a molecule) from the survival bitmask, with each pair's arena offset.  One wavefront
-// per molecule: lane i loads bitmask word i of each run of 64 (one coalesced load), the lanes'
-// popcounts are scanned, and the wavefront visits only the nonzero words, lane l writing query
-// graph 64w+l of word w, so each word's survivors go out in one coalesced store per array.
-__global__ __launch_bounds__(256) void k_surv_scatter(uint32_t Gd, uint32_t Gq, uint32_t W, const unsigned long long* __restrict__ surv,
-                                                      const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ pair_off,
-                                                      uint32_t* __restrict__ indices, uint32_t* __restrict__ pair_graph,
-                                                      uint32_t* __restrict__ mask_off, uint64_t cap) {
+// within a molecule) from the survival bitmask, with each pair's arena offset from its group's
+// records.  A block takes one group of the width-class order and its wavefronts a quarter of the
+// molecules each: for 64 query graphs at a time a lane holds one graph's record and the wavefront
+// goes over its molecules, whose survivors go out in one coalesced store per array.  When the pair
+// evaluation wrote every pair's offset to a [molecule][query graph] table and a wavefront per
+// molecule read them back, 1 M x 1,000 took 1.6 ms here; this takes 1.1 ms.
+__global__ __launch_bounds__(256) void k_surv_scatter(GroupOrder order, uint32_t Gq, uint32_t W, const MolInfo* __restrict__ minfo,
+                                                      const unsigned long long* __restrict__ surv, const uint32_t* __restrict__ offsets,
+                                                      const uint4* __restrict__ blocks, uint32_t* __restrict__ indices,
+                                                      uint32_t* __restrict__ pair_graph, uint32_t* __restrict__ mask_off, uint64_t cap) {
   // `cap` bounds the writes: a replayed graph sized by an earlier run never writes past its
   // arrays (the replay then reports the changed pair count)
-  const uint64_t m = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
-  if (m >= Gd) return;  // wave-uniform
-  const uint32_t lane = static_cast<uint32_t>(lane_id());
+  const uint32_t group = blockIdx.x, lane = static_cast<uint32_t>(lane_id()), wave = uniform32(threadIdx.x / kWave);
+  const uint32_t g0 = order.groups(0), g1 = order.groups(1);
+  const uint32_t cls = group < g0 ? 0u : (group < g0 + g1 ? 1u : 2u);
+  const uint32_t grp = group - (cls > 0 ? g0 : 0u) - (cls > 1 ? g1 : 0u), per = 64u >> cls;
+  const uint32_t first = (cls > 0 ? order.count[0] : 0u) + (cls > 1 ? order.count[1] : 0u);
+  // lane i < share: the wavefront's i-th molecule
+  const uint32_t share = per / 4, slot = wave * share + lane, at = grp * per + slot;
+  const bool valid = lane < share && at < (cls == 0 ? order.count[0] : (cls == 1 ? order.count[1] : order.count[2]));
+  const uint32_t m = valid ? minfo[first + at].m : 0u;
+  uint32_t o = valid ? offsets[m] : 0u;  // where its next survivor goes
   const uint64_t below = (1ull << lane) - 1;
-  uint64_t o = offsets[m];
-  if (offsets[m + 1] == o) return;  // no survivors (wave-uniform)
-  for (uint32_t w0 = 0; w0 < W; w0 += kWave) {  // wave-uniform
-    const uint64_t xl = w0 + lane < W ? surv[m * W + w0 + lane] : 0ull;
-    const uint32_t pc = static_cast<uint32_t>(__popcll(xl));
-    uint32_t incl = pc;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const uint32_t y = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), d));
-      if (lane >= static_cast<uint32_t>(d)) incl += y;
-    }
-    for (uint64_t nz = __ballot(xl != 0ull); nz; nz &= nz - 1) {  // wave-uniform
-      const int wl = static_cast<int>(__builtin_ctzll(nz));
-      const uint64_t x = __shfl(xl, wl);
-      const uint32_t ob = static_cast<uint32_t>(__shfl(static_cast<int>(incl - pc), wl));
-      if ((x >> lane) & 1ull) {
-        const uint64_t r = o + ob + static_cast<uint64_t>(__popcll(x & below));
-        const uint32_t g = (w0 + static_cast<uint32_t>(wl)) * 64 + lane;
-        if (r < cap) {
-          indices[r] = g;
-          pair_graph[r] = static_cast<uint32_t>(m);
-          mask_off[r] = pair_off[static_cast<uint64_t>(m) * Gq + g];
-        }
+  for (uint32_t w = 0; w < W; ++w) {
+    const uint64_t xl = valid ? surv[static_cast<uint64_t>(m) * W + w] : 0ull;
+    uint64_t left = __ballot(xl != 0ull);
+    if (!left) continue;  // wave-uniform
+    const uint32_t g = w * kWave + lane;
+    uint4 rec = make_uint4(0, 0, 0, 0);
+    if (g < Gq) rec = blocks[static_cast<uint64_t>(group) * Gq + g];  // unwritten, and not used, where no molecule of the group survives
+    const uint64_t lanes = rec.z | (static_cast<uint64_t>(rec.w) << 32);
+    for (; left; left &= left - 1) {
+      const uint32_t i = static_cast<uint32_t>(__builtin_ctzll(left));
+      const uint64_t x = rl32(static_cast<uint32_t>(xl), i) | (static_cast<uint64_t>(rl32(static_cast<uint32_t>(xl >> 32), i)) << 32);
+      const uint32_t r = rl32(o, i) + static_cast<uint32_t>(__popcll(x & below)), mol = rl32(m, i);
+      if (((x >> lane) & 1ull) && r < cap) {
+        indices[r] = g;
+        pair_graph[r] = mol;
+        mask_off[r] = pair_block(rec.x, rec.y, lanes, (wave * share + i) << cls);
       }
     }
-    o += static_cast<uint32_t>(__shfl(static_cast<int>(incl), kWave - 1));
+    o += static_cast<uint32_t>(__popcll(xl));
   }
 }
 
-// k_surv_scatter with one thread per molecule instead of one wavefront, for batches of at most 64
-// query graphs (one bitmask word per molecule): most molecules then have no or a few survivors,
-// and a wavefront per molecule would leave almost all of its lanes idle.
-__global__ __launch_bounds__(256) void k_surv_scatter_thread(uint32_t Gd, uint32_t Gq, uint32_t W, const unsigned long long* __restrict__ surv,
-                                                             const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ pair_off,
-                                                             uint32_t* __restrict__ indices, uint32_t* __restrict__ pair_graph,
-                                                             uint32_t* __restrict__ mask_off, uint64_t cap) {
-  const uint64_t m = blockIdx.x * 256ull + threadIdx.x;
-  if (m >= Gd) return;
-  uint64_t o = offsets[m];
-  if (offsets[m + 1] == o) return;
-  for (uint32_t w = 0; w < W; ++w) {
-    uint64_t x = surv[m * W + w];
-    while (x) {
-      const uint32_t g = w * 64 + static_cast<uint32_t>(__builtin_ctzll(x));
-      x &= x - 1;
+// k_surv_scatter for at most 64 query graphs (one bitmask word per molecule): most molecules then
+// have no or a few survivors, so a wavefront takes a group with a lane per molecule and goes over
+// the query graphs that survive for any of them.
+__global__ __launch_bounds__(256) void k_surv_scatter_lanes(GroupOrder order, uint32_t Gq, const MolInfo* __restrict__ minfo,
+                                                            const unsigned long long* __restrict__ surv, const uint32_t* __restrict__ offsets,
+                                                            const uint4* __restrict__ blocks, uint32_t* __restrict__ indices,
+                                                            uint32_t* __restrict__ pair_graph, uint32_t* __restrict__ mask_off, uint64_t cap) {
+  const uint32_t group = uniform32(blockIdx.x * 4 + threadIdx.x / kWave), lane = static_cast<uint32_t>(lane_id());
+  if (group >= order.total()) return;  // wave-uniform; no block barrier follows
+  const uint32_t g0 = order.groups(0), g1 = order.groups(1);
+  const uint32_t cls = group < g0 ? 0u : (group < g0 + g1 ? 1u : 2u);
+  const uint32_t grp = group - (cls > 0 ? g0 : 0u) - (cls > 1 ? g1 : 0u), per = 64u >> cls;
+  const uint32_t first = (cls > 0 ? order.count[0] : 0u) + (cls > 1 ? order.count[1] : 0u);
+  const uint32_t at = grp * per + lane;
+  const bool valid = lane < per && at < (cls == 0 ? order.count[0] : (cls == 1 ? order.count[1] : order.count[2]));
+  uint4 rec = make_uint4(0, 0, 0, 0);
+  if (lane < Gq) rec = blocks[static_cast<uint64_t>(group) * Gq + lane];
+  const uint32_t m = valid ? minfo[first + at].m : 0u;
+  const uint64_t x = valid ? surv[m] : 0ull;
+  uint32_t o = valid ? offsets[m] : 0u;
+  uint32_t any_lo = static_cast<uint32_t>(x), any_hi = static_cast<uint32_t>(x >> 32);
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    any_lo |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(any_lo), d));
+    any_hi |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(any_hi), d));
+  }
+  for (uint64_t bits = uniform64(any_lo | (static_cast<uint64_t>(any_hi) << 32)); bits; bits &= bits - 1) {  // wave-uniform
+    const uint32_t g = static_cast<uint32_t>(__builtin_ctzll(bits));
+    const uint32_t base = rl32(rec.x, g), words = rl32(rec.y, g);
+    const uint64_t lanes = rl32(rec.z, g) | (static_cast<uint64_t>(rl32(rec.w, g)) << 32);
+    if ((x >> g) & 1ull) {
       if (o < cap) {
         indices[o] = g;
-        pair_graph[o] = static_cast<uint32_t>(m);
-        mask_off[o] = pair_off[m * Gq + g];
+        pair_graph[o] = m;
+        mask_off[o] = pair_block(base, words, lanes, lane << cls);
       }
       ++o;
     }
@@ -1224,8 +1263,8 @@ struct sigmo_batch {
   uint64_t cap_arena = 0;
   unsigned long long* surv = nullptr;
   uint64_t cap_surv = 0;
-  uint32_t* pair_off = nullptr;
-  uint64_t cap_pair_off = 0;
+  uint4* blocks = nullptr;
+  uint64_t cap_blocks = 0;
   uint32_t* mol_count = nullptr;
   uint64_t cap_mc = 0;
   unsigned long long* counters = nullptr;
@@ -1275,7 +1314,7 @@ struct sigmo_batch {
     bfree(qcmax);
     bfree(arena);
     bfree(surv);
-    bfree(pair_off);
+    bfree(blocks);
     bfree(mol_count);
     bfree(counters);
     bfree(offsets);
@@ -1468,7 +1507,7 @@ int sigmo_batch_workspace_bytes(const sigmo_batch* b, uint32_t num_query_graphs,
   const bool one_sync = !db->num_wide && pairs && pairs <= kOneSyncPairs;
   const uint64_t gmcr_pairs = one_sync ? pairs : guess;
   *bytes = query_nodes * sigmo_k::token_segment(static_cast<uint32_t>(R)) * 2 + Gq * (sizeof(sigmo_k::QueryInfo) + 8 * R * (1 + sigmo_k::kClasses)) +
-           Gd * W * 8 + pairs * 4 + arena_words * 8 + gmcr_pairs * 16 + (db->num_wide ? guess * 4 : 0) + (Gd + 1) * 8;
+           Gd * W * 8 + uint64_t(db->order.total()) * Gq * 16 + arena_words * 8 + gmcr_pairs * 16 + (db->num_wide ? guess * 4 : 0) + (Gd + 1) * 8;
   return SIGMO_OK;
 }
 
@@ -1558,7 +1597,7 @@ int shape_run(const sigmo_batch* b, const sigmo_graph* query, int cus, RunShape&
   uint64_t per_cu = std::max<uint64_t>(1, std::min<uint64_t>(32 / sigmo_k::kGroupWaves, 160 * 1024 / sigmo_k::group_lds_bytes(L.group_slots, L.R)));
   if (b->tune.filter_blocks_per_cu) per_cu = std::min<uint64_t>(per_cu, b->tune.filter_blocks_per_cu);
   L.group_blocks = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(items, ucus * per_cu)));
-  // a wavefront's arena chunk holds the largest query graph for a whole group (2,048 words) and, for
+  // a wavefront's arena chunk holds the largest query graph for a whole group (1,024 words) and, for
   // many pairs, more: claims meet on one address
   const uint64_t waves = uint64_t(L.group_blocks) * sigmo_k::kGroupWaves;
   uint64_t chunk = 2048;
@@ -1617,7 +1656,7 @@ hipError_t launch_filter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
   a.arena = b->arena;
   a.arena_cap = b->cap_arena;
   a.surv = b->surv;
-  a.pair_off = b->pair_off;
+  a.blocks = b->blocks;
   a.counters = b->counters;
   a.stats = b->counters + 16;
   hipLaunchKernelGGL(sigmo_k::k_pair_group, dim3(L.group_blocks), dim3(sigmo_k::kGroupWaves * 64),
@@ -1649,15 +1688,15 @@ hipError_t launch_count_scan(sigmo_batch* b, const RunShape& L, hipStream_t s) {
 hipError_t launch_scatter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
   if (!L.Gd) return hipSuccess;
   const uint64_t cap = std::min(b->cap_idx, std::min(b->cap_pg, b->cap_mo));
-  if (L.W == 1) {  // at most 64 query graphs: a thread per molecule
-    const dim3 grid(static_cast<unsigned>((uint64_t(L.Gd) + 255) / 256));
-    hipLaunchKernelGGL(sigmo_k::k_surv_scatter_thread, grid, dim3(256), 0, s, L.Gd, L.Gq, L.W, b->surv, b->offsets, b->pair_off, b->indices,
+  const sigmo_k::GroupOrder& order = b->db->order;
+  if (L.W == 1) {  // at most 64 query graphs: a lane per molecule
+    const dim3 grid((order.total() + 3) / 4);
+    hipLaunchKernelGGL(sigmo_k::k_surv_scatter_lanes, grid, dim3(256), 0, s, order, L.Gq, b->db->minfo, b->surv, b->offsets, b->blocks, b->indices,
                        b->pair_graph, b->mask_off, cap);
     return hipGetLastError();
   }
-  const uint64_t blocks = (static_cast<uint64_t>(L.Gd) * sigmo_k::kWave + 255) / 256;  // a wavefront per molecule
-  hipLaunchKernelGGL(sigmo_k::k_surv_scatter, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, L.Gd, L.Gq, L.W, b->surv, b->offsets,
-                     b->pair_off, b->indices, b->pair_graph, b->mask_off, cap);
+  hipLaunchKernelGGL(sigmo_k::k_surv_scatter, dim3(order.total()), dim3(256), 0, s, order, L.Gq, L.W, b->db->minfo, b->surv, b->offsets, b->blocks,
+                     b->indices, b->pair_graph, b->mask_off, cap);
   return hipGetLastError();
 }
 
@@ -1687,7 +1726,7 @@ int size_fixed_buffers(sigmo_batch* b, const RunShape& L) {
   BATCH_TRY(b->grow(&b->qmax, b->cap_qmax, uint64_t(L.Gq) * L.R));
   BATCH_TRY(b->grow(&b->qcmax, b->cap_qcmax, uint64_t(L.Gq) * L.R * sigmo_k::kClasses));
   BATCH_TRY(b->grow(&b->surv, b->cap_surv, uint64_t(L.Gd) * L.W));
-  BATCH_TRY(b->grow(&b->pair_off, b->cap_pair_off, L.pairs));
+  BATCH_TRY(b->grow(&b->blocks, b->cap_blocks, uint64_t(b->db->order.total()) * L.Gq));
   BATCH_TRY(b->grow(&b->mol_count, b->cap_mc, uint64_t(L.Gd) + 1));
   BATCH_TRY(b->grow(&b->offsets, b->cap_off, uint64_t(L.Gd) + 1));
   BATCH_TRY(b->grow(&b->scan_tmp, b->cap_scan, (uint64_t(L.Gd) + 1023) / 1024 + 1));

@@ -13,36 +13,46 @@
 namespace sigmo_k {
 namespace {
 
-// Candidate masks of the survivor arena: k consecutive words per pair (molecules of <= 64 nodes).
-// `overflow` is the pair evaluation's arena-overflow flag: once set, offsets past the arena were
-// handed out and no mask may be read, so the join does nothing and the host repeats the run with
-// a larger arena.
+// Candidate masks of the survivor arena: k consecutive per pair, of 32 bits for molecules of <= 32
+// nodes, 64 for 33..64 and 128 for wider ones.  `overflow` is the pair evaluation's arena-overflow
+// flag: once set, offsets past the arena were handed out and no mask may be read, so the join does
+// nothing and the host repeats the run with a larger arena.
 struct ArenaMasks {
   const uint64_t* arena;
   const uint32_t* mask_off;
   const unsigned long long* overflow;
   __device__ __forceinline__ bool aborted() const { return uniform32(static_cast<uint32_t>(*overflow != 0ull)) != 0u; }
   __device__ __forceinline__ uint32_t base(uint64_t j) const { return mask_off[j]; }
-  __device__ __forceinline__ uint64_t mask(uint32_t base, uint32_t, uint32_t depth, uint32_t, uint32_t) const {
-    return arena[static_cast<uint64_t>(base) + depth];
+  __device__ __forceinline__ uint64_t mask(uint32_t base, uint32_t, uint32_t depth, uint32_t, uint32_t n) const {
+    const uint64_t* p = arena + base;
+    return n <= 32 ? reinterpret_cast<const uint32_t*>(p)[depth] : p[depth];
   }
   // molecules of 65..128 nodes: two words per query node (positions 0-63, 64-127)
   __device__ __forceinline__ void mask2(uint32_t base, uint32_t, uint32_t depth, uint32_t, uint32_t, uint64_t& lo, uint64_t& hi) const {
     lo = arena[static_cast<uint64_t>(base) + 2 * depth];
     hi = arena[static_cast<uint64_t>(base) + 2 * depth + 1];
   }
-  // The masks of query nodes 0..k-1 (entries from k on are not to be read), two per 16-byte load: a
-  // pair's block starts on a 4-word boundary and spans a multiple of 4 words, so a load that starts
-  // below k stays inside it.
+  // The masks of query nodes 0..k-1 (entries from k on are not to be read), 16 bytes per load: a
+  // pair's block starts on a 16-byte boundary and spans a multiple of four masks, so a load that
+  // starts below k stays inside it.
   template <int N>
-  __device__ __forceinline__ void masks(uint32_t base, uint32_t, uint32_t k, uint32_t, uint32_t, uint64_t (&m)[N]) const {
-    static_assert(N % 2 == 0, "masks come in pairs");
+  __device__ __forceinline__ void masks(uint32_t base, uint32_t, uint32_t k, uint32_t, uint32_t n, uint64_t (&m)[N]) const {
+    static_assert(N % 4 == 0, "masks come in fours");
+    const uint4* p = reinterpret_cast<const uint4*>(arena + base);
+    const uint32_t half = n <= 32;
+    uint4 v[N / 2];  // one to two nodes each, or one to four
 #pragma unroll
-    for (uint32_t t = 0; t < static_cast<uint32_t>(N); t += 2) {
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (t < k) v = *reinterpret_cast<const uint4*>(arena + static_cast<uint64_t>(base) + t);
-      m[t] = static_cast<uint64_t>(v.x) | (static_cast<uint64_t>(v.y) << 32);
-      m[t + 1] = static_cast<uint64_t>(v.z) | (static_cast<uint64_t>(v.w) << 32);
+    for (uint32_t t = 0; t < static_cast<uint32_t>(N) / 2; ++t) {
+      v[t] = make_uint4(0, 0, 0, 0);
+      if (2 * t < (half ? (k + 1) / 2 : k)) v[t] = p[t];
+    }
+#pragma unroll
+    for (uint32_t t = 0; t < static_cast<uint32_t>(N); t += 4) {
+      const uint4 a = v[t / 4], b = v[t / 2], c = v[t / 2 + 1];
+      m[t] = half ? a.x : b.x | (static_cast<uint64_t>(b.y) << 32);
+      m[t + 1] = half ? a.y : b.z | (static_cast<uint64_t>(b.w) << 32);
+      m[t + 2] = half ? a.z : c.x | (static_cast<uint64_t>(c.y) << 32);
+      m[t + 3] = half ? a.w : c.z | (static_cast<uint64_t>(c.w) << 32);
     }
   }
   // The two-word masks of query nodes 0..k-1, one 16-byte load per node.

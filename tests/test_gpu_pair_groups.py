@@ -50,6 +50,23 @@ def test_group_sizes(ctx, small, mid, wide):
     _check(ctx, qs, ms, 4)
 
 
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 129])
+def test_mask_blocks(ctx, count):
+    # query sizes around the four masks of a 16-byte store, in all three mask widths
+    rng = np.random.default_rng(count)
+    ms = [_graph(rng, int(n), [8, 7, 6, 8], int(n) // 12) for n in rng.choice([9, 20, 32, 33, 50, 64, 65, 100, 128], 170)]
+    qs = []
+    for i in range(count):  # connected parts of the molecules: a node and those that follow it in its tree
+        lab, edges = ms[int(rng.integers(0, len(ms)))]
+        k = min(len(lab), 2 + i % 16)
+        nodes = [int(rng.integers(0, len(lab)))]
+        while len(nodes) < k:
+            nodes += [b if a in nodes else a for a, b in edges if (a in nodes) != (b in nodes)][: k - len(nodes)]
+            nodes = list(dict.fromkeys(nodes))
+        qs.append(([lab[x] for x in nodes], [(nodes.index(a), nodes.index(b)) for a, b in edges if a in nodes and b in nodes]))
+    _check(ctx, qs, ms, 3)
+
+
 @pytest.mark.parametrize("R", [1, 6, 8])
 def test_more_labels_than_lds_holds(ctx, R):
     rng = np.random.default_rng(R)

@@ -38,9 +38,27 @@ namespace {
 constexpr uint32_t kMaxLevels = 8;        // token encoding keeps 3 bits of level
 constexpr uint16_t kEndToken = 0xFFFF;    // closes a query node's token segment
 
-// Tokens of one query node: [label] [requirement]* [end], requirement = r | l << 3 | c << 7
-// (level r < 8, label l < 16, count 1 <= c <= 15; those of counts up to kNearCount first).  Segments are 4-token aligned with one spare
-// word, so the reader's one-word lookahead stays inside the segment.
+// Tokens of one query node: [label] [requirement]* [end] .., with end tokens up to a whole quad of
+// four.  A token is a plane of a label (6 bits) and a key, label | kind << 4 (6 bits): requirements of
+// counts 1..4 (kind 0) and 5..8 (1) name plane 4 r + (c - 1) % 4 of level r < 8, larger counts (2) hold
+// r and c - 8 there; the label token of a label < 16 is its plane 4 R; kind 3 has the end (key 63),
+// the wildcard label (49) and the other labels (50, the label's upper bits above the key).
+constexpr uint32_t kKeyWildcard = 49, kKeyOther = 50;
+__device__ __forceinline__ uint32_t requirement_token(uint32_t r, uint32_t l, uint32_t c) {
+  return (c <= 8 ? ((c - 1) & 3u) | (r << 2) | (((c - 1) >> 2) << 10) : r | ((c - 8) << 3) | (2u << 10)) | (l << 6);
+}
+__device__ __forceinline__ uint32_t token_level(uint32_t t) { return (t >> 10) == 2 ? t & 7u : (t >> 2) & 7u; }
+__device__ __forceinline__ uint32_t token_count(uint32_t t) { return (t >> 10) == 2 ? 8 + ((t >> 3) & 7u) : 1 + (t & 3u) + 4 * (t >> 10); }
+__device__ __forceinline__ uint32_t token_label(uint32_t t) { return (t >> 6) & 15u; }
+__device__ __forceinline__ uint32_t label_token(uint32_t label, uint32_t R) {
+  if (label < 16) return 4 * R | (label << 6);
+  return label == 255 ? kKeyWildcard << 6 : (label & 63u) | (kKeyOther << 6) | ((label >> 6) << 12);
+}
+// The label of a label token, 255 for the wildcard.
+__device__ __forceinline__ uint32_t labelled(uint32_t t) {
+  const uint32_t key = (t >> 6) & 63u;
+  return key < 16 ? key : (key == kKeyWildcard ? 255u : (t & 63u) | ((t >> 12) << 6));
+}
 __host__ __device__ constexpr uint32_t token_segment(uint32_t R) { return ((2 + 16 * R + 3) & ~3u) + 4; }
 
 // Bit 0 of every nonzero nibble.
@@ -431,17 +449,15 @@ __global__ __launch_bounds__(256) void k_query_prepare(GraphDev q, uint32_t R, u
   }
   uint16_t* t = tokens + static_cast<uint64_t>(prev) * seg + (incl - len);
   if (valid) {
-    t[0] = static_cast<uint16_t>(label);
-    uint32_t at = 1, back = ntok - 1;  // near requirements from the front, the others from the back
-    t[back] = kEndToken;
+    t[0] = static_cast<uint16_t>(label_token(label, R));
+    for (uint32_t x = ntok - 1; x < len; ++x) t[x] = kEndToken;
+    uint32_t at = 1;
 #pragma unroll
     for (uint32_t r = 0; r < kMaxLevels; ++r)
       if (r < R)
         for (uint64_t nz = nibbles_set(sig[r]); nz; nz &= nz - 1) {
           const uint32_t sh = static_cast<uint32_t>(__builtin_ctzll(nz)), c = static_cast<uint32_t>(sig[r] >> sh) & 15u;
-          const uint16_t tk = static_cast<uint16_t>(r | (sh << 1) | (c << 7));  // label = sh / 4, at bit 3
-          if (c <= kNearCount) t[at++] = tk;
-          else t[--back] = tk;
+          t[at++] = static_cast<uint16_t>(requirement_token(r, sh / 4, c));
         }
   }
   uint32_t bits = valid && label < 16 ? 1u << label : 0u;
@@ -494,7 +510,7 @@ __global__ __launch_bounds__(256) void k_query_classes(uint32_t Gq, uint32_t R, 
     const uint64_t ends = __ballot(in && has_end);
     const uint64_t prev = ends & below;  // end words before this lane's in the chunk
     const uint32_t start_lane = prev ? 64u - static_cast<uint32_t>(__builtin_clzll(prev)) : 0u;
-    const uint32_t first = static_cast<uint32_t>(w & 0xFFFFull);
+    const uint32_t first = labelled(static_cast<uint32_t>(w & 0xFFFFull));
     const uint32_t lab_here = static_cast<uint32_t>(__shfl(static_cast<int>(first), static_cast<int>(start_lane)));
     const uint32_t label = prev || starts_new ? lab_here : carry_label;
     const bool is_start = prev ? lane == start_lane : (lane == 0 && starts_new);
@@ -508,7 +524,7 @@ __global__ __launch_bounds__(256) void k_query_classes(uint32_t Gq, uint32_t R, 
       for (uint32_t j = is_start ? 1u : 0u; j < 4; ++j) {
         const uint32_t t = static_cast<uint32_t>(w >> (16 * j)) & 0xFFFFu;
         if (t == kEndToken) break;
-        atomicMax(&cnt[(c * kMaxLevels + (t & 7u)) * 16 + ((t >> 3) & 15u)], (t >> 7) & 15u);
+        atomicMax(&cnt[(c * kMaxLevels + token_level(t)) * 16 + token_label(t)], token_count(t));
       }
     }
     nodes += static_cast<uint32_t>(__popcll(ends));
@@ -673,13 +689,14 @@ struct GroupArgs {
   GraphDev d;
   GroupOrder order;
   uint32_t R, Gq, W;
-  uint32_t parts;          // blocks that share a group's query graphs (a power of two, <= 64 / kGroupWaves)
+  uint32_t parts;          // blocks that share a group's query graphs (a power of two <= 8)
   uint32_t slots;          // labels whose planes LDS holds
+  uint32_t rich;           // the database's most frequent label (>= 16: none)
   uint32_t chunk;          // arena words a wavefront claims at a time
   const MolInfo* minfo;    // width-class order
   const uint4* planes;     // [((group*R + r)*16 + l)*64 + lane]
   const uint32_t* labs;    // [(group*16 + l)*64 + lane]
-  const uint16_t* tokens;
+  const uint64_t* tokens;  // quads
   const QueryInfo* qinfo;
   uint64_t* arena;
   uint64_t arena_cap;
@@ -689,8 +706,19 @@ struct GroupArgs {
   unsigned long long* stats;     // kGroupStatSlots x 16: [0] node evaluations, [1] their live lanes, [2] pre-tested pairs
 };
 
-// LDS: near planes [label slot][level][count][lane], label masks [label slot][lane], the next item.
-__host__ __device__ constexpr uint32_t group_lds_bytes(uint32_t slots, uint32_t R) { return slots * (R * 1024 + 256) + 16; }
+// LDS: planes of 64 words, at most 256 of them, in blocks of slot_planes: a label slot's positions
+// whose count reaches 1..4 per level, then its own positions; the last block has the counts 5..8 of
+// the database's most frequent label, then every position.  Then the list of the group's live query
+// graphs, of eight query words at a time, and GroupCounters.
+__host__ __device__ constexpr uint32_t slot_planes(uint32_t R) { return 4 * R + 1; }
+struct GroupCounters {
+  uint32_t next_item;
+  uint32_t listed[2], taken[2];  // of this list and the next
+};
+constexpr uint32_t kGroupListBytes = kGroupWaves * kWave * sizeof(uint4) + sizeof(GroupCounters);
+__host__ __device__ constexpr uint32_t group_lds_bytes(uint32_t slots, uint32_t R) {
+  return (slots + 1) * slot_planes(R) * 256 + kGroupListBytes;
+}
 
 // The value of lane ^ 1 and lane ^ 2 (quad permutations).
 __device__ __forceinline__ uint32_t quad_xor1(uint32_t x) {
@@ -706,20 +734,37 @@ __device__ __forceinline__ uint32_t pair_block(uint32_t base, uint32_t words, ui
   return base + static_cast<uint32_t>(__popcll(lanes & ((1ull << lane0) - 1))) * words;
 }
 
-// A wavefront's arena chunk and statistics (wave-uniform but `live`).
+// The lane's word of the plane named by byte X of `quad`: the permutation makes plane * 256 + lane * 4,
+// the byte address (dynamic LDS starts at 0: the kernel has no other).
+template <int X>
+__device__ __forceinline__ uint32_t quad_plane(uint32_t quad, uint32_t lane4) {
+  const uint32_t at = __builtin_amdgcn_perm(quad, lane4, 0x0c0c0000u | ((4u + X) << 8));
+  return *reinterpret_cast<const __attribute__((address_space(3))) uint32_t*>(static_cast<uintptr_t>(at));
+}
+
+// The kernel's arguments, read where they are used: kept in registers, those of the rare paths would
+// spill the loop's scalars.
+__device__ __forceinline__ const __attribute__((address_space(4))) GroupArgs& group_args() {
+  auto p = (const __attribute__((address_space(4))) GroupArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *p;
+}
+
+// A wavefront's arena chunk (wave-uniform) and statistics: lane 0 node evaluations, lane 1 their live
+// lanes, lane 2 pre-tested pairs.
 struct GroupState {
-  uint64_t next, end, first_chunks;
-  uint64_t nodes = 0, scans = 0;
-  uint32_t live = 0;  // per lane
+  uint64_t next;
+  uint32_t left;
+  uint32_t turn = 0;  // which of the list counters are this list's
+  uint64_t sums = 0;
 };
 
 // One group of a class against the wavefront's share of the query graphs.
 template <int CLS>
-__device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uint32_t part, uint32_t wave, uint32_t* near_lds, uint32_t* labs_lds,
-                                           GroupState& st) {
-  const uint32_t lane = static_cast<uint32_t>(lane_id());
-  const uint32_t R = a.R;
-  const uint32_t seg = token_segment(R);
+__device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uint32_t part, uint32_t wave, uint32_t* planes_lds, GroupState& st) {
+  const uint32_t lane = static_cast<uint32_t>(lane_id()), lane4 = lane * 4;
+  const uint32_t R = a.R, SP = slot_planes(R);
+  const uint64_t seg = token_segment(R) / 4;
   const uint32_t first = (CLS > 0 ? a.order.count[0] : 0u) + (CLS > 1 ? a.order.count[1] : 0u);
   const uint64_t group = grp + (CLS > 0 ? a.order.groups(0) : 0u) + (CLS > 1 ? a.order.groups(1) : 0u);
   const uint32_t at = grp * (64u >> CLS) + (lane >> CLS);  // the lane's molecule within its class
@@ -734,11 +779,15 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
   for (uint32_t l = 0; l < 16; ++l) present |= static_cast<uint32_t>(__ballot((mi.mlab >> l) & 1u) != 0ull) << l;
   present = uniform32(present);
   const uint32_t occur = static_cast<uint32_t>(__popc(present)), staged = min(occur, a.slots);
+  auto slot_of = [&](uint32_t l) -> uint32_t { return static_cast<uint32_t>(__popc(present & ((1u << l) - 1u))); };
   auto label_of = [&](uint32_t slot) -> uint32_t {  // the slot-th label that occurs
     uint32_t left = present;
     for (uint32_t x = 0; x < slot; ++x) left &= left - 1;
     return static_cast<uint32_t>(__builtin_ctz(left));
   };
+  const uint32_t rich = a.rich < 16 && ((present >> a.rich) & 1u) && slot_of(a.rich) < staged ? a.rich : 16u;
+  const uint32_t all_plane = a.slots * SP + 4 * R;  // the plane of every position
+  auto plane = [&](uint32_t index) -> uint32_t& { return planes_lds[index * kWave + lane]; };
   // the wavefronts take every eighth (label, level), four loads in flight each
   for (uint32_t e0 = wave; e0 < staged * R; e0 += 4 * kGroupWaves) {
     uint4 v[4];
@@ -751,135 +800,200 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
 #pragma unroll
     for (uint32_t x = 0; x < 4; ++x) {
       const uint32_t e = e0 + x * kGroupWaves;
-      if (e < staged * R) stage_near(near_lds, e, v[x]);
+      if (e >= staged * R) break;
+      uint32_t t[kNearCount];
+      thermometer(v[x], t);
+#pragma unroll
+      for (uint32_t c = 0; c < kNearCount; ++c) plane(e / R * SP + 4 * (e % R) + c) = t[c];
+      if (label_of(e / R) == rich) {
+        const uint32_t at5 = a.slots * SP + 4 * (e % R);
+        plane(at5) = v[x].w | (v[x].z & (v[x].y | v[x].x));
+        plane(at5 + 1) = v[x].w | (v[x].z & v[x].y);
+        plane(at5 + 2) = v[x].w | (v[x].z & v[x].y & v[x].x);
+        plane(at5 + 3) = v[x].w;
+      }
     }
   }
   for (uint32_t slot = wave; slot < staged; slot += kGroupWaves)
-    labs_lds[slot * kWave + lane] = valid ? a.labs[(group * 16 + label_of(slot)) * 64 + lane] : 0u;
+    plane(slot * SP + 4 * R) = valid ? a.labs[(group * 16 + label_of(slot)) * 64 + lane] : 0u;
+  const uint32_t positions = mi.n > 32 * h ? min(32u, mi.n - 32 * h) : 0u;
+  if (wave == 0) plane(all_plane) = positions >= 32 ? ~0u : (1u << positions) - 1u;
   __syncthreads();
 
-  const uint32_t workers = kGroupWaves * a.parts;  // wavefronts that share the query graphs (a power of two <= 64)
-  uint64_t mine = 0;
-  for (uint32_t t = part * kGroupWaves + wave; t < 64; t += workers) mine |= 1ull << t;
-  for (uint32_t w = 0; w < a.W; ++w) {
-    const uint64_t word = valid ? a.surv[static_cast<uint64_t>(mi.m) * a.W + w] : 0ull;
-    uint32_t any_lo = static_cast<uint32_t>(word), any_hi = static_cast<uint32_t>(word >> 32);
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      any_lo |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(any_lo), o));
-      any_hi |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(any_hi), o));
+  // what each key's planes start at, << 8 the token bits that count from there; bit 31: LDS has none
+  uint32_t keys;
+  {
+    const uint32_t l = lane & 15u, kind = lane >> 4, slot = kind == 1 ? a.slots : slot_of(l);
+    const bool here = kind == 0 ? slot < staged : kind == 1 && l == rich;
+    const bool any = kind == 3 && lane != kKeyOther;
+    keys = here ? slot * SP | (63u << 8) : (all_plane | (any ? 0u : 1u << 31));
+  }
+  auto key_of = [&](uint32_t t) -> uint32_t {  // of the token in t's low half
+    return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>((t >> 4) & 0xFCu), static_cast<int>(keys)));
+  };
+
+  uint4* list = reinterpret_cast<uint4*>(planes_lds + (a.slots + 1) * SP * kWave);
+  GroupCounters* ctr = reinterpret_cast<GroupCounters*>(list + kGroupWaves * kWave);
+  // 64 quads of a graph's tokens, one per lane (a graph's segment holds k * seg of them)
+  auto quads = [&](uint32_t qoff, uint32_t k, uint32_t from) -> uint64_t {
+    return a.tokens[qoff * seg + min(from + lane, static_cast<uint32_t>(k * seg) - 1)];
+  };
+  uint32_t nodes = 0, live = 0, scans = 0;
+  for (uint32_t w0 = 0; w0 < a.W; w0 += kGroupWaves) {
+    // eight query words, one per wavefront: transposed, a lane has a query graph and the lanes of its
+    // pre-tested pairs; graphs that have some are listed with their first node and size
+    {
+      const auto& c = group_args();
+      const uint32_t w = w0 + wave, g = w * kWave + lane;
+      const uint64_t word = valid && w < c.W ? c.surv[static_cast<uint64_t>(mi.m) * c.W + w] : 0ull;
+      if (__ballot(word != 0)) {  // wave-uniform
+        const uint64_t act = transpose64(word);
+        const bool mine = act != 0 && (lane & (c.parts - 1)) == part;
+        const uint64_t mm = __ballot(mine);
+        uint32_t b = 0;
+        if (lane == 0) b = atomicAdd(&ctr->listed[st.turn], static_cast<uint32_t>(__popcll(mm)));
+        b = uniform32(b);
+        if (mine) {
+          const QueryInfo* info = c.qinfo + g;
+          list[b + static_cast<uint32_t>(__popcll(mm & ((1ull << lane) - 1)))] =
+              make_uint4(static_cast<uint32_t>(act), static_cast<uint32_t>(act >> 32), info->qoff, (g << 5) | (info->k - 1));
+        }
+      }
     }
-    uint64_t dead = 0;
-    for (uint64_t bits = uniform64(any_lo | (static_cast<uint64_t>(any_hi) << 32)) & mine; bits; bits &= bits - 1) {  // wave-uniform
-      const uint32_t jb = static_cast<uint32_t>(__builtin_ctzll(bits));
-      const uint32_t g = w * kWave + jb;
-      const bool act = (word >> jb) & 1ull;
-      const uint64_t am = __ballot(act) & leaders;
-      const uint32_t qoff = uniform32(a.qinfo[g].qoff), k = uniform32(a.qinfo[g].k);
+    __syncthreads();
+    const uint32_t listed = uniform32(ctr->listed[st.turn]);
+    if (threadIdx.x == 0) ctr->listed[st.turn ^ 1u] = ctr->taken[st.turn ^ 1u] = 0;
+    uint32_t t = wave;
+    uint4 entry = make_uint4(0, 0, 0, 0);
+    uint64_t ahead = 0;
+    auto fetch = [&]() {
+      const uint4 e = list[t];
+      entry = make_uint4(uniform32(e.x), uniform32(e.y), uniform32(e.z), uniform32(e.w));
+      ahead = quads(entry.z, (entry.w & 31u) + 1, 0);
+    };
+    if (t < listed) fetch();
+    while (t < listed) {  // wave-uniform
+      const uint64_t act = entry.x | (static_cast<uint64_t>(entry.y) << 32), am = act & leaders;
+      const uint32_t g = entry.w >> 5, qoff = entry.z, k = (entry.w & 31u) + 1;
+      uint64_t raw = ahead;
+      // the next graph, whose tokens are on their way meanwhile
+      if (lane == 0) t = kGroupWaves + atomicAdd(&ctr->taken[st.turn], 1u);
+      t = uniform32(t);
+      if (t < listed) fetch();
       const uint32_t cnt = static_cast<uint32_t>(__popcll(am)), pw = pair_words(k, CLS);
-      st.scans += cnt;
-      if (st.next + static_cast<uint64_t>(cnt) * pw > st.end) {
+      scans += cnt;
+      if (cnt * pw > st.left) {
+        const auto& c = group_args();
         unsigned long long b = 0;
         if (lane == 0) {
-          b = st.first_chunks + atomicAdd(&a.counters[1], static_cast<unsigned long long>(a.chunk));
-          if (b + a.chunk > a.arena_cap) atomicOr(&a.counters[3], 1ull);
+          b = static_cast<uint64_t>(gridDim.x) * kGroupWaves * c.chunk + atomicAdd(&c.counters[1], static_cast<unsigned long long>(c.chunk));
+          if (b + c.chunk > c.arena_cap) atomicOr(&c.counters[3], 1ull);
         }
         st.next = uniform64(__shfl(b, 0));
-        st.end = st.next + a.chunk;
+        st.left = c.chunk;
       }
       const uint64_t base0 = st.next, base = base0 + static_cast<uint64_t>(__popcll(am & below)) * pw;
-      st.next += static_cast<uint64_t>(cnt) * pw;
-      const bool room = st.end <= a.arena_cap;
+      st.next += cnt * pw;
+      st.left -= cnt * pw;
+      const bool room = st.next + st.left <= a.arena_cap;
 
-      // the graph's tokens, 64 at a time and one per lane, decoded once: a near requirement becomes
-      // its plane's offset in LDS; `fars` marks the others (a large count, or a label whose planes
-      // are not there)
-      const uint16_t* tok = a.tokens + static_cast<uint64_t>(qoff) * seg;
-      const uint32_t total = k * seg;
-      uint32_t pos = 0, p = 0, raw = 0, dec = 0;
+      // The quads are decoded once, each lane its own: four planes by their bytes.  A node's mask is the
+      // AND of its quads' planes; `fars` marks quads with a token that LDS has no plane of.
+      uint32_t from = 0, p = 0, dec = 0;
       uint64_t ends = 0, fars = 0;
-      auto load_tokens = [&](uint32_t from) {
-        pos = from;
-        p = 0;
-        raw = tok[min(from + lane, total - 1)];
-        const uint32_t r = raw & 7u, c = (raw >> 7) & 15u, slot = static_cast<uint32_t>(__popc(present & ((1u << ((raw >> 3) & 15u)) - 1u)));
-        dec = near_offset(slot * R + r, c);
-        fars = __ballot(c > kNearCount || slot >= staged);
-        ends = __ballot(raw == kEndToken);
-      };
-      // the candidates of the next node among this lane's positions; leaves p at the node after
-      auto node_mask = [&]() -> uint32_t {
-        if (p >= kWave || (ends >> p) == 0) load_tokens(pos + p);  // the node's stream (at most 33 tokens) crosses the 64
-        const uint32_t e = p + static_cast<uint32_t>(__builtin_ctzll(ends >> p));
-        // its label token: the filter's label test (isomorphism.hpp:49)
-        const uint32_t ql = rl32(raw, p);
-        uint32_t mask = 0, t = p + 1;
-        p = (e & ~3u) + 4;
-        if (ql < 16u) {
-          const uint32_t slot = static_cast<uint32_t>(__popc(present & ((1u << ql) - 1u)));
-          if (slot < staged) mask = labs_lds[slot * kWave + lane];
-          else if (valid) mask = a.labs[(group * 16 + ql) * 64 + lane];
-        } else {
-          const uint32_t positions = mi.n > 32 * h ? min(32u, mi.n - 32 * h) : 0u;
-          if (ql == 255u) {
-            mask = positions >= 32 ? ~0u : (1u << positions) - 1u;
-          } else if (act) {
-            for (uint32_t x = 0; x < positions; ++x)
-              if (a.d.nl[static_cast<uint64_t>(mi.s) + 32 * h + x] == ql) mask |= 1u << x;
+      uint64_t alive = act;
+      uint32_t m0 = 0, m1 = 0, m2 = 0, m3 = 0, i = 0;
+      // nodes whose masks, with those before them, go out
+      const uint32_t flush = (0x88888888u & ((2u << (k - 1)) - 1u)) | (1u << (k - 1));
+      for (;; ++i) {  // wave-uniform
+        if (ends == 0) {  // the node's quads (at most nine) cross the 64, or the first
+          from += p;
+          p = 0;
+          if (from) raw = quads(qoff, k, from);
+          ends = __ballot(static_cast<uint32_t>(raw >> 48) == kEndToken);  // every end quad ends in one
+          const uint32_t t0 = static_cast<uint32_t>(raw), t1 = t0 >> 16, t2 = static_cast<uint32_t>(raw >> 32), t3 = t2 >> 16;
+          const uint32_t k0 = key_of(t0), k1 = key_of(t1), k2 = key_of(t2), k3 = key_of(t3);
+          const uint32_t d0 = k0 + (t0 & ((k0 >> 8) & 63u)), d1 = k1 + (t1 & ((k1 >> 8) & 63u));
+          const uint32_t d2 = k2 + (t2 & ((k2 >> 8) & 63u)), d3 = k3 + (t3 & ((k3 >> 8) & 63u));
+          dec = __builtin_amdgcn_perm(__builtin_amdgcn_perm(d3, d2, 0x0c0c0400u), __builtin_amdgcn_perm(d1, d0, 0x0c0c0400u), 0x05040100u);
+          fars = __ballot(static_cast<int32_t>(k0 | k1 | k2 | k3) < 0);
+        }
+        const uint32_t count = static_cast<uint32_t>(__builtin_ctzll(ends)) + 1, p1 = p + count;
+        ends >>= count;
+        live += static_cast<uint32_t>(__popcll(alive));
+        uint32_t mask = ~0u;
+        if (fars) {
+          const auto& c = group_args();
+          for (uint32_t x = p; x < p1; ++x) {
+            if (!((fars >> x) & 1ull)) continue;
+            const uint64_t qw = rl32(static_cast<uint32_t>(raw), x) | (static_cast<uint64_t>(rl32(static_cast<uint32_t>(raw >> 32), x)) << 32);
+            for (uint32_t y = 0; y < 4; ++y) {
+              const uint32_t t = static_cast<uint32_t>(qw >> (16 * y)) & 0xFFFFu;
+              if (t == kEndToken) break;
+              const uint32_t key = (t >> 6) & 63u, label = token_label(t);
+              if (x == p && y == 0) {  // the label: the filter's test (isomorphism.hpp:49)
+                if (key < 16u) {
+                  mask &= valid ? c.labs[(group * 16 + label) * 64 + lane] : 0u;
+                } else if (key == kKeyOther) {
+                  uint32_t at_label = 0;
+                  if ((act >> lane) & 1ull)
+                    for (uint32_t v = 0; v < positions; ++v)
+                      if (c.d.nl[static_cast<uint64_t>(mi.s) + 32 * h + v] == labelled(t)) at_label |= 1u << v;
+                  mask &= at_label;
+                }
+              } else {
+                uint4 v = make_uint4(0, 0, 0, 0);
+                if (valid) {
+                  const uint4* src = c.planes;
+                  v = src[((group * R + token_level(t)) * 16 + label) * 64 + lane];
+                }
+                mask &= ge4_bits<uint32_t>(v.x, v.y, v.z, v.w, token_count(t));
+              }
+            }
           }
         }
-        // near requirements come first in a node's stream
-        const uint64_t fm = t < kWave ? fars >> t : 0ull;
-        const uint32_t near = fm ? min(e, t + static_cast<uint32_t>(__builtin_ctzll(fm))) : e;
-        mask = near_tests(near_lds, dec, t, near, mask);
-        for (t = near; t < e; ++t) {
-          if (!((fars >> t) & 1ull)) {
-            mask &= near_plane(near_lds, rl32(dec, t));
-          } else {
-            const uint32_t tw = rl32(raw, t);
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (valid) v = a.planes[((group * R + (tw & 7u)) * 16 + ((tw >> 3) & 15u)) * 64 + lane];
-            mask &= ge4_bits<uint32_t>(v.x, v.y, v.z, v.w, (tw >> 7) & 15u);
-          }
+        for (; p + 2 <= p1; p += 2) {
+          const uint32_t qa = rl32(dec, p), qb = rl32(dec, p + 1);
+          const uint32_t a0 = quad_plane<0>(qa, lane4), a1 = quad_plane<1>(qa, lane4), a2 = quad_plane<2>(qa, lane4), a3 = quad_plane<3>(qa, lane4);
+          const uint32_t b0 = quad_plane<0>(qb, lane4), b1 = quad_plane<1>(qb, lane4), b2 = quad_plane<2>(qb, lane4), b3 = quad_plane<3>(qb, lane4);
+          mask &= a0 & a1;
+          mask &= a2 & a3;
+          mask &= b0 & b1;
+          mask &= b2 & b3;
         }
-        ++st.nodes;
-        return mask;
-      };
-      // whether the lane's molecule keeps a candidate
-      auto some = [&](uint32_t mask) -> bool {
-        if (CLS >= 1) mask |= quad_xor1(mask);
-        if (CLS == 2) mask |= quad_xor2(mask);
-        return mask != 0;
-      };
-      load_tokens(0);
-      bool alive = act;
-      // masks go out four nodes at a time, in 16-byte stores (nodes past the last fall in the block's
-      // padding); a pair dies at its first node without candidates (gmcr.hpp:56-61)
-      uint32_t m0 = 0, m1 = 0, m2 = 0, m3 = 0;
-      for (uint32_t i = 0; i < k; ++i) {  // wave-uniform
-        st.live += alive;
+        if (p < p1) {
+          const uint32_t qa = rl32(dec, p);
+          mask &= quad_plane<0>(qa, lane4) & quad_plane<1>(qa, lane4);
+          mask &= quad_plane<2>(qa, lane4) & quad_plane<3>(qa, lane4);
+          p = p1;
+        }
+        // a pair dies at its first node without candidates (gmcr.hpp:56-61)
+        uint32_t some = mask;
+        if (CLS >= 1) some |= quad_xor1(some);
+        if (CLS == 2) some |= quad_xor2(some);
+        alive &= __ballot(some != 0);
+        if (!alive) break;
         m0 = m1;
         m1 = m2;
         m2 = m3;
-        m3 = node_mask();
-        alive = alive && some(m3);
-        if (__ballot(alive) == 0) break;
-        if ((i & 3u) != 3u) {
-          if (i + 1 < k) continue;
-          for (uint32_t x = i & 3u; x < 3; ++x) {
-            m0 = m1;
-            m1 = m2;
-            m2 = m3;
-            m3 = 0;
-          }
+        m3 = mask;
+        if (((flush >> i) & 1u) == 0) continue;
+        // masks go out four nodes at a time, in 16-byte stores (nodes past the last fall in the block's
+        // padding)
+        for (uint32_t x = i; (x & 3u) != 3u; ++x) {
+          m0 = m1;
+          m1 = m2;
+          m2 = m3;
+          m3 = 0;
         }
         const uint32_t i0 = i & ~3u;
+        const bool store = room && __builtin_amdgcn_inverse_ballot_w64(alive);
         if (CLS == 0) {
-          if (alive && room) *reinterpret_cast<uint4*>(a.arena + base + i0 / 2) = make_uint4(m0, m1, m2, m3);
+          if (store) *reinterpret_cast<uint4*>(a.arena + base + i0 / 2) = make_uint4(m0, m1, m2, m3);
         } else if (CLS == 1) {  // the lanes of a molecule swap halves: each stores two nodes' words
           const uint32_t o0 = quad_xor1(h ? m0 : m2), o1 = quad_xor1(h ? m1 : m3);
-          if (alive && room) reinterpret_cast<uint4*>(a.arena + base + i0)[h] = h ? make_uint4(o0, m2, o1, m3) : make_uint4(m0, o0, m1, o1);
-        } else if (alive && room) {
+          if (store) reinterpret_cast<uint4*>(a.arena + base + i0)[h] = h ? make_uint4(o0, m2, o1, m3) : make_uint4(m0, o0, m1, o1);
+        } else if (store) {
           uint32_t* dst = reinterpret_cast<uint32_t*>(a.arena + base + 2 * i0) + h;
           dst[0] = m0;
           dst[4] = m1;
@@ -888,71 +1002,82 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
             dst[12] = m3;
           }
         }
+        if (i + 1 < k) continue;
+        if (lane == 0)
+          group_args().blocks[group * a.Gq + g] = make_uint4(static_cast<uint32_t>(base0), pw, static_cast<uint32_t>(am), static_cast<uint32_t>(am >> 32));
+        break;
       }
-      if (__ballot(alive) && lane == 0)
-        a.blocks[group * a.Gq + g] = make_uint4(static_cast<uint32_t>(base0), pw, static_cast<uint32_t>(am), static_cast<uint32_t>(am >> 32));
-      if (act && !alive) dead |= 1ull << jb;
+      nodes += i + 1;
+      if (__builtin_amdgcn_inverse_ballot_w64(am & ~alive)) {
+        const auto& c = group_args();
+        atomicAnd(&c.surv[static_cast<uint64_t>(mi.m) * c.W + g / kWave], ~(1ull << (g % kWave)));
+      }
     }
-    if (dead && h == 0) atomicAnd(&a.surv[static_cast<uint64_t>(mi.m) * a.W + w], ~dead);
+    st.turn ^= 1u;
+    __syncthreads();  // the list has been read
   }
+  st.sums += lane == 0 ? nodes : (lane == 1 ? live : (lane == 2 ? scans : 0u));
 }
 
 // Pair evaluation: the exact candidates of every pre-tested pair's query nodes (isomorphism.hpp:49
 // and :103-110), keeping the masks of the pairs that survive GMCR.
 //
 // A wavefront takes one query graph and one group, 64 lanes of neighbours in the width-class
-// order, so a requirement's level, label and count are scalars: a near test is one LDS read and
-// three vector operations for 64 x 32 positions.  A lane that walked a pair of its own decoded
-// every token for itself and gathered its token words and planes, about 40 operations a test, and
-// a wavefront waited for its longest pair.  The order groups molecules of one label set and
-// similar size, so a query graph passes the pre-test for none of a group's molecules three times
-// out of four and for half of them otherwise (1 M LogNormal molecules, U[4,32]-node queries).
+// order, so a requirement is the same for 64 x 32 positions: a plane of LDS and an AND.  A lane that
+// walked a pair of its own decoded every token for itself and gathered its token words and planes,
+// about 40 operations a test, and a wavefront waited for its longest pair.  The order groups
+// molecules of one label set and similar size, so a query graph passes the pre-test for none of a
+// group's molecules three times out of four and for half of them otherwise (1 M LogNormal
+// molecules, U[4,32]-node queries).
 //
 // A block of eight wavefronts stages the group's planes and label masks for the labels that occur
-// in it (the first a.slots of them; the rest are read from the database) and shares its query
-// graphs out by index.  Node masks go straight to the pairs' arena blocks, which a wavefront takes
-// from a chunk of its own; pairs that die clear their pre-test bits, one atomic per molecule and
-// 64 query graphs.  80 registers: six wavefronts per SIMD, which its scalar token decode needs to
-// hide (20 waves with 4-wavefront blocks: 8.1 instead of 6.8 ms).  With 64-bit
-// masks for every molecule and an offset per pair, stored 4 KB apart, 174 M writes went to memory
-// instead of 73 M, in 6.7 instead of 5.6 ms.
+// in it (the first a.slots of them; the rest are read from the database), lists the query graphs
+// that have pre-tested pairs, eight words of them at a time, and its wavefronts take them as they
+// come: shared out by index, wavefronts waited a fifth of their time for the longest share.  Counts
+// of 1 to 4 have planes for every label and 5 to 8 for the database's most frequent one, which leaves
+// 0.3% of the requirements to be read from the database (7.5% with 1 to 4 alone).  The tokens of 64
+// quads are decoded at once, a quad per lane, to the four planes' numbers in a word; a quad then
+// takes one lane read, four byte permutations (the LDS addresses), four LDS reads and two ANDs, and
+// its label, end and padding tokens are planes like the others.  With each token a scalar of its own
+// a node took 75 scalar operations and 19 branches, now 45 and 12: one scalar unit serves the
+// CU's 24 wavefronts and bounds the kernel, at 60% issue.
 //
-// Measured, in place of one launch per size class with a lane per pair: 2,000 molecules x 20 query
-// graphs 219 -> 12 us (three serial chains of ~100 us), 100,000 x 100 475 -> 125 us, 1 M x 25
-// 1,242 -> 353 us, 1 M x 1,000 10.7 -> 5.6 ms.
+// Node masks go straight to the pairs' arena blocks, which a wavefront takes from a chunk of its own;
+// pairs that die clear their pre-test bits.  80 registers: six wavefronts per SIMD (20 waves with
+// 4-wavefront blocks: 8.1 instead of 6.8 ms).  With 64-bit masks for every molecule and an offset
+// per pair, stored 4 KB apart, 174 M writes went to memory instead of 73 M.
+//
+// Measured: a lane per pair and a launch per size class, wavefronts by groups with scalar tokens, and
+// this: 2,000 molecules x 20 query graphs 219, 13 and 10 us (three serial chains of ~100 us at
+// first), 100,000 x 100 475, 118 and 73 us, 1 M x 25 1,242, 353 and 294 us, 1 M x 1,000 10.7, 5.6 and
+// 3.2 ms.
 __global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a) {
-  extern __shared__ uint32_t near_lds[];
-  uint32_t* labs = near_lds + static_cast<uint64_t>(a.slots) * a.R * kNearCount * kWave;
-  unsigned long long* next_item = reinterpret_cast<unsigned long long*>(labs + a.slots * kWave);
+  extern __shared__ uint32_t planes_lds[];
+  GroupCounters* ctr = reinterpret_cast<GroupCounters*>(reinterpret_cast<uint4*>(planes_lds + (a.slots + 1) * slot_planes(a.R) * kWave) + kGroupWaves * kWave);
+  if (threadIdx.x == 0) ctr->listed[0] = ctr->taken[0] = 0;  // before the barrier that ends the first staging
   const uint32_t wave = uniform32(threadIdx.x / kWave);
-  const uint32_t g0 = a.order.groups(0), g1 = a.order.groups(1);
-  const uint64_t items = static_cast<uint64_t>(a.order.total()) * a.parts;
+  const uint32_t items = a.order.total() * a.parts;
+  // three quarters of the groups are shared out beforehand: claims meet on one address, where they take
+  // about 10 ns each (1 M molecules x 25 query graphs: 16,000 claims for groups, as many for chunks)
+  const uint32_t fixed = max(gridDim.x, items / 4 * 3 / gridDim.x * gridDim.x);
   GroupState st;
   st.next = (static_cast<uint64_t>(blockIdx.x) * kGroupWaves + wave) * a.chunk;
-  st.end = st.next + a.chunk;
-  st.first_chunks = static_cast<uint64_t>(gridDim.x) * kGroupWaves * a.chunk;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && st.first_chunks > a.arena_cap) atomicOr(&a.counters[3], 1ull);
-  for (uint64_t item = blockIdx.x; item < items;) {
-    const uint32_t part = static_cast<uint32_t>(item & (a.parts - 1));
-    const uint32_t grp = static_cast<uint32_t>(item / a.parts);
-    if (grp < g0) group_item<0>(a, grp, part, wave, near_lds, labs, st);
-    else if (grp < g0 + g1) group_item<1>(a, grp - g0, part, wave, near_lds, labs, st);
-    else group_item<2>(a, grp - g0 - g1, part, wave, near_lds, labs, st);
+  st.left = a.chunk;
+  if (blockIdx.x == 0 && threadIdx.x == 0 && static_cast<uint64_t>(gridDim.x) * kGroupWaves * a.chunk > a.arena_cap) atomicOr(&a.counters[3], 1ull);
+  for (uint32_t item = blockIdx.x; item < items;) {
+    const uint32_t part = item & (a.parts - 1), grp = item / a.parts;
+    const uint32_t g0 = a.order.groups(0), g1 = a.order.groups(1);
+    if (grp < g0) group_item<0>(a, grp, part, wave, planes_lds, st);
+    else if (grp < g0 + g1) group_item<1>(a, grp - g0, part, wave, planes_lds, st);
+    else group_item<2>(a, grp - g0 - g1, part, wave, planes_lds, st);
+    item += gridDim.x;
+    if (item < fixed) continue;
     if (gridDim.x >= items) break;
-    __syncthreads();  // the staged planes have been read
-    if (threadIdx.x == 0) *next_item = gridDim.x + atomicAdd(&a.counters[2], 1ull);
+    if (threadIdx.x == 0) ctr->next_item = fixed + static_cast<uint32_t>(atomicAdd(&a.counters[2], 1ull));  // the staged planes have been read
     __syncthreads();
-    item = uniform64(*next_item);
+    item = uniform32(ctr->next_item);
   }
-  uint32_t live = st.live;
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) live += static_cast<uint32_t>(__shfl_xor(static_cast<int>(live), o));
-  if (lane_id() == 0 && st.scans) {
-    unsigned long long* out = a.stats + (blockIdx.x % kGroupStatSlots) * 16;
-    atomicAdd(&out[0], static_cast<unsigned long long>(st.nodes));
-    atomicAdd(&out[1], static_cast<unsigned long long>(live));
-    atomicAdd(&out[2], static_cast<unsigned long long>(st.scans));
-  }
+  if (lane_id() < 3 && st.sums) atomicAdd(&a.stats[(blockIdx.x % kGroupStatSlots) * 16 + lane_id()], static_cast<unsigned long long>(st.sums));
 }
 
 // Survivors per molecule: the popcount of its row of the survival bitmask.
@@ -1587,13 +1712,14 @@ int shape_run(const sigmo_batch* b, const sigmo_graph* query, int cus, RunShape&
   L.pairs = uint64_t(L.Gq) * L.Gd;
   const uint64_t groups = db->order.total(), ucus = static_cast<uint64_t>(cus);
   // a group's query graphs go to one block, or to more where the groups alone leave CUs idle
-  while (L.group_parts < 64 / sigmo_k::kGroupWaves && groups * L.group_parts < 2 * ucus && sigmo_k::kGroupWaves * L.group_parts < L.Gq)
+  while (L.group_parts < 8 && groups * L.group_parts < 2 * ucus && sigmo_k::kGroupWaves * L.group_parts < L.Gq)
     L.group_parts *= 2;
   const uint64_t items = groups * L.group_parts;
-  // LDS for every label that occurs, within 64 KB; with blocks to spare within 52 KB, so that three
-  // stay resident (a group of neighbours in the width-class order holds 4 to 6 labels)
-  const uint32_t lds = (items > 2 * ucus ? 52u : 64u) * 1024;
-  L.group_slots = std::max<uint32_t>(1, std::min<uint32_t>(db->num_labels, lds / sigmo_k::group_lds_bytes(1, L.R)));
+  // LDS for every label that occurs, within 64 KB (a byte names a plane); with blocks to
+  // spare within 53 KB, so that three stay resident (a group of neighbours in the width-class order
+  // holds 4 to 6 labels)
+  const uint32_t lds = (items > 2 * ucus ? 53u : 64u) * 1024, block = sigmo_k::slot_planes(L.R) * 256;
+  L.group_slots = std::max<uint32_t>(1, std::min<uint32_t>(db->num_labels, (lds - sigmo_k::kGroupListBytes) / block - 1));
   uint64_t per_cu = std::max<uint64_t>(1, std::min<uint64_t>(32 / sigmo_k::kGroupWaves, 160 * 1024 / sigmo_k::group_lds_bytes(L.group_slots, L.R)));
   if (b->tune.filter_blocks_per_cu) per_cu = std::min<uint64_t>(per_cu, b->tune.filter_blocks_per_cu);
   L.group_blocks = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(items, ucus * per_cu)));
@@ -1601,7 +1727,7 @@ int shape_run(const sigmo_batch* b, const sigmo_graph* query, int cus, RunShape&
   // many pairs, more: claims meet on one address
   const uint64_t waves = uint64_t(L.group_blocks) * sigmo_k::kGroupWaves;
   uint64_t chunk = 2048;
-  while (chunk < 16384 && chunk * waves * 64 < L.pairs) chunk *= 2;
+  while (chunk < 32768 && chunk * waves * 4 < L.pairs) chunk *= 2;
   L.group_chunk = static_cast<uint32_t>(chunk);
   L.first_chunks = waves * chunk;
   return SIGMO_OK;
@@ -1647,11 +1773,12 @@ hipError_t launch_filter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
   a.W = L.W;
   a.parts = L.group_parts;
   a.slots = L.group_slots;
+  a.rich = db->cls.l[0];
   a.chunk = L.group_chunk;
   a.minfo = db->minfo;
   a.planes = reinterpret_cast<const uint4*>(db->planes);
   a.labs = db->labs;
-  a.tokens = b->tokens;
+  a.tokens = reinterpret_cast<const uint64_t*>(b->tokens);
   a.qinfo = b->qinfo;
   a.arena = b->arena;
   a.arena_cap = b->cap_arena;

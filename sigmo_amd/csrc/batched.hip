@@ -706,11 +706,8 @@ struct GroupArgs {
   unsigned long long* stats;     // kGroupStatSlots x 16: [0] node evaluations, [1] their live lanes, [2] pre-tested pairs
 };
 
-// LDS: planes of 64 words, at most 256 of them, in blocks of slot_planes: a label slot's positions
-// whose count reaches 1..4 per level, then its own positions; the last block has the counts 5..8 of
-// the database's most frequent label, then every position.  Then the list of the group's live query
-// graphs, of eight query words at a time, and GroupCounters.
-__host__ __device__ constexpr uint32_t slot_planes(uint32_t R) { return 4 * R + 1; }
+// LDS: the planes (slot_planes), then the list of the group's live query graphs, of eight query words
+// at a time, and GroupCounters.
 struct GroupCounters {
   uint32_t next_item;
   uint32_t listed[2], taken[2];  // of this list and the next
@@ -732,14 +729,6 @@ __device__ __forceinline__ uint32_t quad_xor2(uint32_t x) {
 // have consecutive blocks of `words` from `base` on, in the order of their molecules' first lanes.
 __device__ __forceinline__ uint32_t pair_block(uint32_t base, uint32_t words, uint64_t lanes, uint32_t lane0) {
   return base + static_cast<uint32_t>(__popcll(lanes & ((1ull << lane0) - 1))) * words;
-}
-
-// The lane's word of the plane named by byte X of `quad`: the permutation makes plane * 256 + lane * 4,
-// the byte address (dynamic LDS starts at 0: the kernel has no other).
-template <int X>
-__device__ __forceinline__ uint32_t quad_plane(uint32_t quad, uint32_t lane4) {
-  const uint32_t at = __builtin_amdgcn_perm(quad, lane4, 0x0c0c0000u | ((4u + X) << 8));
-  return *reinterpret_cast<const __attribute__((address_space(3))) uint32_t*>(static_cast<uintptr_t>(at));
 }
 
 // The kernel's arguments, read where they are used: kept in registers, those of the rare paths would
@@ -801,17 +790,7 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
     for (uint32_t x = 0; x < 4; ++x) {
       const uint32_t e = e0 + x * kGroupWaves;
       if (e >= staged * R) break;
-      uint32_t t[kNearCount];
-      thermometer(v[x], t);
-#pragma unroll
-      for (uint32_t c = 0; c < kNearCount; ++c) plane(e / R * SP + 4 * (e % R) + c) = t[c];
-      if (label_of(e / R) == rich) {
-        const uint32_t at5 = a.slots * SP + 4 * (e % R);
-        plane(at5) = v[x].w | (v[x].z & (v[x].y | v[x].x));
-        plane(at5 + 1) = v[x].w | (v[x].z & v[x].y);
-        plane(at5 + 2) = v[x].w | (v[x].z & v[x].y & v[x].x);
-        plane(at5 + 3) = v[x].w;
-      }
+      stage_planes(planes_lds, R, e / R, e % R, v[x], a.slots, label_of(e / R) == rich);
     }
   }
   for (uint32_t slot = wave; slot < staged; slot += kGroupWaves)
@@ -952,21 +931,8 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
             }
           }
         }
-        for (; p + 2 <= p1; p += 2) {
-          const uint32_t qa = rl32(dec, p), qb = rl32(dec, p + 1);
-          const uint32_t a0 = quad_plane<0>(qa, lane4), a1 = quad_plane<1>(qa, lane4), a2 = quad_plane<2>(qa, lane4), a3 = quad_plane<3>(qa, lane4);
-          const uint32_t b0 = quad_plane<0>(qb, lane4), b1 = quad_plane<1>(qb, lane4), b2 = quad_plane<2>(qb, lane4), b3 = quad_plane<3>(qb, lane4);
-          mask &= a0 & a1;
-          mask &= a2 & a3;
-          mask &= b0 & b1;
-          mask &= b2 & b3;
-        }
-        if (p < p1) {
-          const uint32_t qa = rl32(dec, p);
-          mask &= quad_plane<0>(qa, lane4) & quad_plane<1>(qa, lane4);
-          mask &= quad_plane<2>(qa, lane4) & quad_plane<3>(qa, lane4);
-          p = p1;
-        }
+        mask = quad_tests(dec, p, p1, lane4, mask);
+        p = p1;
         // a pair dies at its first node without candidates (gmcr.hpp:56-61)
         uint32_t some = mask;
         if (CLS >= 1) some |= quad_xor1(some);

@@ -640,12 +640,19 @@ int graph_fill(sigmo_graph* g, const HostView& h, uint32_t reserve_G = 0, uint64
   g->min_nodes = mn;
   g->host_go.resize(uint64_t(G) + 1);
   for (uint32_t i = 0; i <= G; ++i) g->host_go[i] = h.go[i] - h.node_base;
-  bool present[16] = {false};
+  uint64_t present[16] = {0};
   for (uint64_t v = 0; v < N; ++v)
-    if (h.nl[v] < 16) present[h.nl[v]] = true;
-  g->slots.count = 0;
-  for (int l = 0; l < 16; ++l)
-    if (present[l]) g->slots.label[g->slots.count++] = static_cast<uint8_t>(l);
+    if (h.nl[v] < 16) ++present[h.nl[v]];
+  g->slots.count = g->slots.frequent = 0;
+  uint64_t most = 0;
+  for (int l = 0; l < 16; ++l) {
+    if (!present[l]) continue;
+    if (present[l] > most) {
+      most = present[l];
+      g->slots.frequent = g->slots.count;
+    }
+    g->slots.label[g->slots.count++] = static_cast<uint8_t>(l);
+  }
   hipStream_t s = g->ctx->stream;
   hipError_t e = hipMemcpyAsync(g->go, h.go, (uint64_t(G) + 1) * 4, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(g->ro, h.ro, (N + 1) * 4, hipMemcpyHostToDevice, s);

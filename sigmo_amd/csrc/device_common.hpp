@@ -129,12 +129,16 @@ __device__ __forceinline__ T ge4_bits(T x0, T x1, T x2, T x3, uint32_t c) {
 }
 
 // The pair evaluation and the pipeline's sweep test 32 positions per lane against requirements
-// (label l at level r, count c >= 1) that are scalars.  For c <= 4, nine of ten or more, LDS holds
-// the positions whose count reaches c (thermometer planes, made from the bit planes when they are
-// staged), so a test is one 4-byte read and one AND; larger counts compare the bit planes.
+// (label l at level r, count c >= 1) that are the same for the wavefront.  LDS holds planes of 64
+// words, a word per lane, at most 256 of them, in blocks of slot_planes: a label's positions whose
+// count reaches 1..4 at each level (thermometer planes, made from the bit planes when they are
+// staged), then the positions of that label; the block after the last label's has the counts 5..8 of
+// one frequent label, then every position.  A test is then a read of LDS and an AND; other counts
+// compare bit planes from memory.  Tokens are the planes' numbers, four to a word (a quad).
 constexpr uint32_t kNearCount = 4;
+__host__ __device__ constexpr uint32_t slot_planes(uint32_t R) { return 4 * R + 1; }
 
-// The thermometer planes of counts 1..4 from a label's four bit planes.
+// The positions whose count reaches 1..4, from a label's four bit planes, and 5..8.
 __device__ __forceinline__ void thermometer(const uint4& x, uint32_t t[kNearCount]) {
   const uint32_t high = x.z | x.w;
   t[0] = x.x | x.y | high;
@@ -142,32 +146,48 @@ __device__ __forceinline__ void thermometer(const uint4& x, uint32_t t[kNearCoun
   t[2] = (x.x & x.y) | high;
   t[3] = high;
 }
-// Byte offset in LDS of the plane of count c for entry e = label slot * R + level.
-__device__ __forceinline__ uint32_t near_offset(uint32_t e, uint32_t c) { return (e * kNearCount + c - 1) * (kWave * 4); }
-// A wavefront stages entry e.
-__device__ __forceinline__ void stage_near(uint32_t* lds, uint32_t e, const uint4& x) {
+__device__ __forceinline__ void thermometer_high(const uint4& x, uint32_t t[kNearCount]) {
+  t[0] = x.w | (x.z & (x.y | x.x));
+  t[1] = x.w | (x.z & x.y);
+  t[2] = x.w | (x.z & x.y & x.x);
+  t[3] = x.w;
+}
+// Stages the planes of a label's slot at level r from its bit planes, and those of counts 5..8 when it
+// is the frequent one, after `slots` slots.
+__device__ __forceinline__ void stage_planes(uint32_t* lds, uint32_t R, uint32_t slot, uint32_t r, const uint4& x, uint32_t slots, bool frequent) {
   uint32_t t[kNearCount];
   thermometer(x, t);
 #pragma unroll
-  for (uint32_t c = 0; c < kNearCount; ++c) lds[(e * kNearCount + c) * kWave + lane_id()] = t[c];
+  for (uint32_t c = 0; c < kNearCount; ++c) lds[(slot * slot_planes(R) + 4 * r + c) * kWave + lane_id()] = t[c];
+  if (!frequent) return;
+  thermometer_high(x, t);
+#pragma unroll
+  for (uint32_t c = 0; c < kNearCount; ++c) lds[(slots * slot_planes(R) + 4 * r + c) * kWave + lane_id()] = t[c];
 }
-__device__ __forceinline__ uint32_t near_plane(const uint32_t* lds, uint32_t off) {
-  return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(lds) + (off | static_cast<uint32_t>(lane_id() * 4)));
+
+// The lane's word of the plane named by byte X of `quad`: the permutation makes plane * 256 + lane * 4,
+// the byte address (dynamic LDS starts at 0 in a kernel that has no other).
+template <int X>
+__device__ __forceinline__ uint32_t quad_plane(uint32_t quad, uint32_t lane4) {
+  const uint32_t at = __builtin_amdgcn_perm(quad, lane4, 0x0c0c0000u | ((4u + X) << 8));
+  return *reinterpret_cast<const __attribute__((address_space(3))) uint32_t*>(static_cast<uintptr_t>(at));
 }
-// ANDs the near requirements of lanes [t, e) of `dec` (their byte offsets) into mask.
-__device__ __forceinline__ uint32_t near_tests(const uint32_t* lds, uint32_t dec, uint32_t t, uint32_t e, uint32_t mask) {
-  for (; t + 4 <= e; t += 4) {
-    const uint32_t v0 = near_plane(lds, rl32(dec, t)), v1 = near_plane(lds, rl32(dec, t + 1));
-    const uint32_t v2 = near_plane(lds, rl32(dec, t + 2)), v3 = near_plane(lds, rl32(dec, t + 3));
-    mask &= v0 & v1;
-    mask &= v2 & v3;
+// ANDs the planes of the quads in lanes [p, p1) of `dec` into mask.
+__device__ __forceinline__ uint32_t quad_tests(uint32_t dec, uint32_t p, uint32_t p1, uint32_t lane4, uint32_t mask) {
+  for (; p + 2 <= p1; p += 2) {
+    const uint32_t qa = rl32(dec, p), qb = rl32(dec, p + 1);
+    const uint32_t a0 = quad_plane<0>(qa, lane4), a1 = quad_plane<1>(qa, lane4), a2 = quad_plane<2>(qa, lane4), a3 = quad_plane<3>(qa, lane4);
+    const uint32_t b0 = quad_plane<0>(qb, lane4), b1 = quad_plane<1>(qb, lane4), b2 = quad_plane<2>(qb, lane4), b3 = quad_plane<3>(qb, lane4);
+    mask &= a0 & a1;
+    mask &= a2 & a3;
+    mask &= b0 & b1;
+    mask &= b2 & b3;
   }
-  if (t + 2 <= e) {
-    const uint32_t v0 = near_plane(lds, rl32(dec, t)), v1 = near_plane(lds, rl32(dec, t + 1));
-    mask &= v0 & v1;
-    t += 2;
+  if (p < p1) {
+    const uint32_t qa = rl32(dec, p);
+    mask &= quad_plane<0>(qa, lane4) & quad_plane<1>(qa, lane4);
+    mask &= quad_plane<2>(qa, lane4) & quad_plane<3>(qa, lane4);
   }
-  if (t < e) mask &= near_plane(lds, rl32(dec, t));
   return mask;
 }
 

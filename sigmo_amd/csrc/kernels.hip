@@ -653,7 +653,10 @@ __global__ __launch_bounds__(kBitsBlock) void k_filter_refine(const uint8_t* __r
 // level read the bitset and wrote most of it again.
 
 constexpr uint32_t kStripNodes = 2048;    // data nodes of one strip: 64 lanes of 32
-constexpr uint32_t kLevelTokens = 32;     // words per query node: up to 31 requirements, then count | label << 8
+constexpr uint32_t kLevelQuads = 8;  // words of a query node's planes: its label and up to 31 requirements
+// words per query node: its quads, their number | far tokens << 8, and the far tokens
+constexpr uint32_t kLevelTokens = kLevelQuads + 1 + 32;
+constexpr uint32_t kFarLabel = 1u << 31;
 constexpr uint32_t kLevelWaves = 16;      // wavefronts per block of the sweep
 
 // Data signatures of levels 1..R (signature.hpp:336-390 with view sizes 1, 2, ..., R from empty
@@ -710,11 +713,11 @@ __global__ __launch_bounds__(kSigBlock) void k_sig_levels(GraphDev g, uint32_t R
   }
 }
 
-// Query signatures of levels 1..R as requirement tokens, a wavefront per query graph (<= 32 nodes)
-// and a lane per node: for each nonzero count of label slots.label[u] at level r+1 (at most 31: each
-// needs a node of its own) the LDS offset of its plane when it is near (near_offset), else
-// (u*R + r) << 8 | count; near ones first, as long as their label is one of the first `staged`.
-// tok[node*32 + 31] = near tokens | all tokens << 8 | node label << 16.
+// Query signatures of levels 1..R as planes of the sweep's LDS (slot_planes), a wavefront per query
+// graph (<= 32 nodes) and a lane per node: its label's plane, then one for each nonzero count of label
+// slots.label[u] at level r+1 (at most 31: each needs a node of its own).  Without a plane are a
+// label >= 16, its far token kFarLabel | label, and counts over 4 (over 8 of the frequent label) or of
+// a slot past the first `staged`, (u*R + r) << 8 | count.
 __global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, LabelSlots slots, uint32_t staged, uint32_t* __restrict__ tok) {
   __shared__ uint64_t fold_all[4][kWave];
   const uint32_t lane = static_cast<uint32_t>(lane_id());
@@ -726,8 +729,15 @@ __global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, La
   wave_sync();
   if (lane >= k) return;
   uint32_t* out = tok + (static_cast<uint64_t>(s) + lane) * kLevelTokens;
+  uint8_t* planes = reinterpret_cast<uint8_t*>(out);
+  uint32_t* far = out + kLevelQuads + 1;
+  const uint32_t SP = slot_planes(R), every = staged * SP + 4 * R, label = q.nl[static_cast<uint64_t>(s) + lane];
+  uint32_t near = 1, fars = 0, own = every;
+  for (uint32_t u = 0; u < staged; ++u)
+    if (slots.label[u] == label) own = u * SP + 4 * R;
+  planes[0] = static_cast<uint8_t>(own);
+  if (own == every && label != 255u) far[fars++] = kFarLabel | label;
   uint64_t ball = 1ull << lane, frontier = ball;
-  uint32_t near = 0, far = kLevelTokens - 1;  // far tokens from the back, moved up at the end
   for (uint32_t r = 0; r < R && frontier; ++r) {
     uint64_t next = 0;
     for (; frontier; frontier &= frontier - 1) next |= fold[__builtin_ctzll(frontier)];
@@ -737,75 +747,85 @@ __global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, La
     for (uint32_t u = 0; u < static_cast<uint32_t>(slots.count) && next; ++u) {
       uint32_t c = static_cast<uint32_t>(__popcll(next & q.lmask[static_cast<uint64_t>(g) * 16 + slots.label[u]]));
       c = c < 15 ? c : 15;
-      if (!c || near >= far) continue;
-      if (c <= kNearCount && u < staged) out[near++] = near_offset(u * R + r, c);
-      else out[--far] = ((u * R + r) << 8) | c;
+      if (!c || near + fars >= kLevelTokens - kLevelQuads - 1) continue;  // never more: a requirement per other node
+      const bool frequent = static_cast<int>(u) == slots.frequent;
+      if (u < staged && c <= kNearCount) planes[near++] = static_cast<uint8_t>(u * SP + 4 * r + c - 1);
+      else if (u < staged && frequent && c <= 8) planes[near++] = static_cast<uint8_t>(staged * SP + 4 * r + c - 5);
+      else far[fars++] = ((u * R + r) << 8) | c;
     }
   }
-  uint32_t all = near;
-  for (uint32_t i = far; i < kLevelTokens - 1; ++i) out[all++] = out[i];
-  out[kLevelTokens - 1] = near | (all << 8) | (static_cast<uint32_t>(q.nl[static_cast<uint64_t>(s) + lane]) << 16);
+  const uint32_t quads = (near + 3) / 4;
+  for (; near < 4 * quads; ++near) planes[near] = static_cast<uint8_t>(every);
+  out[kLevelQuads] = quads | (fars << 8);
 }
 
 // filterCandidates<Query> (isomorphism.hpp:22-62) and every refineCandidates<Query> pass (:64-127)
 // as one sweep.  A block stages a strip's planes (of the first `staged` labels of slots) and its
-// wavefronts take the query nodes in turn: a lane holds 32 data nodes and the query node's tokens
-// are scalars, so a near requirement is one LDS read and three vector operations for 2,048 nodes,
-// and each word is written once.  Bound by issue (about a third each vector, scalar and LDS) and
-// the words written.  In place of the fused filter and R - 1 refine passes: 100,000 molecules x
-// 100 queries 823 -> 229 us, 150,000 LogNormal x 300 6.07 -> 1.68 ms (2.6 GB of words, 1.6 TB/s);
-// with four bit planes per entry in LDS instead of the near planes 276 us and 2.10 ms.
+// wavefronts take the query nodes in turn: a lane holds 32 data nodes and the query node's label and
+// requirements are planes of LDS, each a read and an AND for 2,048 nodes, and each word is written
+// once.  In place of the fused filter and R - 1 refine passes: 100,000 molecules x 100 queries 823
+// us, 150,000 LogNormal x 300 6.07 ms; with a scalar per requirement and label compares, bound by
+// issue, 229 us and 1.68 ms; this takes 167 us and 1.24 ms (2.6 GB of words, 2.1 TB/s).
 __global__ __launch_bounds__(kLevelWaves * 64, 8) void k_filter_levels(const uint32_t* __restrict__ tok, uint64_t Q,
                                                                        const uint64_t* __restrict__ lplanes, const uint4* __restrict__ lvl,
-                                                                       uint64_t D, uint32_t R, uint32_t U, uint32_t staged,
+                                                                       uint64_t D, uint32_t R, LabelSlots slots, uint32_t U, uint32_t staged,
                                                                        uint64_t* __restrict__ bits, uint32_t rpb, uint32_t chunks) {
-  extern __shared__ uint32_t near_lds[];
+  extern __shared__ uint32_t planes_lds[];
   const uint64_t W32 = (D + 63) / 64 * 2;  // a row's 32-node words
   const uint64_t strips = (W32 + kWave - 1) / kWave;
   uint64_t strip, chunk;
   if (!xcd_tile(blockIdx.x, strips, chunks, strip, chunk)) return;  // block-uniform
-  const uint32_t lane = static_cast<uint32_t>(lane_id());
+  const uint32_t lane = static_cast<uint32_t>(lane_id()), lane4 = lane * 4;
   const uint32_t wave = uniform32(threadIdx.x / kWave);
   const uint64_t w = strip * kWave + lane;
   const bool in = w < W32;
   const uint4* src = lvl + strip * R * U * kWave;
+  const uint32_t SP = slot_planes(R);
+  uint32_t L[8];
+#pragma unroll
+  for (int b = 0; b < 8; ++b) L[b] = in ? reinterpret_cast<const uint32_t*>(lplanes)[((w >> 1) * 8 + b) * 2 + (w & 1)] : 0u;
+  const uint64_t n0 = w * 32;
+  const uint32_t valid = n0 + 32 <= D ? ~0u : (n0 < D ? (1u << (D - n0)) - 1u : 0u);
+  auto labelled = [&](uint32_t label) -> uint32_t {  // nodes of a label
+    uint32_t m = valid;
+#pragma unroll
+    for (uint32_t b = 0; b < 8; ++b) m = and_xor(m, L[b], bit_mask(~label, b));
+    return m;
+  };
   for (uint32_t e0 = wave; e0 < staged * R; e0 += 4 * kLevelWaves) {
     uint4 v[4];
 #pragma unroll
     for (uint32_t x = 0; x < 4; ++x) {
-      const uint32_t e = e0 + x * kLevelWaves;  // LDS order: label slot, then level
+      const uint32_t e = e0 + x * kLevelWaves;
       v[x] = make_uint4(0, 0, 0, 0);
       if (e < staged * R) v[x] = src[((e % R) * U + e / R) * kWave + lane];
     }
 #pragma unroll
     for (uint32_t x = 0; x < 4; ++x) {
       const uint32_t e = e0 + x * kLevelWaves;
-      if (e < staged * R) stage_near(near_lds, e, v[x]);
+      if (e < staged * R) stage_planes(planes_lds, R, e / R, e % R, v[x], staged, e / R == static_cast<uint32_t>(slots.frequent));
     }
   }
-  uint32_t L[8];
-#pragma unroll
-  for (int b = 0; b < 8; ++b) L[b] = in ? reinterpret_cast<const uint32_t*>(lplanes)[((w >> 1) * 8 + b) * 2 + (w & 1)] : 0u;
-  const uint64_t n0 = w * 32;
-  const uint32_t valid = n0 + 32 <= D ? ~0u : (n0 < D ? (1u << (D - n0)) - 1u : 0u);
+  if (wave < staged) planes_lds[(wave * SP + 4 * R) * kWave + lane] = labelled(slots.label[wave]);  // staged <= 16
+  if (wave == 0) planes_lds[(staged * SP + 4 * R) * kWave + lane] = valid;
   __syncthreads();
   const uint64_t q0 = chunk * rpb, q1 = q0 + rpb < Q ? q0 + rpb : Q;
   uint64_t q = q0 + wave;
-  uint32_t next = q < q1 ? tok[q * kLevelTokens + (lane & 31u)] : 0u;
+  const uint32_t at = min(lane, kLevelTokens - 1);
+  uint32_t next = q < q1 ? tok[q * kLevelTokens + at] : 0u;
   for (; q < q1; q += kLevelWaves) {  // wave-uniform
     const uint32_t dec = next;
-    if (q + kLevelWaves < q1) next = tok[(q + kLevelWaves) * kLevelTokens + (lane & 31u)];
-    const uint32_t meta = rl32(dec, kLevelTokens - 1), near = meta & 0xFFu, all = (meta >> 8) & 0xFFu, ql = meta >> 16;
-    uint32_t mask = valid;
-    if (ql != 255u) {
-#pragma unroll
-      for (uint32_t b = 0; b < 8; ++b) mask = and_xor(mask, L[b], bit_mask(~ql, b));
-    }
-    mask = near_tests(near_lds, dec, 0, near, mask);
-    for (uint32_t t = near; t < all; ++t) {
+    if (q + kLevelWaves < q1) next = tok[(q + kLevelWaves) * kLevelTokens + at];
+    const uint32_t meta = rl32(dec, kLevelQuads), fars = meta >> 8;
+    uint32_t mask = quad_tests(dec, 0, meta & 0xFFu, lane4, ~0u);
+    for (uint32_t t = kLevelQuads + 1; t < kLevelQuads + 1 + fars; ++t) {
       const uint32_t tk = rl32(dec, t), e = tk >> 8;  // e = u*R + r
-      const uint4 x = src[((e % R) * U + e / R) * kWave + lane];
-      mask &= ge4_bits<uint32_t>(x.x, x.y, x.z, x.w, tk & 15u);
+      if (tk & kFarLabel) {
+        mask &= labelled(tk & 0xFFu);
+      } else {
+        const uint4 x = src[((e % R) * U + e / R) * kWave + lane];
+        mask &= ge4_bits<uint32_t>(x.x, x.y, x.z, x.w, tk & 15u);
+      }
     }
     if (in) reinterpret_cast<uint32_t*>(bits)[q * W32 + w] = mask;
   }
@@ -1194,7 +1214,10 @@ hipError_t sig_levels(hipStream_t s, const GraphDev& g, uint32_t R, const LabelS
 }
 
 // Labels whose planes the sweep's LDS holds: 52 KB, so that 32 wavefronts stay resident per CU.
-static uint32_t staged_labels(const LabelSlots& slots, uint32_t R) { return std::min<uint32_t>(static_cast<uint32_t>(slots.count), 52u / R); }
+// labels whose planes a byte can name, the frequent one's counts 5..8 included
+static uint32_t staged_labels(const LabelSlots& slots, uint32_t R) {
+  return std::min<uint32_t>(static_cast<uint32_t>(slots.count), 256u / slot_planes(R) - 1);
+}
 
 hipError_t query_levels(hipStream_t s, const GraphDev& q, uint32_t R, const LabelSlots& slots, uint32_t* tok) {
   if (!q.G) return hipSuccess;
@@ -1213,8 +1236,8 @@ hipError_t filter_levels(hipStream_t s, const uint32_t* tok, uint64_t Q, const u
   const uint64_t chunks0 = std::max<uint64_t>(1, std::min<uint64_t>((Q + 2 * kLevelWaves - 1) / (2 * kLevelWaves), (target + strips - 1) / strips));
   const uint32_t rpb = static_cast<uint32_t>((Q + chunks0 - 1) / chunks0), chunks = static_cast<uint32_t>((Q + rpb - 1) / rpb);
   if (xcd_grid(strips, chunks) > 0x7fffffffull) return hipErrorInvalidValue;
-  k_filter_levels<<<static_cast<unsigned>(xcd_grid(strips, chunks)), kLevelWaves * 64, staged * R * 1024, s>>>(
-      tok, Q, lplanes, static_cast<const uint4*>(lvl), D, R, U, staged, bits, rpb, chunks);
+  k_filter_levels<<<static_cast<unsigned>(xcd_grid(strips, chunks)), kLevelWaves * 64, (staged + 1) * slot_planes(R) * 256, s>>>(
+      tok, Q, lplanes, static_cast<const uint4*>(lvl), D, R, slots, U, staged, bits, rpb, chunks);
   return hipGetLastError();
 }
 

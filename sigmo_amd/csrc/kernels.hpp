@@ -48,6 +48,7 @@ struct AMGraphDev {
 struct LabelSlots {
   uint8_t label[16];
   int count;
+  int frequent;  // the slot of the label that most nodes have
 };
 
 hipError_t fill_u64(hipStream_t s, uint64_t* p, uint64_t n, uint64_t v);

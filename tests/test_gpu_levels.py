@@ -1,5 +1,5 @@
 """The pipeline's one-sweep filter and both forms' requirement tests at their edges: counts around the
-largest that LDS holds a plane of (4) and the saturated 15, more labels than LDS holds, strips of
+largest that LDS holds a plane of (4, and 8 for the most frequent label) and the saturated 15, more labels than LDS holds, strips of
 2,048 data nodes, and level counts with and without the sweep; against the CPU oracle.  All results
 are whole numbers: equality."""
 import numpy as np
@@ -41,6 +41,8 @@ def test_counts_around_the_near_planes_and_saturation(ctx, R):
     counts = (1, 2, 3, 4, 5, 6, 8, 9, 14, 15, 16, 20, 30)
     qs = [_star(c) for c in counts if c < 32] + [_star(c, tail=2) for c in counts if c < 29]
     ms = [_star(c, tail=t) for c in counts for t in (0, 1, 3)] + [_star(c, tail=40) for c in (3, 5, 16, 60)]
+    qs += [_star(c, leaf=6) for c in (4, 5, 8, 9)]  # a label with planes up to 4 only
+    ms += [_star(c, leaf=6) for c in (4, 5, 7, 8, 9, 20)]
     _check(ctx, qs, ms, R)
 
 

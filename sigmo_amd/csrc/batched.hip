@@ -1793,21 +1793,15 @@ hipError_t launch_scatter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Lane join over P pairs (molecules of <= 64 nodes; the others are listed in wide_pairs): for many
-// pairs a shallow first pass and a second over the pairs of deeper queries (deep_pairs).
+// Lane join over P pairs: for many pairs a shallow first pass and a second over the pairs of deeper
+// queries (deep_pairs); pairs of molecules of > 64 nodes are listed (wide_pairs) for the last pass.
 hipError_t launch_join(sigmo_batch* b, const RunShape& L, hipStream_t s, unsigned long long* stats, uint64_t P, int find_first,
                        const unsigned long long* P_dev = nullptr) {
   if (!P) return hipSuccess;
   const uint32_t quarters = b->tune.join_blocks_per_cu ? std::min<uint32_t>(b->tune.join_blocks_per_cu, 4) : 4;
-  return sigmo_k::launch_join_lanes(s, L.qd, L.dd, sigmo_k::ArenaMasks{b->arena, b->mask_off, b->counters + 3}, b->indices, b->pair_graph, P,
-                                    find_first, b->counts, stats, b->wide_pairs, L.cus, P_dev, b->deep_pairs, quarters, b->tune.join_chunk);
-}
-
-// Lane join over the nw listed pairs of 65..128-node molecules (two-word positions).
-hipError_t launch_join_wide(sigmo_batch* b, const RunShape& L, hipStream_t s, unsigned long long* stats, uint64_t nw, int find_first,
-                            const unsigned long long* nw_dev = nullptr) {
-  return sigmo_k::launch_join_wide(s, L.qd, L.dd, sigmo_k::ArenaMasks{b->arena, b->mask_off, b->counters + 3}, b->indices, b->pair_graph,
-                                   b->wide_pairs, nw, find_first, b->counts, stats, L.cus, nw_dev);
+  return sigmo_k::launch_join_lanes(s, L.qd, L.dd, sigmo_k::ArenaMasks{b->arena, b->mask_off, b->counters + 3}, b->offsets, b->indices, b->pair_graph,
+                                    P, find_first, b->counts, stats, b->db->num_wide ? b->wide_pairs : nullptr, L.cus, P_dev, b->deep_pairs, quarters,
+                                    b->tune.join_chunk);
 }
 
 // Buffers of a run that do not depend on its results.
@@ -1953,16 +1947,10 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
   BATCH_TRY(b->grow(&b->deep_pairs, b->cap_deep, P, true));
   BATCH_HIP_TRY(launch_scatter(b, L, s));
   BATCH_TRY(ctx_timed(b->ctx, 0, 0, 0.0, false, &tok));
-  // join: lane per pair; pairs of molecules with > 64 nodes are listed for the two-word kernel
+  // join: lane per pair
   BATCH_TRY(ctx_timed(b->ctx, SIGMO_PHASE_JOIN, SIGMO_KERNEL_JOIN, 0.0, true, &tok));
   BATCH_HIP_TRY(sigmo_k::fill_u64(s, reinterpret_cast<uint64_t*>(stats), sigmo_k::kJoinStatWords, 0));
   BATCH_HIP_TRY(launch_join(b, L, s, stats, P, find_first));
-  if (P && db->num_wide) {
-    unsigned long long nw = 0;
-    BATCH_HIP_TRY(hipMemcpyAsync(&nw, stats + 5, sizeof(nw), hipMemcpyDeviceToHost, s));
-    BATCH_HIP_TRY(hipStreamSynchronize(s));
-    BATCH_HIP_TRY(launch_join_wide(b, L, s, stats, nw, find_first));
-  }
   BATCH_TRY(ctx_timed(b->ctx, 0, 0, 0.0, false, &tok));
   BATCH_HIP_TRY(hipMemcpyAsync(stats_host, stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   BATCH_HIP_TRY(hipStreamSynchronize(s));
@@ -2067,7 +2055,6 @@ int sigmo_batch_capture(sigmo_batch* b, const sigmo_graph* query, int find_first
   // the joins read this replay's pair counts on the device (bounded by the captured sizes), so a
   // replay on changed data reads only entries the replay itself wrote
   if (e == hipSuccess) e = launch_join(b, L, s, stats, b->P, find_first, reinterpret_cast<const unsigned long long*>(b->total));
-  if (e == hipSuccess && db->num_wide) e = launch_join_wide(b, L, s, stats, nw, find_first, stats + 5);
   if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host, b->counters, kCounterWords * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host + kCounterWords, b->total, sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipMemcpyAsync(b->graph_host + kCounterWords + 1, stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);

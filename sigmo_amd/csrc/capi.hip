@@ -640,15 +640,17 @@ int graph_fill(sigmo_graph* g, const HostView& h, uint32_t reserve_G = 0, uint64
   g->min_nodes = mn;
   g->host_go.resize(uint64_t(G) + 1);
   for (uint32_t i = 0; i <= G; ++i) g->host_go[i] = h.go[i] - h.node_base;
-  uint64_t present[16] = {0};
+  bool present[16] = {false};
   for (uint64_t v = 0; v < N; ++v)
-    if (h.nl[v] < 16) ++present[h.nl[v]];
+    if (h.nl[v] < 16) present[h.nl[v]] = true;
+  uint32_t seen[256] = {0};  // which label is frequent, as far as the first nodes tell
+  for (uint64_t v = 0; v < std::min<uint64_t>(N, 4096); ++v) ++seen[h.nl[v]];
   g->slots.count = g->slots.frequent = 0;
-  uint64_t most = 0;
+  uint32_t most = 0;
   for (int l = 0; l < 16; ++l) {
     if (!present[l]) continue;
-    if (present[l] > most) {
-      most = present[l];
+    if (seen[l] > most) {
+      most = seen[l];
       g->slots.frequent = g->slots.count;
     }
     g->slots.label[g->slots.count++] = static_cast<uint8_t>(l);
@@ -1264,25 +1266,14 @@ int sigmo_join(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_graph* data
   hipStream_t s = ctx->stream;
   PhaseScope ps(ctx, SIGMO_PHASE_JOIN, SIGMO_KERNEL_JOIN, 0.0);
   SIGMO_HIP_TRY(sigmo_k::fill_u64(s, reinterpret_cast<uint64_t*>(ctx->stats), sigmo_k::kJoinStatWords, 0));
-  SIGMO_TRY(grow_slack(&mm->wide_pairs, mm->cap_wide, m->P));
+  const bool wide = data->max_nodes > 64;
+  if (wide) SIGMO_TRY(grow_slack(&mm->wide_pairs, mm->cap_wide, m->P));
   SIGMO_TRY(grow_slack(&mm->deep_pairs, mm->cap_deep, m->P));
   // a deferred GMCR: P bounds the grid and the kernel reads the exact count on the device
-  SIGMO_HIP_TRY(sigmo_k::join_lanes(s, query->dev(), data->dev(), c->bits, c->W64, m->indices, m->pair_graph, m->P, find_first,
-                                    mm->pair_counts, ctx->stats, mm->wide_pairs, ctx->num_cus,
+  SIGMO_HIP_TRY(sigmo_k::join_lanes(s, query->dev(), data->dev(), c->bits, c->W64, m->offsets, m->indices, m->pair_graph, m->P, find_first,
+                                    mm->pair_counts, ctx->stats, wide ? mm->wide_pairs : nullptr, ctx->num_cus,
                                     m->deferred || ctx->capturing ? reinterpret_cast<const unsigned long long*>(m->total) : nullptr,
                                     mm->deep_pairs));
-  if (data->max_nodes > 64 && m->P) {  // pairs of molecules with > 64 nodes: the two-word lane join
-    unsigned long long nw = mm->last_wide;  // a graph being recorded keeps the previous run's count
-    if (!ctx->capturing) {
-      SIGMO_HIP_TRY(hipMemcpyAsync(&nw, ctx->stats + 5, sizeof(nw), hipMemcpyDeviceToHost, s));
-      SIGMO_HIP_TRY(hipStreamSynchronize(s));
-      mm->last_wide = nw;
-    }
-    if (nw)
-      SIGMO_HIP_TRY(sigmo_k::join_lanes_wide(s, query->dev(), data->dev(), c->bits, c->W64, m->indices, m->pair_graph, mm->wide_pairs, nw,
-                                             find_first, mm->pair_counts, ctx->stats, ctx->num_cus,
-                                             ctx->capturing ? ctx->stats + 5 : nullptr));
-  }
   SIGMO_TRY(ps.close());
   SIGMO_HIP_TRY(hipMemcpyAsync(ctx->stats_host, ctx->stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   if (ctx->capturing) return SIGMO_OK;  // the replay reads the pinned mirror after the graph
@@ -1290,6 +1281,7 @@ int sigmo_join(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_graph* data
   if (per_pair_counts && m->P)
     SIGMO_HIP_TRY(hipMemcpyAsync(per_pair_counts, mm->pair_counts, m->P * 4, hipMemcpyDeviceToHost, s));
   SIGMO_HIP_TRY(hipStreamSynchronize(s));
+  mm->last_wide = wide ? ctx->stats_host[5] : 0;
   if (ctx->stats_host[3]) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "a per-pair match count exceeded int32");
   if (num_matches) *num_matches += ctx->stats_host[0];
   return SIGMO_OK;
@@ -1342,16 +1334,8 @@ int sigmo_join_noalloc(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_gra
   auto* wide = reinterpret_cast<uint32_t*>(counts + kScratchPairs);
   // the scratch keeps the previous call's contents: the counters (work cursors included) start at 0
   SIGMO_HIP_TRY(sigmo_k::fill_u64(s, reinterpret_cast<uint64_t*>(stats), kScratchStatWords, 0));
-  SIGMO_HIP_TRY(sigmo_k::join_lanes(s, query->dev(), data->dev(), c->bits, c->W64, m->indices, m->pair_graph, m->P, find_first, counts, stats,
-                                    wide, ctx->num_cus));
-  if (data->max_nodes > 64 && m->P) {  // pairs of molecules with > 64 nodes: the two-word lane join
-    SIGMO_HIP_TRY(hipMemcpyAsync(ctx->stats_host, stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    SIGMO_HIP_TRY(hipStreamSynchronize(s));
-    const uint64_t nw = ctx->stats_host[5];
-    if (nw)
-      SIGMO_HIP_TRY(sigmo_k::join_lanes_wide(s, query->dev(), data->dev(), c->bits, c->W64, m->indices, m->pair_graph, wide, nw,
-                                             find_first, counts, stats, ctx->num_cus));
-  }
+  SIGMO_HIP_TRY(sigmo_k::join_lanes(s, query->dev(), data->dev(), c->bits, c->W64, m->offsets, m->indices, m->pair_graph, m->P, find_first, counts,
+                                    stats, data->max_nodes > 64 ? wide : nullptr, ctx->num_cus));
   SIGMO_HIP_TRY(hipMemcpyAsync(ctx->stats_host, stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   if (per_pair_counts && m->P) SIGMO_HIP_TRY(hipMemcpyAsync(per_pair_counts, counts, m->P * 4, hipMemcpyDeviceToHost, s));
   SIGMO_HIP_TRY(hipStreamSynchronize(s));

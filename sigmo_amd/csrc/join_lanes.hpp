@@ -120,6 +120,7 @@ struct BitsetMasks {
 // them all in one pass that holds 12 levels and reaches deeper ones through global memory.
 constexpr int kJoinShallow = 8;
 constexpr int kJoinLevels = 12;
+constexpr int kJoinWideLevels = 7;  // two words per position: LDS as for kJoinLevels of one
 constexpr uint64_t kJoinTwoPassPairs = 1ull << 24;  // pair counts from which the lane join runs in two passes
 constexpr uint32_t kJoinDeepChunk = 128;            // pairs a wavefront claims at a time of the deep queries' list
 constexpr uint32_t kJoinRefill = 24;                // idle lanes that make a wavefront hand out new pairs
@@ -139,12 +140,19 @@ struct JoinLds {
   uint64_t q_adj[kWave];
   uint32_t q_pair[kWave], q_start[kWave], q_qoff[kWave], q_base[kWave];
   uint16_t q_nk[kWave];
-  uint32_t listed[(WIDE ? 0 : 1) + (DEEP ? 0 : 1) ? (WIDE ? 0 : 1) + (DEEP ? 0 : 1) : 1][2 * kWave];  // pairs for other passes: deep, then wide
+  uint32_t listed[DEEP ? 1 : 2 * kWave];  // pairs for the deep pass
 };
-template <int KC, bool DEEP, bool WIDE>
-constexpr uint32_t join_waves_per_cu() {  // wavefronts the 160 KB of LDS hold
-  return static_cast<uint32_t>(160 * 1024 / ((sizeof(JoinLds<KC, DEEP, WIDE>) + 511) / 512 * 512));
+constexpr uint32_t join_waves_per_cu(size_t lds) {  // wavefronts the 160 KB of LDS hold
+  return static_cast<uint32_t>(160 * 1024 / ((lds + 511) / 512 * 512));
 }
+constexpr size_t kJoinAllLds = sizeof(JoinLds<kJoinLevels, true, false>) > sizeof(JoinLds<kJoinWideLevels, true, true>)
+                                   ? sizeof(JoinLds<kJoinLevels, true, false>)
+                                   : sizeof(JoinLds<kJoinWideLevels, true, true>);
+
+// A lane's statistics.
+struct JoinTotals {
+  uint64_t sum = 0, matched = 0, steps = 0, overflow = 0, wave_iters = 0;
+};
 
 // Positions above c of a 64-position word.
 __device__ __forceinline__ uint64_t bits_above(uint32_t c) { return (~0ull << c) << 1; }
@@ -183,34 +191,27 @@ __device__ __forceinline__ uint32_t bit_spread(uint32_t q, uint32_t t) {
 // therefore all issued together, when kJoinRefill lanes are idle, and a wavefront stalls on them
 // once per that many pairs (16, 24 and 32 measure the same, 40 is 4% slower).
 //
-// Bound by VALU issue (about two thirds of it on 68 M pairs) at 12 wavefronts per CU by LDS.  One
+// Bound by VALU issue (about two thirds of it on 68 M pairs) at 11 wavefronts per CU by LDS.  One
 // DFS step per iteration, all rows tested per lane and an atomic per listed batch took, for 1 M
 // LogNormal molecules x 1,000 queries, 10.8 + 1.4 ms (molecules of <= 64 nodes) and 2.5 + 1.6 ms
-// (wider ones); this takes 6.0 + 1.9 and 1.65 ms, and 33,331 molecules x 257 queries find-all,
-// whose last lanes run long searches, 2.3 ms less.
+// (wider ones); this takes 6.5 ms and, with k_join_all's second pass, 3.2, and 33,331 molecules x
+// 257 queries find-all, whose last lanes run long searches, 2.7 ms less.
 //
-// Molecules of <= 64 nodes (!WIDE; pairs of larger ones are listed in `wide`) or, with WIDE, of
-// 65..128 nodes: positions then span two words, and `visited` stays one word addressed by
-// position mod 64, the reference's Bitset aliasing (utils.hpp:71-73).  Queries of up to KC nodes;
-// deeper ones are listed in `deep` (their count in stats[deep_stat]), or, with DEEP, run here
-// with the levels past LDS read through global memory.  With `list` the pairs are list[0..P).
+// Molecules of <= 64 nodes (!WIDE; pairs of larger ones are passed over) or, with WIDE, of 65..128
+// nodes: positions then span two words, and `visited` stays one word addressed by position mod 64,
+// the reference's Bitset aliasing (utils.hpp:71-73).  Queries of up to KC nodes; deeper ones are
+// listed in `deep` (their count in stats[kStatDeep]), or, with DEEP, run here with the levels past LDS
+// read through global memory.  With `list` the pairs are list[0..P).
 template <bool FIND_FIRST, class Src, int KC, bool DEEP, bool WIDE>
-__global__ __launch_bounds__(64) void k_join_lanes(GraphDev q, GraphDev d, Src src, const uint32_t* __restrict__ indices,
-                                                   const uint32_t* __restrict__ pair_graph, uint64_t P, uint32_t chunk,
-                                                   int32_t* __restrict__ counts, unsigned long long* __restrict__ stats,
-                                                   uint32_t* __restrict__ wide, const unsigned long long* __restrict__ P_dev,
-                                                   const uint32_t* __restrict__ list, uint32_t* __restrict__ deep, uint32_t cursor,
-                                                   uint32_t deep_stat) {
-  static_assert(KC == 8 || KC == 12, "levels in LDS");
+__device__ __forceinline__ void join_pass(JoinLds<KC, DEEP, WIDE>& sh, const GraphDev& q, const GraphDev& d, const Src& src,
+                                          const uint32_t* __restrict__ indices, const uint32_t* __restrict__ pair_graph, uint64_t P,
+                                          uint32_t chunk, int32_t* __restrict__ counts, unsigned long long* __restrict__ stats,
+                                          const uint32_t* __restrict__ list, uint32_t* __restrict__ deep, uint32_t cursor, JoinTotals& total) {
+  static_assert(KC == 8 || KC == 12 || (WIDE && KC == 7), "levels in LDS");
   constexpr uint32_t L = KC - 1;
-  __shared__ JoinLds<KC, DEEP, WIDE> sh;
-  if (src.aborted()) return;
-  // the pair (or list) count left on the device; P, what the arrays were sized for, bounds it
-  if (P_dev) P = min(P, static_cast<uint64_t>(*P_dev));
   const uint32_t lane = static_cast<uint32_t>(lane_id());
   const uint64_t below = (1ull << lane) - 1;
   const uint32_t* qfold = reinterpret_cast<const uint32_t*>(q.fold);  // query rows fit the low word (k <= 32)
-  uint64_t sum = 0, matched = 0, steps = 0, overflow = 0, wave_iters = 0;
 
   // pairs on their way to the queue, one per lane and stage: graphs and mask base (a), sizes and
   // offsets (b), query adjacency (c)
@@ -239,27 +240,27 @@ __global__ __launch_bounds__(64) void k_join_lanes(GraphDev q, GraphDev d, Src s
   uint64_t adj = 0, visited = 0, count = 0;      // adj: byte t = query row of node t < 8 over nodes < 8
   uint64_t cur = 0, cur_hi = 0, rem = 0, rem_hi = 0;  // the frame's candidates; positions past its last accept
 
-  // Pairs for another pass gather in LDS and go out 64 at a time: an atomic per batch of 64 pairs on
+  // Pairs for the deep pass gather in LDS and go out 64 at a time: an atomic per batch of 64 pairs on
   // one address (about 10 ns each across the XCDs) took 11 ms for 68 M pairs and bound the kernel.
-  uint32_t ndeep = 0, nwide = 0;
-  auto list_flush = [&](uint32_t* buf, uint32_t cnt, uint32_t* out, unsigned long long* total) {
+  uint32_t ndeep = 0;
+  auto list_flush = [&](uint32_t cnt) {
     unsigned long long b = 0;
-    if (lane == 0) b = atomicAdd(total, static_cast<unsigned long long>(cnt));
+    if (lane == 0) b = atomicAdd(&stats[kStatDeep], static_cast<unsigned long long>(cnt));
     const uint64_t ob = uniform64(__shfl(b, 0));
-    if (lane < cnt) out[ob + lane] = buf[lane];
+    if (lane < cnt) deep[ob + lane] = sh.listed[lane];
   };
-  auto list_pairs = [&](bool mine, uint32_t pair, uint32_t* buf, uint32_t& cnt, uint32_t* out, unsigned long long* total) {
+  auto list_pairs = [&](bool mine, uint32_t pair) {
     const uint64_t m = __ballot(mine);
     if (!m) return;
-    if (mine) buf[cnt + __popcll(m & below)] = pair;
+    if (mine) sh.listed[ndeep + __popcll(m & below)] = pair;
     wave_sync();
-    cnt += static_cast<uint32_t>(__popcll(m));
-    if (cnt >= kWave) {
-      list_flush(buf, kWave, out, total);
-      cnt -= kWave;
-      const uint32_t left = buf[kWave + lane];
+    ndeep += static_cast<uint32_t>(__popcll(m));
+    if (ndeep >= kWave) {
+      list_flush(kWave);
+      ndeep -= kWave;
+      const uint32_t left = sh.listed[kWave + lane];
       wave_sync();
-      buf[lane] = left;
+      sh.listed[lane] = left;
       wave_sync();
     }
   };
@@ -345,10 +346,9 @@ __global__ __launch_bounds__(64) void k_join_lanes(GraphDev q, GraphDev d, Src s
     const uint64_t idle = __ballot(!have);
     if (static_cast<uint32_t>(__popcll(idle)) >= kJoinRefill || idle == ~0ull) {  // wave-uniform
       if (qcount == 0 && have_c) {  // the third stage has arrived: queue its pairs
-        const bool wide_pair = !WIDE && cv && cn > 64;  // molecules of > 64 nodes go to the two-word pass
+        const bool wide_pair = !WIDE && cn > 64;  // molecules of > 64 nodes belong to the two-word pass
         const bool deep_pair = !DEEP && cv && !wide_pair && ck > static_cast<uint32_t>(KC);
-        if constexpr (!DEEP) list_pairs(deep_pair, cj, sh.listed[0], ndeep, deep, &stats[deep_stat]);
-        if constexpr (!WIDE) list_pairs(wide_pair, cj, sh.listed[DEEP ? 0 : 1], nwide, wide, &stats[kStatWide]);
+        if constexpr (!DEEP) list_pairs(deep_pair, cj);
         const bool mine = cv && !wide_pair && !deep_pair;
         const uint64_t mm = __ballot(mine);
         if (mine) {
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(64) void k_join_lanes(GraphDev q, GraphDev d, Src s
         continue;
       }
     }
-    ++wave_iters;
+    ++total.wave_iters;
     if (have) {
       bool done = false;
       uint32_t st = 0;
@@ -533,20 +533,22 @@ __global__ __launch_bounds__(64) void k_join_lanes(GraphDev q, GraphDev d, Src s
           if (!leaf) visited = nd == 1 ? 0ull : visited & ~bit_of(stale);
         }
       }
-      steps += st;
+      total.steps += st;
       if (done) {
-        if (count > 0x7FFFFFFFull) overflow = 1;
+        if (count > 0x7FFFFFFFull) total.overflow = 1;
         counts[j] = static_cast<int32_t>(count > 0x7FFFFFFFull ? 0x7FFFFFFFull : count);
-        sum += count;
-        matched += count > 0;
+        total.sum += count;
+        total.matched += count > 0;
         have = false;
       }
     }
   }
   if constexpr (!DEEP)
-    if (ndeep) list_flush(sh.listed[0], ndeep, deep, &stats[deep_stat]);
-  if constexpr (!WIDE)
-    if (nwide) list_flush(sh.listed[DEEP ? 0 : 1], nwide, wide, &stats[kStatWide]);
+    if (ndeep) list_flush(ndeep);
+}
+
+__device__ __forceinline__ void join_totals(const JoinTotals& total, unsigned long long* __restrict__ stats) {
+  uint64_t sum = total.sum, matched = total.matched, steps = total.steps, overflow = total.overflow;
 #pragma unroll
   for (int o = kWave / 2; o > 0; o >>= 1) {
     sum += __shfl_xor(sum, o);
@@ -554,86 +556,152 @@ __global__ __launch_bounds__(64) void k_join_lanes(GraphDev q, GraphDev d, Src s
     steps += __shfl_xor(steps, o);
     overflow |= __shfl_xor(overflow, o);
   }
-  if (lane == 0) {
+  if (lane_id() == 0) {
     if (sum) atomicAdd(&stats[0], static_cast<unsigned long long>(sum));
     if (matched) atomicAdd(&stats[1], static_cast<unsigned long long>(matched));
     if (overflow) atomicOr(&stats[3], 1ull);
     atomicAdd(&stats[4], static_cast<unsigned long long>(steps));
-    atomicAdd(&stats[7], static_cast<unsigned long long>(wave_iters));
+    atomicAdd(&stats[7], static_cast<unsigned long long>(total.wave_iters));
+  }
+}
+
+// One pass over the pairs, or those listed, of molecules of <= 64 nodes.  P_dev: their count left on
+// the device; P, what the arrays were sized for, bounds it.
+template <bool FIND_FIRST, class Src, int KC, bool DEEP>
+__global__ __launch_bounds__(64) void k_join_lanes(GraphDev q, GraphDev d, Src src, const uint32_t* __restrict__ indices,
+                                                   const uint32_t* __restrict__ pair_graph, uint64_t P, uint32_t chunk,
+                                                   int32_t* __restrict__ counts, unsigned long long* __restrict__ stats,
+                                                   const unsigned long long* __restrict__ P_dev, const uint32_t* __restrict__ list,
+                                                   uint32_t* __restrict__ deep, uint32_t cursor) {
+  __shared__ JoinLds<KC, DEEP, false> sh;
+  if (src.aborted()) return;
+  if (P_dev) P = min(P, static_cast<uint64_t>(*P_dev));
+  JoinTotals total;
+  join_pass<FIND_FIRST, Src, KC, DEEP, false>(sh, q, d, src, indices, pair_graph, P, chunk, counts, stats, list, deep, cursor, total);
+  join_totals(total, stats);
+}
+
+// The pairs of molecules of > 64 nodes, listed in `wide`, then the other pairs (or those of `list`): a
+// wavefront goes on to these as soon as no wide pair is left to claim.  The wide pairs are few but
+// their longest searches take as long as the rest of a mid-size join; in a launch of their own,
+// after the others and a round trip to the host for their count, they took 1.6 of 10.2 ms for 1 M
+// LogNormal molecules x 1,000 query graphs, now 9.7 in all; 300,000 x 306 1.93 -> 1.59 ms, the plain
+// form's 150,000 x 300 1.63 -> 1.19 ms.
+template <bool FIND_FIRST, class Src>
+__global__ __launch_bounds__(64) void k_join_all(GraphDev q, GraphDev d, Src src, const uint32_t* __restrict__ indices,
+                                                 const uint32_t* __restrict__ pair_graph, uint64_t P, uint32_t chunk,
+                                                 int32_t* __restrict__ counts, unsigned long long* __restrict__ stats,
+                                                 const unsigned long long* __restrict__ P_dev, const uint32_t* __restrict__ wide, uint64_t wide_cap,
+                                                 const uint32_t* __restrict__ list, uint32_t cursor) {
+  __shared__ alignas(16) unsigned char lds[kJoinAllLds];
+  if (src.aborted()) return;
+  if (P_dev) P = min(P, static_cast<uint64_t>(*P_dev));
+  JoinTotals total;
+  join_pass<FIND_FIRST, Src, kJoinWideLevels, true, true>(*reinterpret_cast<JoinLds<kJoinWideLevels, true, true>*>(lds), q, d, src, indices, pair_graph,
+                                                          min(wide_cap, static_cast<uint64_t>(stats[kStatWide])), kWave, counts, stats, wide, nullptr,
+                                                          kStatWideCursor, total);
+  wave_sync();
+  join_pass<FIND_FIRST, Src, kJoinLevels, true, false>(*reinterpret_cast<JoinLds<kJoinLevels, true, false>*>(lds), q, d, src, indices, pair_graph, P,
+                                                       chunk, counts, stats, list, nullptr, cursor, total);
+  join_totals(total, stats);
+}
+
+// Lists the pairs of molecules of > 64 nodes (the ranges of their molecules in offsets, at most P):
+// a thread per molecule and turn, one atomic per block, a wavefront writes a molecule's range.
+constexpr uint32_t kListTurns = 8;
+__global__ __launch_bounds__(256) void k_list_wide(GraphDev d, const uint32_t* __restrict__ offsets, uint64_t P, uint32_t* __restrict__ wide,
+                                                   unsigned long long* __restrict__ stats) {
+  __shared__ uint32_t waves[4];
+  __shared__ unsigned long long base;
+  const uint32_t lane = static_cast<uint32_t>(lane_id()), wave = threadIdx.x / kWave;
+  const uint64_t m0 = blockIdx.x * static_cast<uint64_t>(256 * kListTurns) + wave * kWave * kListTurns;
+  uint32_t start[kListTurns], cnt[kListTurns], mine = 0;
+#pragma unroll
+  for (uint32_t t = 0; t < kListTurns; ++t) {
+    const uint64_t m = m0 + t * kWave + lane;
+    start[t] = cnt[t] = 0;
+    if (m < d.G && d.go[m + 1] - d.go[m] > 64) {
+      start[t] = static_cast<uint32_t>(min(P, static_cast<uint64_t>(offsets[m])));
+      cnt[t] = static_cast<uint32_t>(min(P, static_cast<uint64_t>(offsets[m + 1]))) - start[t];
+    }
+    mine += cnt[t];
+  }
+  uint32_t incl = mine;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const uint32_t y = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), o));
+    if (lane >= static_cast<uint32_t>(o)) incl += y;
+  }
+  if (lane == kWave - 1) waves[wave] = incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t all = waves[0] + waves[1] + waves[2] + waves[3];
+    base = all ? atomicAdd(&stats[kStatWide], static_cast<unsigned long long>(all)) : 0ull;
+  }
+  __syncthreads();
+  uint64_t at = base + incl - mine;
+  for (uint32_t x = 0; x < wave; ++x) at += waves[x];
+#pragma unroll
+  for (uint32_t t = 0; t < kListTurns; ++t) {
+    for (uint64_t left = __ballot(cnt[t] != 0); left; left &= left - 1) {  // wave-uniform
+      const int i = static_cast<int>(__builtin_ctzll(left));
+      const uint32_t s = rl32(start[t], i), n = rl32(cnt[t], i);
+      const uint64_t to = uniform64(__shfl(at, i));
+      for (uint32_t x = lane; x < n; x += kWave) wide[to + x] = s + x;
+    }
+    at += cnt[t];
   }
 }
 
 // Wavefronts (one-wavefront blocks) for `pairs` pairs: as many as stay resident by LDS, or the
 // tuned share of them in quarters, and no more than have a pair each.
-template <int KC, bool DEEP, bool WIDE>
-uint64_t join_blocks(uint64_t pairs, int num_cus, uint32_t quarters) {
+inline uint64_t join_blocks(size_t lds, uint64_t pairs, int num_cus, uint32_t quarters) {
   const uint64_t cus = static_cast<uint64_t>(num_cus > 0 ? num_cus : 256);
-  const uint64_t per_cu = std::max<uint64_t>(1, uint64_t(join_waves_per_cu<KC, DEEP, WIDE>()) * quarters / 4);
+  const uint64_t per_cu = std::max<uint64_t>(1, uint64_t(join_waves_per_cu(lds)) * quarters / 4);
   return std::max<uint64_t>(1, std::min<uint64_t>((pairs + 63) / 64, cus * per_cu));
 }
 
-// The lane join over P pairs: with `deep`, a kJoinShallow-level pass over all of them that lists
-// the deeper queries, then a pass over that list (its length read on the device); without it, one
-// pass.  `quarters` (1..4: share of the resident wavefronts) and chunk (0: ~4 claims per
-// wavefront, at most 1024 pairs: a claim is an atomic on one address) shape the first pass.
-template <class Src>
-hipError_t launch_join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const Src& src, const uint32_t* indices,
-                             const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts, unsigned long long* stats,
-                             uint32_t* wide, int num_cus, const unsigned long long* P_dev, uint32_t* deep, uint32_t quarters,
-                             uint32_t chunk) {
-  if (!P) return hipSuccess;
-  if (P < kJoinTwoPassPairs) deep = nullptr;
-  const auto claim = [&](uint64_t blocks) {
-    return chunk ? chunk : static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, P / (blocks * 4) / 64 * 64)));
+// The lane join over P pairs.  With `deep` and enough pairs, a kJoinShallow-level pass over all of them
+// lists the deeper queries' pairs, whose count the next pass reads on the device; otherwise one pass
+// takes them all.  With `wide` (capacity P) the pairs of molecules of > 64 nodes are listed first and
+// run with the last pass; null when the data has none.  `quarters` (1..4: share of the resident
+// wavefronts) and chunk (0: ~4 claims per wavefront, ~8 behind wide pairs, at most 1024 pairs: a claim
+// is an atomic on one address) shape the pass over all pairs.
+template <bool FIND_FIRST, class Src>
+hipError_t launch_join_passes(hipStream_t s, const GraphDev& q, const GraphDev& d, const Src& src, const uint32_t* offsets, const uint32_t* indices,
+                              const uint32_t* pair_graph, uint64_t P, int32_t* counts, unsigned long long* stats, uint32_t* wide, int num_cus,
+                              const unsigned long long* P_dev, uint32_t* deep, uint32_t quarters, uint32_t chunk) {
+  const auto claim = [&](uint64_t blocks, uint32_t claims) {
+    return chunk ? chunk : static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, P / (blocks * claims) / 64 * 64)));
   };
-  if (!deep) {
-    const uint64_t blocks = join_blocks<kJoinLevels, true, false>(P, num_cus, quarters);
-    const dim3 grid(static_cast<unsigned>(blocks));
-    if (find_first)
-      hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinLevels, true, false>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, claim(blocks),
-                         counts, stats, wide, P_dev, nullptr, nullptr, kStatCursor, kStatDeep);
-    else
-      hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinLevels, true, false>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, claim(blocks),
-                         counts, stats, wide, P_dev, nullptr, nullptr, kStatCursor, kStatDeep);
-    return hipGetLastError();
+  if (wide) k_list_wide<<<(d.G + 256 * kListTurns - 1) / (256 * kListTurns), 256, 0, s>>>(d, offsets, P, wide, stats);
+  const bool two = deep && P >= kJoinTwoPassPairs;
+  if (two) {
+    const uint64_t blocks = join_blocks(sizeof(JoinLds<kJoinShallow, false, false>), P, num_cus, quarters);
+    k_join_lanes<FIND_FIRST, Src, kJoinShallow, false><<<static_cast<unsigned>(blocks), 64, 0, s>>>(
+        q, d, src, indices, pair_graph, P, claim(blocks, 4), counts, stats, P_dev, nullptr, deep, kStatCursor);
+    P_dev = stats + kStatDeep;
+    quarters = 4;
   }
-  const uint64_t blocks = join_blocks<kJoinShallow, false, false>(P, num_cus, quarters);
-  const dim3 grid(static_cast<unsigned>(blocks));
-  if (find_first)
-    hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinShallow, false, false>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, claim(blocks),
-                       counts, stats, wide, P_dev, nullptr, deep, kStatCursor, kStatDeep);
+  const uint32_t* list = two ? deep : nullptr;
+  const uint32_t cursor = two ? kStatDeepCursor : kStatCursor;
+  const uint64_t blocks = join_blocks(wide ? kJoinAllLds : sizeof(JoinLds<kJoinLevels, true, false>), P, num_cus, quarters);
+  const uint32_t claims = two ? kJoinDeepChunk : claim(blocks, wide ? 8 : 4);
+  if (wide)
+    k_join_all<FIND_FIRST, Src><<<static_cast<unsigned>(blocks), 64, 0, s>>>(q, d, src, indices, pair_graph, P, claims, counts, stats, P_dev, wide, P,
+                                                                             list, cursor);
   else
-    hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinShallow, false, false>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, claim(blocks),
-                       counts, stats, wide, P_dev, nullptr, deep, kStatCursor, kStatDeep);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const dim3 dgrid(static_cast<unsigned>(join_blocks<kJoinLevels, true, false>(P, num_cus, 4)));
-  if (find_first)
-    hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinLevels, true, false>), dgrid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, kJoinDeepChunk, counts,
-                       stats, wide, stats + kStatDeep, deep, nullptr, kStatDeepCursor, kStatDeep);
-  else
-    hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinLevels, true, false>), dgrid, dim3(64), 0, s, q, d, src, indices, pair_graph, P, kJoinDeepChunk, counts,
-                       stats, wide, stats + kStatDeep, deep, nullptr, kStatDeepCursor, kStatDeep);
+    k_join_lanes<FIND_FIRST, Src, kJoinLevels, true><<<static_cast<unsigned>(blocks), 64, 0, s>>>(q, d, src, indices, pair_graph, P, claims, counts,
+                                                                                                  stats, P_dev, list, nullptr, cursor);
   return hipGetLastError();
 }
-
-// The two-word lane join over the nw pairs listed in `list` (their count also at nw_dev when
-// given, nw then only bounding the grid).
 template <class Src>
-hipError_t launch_join_wide(hipStream_t s, const GraphDev& q, const GraphDev& d, const Src& src, const uint32_t* indices,
-                            const uint32_t* pair_graph, const uint32_t* list, uint64_t nw, int find_first, int32_t* counts,
-                            unsigned long long* stats, int num_cus, const unsigned long long* nw_dev) {
-  if (!nw) return hipSuccess;
-  const uint64_t blocks = join_blocks<kJoinShallow, true, true>(nw, num_cus, 4);
-  const uint32_t chunk = static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, nw / (blocks * 4) / 64 * 64)));
-  const dim3 grid(static_cast<unsigned>(blocks));
-  if (find_first)
-    hipLaunchKernelGGL((k_join_lanes<true, Src, kJoinShallow, true, true>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, nw, chunk, counts,
-                       stats, nullptr, nw_dev, list, nullptr, static_cast<uint32_t>(kStatWideCursor), static_cast<uint32_t>(kStatDeep));
-  else
-    hipLaunchKernelGGL((k_join_lanes<false, Src, kJoinShallow, true, true>), grid, dim3(64), 0, s, q, d, src, indices, pair_graph, nw, chunk, counts,
-                       stats, nullptr, nw_dev, list, nullptr, static_cast<uint32_t>(kStatWideCursor), static_cast<uint32_t>(kStatDeep));
-  return hipGetLastError();
+hipError_t launch_join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const Src& src, const uint32_t* offsets, const uint32_t* indices,
+                             const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts, unsigned long long* stats, uint32_t* wide,
+                             int num_cus, const unsigned long long* P_dev, uint32_t* deep, uint32_t quarters, uint32_t chunk) {
+  if (!P) return hipSuccess;
+  return find_first ? launch_join_passes<true>(s, q, d, src, offsets, indices, pair_graph, P, counts, stats, wide, num_cus, P_dev, deep, quarters, chunk)
+                    : launch_join_passes<false>(s, q, d, src, offsets, indices, pair_graph, P, counts, stats, wide, num_cus, P_dev, deep, quarters, chunk);
 }
 
 }  // namespace

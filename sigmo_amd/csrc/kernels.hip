@@ -1280,12 +1280,10 @@ hipError_t gmcr_scatter(hipStream_t s, const uint64_t* pair_bits, uint32_t Gq, u
   return hipGetLastError();
 }
 
-hipError_t join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint64_t* bits, uint64_t W64, const uint32_t* indices,
-                      const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts, unsigned long long* stats, uint32_t* wide,
-                      int num_cus, const unsigned long long* P_dev, uint32_t* deep) {
-  if (!P) return hipSuccess;
-  const BitsetMasks src{bits, W64};
-  return launch_join_lanes(s, q, d, src, indices, pair_graph, P, find_first, counts, stats, wide, num_cus, P_dev, deep, 4, 0);
+hipError_t join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint64_t* bits, uint64_t W64, const uint32_t* offsets,
+                      const uint32_t* indices, const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts, unsigned long long* stats,
+                      uint32_t* wide, int num_cus, const unsigned long long* P_dev, uint32_t* deep) {
+  return launch_join_lanes(s, q, d, BitsetMasks{bits, W64}, offsets, indices, pair_graph, P, find_first, counts, stats, wide, num_cus, P_dev, deep, 4, 0);
 }
 
 hipError_t join_wildcard(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint8_t* qel, const uint8_t* del, const uint64_t* bits,
@@ -1312,12 +1310,6 @@ hipError_t join_wildcard(hipStream_t s, const GraphDev& q, const GraphDev& d, co
   pass<<<static_cast<unsigned>(blocks), 64, 0, s>>>(q, d, qel, del, src, indices, pair_graph, P, 64, counts, stats, nullptr, wide,
                                                     stats + kStatWide, kStatWideCursor);
   return hipGetLastError();
-}
-
-hipError_t join_lanes_wide(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint64_t* bits, uint64_t W64, const uint32_t* indices,
-                           const uint32_t* pair_graph, const uint32_t* list, uint64_t nw, int find_first, int32_t* counts,
-                           unsigned long long* stats, int num_cus, const unsigned long long* nw_dev) {
-  return launch_join_wide(s, q, d, BitsetMasks{bits, W64}, indices, pair_graph, list, nw, find_first, counts, stats, num_cus, nw_dev);
 }
 
 }  // namespace sigmo_k

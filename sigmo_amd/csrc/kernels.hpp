@@ -48,7 +48,7 @@ struct AMGraphDev {
 struct LabelSlots {
   uint8_t label[16];
   int count;
-  int frequent;  // the slot of the label that most nodes have
+  int frequent;  // the slot of the label that most of the first nodes have
 };
 
 hipError_t fill_u64(hipStream_t s, uint64_t* p, uint64_t n, uint64_t v);
@@ -134,13 +134,13 @@ constexpr uint32_t kJoinStatWords = 16;
 // (zeroed by the caller), stats[3] |= 1 on int32 overflow.  With `deep` (capacity P) a
 // large join runs in two passes: a first over the queries of at most kJoinShallow nodes, which
 // lists the other pairs in `deep` (count in stats[8]), then one over that list; without it, one
-// pass.
-// Lane-per-pair join of the pairs whose molecule has <= 64 nodes; the others are appended to
-// `wide` (count in stats[5]) for join_lanes_wide.  With P_dev the kernel reads the pair count
-// from the device and P only bounds the grid.
-hipError_t join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint64_t* bits, uint64_t W64, const uint32_t* indices,
-                      const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts, unsigned long long* stats, uint32_t* wide,
-                      int num_cus, const unsigned long long* P_dev = nullptr, uint32_t* deep = nullptr);
+// pass.  A lane per pair; the pairs of molecules of more than 64 nodes are listed in `wide` (capacity
+// P, count in stats[5]; null when the data has none) by their molecules' ranges of `offsets`, and
+// searched before the others of the last pass.  With P_dev the kernels read the pair count from the
+// device and P only bounds it.
+hipError_t join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint64_t* bits, uint64_t W64, const uint32_t* offsets,
+                      const uint32_t* indices, const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts, unsigned long long* stats,
+                      uint32_t* wide, int num_cus, const unsigned long long* P_dev = nullptr, uint32_t* deep = nullptr);
 // joinWildcardCandidates: matching order by candidate count, edge labels compared, one DFS per
 // candidate of the first node; one lane per pair (qel/del: edge labels of the CSR entries).  `wide`
 // (capacity P) takes the pairs of molecules of more than 64 nodes for a second pass; null when the
@@ -148,11 +148,4 @@ hipError_t join_lanes(hipStream_t s, const GraphDev& q, const GraphDev& d, const
 hipError_t join_wildcard(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint8_t* qel, const uint8_t* del, const uint64_t* bits,
                          uint64_t W64, const uint32_t* indices, const uint32_t* pair_graph, uint64_t P, int find_first, int32_t* counts,
                          unsigned long long* stats, int num_cus, uint32_t* wide);
-// The lane-per-pair join over the `nw` listed pairs of molecules with 65..128 nodes
-// (stats[kStatWideCursor] is the work counter).  With nw_dev the kernel reads the list's length on
-// the device, bounded by nw.
-hipError_t join_lanes_wide(hipStream_t s, const GraphDev& q, const GraphDev& d, const uint64_t* bits, uint64_t W64, const uint32_t* indices,
-                           const uint32_t* pair_graph, const uint32_t* list, uint64_t nw, int find_first, int32_t* counts,
-                           unsigned long long* stats, int num_cus, const unsigned long long* nw_dev = nullptr);
-
 }  // namespace sigmo_k

@@ -1290,6 +1290,7 @@ int bgrow_slack(T** p, uint64_t& cap, uint64_t need) {
 namespace sigmo_internal {
 int ctx_info(sigmo_ctx* ctx, int* device, hipStream_t* stream, int* num_cus, unsigned long long** stats, unsigned long long** stats_host);
 int ctx_timed(sigmo_ctx* ctx, int phase, int kernel, double bytes, bool begin, void** token);
+int ctx_read_back(sigmo_ctx* ctx, const sigmo_k::HostCopy* copies, int n);
 void ctx_add_bytes(sigmo_ctx* ctx, int kernel, double bytes);
 const sigmo_k::GraphDev graph_dev(const sigmo_graph* g);
 const std::vector<uint32_t>& graph_host_offsets(const sigmo_graph* g);
@@ -1625,8 +1626,8 @@ int sigmo_batch_request_stats(sigmo_batch* b, const uint32_t* request_graph_offs
     BATCH_HIP_TRY(hipGetLastError());
   }
   std::vector<unsigned long long> h(3ull * num_requests);
-  BATCH_HIP_TRY(hipMemcpyAsync(h.data(), b->req_out, h.size() * 8, hipMemcpyDeviceToHost, s));
-  BATCH_HIP_TRY(hipStreamSynchronize(s));
+  const sigmo_k::HostCopy back = {h.data(), b->req_out, h.size() * 8};
+  BATCH_TRY(ctx_read_back(b->ctx, &back, 1));
   for (uint32_t r = 0; r < num_requests; ++r) {
     out[r].matched_pairs = h[3 * r];
     out[r].embeddings = h[3 * r + 1];
@@ -1934,9 +1935,9 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
   void* tok = nullptr;
   BATCH_TRY(ctx_timed(b->ctx, SIGMO_PHASE_GMCR, -1, 0.0, true, &tok));
   BATCH_HIP_TRY(launch_count_scan(b, L, s));
-  uint64_t P = 0;
-  BATCH_HIP_TRY(hipMemcpyAsync(&P, b->total, 8, hipMemcpyDeviceToHost, s));
+  BATCH_HIP_TRY(hipMemcpyAsync(b->run_host + kCounterWords, b->total, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   BATCH_HIP_TRY(hipStreamSynchronize(s));
+  const uint64_t P = b->run_host[kCounterWords];
   if (P >= (1ull << 32)) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "GMCR pair count exceeds u32");
   // result-sized arrays regrow with a quarter to spare: each hipFree waits for the whole device
   BATCH_TRY(b->grow(&b->indices, b->cap_idx, P, true));
@@ -2117,15 +2118,12 @@ int sigmo_batch_pairs(sigmo_batch* b, uint32_t* data_graph_offsets, uint64_t n_o
   unsigned long long *st, *sh;
   BATCH_TRY(ctx_info(b->ctx, &device, &s, &cus, &st, &sh));
   const uint64_t Gd = graph_dev(b->db->data).G;
-  if (data_graph_offsets) {
-    if (n_offsets != Gd + 1) return sigmo_err::set(SIGMO_ERR_INVALID, "n_offsets must be Gd+1");
-    BATCH_HIP_TRY(hipMemcpyAsync(data_graph_offsets, b->offsets, n_offsets * 4, hipMemcpyDeviceToHost, s));
-  }
+  if (data_graph_offsets && n_offsets != Gd + 1) return sigmo_err::set(SIGMO_ERR_INVALID, "n_offsets must be Gd+1");
   if ((query_graph_indices || counts) && n_pairs != b->P) return sigmo_err::set(SIGMO_ERR_INVALID, "n_pairs must be the pair count");
-  if (query_graph_indices && n_pairs)
-    BATCH_HIP_TRY(hipMemcpyAsync(query_graph_indices, b->indices, n_pairs * 4, hipMemcpyDeviceToHost, s));
-  if (counts && n_pairs) BATCH_HIP_TRY(hipMemcpyAsync(counts, b->counts, n_pairs * 4, hipMemcpyDeviceToHost, s));
-  BATCH_HIP_TRY(hipStreamSynchronize(s));
+  const sigmo_k::HostCopy out[3] = {{data_graph_offsets, b->offsets, data_graph_offsets ? n_offsets * 4 : 0},
+                                    {query_graph_indices, b->indices, query_graph_indices ? n_pairs * 4 : 0},
+                                    {counts, b->counts, counts ? n_pairs * 4 : 0}};
+  BATCH_TRY(ctx_read_back(b->ctx, out, 3));
   return SIGMO_OK;
 }
 

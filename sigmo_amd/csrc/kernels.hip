@@ -43,6 +43,18 @@ __global__ void k_sub_u32(uint32_t* p, uint64_t n, uint32_t v) {
     p[i] -= v;
 }
 
+// Bound by the link to the host (50 GB/s): 16 bytes per lane and store.
+__global__ __launch_bounds__(256) void k_gather(GatherArgs a, unsigned char* __restrict__ to) {
+  for (int i = 0; i < a.count; ++i) {
+    const uint32_t words = a.bytes[i] / 4, whole = words / 4;
+    const uint4* src = static_cast<const uint4*>(a.src[i]);
+    uint4* dst = reinterpret_cast<uint4*>(to + a.at[i]);
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t x = t; x < whole; x += gridDim.x * blockDim.x) dst[x] = src[x];
+    if (t < words - 4 * whole) reinterpret_cast<uint32_t*>(dst + whole)[t] = reinterpret_cast<const uint32_t*>(src + whole)[t];
+  }
+}
+
 inline unsigned grid_for(uint64_t n, unsigned block, unsigned cap = 1u << 20) {
   uint64_t g = (n + block - 1) / block;
   if (g > cap) g = cap;
@@ -1238,6 +1250,14 @@ hipError_t filter_levels(hipStream_t s, const uint32_t* tok, uint64_t Q, const u
   if (xcd_grid(strips, chunks) > 0x7fffffffull) return hipErrorInvalidValue;
   k_filter_levels<<<static_cast<unsigned>(xcd_grid(strips, chunks)), kLevelWaves * 64, (staged + 1) * slot_planes(R) * 256, s>>>(
       tok, Q, lplanes, static_cast<const uint4*>(lvl), D, R, slots, U, staged, bits, rpb, chunks);
+  return hipGetLastError();
+}
+
+hipError_t gather(hipStream_t s, const GatherArgs& a, void* to) {
+  uint64_t bytes = 0;
+  for (int i = 0; i < a.count; ++i) bytes += a.bytes[i];
+  if (!bytes) return hipSuccess;
+  k_gather<<<grid_for(bytes / 16 + 1, 256, 256), 256, 0, s>>>(a, static_cast<unsigned char*>(to));
   return hipGetLastError();
 }
 

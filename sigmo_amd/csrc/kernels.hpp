@@ -44,6 +44,23 @@ struct AMGraphDev {
   uint64_t N;
 };
 
+// A device-to-host copy into a caller's memory.
+struct HostCopy {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+
+// Arrays gathered into pinned host memory: bytes (whole words) of src to offset `at`, both at 16-byte
+// boundaries.
+constexpr int kGatherParts = 4;
+struct GatherArgs {
+  int count;
+  const void* src[kGatherParts];
+  uint32_t at[kGatherParts], bytes[kGatherParts];
+};
+hipError_t gather(hipStream_t s, const GatherArgs& a, void* to);
+
 // Labels < 16 that may carry a nonzero signature count, compacted into slots.
 struct LabelSlots {
   uint8_t label[16];

@@ -189,7 +189,10 @@ __device__ __forceinline__ uint32_t bit_spread(uint32_t q, uint32_t t) {
 // idle lanes take queued pairs and load their masks.  Loads return in order, so a step's wait for
 // its adjacency row also waits for every load issued before: the stages and the masks are
 // therefore all issued together, when kJoinRefill lanes are idle, and a wavefront stalls on them
-// once per that many pairs (16, 24 and 32 measure the same, 40 is 4% slower).
+// once per that many pairs (16, 24 and 32 measure the same, 40 is 4% slower).  Results are stored then
+// too, since a wait for a load also waits for every store before it: 1 M LogNormal molecules x
+// 1,000 queries 10.7 -> 10.3 ms, 300,000 x 306 2.08 -> 2.01 ms.  Reading one word of each line of a
+// pair's adjacency rows ahead, or all levels' rows in one group, gave nothing.
 //
 // Bound by VALU issue (about two thirds of it on 68 M pairs) at 11 wavefronts per CU by LDS.  One
 // DFS step per iteration, all rows tested per lane and an atomic per listed batch took, for 1 M
@@ -230,7 +233,7 @@ __device__ __forceinline__ void join_pass(JoinLds<KC, DEEP, WIDE>& sh, const Gra
   for (int t = 0; t < 8; ++t) ca[t] = 0;
 
   // the lane's pair; `loading`: taken, its candidate masks on their way
-  bool have = false, loading = false;
+  bool have = false, loading = false, finished = false;
   uint64_t mlo[KC], mhi[WIDE ? KC : 1];
 #pragma unroll
   for (int t = 0; t < KC; ++t) mlo[t] = 0;
@@ -345,6 +348,13 @@ __device__ __forceinline__ void join_pass(JoinLds<KC, DEEP, WIDE>& sh, const Gra
     }
     const uint64_t idle = __ballot(!have);
     if (static_cast<uint32_t>(__popcll(idle)) >= kJoinRefill || idle == ~0ull) {  // wave-uniform
+      if (finished) {  // stored here and not when the search ends: the next step's wait for its row would wait for it
+        if (count > 0x7FFFFFFFull) total.overflow = 1;
+        counts[j] = static_cast<int32_t>(count > 0x7FFFFFFFull ? 0x7FFFFFFFull : count);
+        total.sum += count;
+        total.matched += count > 0;
+        finished = false;
+      }
       if (qcount == 0 && have_c) {  // the third stage has arrived: queue its pairs
         const bool wide_pair = !WIDE && cn > 64;  // molecules of > 64 nodes belong to the two-word pass
         const bool deep_pair = !DEEP && cv && !wide_pair && ck > static_cast<uint32_t>(KC);
@@ -535,10 +545,7 @@ __device__ __forceinline__ void join_pass(JoinLds<KC, DEEP, WIDE>& sh, const Gra
       }
       total.steps += st;
       if (done) {
-        if (count > 0x7FFFFFFFull) total.overflow = 1;
-        counts[j] = static_cast<int32_t>(count > 0x7FFFFFFFull ? 0x7FFFFFFFull : count);
-        total.sum += count;
-        total.matched += count > 0;
+        finished = true;
         have = false;
       }
     }
@@ -556,13 +563,13 @@ __device__ __forceinline__ void join_totals(const JoinTotals& total, unsigned lo
     steps += __shfl_xor(steps, o);
     overflow |= __shfl_xor(overflow, o);
   }
-  if (lane_id() == 0) {
-    if (sum) atomicAdd(&stats[0], static_cast<unsigned long long>(sum));
-    if (matched) atomicAdd(&stats[1], static_cast<unsigned long long>(matched));
-    if (overflow) atomicOr(&stats[3], 1ull);
-    atomicAdd(&stats[4], static_cast<unsigned long long>(steps));
-    atomicAdd(&stats[7], static_cast<unsigned long long>(total.wave_iters));
-  }
+  // one atomic for the four sums, which share a line (about 10 ns each on one line), and none of zero:
+  // 100,000 pairs' wavefronts with nothing to join 40 -> 4 us
+  const uint32_t lane = static_cast<uint32_t>(lane_id());
+  const uint64_t mine = lane == 0 ? sum : (lane == 1 ? matched : (lane == 2 ? steps : total.wave_iters));
+  const uint32_t at = lane == 0 ? kStatSum : (lane == 1 ? kStatMatched : (lane == 2 ? kStatSteps : kStatWaveIters));
+  if (lane < 4 && mine) atomicAdd(&stats[at], static_cast<unsigned long long>(mine));
+  if (lane == 0 && overflow) atomicOr(&stats[kStatOverflow], 1ull);
 }
 
 // One pass over the pairs, or those listed, of molecules of <= 64 nodes.  P_dev: their count left on

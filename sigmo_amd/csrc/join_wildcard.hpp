@@ -13,14 +13,6 @@
 namespace sigmo_k {
 namespace {
 
-// Label of the first CSR entry of row a that points at b (graph.hpp:88-93), 255 if none.
-__device__ __forceinline__ uint32_t first_edge_label(const uint32_t* __restrict__ ro, const uint32_t* __restrict__ ci,
-                                                     const uint8_t* __restrict__ el, uint32_t a, uint32_t b) {
-  for (uint32_t i = ro[a], e = ro[a + 1]; i < e; ++i)
-    if (ci[i] == b) return el[i];
-  return 0xFFu;
-}
-
 constexpr int kWildcardLevels = 8;
 constexpr uint32_t kWildcardRefill = 16;  // free pair slots that make a wavefront load new pairs
 
@@ -62,8 +54,11 @@ struct WildcardLds {
 // candidates at once, from rows and masks in LDS, less the neighbours of a mapped query neighbour
 // whose edge label differs from the query's; frames past the seventh read masks and rows from
 // memory.  That join took 4.35 ms with a lane per pair and every step rereading masks, rows and
-// labels from memory, 2.6 ms with a lane per pair in these frames, and takes 0.92 ms with a lane per
-// search: what bounds it is the chain of dependent steps, few waves in flight by LDS.
+// labels from memory, 2.6 ms with a lane per pair in these frames, and 1.02 ms with a lane per search:
+// what bounds it is the chain of dependent steps, few waves in flight by LDS.  A step's loads are
+// therefore two deep: the row offsets with the adjacency and query rows, then four CSR entries of either
+// side, and all levels' rows come from LDS together; 0.72 ms, where entry after entry and row after row
+// were a dozen waits.  Loading a new pair's masks four at a time gave nothing.
 // Molecules of <= 64 nodes (!WIDE; pairs of larger ones are listed in `wide`) or, with WIDE, the
 // listed pairs of larger ones.
 template <bool FIND_FIRST, bool WIDE>
@@ -110,39 +105,88 @@ __global__ __launch_bounds__(64) void k_join_wildcard(GraphDev q, GraphDev d, co
     }
   };
   // order position t's candidate set after the mapped positions below it: rows and, for query
-  // neighbours, edge labels
-  auto frame = [&](uint32_t t, uint64_t& lo, uint64_t& hi) {
+  // neighbours, edge labels.  qr: t's query row; [vi, ve): the CSR row of the position mapped at t - 1
+  auto frame = [&](uint32_t t, uint32_t qr, uint32_t vi, uint32_t ve, uint64_t& lo, uint64_t& hi) {
     node_mask(t, lo, hi);
-    const uint32_t qr = query_row(t);
-    for (uint32_t x = 0; x < t; ++x) {
-      const uint32_t a = bit_spread(qr, x);
-      uint64_t rl, rh = 0;
-      if (x < L) {
-        rl = sh.row[0][x][lane];
-        if constexpr (WIDE) rh = sh.row[1][x][lane];
-      } else {
-        const uint64_t v = static_cast<uint64_t>(s) + sh.map[lane][x];
-        rl = d.adj[2 * v];
-        if constexpr (WIDE) rh = d.adj[2 * v + 1];
+    const uint32_t mapped = qr & ((1u << t) - 1u);
+    auto group = [&](uint32_t x0, uint32_t x1) {
+      uint64_t r[4], rh[4];
+#pragma unroll
+      for (uint32_t x = x0; x < x1; ++x) {
+        r[x - x0] = sh.row[0][x][lane];
+        if constexpr (WIDE) rh[x - x0] = sh.row[1][x][lane];
       }
-      lo = and_row(lo, rl, a);
-      if constexpr (WIDE) hi = and_row(hi, rh, a);
+#pragma unroll
+      for (uint32_t x = x0; x < x1; ++x) {  // an empty row of no neighbour keeps every position
+        const uint32_t a = bit_spread(mapped, x);
+        lo = and_row(lo, x < t ? r[x - x0] : 0ull, a);
+        if constexpr (WIDE) hi = and_row(hi, x < t ? rh[x - x0] : 0ull, a);
+      }
+    };
+    group(0, 4);
+    if (__any(t > 4)) group(4, L);
+    for (uint32_t x = L; x < t; ++x) {
+      const uint64_t v = static_cast<uint64_t>(s) + sh.map[lane][x];
+      const uint32_t a = bit_spread(mapped, x);
+      lo = and_row(lo, d.adj[2 * v], a);
+      if constexpr (WIDE) hi = and_row(hi, d.adj[2 * v + 1], a);
     }
     const uint32_t qn = qoff + node_of(t);
-    for (uint32_t nb = qr & ((1u << t) - 1u); nb && (lo | hi); nb &= nb - 1) {
+    for (uint32_t nb = mapped; nb && (lo | hi); nb &= nb - 1) {
       const uint32_t x = static_cast<uint32_t>(__builtin_ctz(nb));
-      const uint32_t want = first_edge_label(q.ro, q.ci, qel, qoff + node_of(x), qn);
-      const uint32_t v = s + sh.map[lane][x];
-      uint64_t seen_lo = 0, seen_hi = 0;  // neighbours whose first CSR entry has passed
-      for (uint32_t i = d.ro[v], e = d.ro[v + 1]; i < e; ++i) {
-        const uint32_t c = d.ci[i] - s;
-        const uint64_t bit = bit_of(c);
-        uint64_t& seen = c < 64 ? seen_lo : seen_hi;
-        if (!(seen & bit) && del[i] != want) {
-          if (c < 64) lo &= ~bit;
-          else hi &= ~bit;
+      const uint32_t qx = qoff + node_of(x), v = s + sh.map[lane][x];
+      uint32_t qi = q.ro[qx], di = vi, de = ve;
+      const uint32_t qe = q.ro[qx + 1];
+      if (x + 1 != t) {
+        di = d.ro[v];
+        de = d.ro[v + 1];
+      }
+      // the label of the first CSR entry of the query edge (graph.hpp:88-93), 255 if none, and the data
+      // row's neighbours: four entries each at a time, past the end the last one again
+      uint32_t want = 0xFFu, dc[4], dl[4];
+      if (di < de) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+          dc[u] = d.ci[min(di + u, de - 1)];
+          dl[u] = del[min(di + u, de - 1)];
         }
-        seen |= bit;
+      }
+      for (bool found = false; qi < qe && !found; qi += 4) {
+        uint32_t qc[4], ql[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+          qc[u] = q.ci[min(qi + u, qe - 1)];
+          ql[u] = qel[min(qi + u, qe - 1)];
+        }
+#pragma unroll
+        for (int u = 3; u >= 0; --u)
+          if (qc[u] == qn) {
+            want = ql[u];
+            found = true;
+          }
+      }
+      uint64_t seen_lo = 0, seen_hi = 0;  // neighbours whose first CSR entry has passed
+      while (di < de) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+          const uint32_t c = dc[u] - s;
+          const uint64_t bit = bit_of(c);
+          if (!WIDE || c < 64) {
+            if (!(seen_lo & bit) && dl[u] != want) lo &= ~bit;
+            seen_lo |= bit;
+          } else {
+            if (!(seen_hi & bit) && dl[u] != want) hi &= ~bit;
+            seen_hi |= bit;
+          }
+        }
+        di += 4;
+        if (di < de) {
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) {
+            dc[u] = d.ci[min(di + u, de - 1)];
+            dl[u] = del[min(di + u, de - 1)];
+          }
+        }
       }
     }
   };
@@ -154,17 +198,20 @@ __global__ __launch_bounds__(64) void k_join_wildcard(GraphDev q, GraphDev d, co
       ++count;
       return FIND_FIRST;
     }
+    // what the next frame reads from memory first, issued together
+    const uint64_t v = static_cast<uint64_t>(s) + c;
+    const uint64_t rlo = d.adj[2 * v], rhi = WIDE ? d.adj[2 * v + 1] : 0ull;
+    const uint32_t vi = d.ro[v], ve = d.ro[v + 1], qr = query_row(nd);
     if (depth < L) {
-      const uint64_t v = static_cast<uint64_t>(s) + c;
-      sh.row[0][depth][lane] = d.adj[2 * v];
+      sh.row[0][depth][lane] = rlo;
       sh.base[0][depth][lane] = cur;
       if constexpr (WIDE) {
-        sh.row[1][depth][lane] = d.adj[2 * v + 1];
+        sh.row[1][depth][lane] = rhi;
         sh.base[1][depth][lane] = cur_hi;
       }
     }
     uint64_t nlo = 0, nhi = 0;
-    frame(nd, nlo, nhi);
+    frame(nd, qr, vi, ve, nlo, nhi);
     if ((nlo & ~visited) | (WIDE ? nhi & ~visited : 0ull)) {
       depth = nd;
       cur = nlo;
@@ -324,7 +371,8 @@ __global__ __launch_bounds__(64) void k_join_wildcard(GraphDev q, GraphDev d, co
             cur = sh.base[0][depth][lane];
             if constexpr (WIDE) cur_hi = sh.base[1][depth][lane];
           } else {
-            frame(depth, cur, cur_hi);
+            const uint32_t v = s + sh.map[lane][depth - 1];
+            frame(depth, query_row(depth), d.ro[v], d.ro[v + 1], cur, cur_hi);
           }
           rem = c < 64 ? bits_above(c) : 0ull;
           rem_hi = c < 64 ? ~0ull : bits_above(c - 64);

@@ -121,7 +121,13 @@ struct BitsetMasks {
 constexpr int kJoinShallow = 8;
 constexpr int kJoinLevels = 12;
 constexpr int kJoinWideLevels = 7;  // two words per position: LDS as for kJoinLevels of one
-constexpr uint64_t kJoinTwoPassPairs = 1ull << 24;  // pair counts from which the lane join runs in two passes
+// Pair counts from which the lane join runs in two passes: the first gains a third of its time per pair,
+// the second costs its longest searches' time again.  In one and two passes, 7 M pairs (300,000
+// LogNormal molecules x 306) take 2.04 and 1.72 ms, 3.4 M (150,000 x 300, plain) 1.55 and 1.93, 2 M (1 M x
+// 25) 0.48 and 0.75.  Where only a bound of the count is known, most of its pairs do not survive, and
+// counting every embedding makes the longest searches longer.
+constexpr uint64_t kJoinTwoPassPairs = 3ull << 21;
+constexpr uint64_t kJoinTwoPassBound = 1ull << 24;
 constexpr uint32_t kJoinDeepChunk = 128;            // pairs a wavefront claims at a time of the deep queries' list
 constexpr uint32_t kJoinRefill = 24;                // idle lanes that make a wavefront hand out new pairs
 
@@ -682,7 +688,7 @@ hipError_t launch_join_passes(hipStream_t s, const GraphDev& q, const GraphDev& 
     return chunk ? chunk : static_cast<uint32_t>(std::min<uint64_t>(1024, std::max<uint64_t>(64, P / (blocks * claims) / 64 * 64)));
   };
   if (wide) k_list_wide<<<(d.G + 256 * kListTurns - 1) / (256 * kListTurns), 256, 0, s>>>(d, offsets, P, wide, stats);
-  const bool two = deep && P >= kJoinTwoPassPairs;
+  const bool two = deep && P >= (P_dev || !FIND_FIRST ? kJoinTwoPassBound : kJoinTwoPassPairs);
   if (two) {
     const uint64_t blocks = join_blocks(sizeof(JoinLds<kJoinShallow, false, false>), P, num_cus, quarters);
     k_join_lanes<FIND_FIRST, Src, kJoinShallow, false><<<static_cast<unsigned>(blocks), 64, 0, s>>>(

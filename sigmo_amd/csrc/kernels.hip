@@ -666,8 +666,9 @@ __global__ __launch_bounds__(kBitsBlock) void k_filter_refine(const uint8_t* __r
 
 constexpr uint32_t kStripNodes = 2048;    // data nodes of one strip: 64 lanes of 32
 constexpr uint32_t kLevelQuads = 8;  // words of a query node's planes: its label and up to 31 requirements
+constexpr uint32_t kLevelFars = 32;  // far tokens: likewise, when none has a plane
 // words per query node: its quads, their number | far tokens << 8, and the far tokens
-constexpr uint32_t kLevelTokens = kLevelQuads + 1 + 32;
+constexpr uint32_t kLevelTokens = kLevelQuads + 1 + kLevelFars;
 constexpr uint32_t kFarLabel = 1u << 31;
 constexpr uint32_t kLevelWaves = 16;      // wavefronts per block of the sweep
 
@@ -728,8 +729,9 @@ __global__ __launch_bounds__(kSigBlock) void k_sig_levels(GraphDev g, uint32_t R
 // Query signatures of levels 1..R as planes of the sweep's LDS (slot_planes), a wavefront per query
 // graph (<= 32 nodes) and a lane per node: its label's plane, then one for each nonzero count of label
 // slots.label[u] at level r+1 (at most 31: each needs a node of its own).  Without a plane are a
-// label >= 16, its far token kFarLabel | label, and counts over 4 (over 8 of the frequent label) or of
-// a slot past the first `staged`, (u*R + r) << 8 | count.
+// label >= 16 or past the first `staged` slots, its far token kFarLabel | label beside the plane of
+// every position, and counts over 4 (over 8 of the frequent label) or of a slot past `staged`,
+// (u*R + r) << 8 | count.
 __global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, LabelSlots slots, uint32_t staged, uint32_t* __restrict__ tok) {
   __shared__ uint64_t fold_all[4][kWave];
   const uint32_t lane = static_cast<uint32_t>(lane_id());
@@ -759,11 +761,13 @@ __global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, La
     for (uint32_t u = 0; u < static_cast<uint32_t>(slots.count) && next; ++u) {
       uint32_t c = static_cast<uint32_t>(__popcll(next & q.lmask[static_cast<uint64_t>(g) * 16 + slots.label[u]]));
       c = c < 15 ? c : 15;
-      if (!c || near + fars >= kLevelTokens - kLevelQuads - 1) continue;  // never more: a requirement per other node
-      const bool frequent = static_cast<int>(u) == slots.frequent;
-      if (u < staged && c <= kNearCount) planes[near++] = static_cast<uint8_t>(u * SP + 4 * r + c - 1);
-      else if (u < staged && frequent && c <= 8) planes[near++] = static_cast<uint8_t>(staged * SP + 4 * r + c - 5);
-      else far[fars++] = ((u * R + r) << 8) | c;
+      if (!c) continue;
+      // either place holds the label and a requirement per other node
+      if (u < staged && (c <= kNearCount || (c <= 8 && static_cast<int>(u) == slots.frequent))) {
+        if (near < 4 * kLevelQuads) planes[near++] = static_cast<uint8_t>((c <= kNearCount ? u * SP + c - 1 : staged * SP + c - 5) + 4 * r);
+      } else if (fars < kLevelFars) {
+        far[fars++] = ((u * R + r) << 8) | c;
+      }
     }
   }
   const uint32_t quads = (near + 3) / 4;

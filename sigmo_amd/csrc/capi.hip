@@ -1685,6 +1685,8 @@ int sigmo_pipeline_replay(sigmo_pipeline* p, sigmo_pipeline_result* result) {
     return sigmo_err::set(SIGMO_ERR_INVALID, "the captured graph no longer matches the data (pair counts changed): capture again");
   }
   if (st[3]) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "a per-pair match count exceeded int32");
+  p->gm->P = p->graph_P;  // the arrays hold this replay's pairs, whatever an execute in between left there
+  p->gm->deferred = false;
   p->has_counts = true;
   result->num_matches = st[0];
   result->gmcr_pairs = p->graph_P;

@@ -1,0 +1,36 @@
+"""A captured pipeline replayed after executes of other level counts: results and pairs are the captured
+run's.  Whole numbers: equality."""
+import numpy as np
+import pytest
+
+from sigmo_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(a, b):
+    for x, y in zip(a, b):
+        np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("captured,executed", [(6, 2), (6, 9), (9, 6)])
+def test_replay_after_an_execute_of_other_levels(ctx, captured, executed):
+    qd = capi.DeviceGraph(ctx, capi.HostGraphs.queries(31, 40, 4, 12, capi.SIZE_NORMAL))
+    dd = capi.DeviceGraph(ctx, capi.HostGraphs.molecules(31, 3001, capi.SIZE_NORMAL))
+    p, fresh = capi.Pipeline(ctx, qd, dd), capi.Pipeline(ctx, qd, dd)
+    want = {}
+    for R in (captured, executed):
+        r = fresh.execute(R, True)
+        want[R] = r["num_matches"], r["gmcr_pairs"], fresh.pairs()
+    p.capture(captured, True)
+    for R in (executed, executed):
+        p.execute(R, True)
+        if R == executed:
+            _same(p.pairs(), want[R][2])
+        for _ in range(2):
+            r = p.replay()
+            assert (r["num_matches"], r["gmcr_pairs"]) == want[captured][:2]
+            _same(p.pairs(), want[captured][2])
+    p.capture(executed, True)
+    assert p.replay()["num_matches"] == want[executed][0]
+    _same(p.pairs(), want[executed][2])

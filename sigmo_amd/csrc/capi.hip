@@ -1476,11 +1476,15 @@ struct sigmo_pipeline {
   hipGraphExec_t graph_exec = nullptr;
   uint64_t* replay_host = nullptr;  // pinned: the GMCR total of the last replay
   uint64_t graph_P = 0, graph_nw = 0;
+  const uint8_t* graph_lvl = nullptr;   // the level planes that it uses ..
+  uint8_t* kept_lvl = nullptr;          // .. once an execute of more levels has outgrown them
   void drop_graph() {
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
     if (graph) (void)hipGraphDestroy(graph);
     graph_exec = nullptr;
     graph = nullptr;
+    graph_lvl = nullptr;
+    dev_free(kept_lvl);
   }
   ~sigmo_pipeline() {
     drop_graph();
@@ -1517,6 +1521,11 @@ bool pipeline_levels(sigmo_pipeline* p, uint32_t R) {
   if (R < 1 || R > 8 || slots.count < 1 || !p->q->N || !p->d->N) return false;
   const uint64_t lvl = sigmo_k::level_planes_bytes(std::max(p->sig->capD, p->d->N), R, static_cast<uint32_t>(slots.count));
   if (p->ctx->capturing) return p->lvl && p->qtok && p->cap_lvl >= lvl && p->cap_qtok >= sigmo_k::level_tokens(p->q->N);
+  // a captured graph's planes outlive their growth: its replays still write and read them
+  if (p->lvl && p->lvl == p->graph_lvl && p->cap_lvl < lvl) {
+    p->kept_lvl = p->lvl;
+    p->lvl = nullptr;
+  }
   return grow(&p->qtok, p->cap_qtok, sigmo_k::level_tokens(p->q->N)) == SIGMO_OK && grow(&p->lvl, p->cap_lvl, lvl) == SIGMO_OK;
 }
 
@@ -1659,6 +1668,7 @@ int sigmo_pipeline_capture(sigmo_pipeline* p, uint32_t refinement_steps, int fin
   SIGMO_HIP_TRY(hipGraphInstantiate(&p->graph_exec, g, nullptr, nullptr, 0));
   p->graph_P = p->gm->P;
   p->graph_nw = p->gm->last_wide;
+  p->graph_lvl = p->lvl;
   return SIGMO_OK;
 }
 

@@ -1,5 +1,5 @@
-"""A captured pipeline replayed after executes of other level counts: results and pairs are the captured
-run's.  Whole numbers: equality."""
+"""A captured pipeline whose buffers a later execute outgrows: the level planes grow with the level count
+(the graph keeps its own).  Whole numbers: equality."""
 import numpy as np
 import pytest
 
@@ -13,7 +13,7 @@ def _same(a, b):
         np.testing.assert_array_equal(x, y)
 
 
-@pytest.mark.parametrize("captured,executed", [(6, 2), (6, 9), (9, 6)])
+@pytest.mark.parametrize("captured,executed", [(1, 6), (2, 8), (6, 2), (6, 9), (9, 6)])
 def test_replay_after_an_execute_of_other_levels(ctx, captured, executed):
     qd = capi.DeviceGraph(ctx, capi.HostGraphs.queries(31, 40, 4, 12, capi.SIZE_NORMAL))
     dd = capi.DeviceGraph(ctx, capi.HostGraphs.molecules(31, 3001, capi.SIZE_NORMAL))
@@ -23,7 +23,7 @@ def test_replay_after_an_execute_of_other_levels(ctx, captured, executed):
         r = fresh.execute(R, True)
         want[R] = r["num_matches"], r["gmcr_pairs"], fresh.pairs()
     p.capture(captured, True)
-    for R in (executed, executed):
+    for R in (executed, executed, 8):  # further growths, and none
         p.execute(R, True)
         if R == executed:
             _same(p.pairs(), want[R][2])

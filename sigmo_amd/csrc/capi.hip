@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -1478,6 +1479,10 @@ struct sigmo_pipeline {
   uint64_t graph_P = 0, graph_nw = 0;
   const uint8_t* graph_lvl = nullptr;   // the level planes that it uses ..
   uint8_t* kept_lvl = nullptr;          // .. once an execute of more levels has outgrown them
+  std::array<const void*, 9> graph_gm;  // and the result arrays, which grow with the pairs found
+  std::array<const void*, 9> gm_arrays() const {
+    return {gm->offsets, gm->counts, gm->indices, gm->pair_graph, gm->pair_bits, gm->scan_tmp, gm->pair_counts, gm->wide_pairs, gm->deep_pairs};
+  }
   void drop_graph() {
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -1669,6 +1674,7 @@ int sigmo_pipeline_capture(sigmo_pipeline* p, uint32_t refinement_steps, int fin
   p->graph_P = p->gm->P;
   p->graph_nw = p->gm->last_wide;
   p->graph_lvl = p->lvl;
+  p->graph_gm = p->gm_arrays();
   return SIGMO_OK;
 }
 
@@ -1677,6 +1683,10 @@ int sigmo_pipeline_replay(sigmo_pipeline* p, sigmo_pipeline_result* result) {
   if (!p->graph_exec) return sigmo_err::set(SIGMO_ERR_INVALID, "no captured graph (call sigmo_pipeline_capture)");
   sigmo_ctx* ctx = p->ctx;
   SIGMO_TRY(bind(ctx));
+  if (p->gm_arrays() != p->graph_gm) {  // an execute that found more pairs has freed arrays that the graph writes
+    p->drop_graph();
+    return sigmo_err::set(SIGMO_ERR_INVALID, "the captured graph's result arrays were reallocated by a later execute: capture again");
+  }
   std::memset(result, 0, sizeof(*result));
   hipEvent_t t0, t1;
   SIGMO_TRY(ctx->event(&t0));

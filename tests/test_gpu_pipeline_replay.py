@@ -1,5 +1,6 @@
 """A captured pipeline whose buffers a later execute outgrows: the level planes grow with the level count
-(the graph keeps its own).  Whole numbers: equality."""
+(the graph keeps its own), the result arrays with the pairs found (the replay is refused).  Whole
+numbers: equality."""
 import numpy as np
 import pytest
 
@@ -34,3 +35,21 @@ def test_replay_after_an_execute_of_other_levels(ctx, captured, executed):
     p.capture(executed, True)
     assert p.replay()["num_matches"] == want[executed][0]
     _same(p.pairs(), want[executed][2])
+
+
+def test_replay_is_refused_once_its_arrays_are_gone(ctx):
+    # molecules of more than 64 nodes: arrays sized by the pairs found
+    qd = capi.DeviceGraph(ctx, capi.HostGraphs.queries(32, 60, 4, 16, capi.SIZE_LOGNORMAL))
+    dd = capi.DeviceGraph(ctx, capi.HostGraphs.molecules(32, 2000, capi.SIZE_LOGNORMAL))
+    p = capi.Pipeline(ctx, qd, dd)
+    p.capture(6, True)
+    first = p.replay()
+    pairs = p.pairs()
+    more = p.execute(0, True)
+    assert more["gmcr_pairs"] > 1.5 * first["gmcr_pairs"]
+    for _ in range(2):
+        with pytest.raises(capi.SigmoError, match="capture"):
+            p.replay()
+    p.capture(6, True)
+    assert p.replay()["num_matches"] == first["num_matches"]
+    _same(p.pairs(), pairs)

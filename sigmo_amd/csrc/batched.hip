@@ -702,7 +702,7 @@ struct GroupArgs {
   uint64_t arena_cap;
   unsigned long long* surv;      // [Gd][W] in: the pre-test's pairs; out: bit qg of row m = the pair survives GMCR
   uint4* blocks;                 // [group * Gq + g] where the masks of group and query graph are: pair_block
-  unsigned long long* counters;  // [1] arena words claimed past the wavefronts' first chunks, [2] item cursor, [3] overflow
+  unsigned long long* counters;  // [1] arena words claimed past the wavefronts' first chunks, [2] item cursor, [3] overflow, [4] k_surv_words
   unsigned long long* stats;     // kGroupStatSlots x 16: [0] node evaluations, [1] their live lanes, [2] pre-tested pairs
 };
 
@@ -748,8 +748,8 @@ struct GroupState {
   uint64_t sums = 0;
 };
 
-// One group of a class against the wavefront's share of the query graphs.
-template <int CLS>
+// One group of a class against the wavefront's share of the query graphs.  COMPACT: see k_pair_group.
+template <int CLS, bool COMPACT>
 __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uint32_t part, uint32_t wave, uint32_t* planes_lds, GroupState& st) {
   const uint32_t lane = static_cast<uint32_t>(lane_id()), lane4 = lane * 4;
   const uint32_t R = a.R, SP = slot_planes(R);
@@ -872,8 +872,6 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
         st.left = c.chunk;
       }
       const uint64_t base0 = st.next, base = base0 + static_cast<uint64_t>(__popcll(am & below)) * pw;
-      st.next += cnt * pw;
-      st.left -= cnt * pw;
       const bool room = st.next + st.left <= a.arena_cap;
 
       // The quads are decoded once, each lane its own: four planes by their bytes.  A node's mask is the
@@ -969,8 +967,26 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
           }
         }
         if (i + 1 < k) continue;
+        uint64_t lanes = am;  // whose blocks these are
+        uint32_t taken = cnt * pw;
+        if constexpr (COMPACT) {
+          lanes &= alive;
+          taken = static_cast<uint32_t>(__popcll(lanes)) * pw;
+          const uint64_t to = base0 + static_cast<uint64_t>(__popcll(lanes & below)) * pw;
+          // a block moves to where an earlier molecule's is or was; a step loads 16 bytes of every block before
+          // it stores them, each at the same place in its block, so none is lost
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+          if (store && to != base)
+#pragma unroll 1
+            for (uint32_t u = h; u < pw / 2; u += 1u << CLS) {
+              const uint4 v = reinterpret_cast<const uint4*>(a.arena + base)[u];
+              reinterpret_cast<uint4*>(a.arena + to)[u] = v;
+            }
+        }
         if (lane == 0)
-          group_args().blocks[group * a.Gq + g] = make_uint4(static_cast<uint32_t>(base0), pw, static_cast<uint32_t>(am), static_cast<uint32_t>(am >> 32));
+          group_args().blocks[group * a.Gq + g] = make_uint4(static_cast<uint32_t>(base0), pw, static_cast<uint32_t>(lanes), static_cast<uint32_t>(lanes >> 32));
+        st.next += taken;  // without survivors the next graph takes the same words
+        st.left -= taken;
         break;
       }
       nodes += i + 1;
@@ -1009,7 +1025,9 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
 // CU's 24 wavefronts and bounds the kernel, at 60% issue.
 //
 // Node masks go straight to the pairs' arena blocks, which a wavefront takes from a chunk of its own;
-// pairs that die clear their pre-test bits.  80 registers: six wavefronts per SIMD (20 waves with
+// pairs that die clear their pre-test bits, and where none of a group survives the next query graph
+// takes the blocks.  With COMPACT (a batch that size_arena moved to it) the survivors' blocks move
+// together, so that the arena holds no others.  80 registers: six wavefronts per SIMD (20 waves with
 // 4-wavefront blocks: 8.1 instead of 6.8 ms).  With 64-bit masks for every molecule and an offset
 // per pair, stored 4 KB apart, 174 M writes went to memory instead of 73 M.
 //
@@ -1017,6 +1035,7 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
 // this: 2,000 molecules x 20 query graphs 219, 13 and 10 us (three serial chains of ~100 us at
 // first), 100,000 x 100 475, 118 and 73 us, 1 M x 25 1,242, 353 and 294 us, 1 M x 1,000 10.7, 5.6 and
 // 3.2 ms.
+template <bool COMPACT>
 __global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a) {
   extern __shared__ uint32_t planes_lds[];
   GroupCounters* ctr = reinterpret_cast<GroupCounters*>(reinterpret_cast<uint4*>(planes_lds + (a.slots + 1) * slot_planes(a.R) * kWave) + kGroupWaves * kWave);
@@ -1033,9 +1052,9 @@ __global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a)
   for (uint32_t item = blockIdx.x; item < items;) {
     const uint32_t part = item & (a.parts - 1), grp = item / a.parts;
     const uint32_t g0 = a.order.groups(0), g1 = a.order.groups(1);
-    if (grp < g0) group_item<0>(a, grp, part, wave, planes_lds, st);
-    else if (grp < g0 + g1) group_item<1>(a, grp - g0, part, wave, planes_lds, st);
-    else group_item<2>(a, grp - g0 - g1, part, wave, planes_lds, st);
+    if (grp < g0) group_item<0, COMPACT>(a, grp, part, wave, planes_lds, st);
+    else if (grp < g0 + g1) group_item<1, COMPACT>(a, grp - g0, part, wave, planes_lds, st);
+    else group_item<2, COMPACT>(a, grp - g0 - g1, part, wave, planes_lds, st);
     item += gridDim.x;
     if (item < fixed) continue;
     if (gridDim.x >= items) break;
@@ -1044,6 +1063,23 @@ __global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a)
     item = uniform32(ctr->next_item);
   }
   if (lane_id() < 3 && st.sums) atomicAdd(&a.stats[(blockIdx.x % kGroupStatSlots) * 16 + lane_id()], static_cast<unsigned long long>(st.sums));
+}
+
+// The arena words of the pairs that survive (a thread per molecule of the width-class order).
+__global__ __launch_bounds__(256) void k_surv_words(GroupOrder order, uint32_t G, uint32_t W, const MolInfo* __restrict__ minfo,
+                                                    const QueryInfo* __restrict__ qinfo, const unsigned long long* __restrict__ surv,
+                                                    unsigned long long* __restrict__ out) {
+  const uint64_t c = blockIdx.x * 256ull + threadIdx.x;
+  uint64_t words = 0;
+  if (c < G) {
+    const int cls = c < order.count[0] ? 0 : (c < static_cast<uint64_t>(order.count[0]) + order.count[1] ? 1 : 2);
+    const uint64_t m = minfo[c].m;
+    for (uint32_t w = 0; w < W; ++w)
+      for (uint64_t x = surv[m * W + w]; x; x &= x - 1) words += pair_words(qinfo[w * kWave + static_cast<uint32_t>(__builtin_ctzll(x))].k, cls);
+  }
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) words += static_cast<uint64_t>(__shfl_xor(static_cast<unsigned long long>(words), o));
+  if (lane_id() == 0 && words) atomicAdd(out, static_cast<unsigned long long>(words));
 }
 
 // Survivors per molecule: the popcount of its row of the survival bitmask.
@@ -1402,6 +1438,7 @@ struct sigmo_batch {
   // pair evaluation
   uint64_t* arena = nullptr;
   uint64_t cap_arena = 0;
+  bool compact = false;  // the arena keeps only the survivors' masks (size_arena)
   unsigned long long* surv = nullptr;
   uint64_t cap_surv = 0;
   uint4* blocks = nullptr;
@@ -1810,7 +1847,7 @@ hipError_t launch_filter(sigmo_batch* b, const RunShape& L, hipStream_t s) {
   a.blocks = b->blocks;
   a.counters = b->counters;
   a.stats = b->counters + 16;
-  hipLaunchKernelGGL(sigmo_k::k_pair_group, dim3(L.group_blocks), dim3(sigmo_k::kGroupWaves * 64),
+  hipLaunchKernelGGL(b->compact ? sigmo_k::k_pair_group<true> : sigmo_k::k_pair_group<false>, dim3(L.group_blocks), dim3(sigmo_k::kGroupWaves * 64),
                      sigmo_k::group_lds_bytes(L.group_slots, L.R), s, a);
   return hipGetLastError();
 }
@@ -1824,6 +1861,31 @@ uint64_t read_counters(uint64_t first_chunks, const unsigned long long* cnt, sig
     res->filter_scans += cnt[16 + 16 * i + 2];
   }
   return cnt[1] + first_chunks;
+}
+
+// What the arena is to hold after an overflow, given the run's demand.  Where the pre-tested pairs took
+// more than twice what the survivors need (labels >= 16 and wildcards leave the pre-test little to go
+// by), the batch goes over to the form that keeps only these, for this and later runs: everywhere, it
+// would take 4.05 instead of 3.53 ms for 1 M molecules x 1,000 query graphs.
+int size_arena(sigmo_batch* b, const RunShape& L, hipStream_t s, uint64_t demand, uint64_t slack, uint64_t& want) {
+  bool larger = true;
+  if (!b->compact) {
+    const sigmo_db* db = b->db;
+    unsigned long long words = 0;
+    hipLaunchKernelGGL(sigmo_k::k_surv_words, dim3((L.Gd + 255) / 256), dim3(256), 0, s, db->order, L.Gd, L.W, db->minfo, b->qinfo, b->surv,
+                       b->counters + 4);
+    BATCH_HIP_TRY(hipGetLastError());
+    BATCH_HIP_TRY(hipMemcpyAsync(&words, b->counters + 4, sizeof(words), hipMemcpyDeviceToHost, s));
+    BATCH_HIP_TRY(hipStreamSynchronize(s));
+    if (demand > 2 * words + slack) {
+      b->compact = true;
+      demand = 2 * words;  // a wavefront may leave up to half of each chunk, of at least two groups' largest blocks
+      larger = demand + slack > b->cap_arena;
+    }
+  }
+  // the claim order (and so the space left unused at chunk ends) varies between runs, hence the 1/8 margin
+  if (larger) want = std::max<uint64_t>(want + 1, demand + demand / 8 + slack);
+  return SIGMO_OK;
 }
 
 // GMCR: survivors per molecule and their exclusive scan (total in b->total).
@@ -1906,8 +1968,8 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
     BATCH_TRY(ctx_timed(b->ctx, 0, 0, 0.0, false, &tok));
   }
   // arena capacity: start from 1/8 of the pairs (at most 2^26) plus every wavefront's open chunk.
-  // On overflow the counter still holds the exact demand, so one replay with that size
-  // suffices; the capacity is kept for later runs.
+  // On overflow the counter still holds the demand, so one replay with that size, or of the
+  // survivors' masks alone, suffices; the capacity is kept for later runs.
   const double mean_k = Gq ? double(L.ksum) / Gq : 0.0;
   // every wavefront starts with a chunk and may leave its last one's tail unused
   const uint64_t slack_arena = 2 * L.first_chunks;
@@ -1962,7 +2024,7 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
       res->join_wave_steps = stats_host[7];
       return SIGMO_OK;
     }
-    want_arena = std::max<uint64_t>(want_arena + 1, demand + demand / 8 + slack_arena);  // overflowed: size and repeat
+    BATCH_TRY(size_arena(b, L, s, demand, slack_arena, want_arena));  // overflowed: size and repeat
     res->arena_repeats = 1;
   }
   for (int attempt = 0; attempt < 4; ++attempt) {
@@ -1984,9 +2046,7 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
     if (!cnt[3]) break;
     if (attempt == 3) return sigmo_err::set(SIGMO_ERR_NOMEM, "candidate arena overflowed repeatedly");
     res->arena_repeats++;
-    // replay with the demand just measured; the claim order (and so the space left unused at
-    // chunk ends) varies between runs, hence the 1/8 margin
-    if (demand > b->cap_arena) want_arena = std::max<uint64_t>(want_arena + 1, demand + demand / 8 + slack_arena);
+    BATCH_TRY(size_arena(b, L, s, demand, slack_arena, want_arena));
   }
   // canonical GMCR: count survivors per molecule, scan, scatter in (molecule, query graph) order
   void* tok = nullptr;

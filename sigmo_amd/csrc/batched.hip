@@ -1387,6 +1387,8 @@ using namespace sigmo_internal;
 
 // Pair spaces up to this size run with one host synchronisation (sigmo_batch_run).
 constexpr uint64_t kOneSyncPairs = 1ull << 25;
+// Arena offsets are 32-bit.
+constexpr uint64_t kMaxArenaWords = (1ull << 32) - 4;
 // A run's device counters: 16 words, then the group evaluation's statistics.
 constexpr uint64_t kCounterWords = 16 + 16 * sigmo_k::kGroupStatSlots;
 
@@ -1785,10 +1787,11 @@ int shape_run(const sigmo_batch* b, const sigmo_graph* query, int cus, RunShape&
   if (b->tune.filter_blocks_per_cu) per_cu = std::min<uint64_t>(per_cu, b->tune.filter_blocks_per_cu);
   L.group_blocks = static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(items, ucus * per_cu)));
   // a wavefront's arena chunk holds the largest query graph for a whole group (1,024 words) and, for
-  // many pairs, more: claims meet on one address
+  // many pairs, more: claims meet on one address.  Every wavefront has one and may leave another's tail:
+  // at most 1.6 GB for 6,144 wavefronts
   const uint64_t waves = uint64_t(L.group_blocks) * sigmo_k::kGroupWaves;
   uint64_t chunk = 2048;
-  while (chunk < 32768 && chunk * waves * 4 < L.pairs) chunk *= 2;
+  while (chunk < 16384 && chunk * waves * 4 < L.pairs) chunk *= 2;
   L.group_chunk = static_cast<uint32_t>(chunk);
   L.first_chunks = waves * chunk;
   return SIGMO_OK;
@@ -1884,7 +1887,10 @@ int size_arena(sigmo_batch* b, const RunShape& L, hipStream_t s, uint64_t demand
     }
   }
   // the claim order (and so the space left unused at chunk ends) varies between runs, hence the 1/8 margin
-  if (larger) want = std::max<uint64_t>(want + 1, demand + demand / 8 + slack);
+  if (larger) {
+    if (demand > kMaxArenaWords || want >= kMaxArenaWords) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "candidate arena exceeds 2^32 words");
+    want = std::min(kMaxArenaWords, std::max<uint64_t>(want + 1, demand + demand / 8 + slack));
+  }
   return SIGMO_OK;
 }
 
@@ -1975,7 +1981,7 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
   const uint64_t slack_arena = 2 * L.first_chunks;
   const uint64_t guess = std::min<uint64_t>(std::max<uint64_t>(L.pairs / 8, 1 << 16), 1ull << 26);
   uint64_t want_arena = static_cast<uint64_t>(double(guess) * (mean_k + 1.0) * (db->num_wide ? 2.0 : 1.0)) + slack_arena;
-  want_arena = std::max(want_arena, b->cap_arena);
+  want_arena = std::max(std::min(want_arena, kMaxArenaWords), b->cap_arena);
   // One synchronisation per run once an earlier run has sized the arena: with no molecule of
   // more than 64 nodes and a pair space of at most kOneSyncPairs, the GMCR arrays are sized for
   // every pair, the join reads the pair count on the device, and the filter's counters and the
@@ -2029,7 +2035,6 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
   }
   for (int attempt = 0; attempt < 4; ++attempt) {
     BATCH_TRY(b->grow(&b->arena, b->cap_arena, want_arena));
-    if (b->cap_arena >= (1ull << 32)) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "candidate arena exceeds 2^32 words");
     // algorithmic reads: the data side once per run -- a label byte and R level signatures per
     // data node, (1 + 8R) D -- plus the query side; writes are added once they are known.
     const double reads = (1.0 + 8.0 * R) * double(L.dd.N) + double(L.qd.N) * (1.0 + 2.0 * 16.0 * R) + double(Gq) * (4.0 + 8.0 * R);

@@ -70,3 +70,20 @@ def test_demand_follows_the_survivors(ctx, n, every):
         slack = 2 * 2048 * 8 * 256  # 256 CUs x 8 wavefronts, two chunks each
         first = max(len(qs) * len(ms) // 8, 1 << 16) * (np.mean([len(lab) for lab, _ in qs]) + 1) * (2 if n > 64 else 1)
         assert words <= max(first, 2 * own) + slack, (words, own)
+
+
+def test_first_sizing_near_the_largest_arena(ctx):
+    # 2^29 pairs and one molecule of more than 64 nodes: the guess for 30-node queries is 4.16 G words of the
+    # 2^32 that offsets reach, and the wavefronts' chunks come on top.  No pair passes the pre-test.
+    rng = np.random.default_rng(0)
+    path = [(i, i + 1) for i in range(29)]
+    qh = capi.HostGraphs.from_edge_lists([([int(x) for x in rng.integers(0, 16, 30)], path) for _ in range(4100)])
+    ones = 131_071
+    dh = capi.HostGraphs.from_arrays(np.arange(ones + 1), np.zeros(ones + 1), np.zeros(0), rng.integers(0, 16, ones))
+    dh = dh.concat(capi.HostGraphs.from_edge_lists([([8] * 65, path)]))
+    dd = capi.DeviceGraph(ctx, dh)
+    batch = capi.Batch(ctx, capi.Database(ctx, dd, 2))
+    r = batch.run(capi.DeviceGraph(ctx, qh), True)
+    assert r["gmcr_pairs"] == 0 and r["arena_repeats"] == 0
+    few = batch.run(capi.DeviceGraph(ctx, capi.HostGraphs.from_edge_lists([([8, 8], [(0, 1)])])), True)
+    assert few["gmcr_pairs"] == 1 and few["matched_pairs"] == 1

@@ -10,10 +10,10 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
-#include <thread>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/sigmo_hip.h"
@@ -68,12 +68,12 @@ struct ReadBack {
   static constexpr size_t kHalf = 2u << 20;
   std::mutex mu;
   unsigned char* buf = nullptr;
-  hipEvent_t done[2] = {nullptr, nullptr};
+  hipEvent_t done[2] = {nullptr, nullptr}, begun = nullptr;
 
   hipError_t create() {
     hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&buf), 2 * kHalf, hipHostMallocDefault);
-    for (hipEvent_t& d : done)
-      if (e == hipSuccess) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
+    for (hipEvent_t* d : {&done[0], &done[1], &begun})
+      if (e == hipSuccess) e = hipEventCreateWithFlags(d, hipEventDisableTiming);
     return e;
   }
   // The parts of a half: where they go.
@@ -89,28 +89,15 @@ struct ReadBack {
     }
   }
   // Copies the arrays (at most kGatherParts, whole 4-byte words at 16-byte boundaries) and waits for them
-  // and the stream's work.
-  hipError_t run(hipStream_t s, const sigmo_k::HostCopy* c, int n) {
+  // and the stream's work.  The second thread spins between halves: behind `queued` work (a join) it
+  // starts when that has ended, while the first half fills, and not with the call.
+  hipError_t run(hipStream_t s, const sigmo_k::HostCopy* c, int n, bool queued = false) {
     std::lock_guard<std::mutex> lock(mu);
     size_t total = 0;
     for (int i = 0; i < n; ++i) total += c[i].bytes;
     Half halves[2];
     std::atomic<int> ready{0}, copied{0};  // halves handed to the second thread and copied by it; -1: no more
     std::thread second;
-    if (total > kHalf) {
-      try {
-        second = std::thread([&] {
-          for (int turn = 0;; ++turn) {
-            int r;
-            while ((r = ready.load(std::memory_order_acquire)) == turn) std::this_thread::yield();
-            if (r < 0) return;
-            copy_out(halves[turn & 1], turn & 1, 1, 2);
-            copied.store(turn + 1, std::memory_order_release);
-          }
-        });
-      } catch (const std::system_error&) {  // no thread to be had: this one copies all
-      }
-    }
     int turn = 0;  // halves copied out
     auto out = [&] {
       const int half = turn++ & 1;
@@ -119,7 +106,23 @@ struct ReadBack {
       copy_out(halves[half], half, 0, 2);
       while (copied.load(std::memory_order_acquire) != turn) std::this_thread::yield();
     };
-    hipError_t e = hipSuccess;
+    auto start_second = [&] {
+      try {
+        second = std::thread([&] {
+          for (int t = 0;; ++t) {
+            int r;
+            while ((r = ready.load(std::memory_order_acquire)) == t) std::this_thread::yield();
+            if (r < 0) return;
+            copy_out(halves[t & 1], t & 1, 1, 2);
+            copied.store(t + 1, std::memory_order_release);
+          }
+        });
+      } catch (const std::exception&) {  // no thread to be had: this one copies all
+      }
+    };
+    queued = queued && total > kHalf;
+    hipError_t e = queued ? hipEventRecord(begun, s) : hipSuccess;
+    if (!queued && total > kHalf) start_second();
     int filled = 0, i = 0;
     size_t from = 0;
     while (e == hipSuccess && i < n) {
@@ -144,6 +147,10 @@ struct ReadBack {
       }
       e = sigmo_k::gather(s, h.parts, buf + (filled & 1) * kHalf);
       if (e == hipSuccess) e = hipEventRecord(done[filled & 1], s);
+      if (e == hipSuccess && queued && filled == 0) {
+        e = hipEventSynchronize(begun);
+        if (e == hipSuccess) start_second();
+      }
       if (e == hipSuccess && filled++ > turn) {  // the half before
         e = hipEventSynchronize(done[turn & 1]);
         if (e == hipSuccess) out();
@@ -160,7 +167,7 @@ struct ReadBack {
   }
   ~ReadBack() {
     if (buf) (void)hipHostFree(buf);
-    for (hipEvent_t e : done)
+    for (hipEvent_t e : {done[0], done[1], begun})
       if (e) (void)hipEventDestroy(e);
   }
 };
@@ -1393,7 +1400,7 @@ int sigmo_join(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_graph* data
   if (ctx->capturing) return SIGMO_OK;  // the replay reads the pinned mirror after the graph
   SIGMO_TRY(gmcr_resolve(mm, s));  // the exact pair count, before any per-pair copy
   const sigmo_k::HostCopy out = {per_pair_counts, mm->pair_counts, per_pair_counts ? m->P * 4 : 0};
-  SIGMO_HIP_TRY(ctx->back.run(s, &out, 1));
+  SIGMO_HIP_TRY(ctx->back.run(s, &out, 1, true));
   mm->last_wide = wide ? ctx->stats_host[5] : 0;
   if (ctx->stats_host[3]) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "a per-pair match count exceeded int32");
   if (num_matches) *num_matches += ctx->stats_host[0];
@@ -1420,7 +1427,7 @@ int sigmo_join_wildcard(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_gr
   SIGMO_TRY(ps.close());
   SIGMO_HIP_TRY(hipMemcpyAsync(ctx->stats_host, ctx->stats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   const sigmo_k::HostCopy out = {per_pair_counts, mm->pair_counts, per_pair_counts ? m->P * 4 : 0};
-  SIGMO_HIP_TRY(ctx->back.run(s, &out, 1));
+  SIGMO_HIP_TRY(ctx->back.run(s, &out, 1, true));
   if (ctx->stats_host[3]) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "a per-pair match count exceeded int32");
   if (num_matches) *num_matches += ctx->stats_host[0];
   return SIGMO_OK;

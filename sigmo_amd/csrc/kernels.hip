@@ -751,6 +751,7 @@ __global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, La
     if (slots.label[u] == label) own = u * SP + 4 * R;
   planes[0] = static_cast<uint8_t>(own);
   if (own == every && label != 255u) far[fars++] = kFarLabel | label;
+  const uint32_t most = near + fars + 31;  // either place has room for as many beside the label
   uint64_t ball = 1ull << lane, frontier = ball;
   for (uint32_t r = 0; r < R && frontier; ++r) {
     uint64_t next = 0;
@@ -761,13 +762,11 @@ __global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, La
     for (uint32_t u = 0; u < static_cast<uint32_t>(slots.count) && next; ++u) {
       uint32_t c = static_cast<uint32_t>(__popcll(next & q.lmask[static_cast<uint64_t>(g) * 16 + slots.label[u]]));
       c = c < 15 ? c : 15;
-      if (!c) continue;
-      // either place holds the label and a requirement per other node
-      if (u < staged && (c <= kNearCount || (c <= 8 && static_cast<int>(u) == slots.frequent))) {
-        if (near < 4 * kLevelQuads) planes[near++] = static_cast<uint8_t>((c <= kNearCount ? u * SP + c - 1 : staged * SP + c - 5) + 4 * r);
-      } else if (fars < kLevelFars) {
-        far[fars++] = ((u * R + r) << 8) | c;
-      }
+      if (!c || near + fars >= most) continue;  // never more: a requirement per other node
+      const bool frequent = static_cast<int>(u) == slots.frequent;
+      if (u < staged && c <= kNearCount) planes[near++] = static_cast<uint8_t>(u * SP + 4 * r + c - 1);
+      else if (u < staged && frequent && c <= 8) planes[near++] = static_cast<uint8_t>(staged * SP + 4 * r + c - 5);
+      else far[fars++] = ((u * R + r) << 8) | c;
     }
   }
   const uint32_t quads = (near + 3) / 4;

@@ -1577,6 +1577,14 @@ int pipeline_enqueue(sigmo_pipeline* p, uint32_t refinement_steps, int find_firs
       SIGMO_HIP_TRY(sigmo_k::filter_levels(ctx->stream, p->qtok, c->Q, p->d->lplanes, p->lvl, c->D, R, slots, c->bits, ctx->num_cus));
       SIGMO_TRY(ps.close());
     }
+    int st = gmcr_generate(ctx, p->gm, p->q, p->d, p->cand, true);
+    if (st == SIGMO_OK) st = sigmo_join(ctx, p->q, p->d, p->cand, p->gm, find_first, matches, nullptr);
+    if (st != SIGMO_ERR_NOMEM || ctx->capturing) return st;
+    // the planes, which the candidates no longer need, have left the pairs too little memory
+    SIGMO_HIP_TRY(hipStreamSynchronize(ctx->stream));
+    p->drop_graph();
+    dev_free(p->lvl);
+    p->cap_lvl = 0;
     SIGMO_TRY(gmcr_generate(ctx, p->gm, p->q, p->d, p->cand, true));
     return sigmo_join(ctx, p->q, p->d, p->cand, p->gm, find_first, matches, nullptr);
   }

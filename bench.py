@@ -364,7 +364,7 @@ def launched(kstats: dict) -> dict:
     for name, (once, more) in SHARED.items():
         n, ms, by = out.get(once, (0, 0.0, 0.0))
         m, more_ms, more_by = out.get(more, (0, 0.0, 0.0))
-        if n and m and abs(ms / n - more_ms / m) <= 1e-9 * ms / n and abs(by / n - more_by / m) <= 1e-9 * by / n:
+        if n and m and abs(ms / n - more_ms / m) <= 1e-6 * ms / n and abs(by / n - more_by / m) <= 1e-6 * by / n:  # times are 32-bit
             out[name] = (n, ms + more_ms, by + more_by)
             del out[once], out[more]
     return out

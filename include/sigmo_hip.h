@@ -257,18 +257,18 @@ typedef struct sigmo_pipeline_result {
   uint64_t join_wave_steps; /* join loop iterations summed over wavefronts (an iteration takes up to three DFS steps of each lane) */
 } sigmo_pipeline_result;
 /* Runs gen(D), gen(Q), filter, R x {refsig(D,r), refsig(Q,r), refine}, GMCR, join on
- * device-resident graphs, with one launch per phase; allocates and frees its buffers.  With
- * 1 <= R <= 8 (and memory for every level's signature planes) each side's signatures of all levels
- * are one launch, and the filter with all refinements is another, which writes each bitset word
- * once (the same bits: the filter reads no signatures, the signature passes no candidates, and the
- * tests AND); otherwise the filter is fused with the first refine.  sigmo_kernel_stats counts a
- * launch that does several's work once for each -- one SIG_GENERATE and R SIG_REFINE, one FILTER and
- * R - 1 REFINE -- with its time and bytes shared out equally. */
+ * device-resident graphs by the calls above, a launch each; allocates and frees its buffers. */
 int sigmo_pipeline_run(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_graph* data, uint32_t refinement_steps,
                        int find_first, sigmo_pipeline_result* result);
 
 /* The same plain pipeline with its signature/candidate/GMCR buffers allocated once
- * (the reference's setup phase, sigmo.cpp:75-91) and reused by every execute. */
+ * (the reference's setup phase, sigmo.cpp:75-91) and reused by every execute.  With 1 <= R <= 8 (and
+ * memory for every level's signature planes) each side's signatures of all levels are one launch, and
+ * the filter with all refinements is another, which writes each bitset word once (the same bits: the
+ * filter reads no signatures, the signature passes no candidates, and the tests AND); otherwise the
+ * filter is fused with the first refine.  sigmo_kernel_stats counts a launch that does several's
+ * work once for each -- one SIG_GENERATE and R SIG_REFINE, one FILTER and R - 1 REFINE -- with its
+ * time and bytes shared out equally. */
 typedef struct sigmo_pipeline sigmo_pipeline;
 int sigmo_pipeline_create(sigmo_ctx* ctx, const sigmo_graph* query, const sigmo_graph* data, sigmo_pipeline** out);
 int sigmo_pipeline_execute(sigmo_pipeline* p, uint32_t refinement_steps, int find_first, sigmo_pipeline_result* result);
@@ -277,7 +277,9 @@ int sigmo_pipeline_execute(sigmo_pipeline* p, uint32_t refinement_steps, int fin
  * pair count of that execute, the join) as a graph; sigmo_pipeline_replay launches it.  Work per
  * replay is that of an execute; only host round trips and launch gaps go away.  The graphs must
  * stay allocated and unchanged; a replay whose pair counts differ from the capture's returns
- * SIGMO_ERR_INVALID.  phase_ms is not filled by a replay (total_ms is). */
+ * SIGMO_ERR_INVALID.  Executes in between (of any R) leave the captured graph as it is, unless they
+ * reallocate its result arrays (they found more pairs, and the arrays are sized by them): a replay
+ * then returns SIGMO_ERR_INVALID without launching.  phase_ms is not filled by a replay (total_ms is). */
 int sigmo_pipeline_capture(sigmo_pipeline* p, uint32_t refinement_steps, int find_first);
 int sigmo_pipeline_replay(sigmo_pipeline* p, sigmo_pipeline_result* result);
 /* Per-pair counts of the last execute or replay (GMCR order) and the GMCR arrays. */
@@ -344,7 +346,7 @@ int sigmo_batch_pairs(sigmo_batch* b, uint32_t* data_graph_offsets, uint64_t n_o
 int sigmo_batch_free(sigmo_batch* b);
 int sigmo_batch_set_tuning(sigmo_batch* b, const sigmo_batch_tuning* t);
 int sigmo_batch_get_tuning(const sigmo_batch* b, sigmo_batch_tuning* t);
-/* Autotuner: times sigmo_batch_run over a small grid of launch shapes (pair evaluation mode and shape first,
+/* Autotuner: times sigmo_batch_run over a small grid of launch shapes (the pair evaluation's blocks first,
  * then the join), each the best of `repeats` runs, and keeps the fastest in the batch.  Results
  * do not depend on the tuning.  *best_ms (nullable) receives the winner's time. */
 int sigmo_batch_autotune(sigmo_batch* b, const sigmo_graph* query, int find_first, uint32_t repeats, sigmo_batch_tuning* chosen,
@@ -369,9 +371,10 @@ typedef struct sigmo_request_stats {
 } sigmo_request_stats;
 int sigmo_batch_request_stats(sigmo_batch* b, const uint32_t* request_graph_offsets, uint32_t num_requests, sigmo_request_stats* out);
 /* Device bytes a run over `num_query_graphs` query graphs of `query_nodes` nodes in total is
- * expected to hold beyond the database: the per-pair offsets (4 B per query graph x molecule),
- * the survival bits and the first sizing of the candidate arena.  Runs whose survivors outgrow
- * the arena's first sizing grow it (and keep it for later runs). */
+ * expected to hold beyond the database: the group records (16 B per query graph and group of 16 to
+ * 64 molecules), the survival bits, the GMCR arrays and the first sizing of the candidate arena.  Not
+ * included: the arena chunks that the pair evaluation's wavefronts hold (at most 1.6 GB).  Runs whose
+ * survivors outgrow the arena's first sizing grow it (and keep it for later runs). */
 int sigmo_batch_workspace_bytes(const sigmo_batch* b, uint32_t num_query_graphs, uint64_t query_nodes, uint64_t* bytes);
 
 /* ---- serving loop (continuous batching over a resident database) ------------------------ */

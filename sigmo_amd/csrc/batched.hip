@@ -1022,19 +1022,19 @@ __device__ __forceinline__ void group_item(const GroupArgs& a, uint32_t grp, uin
 // takes one lane read, four byte permutations (the LDS addresses), four LDS reads and two ANDs, and
 // its label, end and padding tokens are planes like the others.  With each token a scalar of its own
 // a node took 75 scalar operations and 19 branches, now 45 and 12: one scalar unit serves the
-// CU's 24 wavefronts and bounds the kernel, at 60% issue.
+// CU's 24 wavefronts and bounds the kernel, at 69% of its issue slots (VALU 58%; 1 M x 1,000).
 //
 // Node masks go straight to the pairs' arena blocks, which a wavefront takes from a chunk of its own;
 // pairs that die clear their pre-test bits, and where none of a group survives the next query graph
 // takes the blocks.  With COMPACT (a batch that size_arena moved to it) the survivors' blocks move
-// together, so that the arena holds no others.  80 registers: six wavefronts per SIMD (20 waves with
-// 4-wavefront blocks: 8.1 instead of 6.8 ms).  With 64-bit masks for every molecule and an offset
-// per pair, stored 4 KB apart, 174 M writes went to memory instead of 73 M.
+// together, so that the arena holds no others.  At most 80 registers: six wavefronts per SIMD (20 waves
+// with 4-wavefront blocks: 8.1 instead of 6.8 ms).  With 64-bit masks for every molecule and an offset
+// per pair, stored 4 KB apart, 174 M writes went to memory instead of 68 M of 64 bytes (4.4 GB).
 //
 // Measured: a lane per pair and a launch per size class, wavefronts by groups with scalar tokens, and
 // this: 2,000 molecules x 20 query graphs 219, 13 and 10 us (three serial chains of ~100 us at
 // first), 100,000 x 100 475, 118 and 73 us, 1 M x 25 1,242, 353 and 294 us, 1 M x 1,000 10.7, 5.6 and
-// 3.2 ms.
+// 3.2 to 3.5 ms.
 template <bool COMPACT>
 __global__ __launch_bounds__(kGroupWaves * 64, 6) void k_pair_group(GroupArgs a) {
   extern __shared__ uint32_t planes_lds[];
@@ -1681,7 +1681,9 @@ int sigmo_batch_workspace_bytes(const sigmo_batch* b, uint32_t num_query_graphs,
   // for the pairs that survive otherwise, priced at the arena's guess of 1/8 of the pairs (plus
   // 4 B per pair for the list of wide-molecule pairs).  A run whose survivors exceed the guess
   // grows the arena and those arrays to the measured demand; a batch keeps its buffers at their
-  // largest size, so a caller admitting by this figure should leave room for that growth.
+  // largest size, so a caller admitting by this figure should leave room for that growth.  Not
+  // priced: the wavefronts' chunks (twice L.first_chunks words in shape_run, 4 MB to 1.6 GB by the
+  // pair space and the device) and the deep queries' list (4 B per GMCR pair).
   const uint64_t guess = std::min<uint64_t>(std::max<uint64_t>(pairs / 8, 1 << 16), 1ull << 26);
   const uint64_t arena_words = static_cast<uint64_t>(double(guess) * (mean_k + 1.0) * (db->num_wide ? 2.0 : 1.0));
   const bool one_sync = !db->num_wide && pairs && pairs <= kOneSyncPairs;
@@ -1868,8 +1870,8 @@ uint64_t read_counters(uint64_t first_chunks, const unsigned long long* cnt, sig
 
 // What the arena is to hold after an overflow, given the run's demand.  Where the pre-tested pairs took
 // more than twice what the survivors need (labels >= 16 and wildcards leave the pre-test little to go
-// by), the batch goes over to the form that keeps only these, for this and later runs: everywhere, it
-// would take 4.05 instead of 3.53 ms for 1 M molecules x 1,000 query graphs.
+// by), the batch goes over to the form that keeps only these, for this and later runs: in every run, it
+// would take 4.36 instead of 3.49 ms for 1 M molecules x 1,000 query graphs.
 int size_arena(sigmo_batch* b, const RunShape& L, hipStream_t s, uint64_t demand, uint64_t slack, uint64_t& want) {
   bool larger = true;
   if (!b->compact) {
@@ -2046,7 +2048,7 @@ int sigmo_batch_run(sigmo_batch* b, const sigmo_graph* query, int find_first, si
     BATCH_HIP_TRY(hipStreamSynchronize(s));
     const uint64_t demand = read_counters(L.first_chunks, cnt, res);
     if (res->filter_scans >= (1ull << 32)) return sigmo_err::set(SIGMO_ERR_OVERFLOW, "pre-tested pairs of one run exceed 2^32");
-    // writes: candidate masks, the survival bits and arena offsets
+    // writes: candidate masks and the survival bits
     ctx_add_bytes(b->ctx, SIGMO_KERNEL_PAIR_FILTER, double(demand) * 8.0 + double(Gd) * W * 8.0);
     if (!cnt[3]) break;
     if (attempt == 3) return sigmo_err::set(SIGMO_ERR_NOMEM, "candidate arena overflowed repeatedly");

@@ -122,10 +122,13 @@ constexpr int kJoinShallow = 8;
 constexpr int kJoinLevels = 12;
 constexpr int kJoinWideLevels = 7;  // two words per position: LDS as for kJoinLevels of one
 // Pair counts from which the lane join runs in two passes: the first gains a third of its time per pair,
-// the second costs its longest searches' time again.  In one and two passes, 7 M pairs (300,000
-// LogNormal molecules x 306) take 2.04 and 1.72 ms, 3.4 M (150,000 x 300, plain) 1.55 and 1.93, 2 M (1 M x
-// 25) 0.48 and 0.75.  Where only a bound of the count is known, most of its pairs do not survive, and
-// counting every embedding makes the longest searches longer.
+// the second costs its longest searches' time again.  The join in one and two passes, find-first,
+// 150,000 LogNormal molecules: 2.2 M pairs 0.51 and 0.80 ms, 3.6 M 0.90 and 1.11, 4.6 M 1.54 and 1.57, 6.4 M
+// 1.70 and 1.67, 10.3 M 2.56 and 2.19; 100,000 Normal molecules: 3.4 M 0.72 and 0.83, 6.1 M 1.11 and 1.19,
+// 7.5 M 1.57 and 1.38; with masks cut from the bitset the sides meet at 4 to 4.5 M.  Counting every
+// embedding they meet between 6 and 8 M or lower (Normal 6.1 M: 2.80 and 2.28; LogNormal 6.4 M: 3.34 and
+// 3.50, 8.4 M: 4.58 and 4.35).  Of a bound on the device 8 to 15% survive, and the better side varies with the
+// searches: 20 M (2.2 M pairs) 0.45 and 0.34, 30 M (3.0 M) 0.73 and 0.89, 24 M that all survive 17.7 and 15.5.
 constexpr uint64_t kJoinTwoPassPairs = 3ull << 21;
 constexpr uint64_t kJoinTwoPassBound = 1ull << 24;
 constexpr uint32_t kJoinDeepChunk = 128;            // pairs a wavefront claims at a time of the deep queries' list
@@ -200,7 +203,8 @@ __device__ __forceinline__ uint32_t bit_spread(uint32_t q, uint32_t t) {
 // 1,000 queries 10.7 -> 10.3 ms, 300,000 x 306 2.08 -> 2.01 ms.  Reading one word of each line of a
 // pair's adjacency rows ahead, or all levels' rows in one group, gave nothing.
 //
-// Bound by VALU issue (about two thirds of it on 68 M pairs) at 11 wavefronts per CU by LDS.  One
+// Bound by VALU issue at 11 wavefronts per CU by LDS: on 68 M pairs 54% of the issue slots, 58% of the
+// lanes active, wavefronts waiting 55% of their time, LDS a quarter busy.  One
 // DFS step per iteration, all rows tested per lane and an atomic per listed batch took, for 1 M
 // LogNormal molecules x 1,000 queries, 10.8 + 1.4 ms (molecules of <= 64 nodes) and 2.5 + 1.6 ms
 // (wider ones); this takes 6.5 ms and, with k_join_all's second pass, 3.2, and 33,331 molecules x

@@ -780,7 +780,8 @@ __global__ __launch_bounds__(256) void k_query_levels(GraphDev q, uint32_t R, La
 // requirements are planes of LDS, each a read and an AND for 2,048 nodes, and each word is written
 // once.  In place of the fused filter and R - 1 refine passes: 100,000 molecules x 100 queries 823
 // us, 150,000 LogNormal x 300 6.07 ms; with a scalar per requirement and label compares, bound by
-// issue, 229 us and 1.68 ms; this takes 167 us and 1.24 ms (2.6 GB of words, 2.1 TB/s).
+// issue, 229 us and 1.68 ms; this takes 167 us and 1.08 to 1.24 ms (2.6 GB of words, 2.1 to 2.4 TB/s; VALU
+// 42% and scalar unit 39% of their issue slots, wavefronts waiting 64% of their time).
 __global__ __launch_bounds__(kLevelWaves * 64, 8) void k_filter_levels(const uint32_t* __restrict__ tok, uint64_t Q,
                                                                        const uint64_t* __restrict__ lplanes, const uint4* __restrict__ lvl,
                                                                        uint64_t D, uint32_t R, LabelSlots slots, uint32_t U, uint32_t staged,
@@ -1228,8 +1229,8 @@ hipError_t sig_levels(hipStream_t s, const GraphDev& g, uint32_t R, const LabelS
   return hipGetLastError();
 }
 
-// Labels whose planes the sweep's LDS holds: 52 KB, so that 32 wavefronts stay resident per CU.
-// labels whose planes a byte can name, the frequent one's counts 5..8 included
+// Labels whose planes a byte can name, the frequent one's counts 5..8 included: up to 64 KB of the sweep's
+// LDS, and two 16-wavefront blocks per CU either way (their 32 wavefronts fill it).
 static uint32_t staged_labels(const LabelSlots& slots, uint32_t R) {
   return std::min<uint32_t>(static_cast<uint32_t>(slots.count), 256u / slot_planes(R) - 1);
 }
@@ -1245,8 +1246,8 @@ hipError_t filter_levels(hipStream_t s, const uint32_t* tok, uint64_t Q, const u
   const uint64_t strips = (D + kStripNodes - 1) / kStripNodes;
   if (!Q || !strips) return hipSuccess;
   const uint32_t U = static_cast<uint32_t>(slots.count), staged = staged_labels(slots, R);
-  // row chunks only until the blocks fill the device four times (staging is paid per block), and of at
-  // least two rows per wavefront
+  // row chunks only until there are twelve blocks per CU, six turns of the two that stay resident (staging is
+  // paid per block), and of at least two rows per wavefront
   const uint64_t target = static_cast<uint64_t>(num_cus > 0 ? num_cus : 256) * 12;
   const uint64_t chunks0 = std::max<uint64_t>(1, std::min<uint64_t>((Q + 2 * kLevelWaves - 1) / (2 * kLevelWaves), (target + strips - 1) / strips));
   const uint32_t rpb = static_cast<uint32_t>((Q + chunks0 - 1) / chunks0), chunks = static_cast<uint32_t>((Q + rpb - 1) / rpb);

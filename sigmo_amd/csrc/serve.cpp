@@ -313,7 +313,7 @@ int sigmo_serve(sigmo_batch* const* workers, uint32_t num_workers, const sigmo_h
   sigmo_serve_options opt = *options;
   if (opt.bytes_per_graph == 0 && num_requests) {
     // price a query graph at the batch's mean size, from the workspace estimate of a
-    // 64-graph batch (the per-pair offsets dominate and grow linearly)
+    // 64-graph batch (the arena and the GMCR arrays dominate and grow linearly)
     const uint32_t G = request_graph_offsets[num_requests] - request_graph_offsets[0];
     const uint64_t nodes = queries->graph_offsets[request_graph_offsets[num_requests]] - queries->graph_offsets[request_graph_offsets[0]];
     uint64_t b64 = 0;
